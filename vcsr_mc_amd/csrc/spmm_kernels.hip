@@ -43,6 +43,8 @@ namespace vcsrmc {
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
+// Four floats of C at any float (a ragged O, an unaligned C): one 128-bit access either way.
+typedef floatx4 floatx4_any __attribute__((aligned(4)));
 
 constexpr int kApitch = 40;  // FP16 A tile row pitch in halves (80 B: conflict-free b128 reads)
 // FP32 A tile in LDS: four K groups (k & 3) of 16 rows, each row the 8 values k >> 2 a lane
@@ -61,34 +63,41 @@ struct BRows {
     vec_t r[8];
 };
 
-// Zeros read in place of a B row by padding columns and by lanes past O.  Never written; not
-// `const`, so that it lives in the global address space like B and the loads stay global loads
-// (a constant-space operand would turn them into flat loads, which also count against the LDS
-// wait counter).
+// Zeros read in place of a B row by padding columns.  Never written; not `const`, so that it lives
+// in the global address space like B and the loads stay global loads (a constant-space operand
+// would turn them into flat loads, which also count against the LDS wait counter).
 __device__ __attribute__((aligned(16))) float kZeroRow[16];
 
-// Every load is issued unconditionally (padding columns and lanes past O read kZeroRow): the
-// number of loads in flight is then the same on every path, which lets the compiler wait for
-// exactly the older loads it needs, and no select is needed after a load.
+// The first of the VEC output columns a lane multiplies: c0, or O - VEC where that is lower (O >=
+// VEC: an O tile is never more than twice as wide as O, or 16 wide).  A lane's columns are then
+// always VEC columns of the row, read with one load.  Where O ends inside a lane's columns, the
+// ones it takes below c0 are a neighbour's too: both hold the same sums, and the epilogue writes
+// c0 .. O - 1.  Lanes past O repeat the row's last columns, and nothing they hold is written: read
+// from kZeroRow instead, they cost every load of a B row a second cache line (FP16 power-law
+// 100,000^2, O = 7: 18.8 us with the zeros, 12.7 without; FP32 27-point stencil 60^3, O = 24,
+// C += A.B: 30.4 -> 26.5).
+template <int VEC>
+__device__ __forceinline__ int lane_column(int c0, int O) { return min(c0, O - VEC); }
+
+// Every load is issued unconditionally (padding columns read kZeroRow): the number of loads in
+// flight is then the same on every path, which lets the compiler wait for exactly the older loads
+// it needs, and no select is needed after a load.  Rows of a ragged O, or of an unaligned B, start
+// at any element: the same one load at element alignment (global loads need no more on gfx950).
+// Measured against a load per element: FP16 power-law 100,000^2 with 12 per row, C = A.B, O = 100
+// 142 -> 36 us, 33 45 -> 24, 130 281 -> 65; FP32 the same, O = 130 180 -> 106; FP32 27-point
+// stencil 60^3, C += A.B, O = 100 246 -> 71.
 template <int VEC, typename TB, bool ALIGNED>
 __device__ __forceinline__ void load_b_rows(const TB* __restrict__ B, const int (&cols)[8],
-                                            long long O, int c0, BRows<VEC, TB>& R) {
+                                            long long ld, int c0, BRows<VEC, TB>& R) {
     typedef typename BRows<VEC, TB>::vec_t vec_t;
-    const bool lane_ok = c0 < O;
+    typedef vec_t vec_any __attribute__((aligned(sizeof(TB))));
     const TB* zero = reinterpret_cast<const TB*>(kZeroRow);
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         const int col = cols[i];
-        const bool ok = col >= 0 && lane_ok;
-        const TB* src = ok ? B + (long long)col * O + c0 : zero;
-        if constexpr (ALIGNED && VEC * sizeof(TB) >= 4) {
-            R.r[i] = *reinterpret_cast<const vec_t*>(src);
-        } else {
-            vec_t x;
-#pragma unroll
-            for (int q = 0; q < VEC; ++q) x[q] = (ok && c0 + q < O) ? src[q] : (TB)0;
-            R.r[i] = x;
-        }
+        const TB* src = col >= 0 ? B + (long long)col * ld + c0 : zero;
+        if constexpr (ALIGNED) R.r[i] = *reinterpret_cast<const vec_t*>(src);
+        else R.r[i] = *reinterpret_cast<const vec_any*>(src);
     }
 }
 
@@ -140,18 +149,15 @@ __device__ __forceinline__ PanelRows<MAPPED> panel_rows(const int4& U,
 }
 
 // C of a unit's output tile, read ahead of the merge (C += A.B needs it) so that its latency
-// overlaps the tile loop.  W == 1 (light): just before the wave's last tile is multiplied; for a
-// whole, aligned, unsplit tile (the staged merge below) lane l reads the float4s at l*4 + 256 j of
-// the 16 x TK tile, row-major; otherwise lane (n, g) reads rows 4g..4g+3 at columns
-// k0 + VEC n .. + VEC - 1 (VEC / 4 float4 per row).  W > 1 (heavy): thread t reads the float4 at
-// t*4 + 256 W j of the tile when the unit starts.  The loads are always issued -- rows outside
-// the mask, split panels, unaligned C, columns past O and overwriting launches read kZeroRow
-// instead -- so their number is fixed and a wait for an older load never has to cover them.
+// overlaps the tile loop: thread t of the W waves reads the float4 at t*4 + 256 W j of the 16 x TK
+// tile, row-major, as the merge writes it back -- W == 1 (light) just before the wave's last tile
+// is multiplied, W > 1 (heavy) when the unit starts.  The loads are always issued -- rows outside
+// the mask, split panels, pieces that end past O and overwriting launches read kZeroRow instead
+// -- so their number is fixed and a wait for an older load never has to cover them.
 template <int TK, int W>
 struct CAhead {
-    static constexpr int VEC = TK / 16;
-    static constexpr int N = W == 1 ? TK / 16 : (16 * TK + 256 * W - 1) / (256 * W);
-    floatx4 v[N > 0 ? N : 1];
+    static constexpr int N = (16 * TK + 256 * W - 1) / (256 * W);
+    floatx4 v[N];
 };
 
 // Sixteen bytes of C read ahead: an ordinary load, or (NT) a non-temporal one, which neither L2
@@ -164,56 +170,26 @@ struct CAhead {
 // load whose kind a run-time flag selects into one ordinary load.)
 template <bool NT>
 __device__ __forceinline__ floatx4 load_c4(const float* p) {
-    if constexpr (NT) return __builtin_nontemporal_load(reinterpret_cast<const floatx4*>(p));
-    else return *reinterpret_cast<const floatx4*>(p);
+    if constexpr (NT) return __builtin_nontemporal_load(reinterpret_cast<const floatx4_any*>(p));
+    else return *reinterpret_cast<const floatx4_any*>(p);
 }
 
 template <int TK, int W, bool NT = false, typename PR>
 __device__ __forceinline__ void read_c_ahead(CAhead<TK, W>& ca, const int4& U,
-                                             const PR& pr, int k0, int O, bool c4,
-                                             bool accumulate, const float* __restrict__ C) {
-    constexpr int VEC = TK / 16;
-    constexpr int N = CAhead<TK, W>::N;
-    const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
+                                             const PR& pr, int k0, int O, bool accumulate,
+                                             const float* __restrict__ C) {
+    const int t = W == 1 ? (threadIdx.x & 63) : threadIdx.x;
     // Overwrite launches (C = A.B) read zeros instead of C; split panels merge through atomics.
-    const bool ok = c4 && accumulate && !(U.w & kUnitSplit);
+    const bool ok = accumulate && !(U.w & kUnitSplit);
     const long long OL = O;
-    if constexpr (W == 1) {
-        if (c4 && !(U.w & kUnitSplit) && k0 + TK <= O) {
-            // staged merge: lane-contiguous 16-byte pieces, as merge_into_c writes them back
 #pragma unroll
-            for (int j = 0; j < N; ++j) {
-                const int e = lane * 4 + 256 * j;
-                const int row = e / TK, col = e % TK;
-                const long long cr = pr.row(row);
-                const bool in = accumulate && ((U.w >> row) & 1);
-                const float* src = in ? C + cr * OL + k0 + col : kZeroRow;
-                ca.v[j] = load_c4<NT>(src);
-            }
-        } else if constexpr (VEC >= 4) {
-            const int c0 = k0 + VEC * n;
-            const bool lane_ok = ok && c0 + VEC <= O;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int rl = 4 * g + i;
-                const long long cr = pr.row(rl);
-                const bool in = lane_ok && ((U.w >> rl) & 1);
-                const float* src = in ? C + cr * OL + c0 : kZeroRow;
-#pragma unroll
-                for (int h = 0; h < VEC / 4; ++h)
-                    ca.v[i * (VEC / 4) + h] = load_c4<NT>(src + 4 * h);
-            }
-        }
-    } else {
-#pragma unroll
-        for (int j = 0; j < N; ++j) {
-            const int e = threadIdx.x * 4 + j * 256 * W;
-            const int row = (e / TK) & 15, cc = k0 + e % TK;
-            const long long cr = pr.row(row);
-            const bool in = ok && e < 16 * TK && ((U.w >> row) & 1) && cc + 4 <= O;
-            const float* src = in ? C + cr * OL + cc : kZeroRow;
-            ca.v[j] = load_c4<NT>(src);
-        }
+    for (int j = 0; j < CAhead<TK, W>::N; ++j) {
+        const int e = t * 4 + j * 256 * W;
+        const int row = (e / TK) & 15, cc = k0 + e % TK;
+        const long long cr = pr.row(row);
+        const bool in = ok && e < 16 * TK && ((U.w >> row) & 1) && cc + 4 <= O;
+        const float* src = in ? C + cr * OL + cc : kZeroRow;
+        ca.v[j] = load_c4<NT>(src);
     }
 }
 
@@ -224,8 +200,8 @@ __device__ __forceinline__ void read_c_ahead(CAhead<TK, W>& ca, const int4& U,
 // stores into one ordinary store.)
 template <bool ACC>
 __device__ __forceinline__ void store_c4(float* p, const floatx4& v) {
-    if constexpr (ACC) *reinterpret_cast<floatx4*>(p) = v;
-    else __builtin_nontemporal_store(v, reinterpret_cast<floatx4*>(p));
+    if constexpr (ACC) *reinterpret_cast<floatx4_any*>(p) = v;
+    else __builtin_nontemporal_store(v, reinterpret_cast<floatx4_any*>(p));
 }
 
 // Parks a wave's 16 x TK tile row-major in P (row pitch TK floats): lane (n, g) holds rows
@@ -237,10 +213,22 @@ __device__ __forceinline__ void store_c4(float* p, const floatx4& v) {
 // lanes n and n + 4 on the same four banks.  Lanes with n & 4 therefore write their two pieces
 // in the other order, and each 8-lane pass covers all 32 banks once; the layout, and so the
 // contiguous reads of the merge, are unchanged.  (At VEC = 4 a pass is already conflict-free.)
-template <int TK>
+// A lane whose columns were moved left to end at O (lane_column) writes the ones it owns singly.
+template <int TK, bool ALIGNED>
 __device__ __forceinline__ void park_tile(float* Pw, const floatx4 (&acc)[TK / 16], float scale,
-                                          int n, int g) {
+                                          int n, int g, int k0, int O) {
     constexpr int VEC = TK / 16;
+    if constexpr (!ALIGNED) {
+        const int c0 = k0 + VEC * n, moved = c0 - lane_column<VEC>(c0, O);
+        if (moved > 0) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int q = 0; q < VEC; ++q)
+                    if (q >= moved) Pw[(4 * g + i) * TK + VEC * n + q - moved] = acc[q][i] * scale;
+            return;
+        }
+    }
     if constexpr (VEC == 8) {
         const bool sw = (n & 4) != 0;
 #pragma unroll
@@ -259,102 +247,60 @@ __device__ __forceinline__ void park_tile(float* Pw, const floatx4 (&acc)[TK / 1
     }
 }
 
-// Adds the unit's 16 x TK result into C (ACC) or writes it (overwrite).  W == 1, staged merge
-// (a whole, aligned tile of an unsplit panel): the wave parks its tile in its slice of P (lane
-// (n, g) owns rows 4g..4g+3, columns k0 + VEC n .. + VEC - 1), reads it back with consecutive
-// lanes on consecutive 16-byte pieces, adds the C read ahead in that order, and stores each run of
-// 1 KB non-temporally.  From the accumulators, one store instruction covered every other 16
-// bytes of a row at O tiles of 128, which non-temporal stores turned into 1.5x the C bytes.
+// Adds the unit's 16 x TK result into C (ACC) or writes it (overwrite).  W == 1 (light): the wave
+// parks its tile in its slice of P, reads it back with consecutive lanes on consecutive 16-byte
+// pieces, adds the C read ahead in that order, and stores runs of up to 1 KB, non-temporally where
+// the rows of C keep every store instruction on whole lines (ALIGNED).  From the accumulators, one
+// store instruction covered every other 16 bytes of a row at O tiles of 128, which non-temporal
+// stores turned into 1.5x the C bytes.
 // Measured on gfx950 against the register epilogue with ordinary stores: overwrite power-law
 // 36,692^2 14.4 -> 12.8 us, 32 x 32 blocks 174 -> 140 us, 27-point stencil 543 -> 508 us, R-MAT
 // scale 22 2.46 -> 2.38 ms; accumulate blocks 189 -> 178 us, stencil 584 -> 565 us, the others
-// within 1%.  Other W == 1 tiles: straight from the accumulators.  W > 1: every wave parks its
+// within 1%.  W > 1: every wave parks its
 // partial tile in LDS, then the work-group sums the W partials and writes each row with
-// consecutive threads on consecutive columns.  Split panels merge through atomics; other rows
-// are a read-modify-write (C += A.B) whose read came from read_c_ahead.  Rows outside the
-// panel's row mask are never touched.
-template <int TK, int W, bool ACC, typename PR>
+// consecutive threads on consecutive columns.  Split panels (heavy units only) merge through
+// atomics; other rows are a read-modify-write (C += A.B) whose read came from read_c_ahead; the
+// last piece of a row of a ragged O goes element by element.  Rows outside the panel's row mask
+// are never touched.
+template <int TK, int W, bool ALIGNED, bool ACC, typename PR>
 __device__ __forceinline__ void merge_into_c(const floatx4 (&acc)[TK / 16], float scale,
                                              const int4& U, const PR& pr, int k0, int O,
-                                             bool c4, float* __restrict__ C, float* P,
+                                             float* __restrict__ C, float* P,
                                              const CAhead<TK, W>& ca) {
-    constexpr int VEC = TK / 16;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = lane & 15, g = lane >> 4;
-    const bool split = U.w & kUnitSplit;
+    const int t = W == 1 ? lane : threadIdx.x;
+    const bool split = W > 1 && (U.w & kUnitSplit);
     const long long OL = O;
-    if constexpr (W == 1) {
-        if (!split && c4 && k0 + TK <= O) {  // staged merge
-            park_tile<TK>(P + wave * 16 * TK, acc, scale, n, g);
-            wave_lds_sync();
-            const float* Pw = P + wave * 16 * TK;
+    float* const mine = P + wave * 16 * TK;
+    park_tile<TK, ALIGNED>(mine, acc, W == 1 ? scale : 1.0f, n, g, k0, O);
+    if constexpr (W == 1) wave_lds_sync();
+    else __syncthreads();
+    const float* const first = W == 1 ? mine : P;
 #pragma unroll
-            for (int j = 0; j < 16 * TK / 256; ++j) {
-                const int e = lane * 4 + 256 * j;
-                const int row = e / TK, col = e % TK;
-                const long long cr = pr.row(row);
-                floatx4 v = *reinterpret_cast<const floatx4*>(Pw + e);
-                if constexpr (ACC) v += ca.v[j];
-                if ((U.w >> row) & 1) store_c4<false>(C + cr * OL + k0 + col, v);
-            }
-            return;
+    for (int j = 0; j < CAhead<TK, W>::N; ++j) {
+        const int e = t * 4 + j * 256 * W;
+        if (W > 1 && e >= 16 * TK) break;
+        const int row = e / TK, cc = k0 + e % TK;
+        const long long cr = pr.row(row);
+        if (!((U.w >> row) & 1) || cc >= O) continue;
+        floatx4 v = *reinterpret_cast<const floatx4*>(first + e);
+        if constexpr (W > 1) {
+#pragma unroll
+            for (int w = 1; w < W; ++w) v += *reinterpret_cast<const floatx4*>(P + w * 16 * TK + e);
+            v *= scale;
         }
-        const int c0 = k0 + VEC * n;
+        float* crow = C + cr * OL + cc;
+        if (split) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int rl = 4 * g + i;
-            const long long cr = pr.row(rl);
-            if (!((U.w >> rl) & 1)) continue;
-            float* crow = C + cr * OL + c0;
-            if (split) {
+            for (int q = 0; q < 4; ++q)
+                if (cc + q < O) atomicAdd(crow + q, v[q]);
+        } else if (cc + 4 <= O) {
+            if constexpr (ACC) v += ca.v[j];
+            store_c4<(W > 1 && ACC) || !ALIGNED>(crow, v);
+        } else {
 #pragma unroll
-                for (int q = 0; q < VEC; ++q)
-                    if (c0 + q < O) atomicAdd(crow + q, acc[q][i] * scale);
-            } else if (VEC >= 4 && c4 && c0 + VEC <= O) {
-#pragma unroll
-                for (int h = 0; h < VEC; h += 4) {
-                    floatx4 v = ca.v[(i * (VEC / 4) + h / 4) % CAhead<TK, W>::N];
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) v[q] += acc[(h + q) % VEC][i] * scale;
-                    store_c4<ACC>(crow + h, v);
-                }
-            } else {
-#pragma unroll
-                for (int q = 0; q < VEC; ++q)
-                    if (c0 + q < O) crow[q] = (ACC ? crow[q] : 0.0f) + acc[q][i] * scale;
-            }
-        }
-    } else {
-        park_tile<TK>(P + wave * 16 * TK, acc, 1.0f, n, g);
-        __syncthreads();
-#pragma unroll
-        for (int j = 0; j < CAhead<TK, W>::N; ++j) {
-            const int e = threadIdx.x * 4 + j * 256 * W;
-            if (e >= 16 * TK) break;
-            const int row = e / TK, col = e % TK;
-            const long long cr = pr.row(row);
-            if (!((U.w >> row) & 1)) continue;
-            floatx4 sum = *reinterpret_cast<const floatx4*>(P + e);
-#pragma unroll
-            for (int w = 1; w < W; ++w) {
-                const floatx4 x = *reinterpret_cast<const floatx4*>(P + w * 16 * TK + e);
-                sum += x;
-            }
-            const int cc = k0 + col;
-            if (cc >= O) continue;
-            float* crow = C + cr * OL + cc;
-            if (split) {
-#pragma unroll
-                for (int jj = 0; jj < 4; ++jj)
-                    if (cc + jj < O) atomicAdd(crow + jj, sum[jj] * scale);
-            } else if (c4 && cc + 4 <= O) {
-                floatx4 v = ca.v[j];
-                v += sum * scale;
-                store_c4<ACC>(crow, v);
-            } else {
-#pragma unroll
-                for (int jj = 0; jj < 4; ++jj)
-                    if (cc + jj < O) crow[jj] = (ACC ? crow[jj] : 0.0f) + sum[jj] * scale;
-            }
+            for (int q = 0; q < 4; ++q)
+                if (cc + q < O) crow[q] = (ACC ? crow[q] : 0.0f) + v[q];
         }
     }
 }
@@ -459,7 +405,8 @@ __device__ __forceinline__ void mma_tile_f16(const TileMeta& m, const uint4& st,
 //   * every iteration issues the same loads (column indices past the last tile are clamped).
 template <int TK, typename TB, bool ALIGNED, typename Pre>
 __device__ __forceinline__ void tiles_f16(int first, int end, int W, int lane, int n, int g,
-                                          int c0, long long OL, const int* __restrict__ chunk_eptr,
+                                          int c0, long long OL,
+                                          const int* __restrict__ chunk_eptr,
                                           const int* __restrict__ chunk_cols,
                                           const int* __restrict__ chunk_dense,
                                           const uint32_t* __restrict__ entries,
@@ -515,19 +462,18 @@ __device__ __forceinline__ void tiles_f16(int first, int end, int W, int lane, i
     }
 }
 
-// Register budget: FP16 B with aligned rows fits three waves per SIMD without spilling; the
-// FP32-B and unaligned variants hold more B data and are given two (at O tiles of 64 or less
-// they still fit three: 139 VGPRs for FP32 B).
-template <typename TB, bool ALIGNED>
-constexpr int f16_min_waves() { return (sizeof(TB) == 2 && ALIGNED) ? 3 : 2; }
+// Register budget: FP16 B fits three waves per SIMD without spilling; the FP32-B variants hold
+// more B data and are given two (at O tiles of 64 or less they still fit three: 139 VGPRs).
+template <typename TB>
+constexpr int f16_min_waves() { return sizeof(TB) == 2 ? 3 : 2; }
 
 template <int TK, typename TB, bool ALIGNED, bool ACC, bool MAPPED, bool NTC>
-__global__ __launch_bounds__(64 * kWaves, (f16_min_waves<TB, ALIGNED>())) void k_spmm_f16(
+__global__ __launch_bounds__(64 * kWaves, (f16_min_waves<TB>())) void k_spmm_f16(
     const int4* __restrict__ units, const int* __restrict__ rmap, int num_heavy, XcdSplit xs,
     const int* __restrict__ chunk_eptr, const int* __restrict__ chunk_cols,
     const int* __restrict__ chunk_dense, const uint32_t* __restrict__ entries,
     const _Float16* __restrict__ dense_a, const TB* __restrict__ B, int O, int tiled_n,
-    float scale, bool c4, float* __restrict__ C) {
+    float scale, float* __restrict__ C) {
     constexpr int VEC = TK / 16;
     __shared__ __attribute__((aligned(16))) _Float16 As[kWaves][16 * kApitch];
     __shared__ __attribute__((aligned(16))) float P[kWaves * 16 * TK];
@@ -548,7 +494,7 @@ __global__ __launch_bounds__(64 * kWaves, (f16_min_waves<TB, ALIGNED>())) void k
     // memory instead of every other half of the 256-byte rows).
     const TB* Bt = tiled_n > 0 ? B + (long long)(k0 / TK) * tiled_n * TK : B;
     const long long ldb = tiled_n > 0 ? TK : O;
-    const int cb = tiled_n > 0 ? VEC * n : c0;
+    const int cb = tiled_n > 0 ? VEC * n : lane_column<VEC>(c0, O);
     floatx4 acc[VEC];
 #pragma unroll
     for (int q = 0; q < VEC; ++q) acc[q] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -556,17 +502,17 @@ __global__ __launch_bounds__(64 * kWaves, (f16_min_waves<TB, ALIGNED>())) void k
     // counting sees one fixed sequence of loads on each.
     if (heavy) {
         CAhead<TK, kWaves> ca;
-        read_c_ahead<TK, kWaves, NTC>(ca, U, pr, k0, O, c4, ACC, C);
+        read_c_ahead<TK, kWaves, NTC>(ca, U, pr, k0, O, ACC, C);
         tiles_f16<TK, TB, ALIGNED>(U.y + wave, U.z, kWaves, lane, n, g, cb, ldb,
                                    chunk_eptr, chunk_cols, chunk_dense, entries, dense_a, Bt,
                                    As[wave], acc, [] {});
-        merge_into_c<TK, kWaves, ACC>(acc, scale, U, pr, k0, O, c4, C, P, ca);
+        merge_into_c<TK, kWaves, ALIGNED, ACC>(acc, scale, U, pr, k0, O, C, P, ca);
     } else {
         CAhead<TK, 1> ca;
         tiles_f16<TK, TB, ALIGNED>(U.y, U.z, 1, lane, n, g, cb, ldb, chunk_eptr,
                                    chunk_cols, chunk_dense, entries, dense_a, Bt, As[wave], acc,
-                                   [&] { read_c_ahead<TK, 1, NTC>(ca, U, pr, k0, O, c4, ACC, C); });
-        merge_into_c<TK, 1, ACC>(acc, scale, U, pr, k0, O, c4, C, P, ca);
+                                   [&] { read_c_ahead<TK, 1, NTC>(ca, U, pr, k0, O, ACC, C); });
+        merge_into_c<TK, 1, ALIGNED, ACC>(acc, scale, U, pr, k0, O, C, P, ca);
     }
 }
 
@@ -582,25 +528,18 @@ struct FRows {
 
 // Half a tile of B rows (K steps s0 .. s0 + 3 of the lane's column group): row s holds the VEC
 // output columns c0 .. c0 + VEC - 1 of B row cols[s0 + s].  Loads are unconditional like
-// load_b_rows (padding and lanes past O read kZeroRow).
+// load_b_rows (padding reads kZeroRow).
 template <int VEC, bool ALIGNED>
 __device__ __forceinline__ void load_b_half_f32(const float* __restrict__ B, const int (&cols)[8],
-                                                int s0, long long O, int c0, FRows<VEC>& R) {
+                                                int s0, long long ld, int c0, FRows<VEC>& R) {
     typedef typename FRows<VEC>::vec_t vec_t;
-    const bool lane_ok = c0 < O;
+    typedef vec_t vec_any __attribute__((aligned(4)));
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
         const int col = cols[s0 + s];
-        const bool ok = col >= 0 && lane_ok;
-        const float* src = ok ? B + (long long)col * O + c0 : kZeroRow;
-        if constexpr (ALIGNED) {
-            R.r[s] = *reinterpret_cast<const vec_t*>(src);
-        } else {
-            vec_t x;
-#pragma unroll
-            for (int q = 0; q < VEC; ++q) x[q] = (ok && c0 + q < O) ? src[q] : 0.0f;
-            R.r[s] = x;
-        }
+        const float* src = col >= 0 ? B + (long long)col * ld + c0 : kZeroRow;
+        if constexpr (ALIGNED) R.r[s] = *reinterpret_cast<const vec_t*>(src);
+        else R.r[s] = *reinterpret_cast<const vec_any*>(src);
     }
 }
 
@@ -726,7 +665,8 @@ __device__ __forceinline__ void a_operand_f32(const TileMeta& m, const AState32&
 // the same loads of columns and B rows and mfma_half_rs as the product.
 template <int TK, bool ALIGNED, bool RS, typename Pre>
 __device__ __forceinline__ void tiles_f32(int first, int end, int W, int lane, int n, int g,
-                                          int c0, long long OL, const int* __restrict__ chunk_eptr,
+                                          int c0, long long OL,
+                                          const int* __restrict__ chunk_eptr,
                                           const int* __restrict__ chunk_cols,
                                           const int* __restrict__ chunk_dense,
                                           const uint32_t* __restrict__ entries,
@@ -828,7 +768,7 @@ __global__ __launch_bounds__(64 * kWaves, 3) void k_spmm_f32(
     const int* __restrict__ chunk_eptr, const int* __restrict__ chunk_cols,
     const int* __restrict__ chunk_dense, const uint32_t* __restrict__ entries,
     const float* __restrict__ dense_a, const int* __restrict__ rs_cols,
-    const float* __restrict__ rs_vals, const float* __restrict__ B, int O, bool c4,
+    const float* __restrict__ rs_vals, const float* __restrict__ B, int O,
     float* __restrict__ C) {
     constexpr int VEC = TK / 16;
     __shared__ __attribute__((aligned(16))) float At[kWaves][4 * kAgroup32];
@@ -841,7 +781,7 @@ __global__ __launch_bounds__(64 * kWaves, 3) void k_spmm_f32(
     const int4 U = units[u];
     const PanelRows<MAPPED> pr = panel_rows<MAPPED>(U, rmap);
     const int k0 = ((blockIdx.y << (3 - xs.lgp)) + ot) * TK;
-    const int c0 = k0 + VEC * n;
+    const int c0 = lane_column<VEC>(k0 + VEC * n, O);
     floatx4 acc[VEC];
 #pragma unroll
     for (int q = 0; q < VEC; ++q) acc[q] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -859,19 +799,19 @@ __global__ __launch_bounds__(64 * kWaves, 3) void k_spmm_f32(
                 return;
             }
         }
-        tiles_f32<TK, ALIGNED, false>(first, U.z, W, lane, n, g, c0, (long long)O, chunk_eptr,
-                                      chunk_cols, chunk_dense, entries, dense_a, B, At[wave], acc,
-                                      pre);
+        tiles_f32<TK, ALIGNED, false>(first, U.z, W, lane, n, g, c0, (long long)O,
+                                      chunk_eptr, chunk_cols, chunk_dense, entries, dense_a, B,
+                                      At[wave], acc, pre);
     };
     if (heavy) {
         CAhead<TK, kWaves> ca;
-        read_c_ahead<TK, kWaves, NTC>(ca, U, pr, k0, O, c4, ACC, C);
+        read_c_ahead<TK, kWaves, NTC>(ca, U, pr, k0, O, ACC, C);
         run(U.y + wave, kWaves, [] {});
-        merge_into_c<TK, kWaves, ACC>(acc, 1.0f, U, pr, k0, O, c4, C, P, ca);
+        merge_into_c<TK, kWaves, ALIGNED, ACC>(acc, 1.0f, U, pr, k0, O, C, P, ca);
     } else {
         CAhead<TK, 1> ca;
-        run(U.y, 1, [&] { read_c_ahead<TK, 1, NTC>(ca, U, pr, k0, O, c4, ACC, C); });
-        merge_into_c<TK, 1, ACC>(acc, 1.0f, U, pr, k0, O, c4, C, P, ca);
+        run(U.y, 1, [&] { read_c_ahead<TK, 1, NTC>(ca, U, pr, k0, O, ACC, C); });
+        merge_into_c<TK, 1, ALIGNED, ACC>(acc, 1.0f, U, pr, k0, O, C, P, ca);
     }
 }
 
@@ -881,9 +821,10 @@ template <int TK, bool ACC, bool MAPPED, bool NTC>
 static void launch_tk_mode(const DeviceFormat& F, const void* dB, bool b_f16, bool b_tiled, int O,
                            float* dC, hipStream_t st) {
     constexpr int VEC = TK / 16;
-    // Vector loads of B need O % VEC == 0 and a 16-byte aligned base.
-    const bool aligned = (O % VEC) == 0 && ((uintptr_t)dB % 16) == 0;
-    const bool c4 = (O % 4) == 0 && ((uintptr_t)dC % 16) == 0;
+    // Rows of B and C on their vectors' natural boundaries; other launches take the variants with
+    // element-aligned loads, lane_column's shift and ordinary stores of C.
+    const bool aligned = (O % VEC) == 0 && (O % 4) == 0 && ((uintptr_t)dB % 16) == 0 &&
+                         ((uintptr_t)dC % 16) == 0;
     // O tiles: G = the largest power of two <= 8 dividing their count go to separate XCD
     // groups; the rest are launch rows (blockIdx.y).
     const int otiles = (O + TK - 1) / TK;
@@ -914,36 +855,34 @@ static void launch_tk_mode(const DeviceFormat& F, const void* dB, bool b_f16, bo
         const float* rsv = F.rs_vals.p;
         if (aligned)
             hipLaunchKernelGGL((k_spmm_f32<TK, true, ACC, MAPPED, NTC>), grid, block, 0, st, U, rmap,
-                               NH, xs, eptr, cols, dense, ent, F.dense_a32.p, rsc, rsv, B, O, c4,
-                               dC);
+                               NH, xs, eptr, cols, dense, ent, F.dense_a32.p, rsc, rsv, B, O, dC);
         else
             hipLaunchKernelGGL((k_spmm_f32<TK, false, ACC, MAPPED, false>), grid, block, 0, st, U, rmap,
-                               NH, xs, eptr, cols, dense, ent, F.dense_a32.p, rsc, rsv, B, O, c4,
-                               dC);
+                               NH, xs, eptr, cols, dense, ent, F.dense_a32.p, rsc, rsv, B, O, dC);
     } else if (b_f16) {
         const _Float16* B = static_cast<const _Float16*>(dB);
         // O-tile-major B (written by the conversion pass) only with every O tile full
-        if (b_tiled && (O % TK != 0 || !aligned))
-            throw Error(VCSRMC_ERR_STATE, "O-tile-major B needs full, aligned O tiles");
+        if (b_tiled && O % TK != 0)
+            throw Error(VCSRMC_ERR_STATE, "O-tile-major B needs full O tiles");
         const int tiled_n = b_tiled ? F.N : 0;
         if (aligned)
             hipLaunchKernelGGL((k_spmm_f16<TK, _Float16, true, ACC, MAPPED, NTC>), grid, block, 0, st,
                                U, rmap, NH, xs, eptr, cols, dense, ent, F.dense_a16.p, B, O,
-                               tiled_n, F.scale, c4, dC);
+                               tiled_n, F.scale, dC);
         else
             hipLaunchKernelGGL((k_spmm_f16<TK, _Float16, false, ACC, MAPPED, false>), grid, block, 0, st,
-                               U, rmap, NH, xs, eptr, cols, dense, ent, F.dense_a16.p, B, O, 0,
-                               F.scale, c4, dC);
+                               U, rmap, NH, xs, eptr, cols, dense, ent, F.dense_a16.p, B, O,
+                               tiled_n, F.scale, dC);
     } else if constexpr (TK <= 64) {
         const float* B = static_cast<const float*>(dB);
         if (aligned)
             hipLaunchKernelGGL((k_spmm_f16<TK, float, true, ACC, MAPPED, NTC>), grid, block, 0, st, U,
                                rmap, NH, xs, eptr, cols, dense, ent, F.dense_a16.p, B, O, 0,
-                               F.scale, c4, dC);
+                               F.scale, dC);
         else
             hipLaunchKernelGGL((k_spmm_f16<TK, float, false, ACC, MAPPED, false>), grid, block, 0, st, U,
                                rmap, NH, xs, eptr, cols, dense, ent, F.dense_a16.p, B, O, 0,
-                               F.scale, c4, dC);
+                               F.scale, dC);
     } else {
         // o_tile_width never gives an FP16 format reading FP32 B an O tile of 128.
         throw Error(VCSRMC_ERR_STATE, "no O tile of 128 for FP32 B with an FP16 format");
