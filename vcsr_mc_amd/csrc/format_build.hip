@@ -55,7 +55,8 @@ __global__ __launch_bounds__(256) void k_absmax_bits(const float* __restrict__ v
 }
 
 float device_absmax(const float* d_val, long long n, hipStream_t st) {
-    DevBuf<unsigned> bits(1);
+    ScratchScope scratch(0);
+    TmpBuf<unsigned> bits(1);
     VCSRMC_HIP(hipMemsetAsync(bits.p, 0, sizeof(unsigned), st));
     if (n > 0) {
         const unsigned grid = (unsigned)std::min<long long>(grid_for(n, 256), 4096);
@@ -646,14 +647,14 @@ static void build_exec_layout_k(DeviceFormat& F, const int* trow, const int* tco
     const int pbits = bits_for(num_panels_all > 0 ? (unsigned long long)(num_panels_all - 1) : 0ull);
     const int kbits = pbits + cbits + 4;
 
-    DevBuf<K> k1(n), k2(n);
-    DevBuf<uint32_t> v1(n), v2(n);
+    TmpBuf<K> k1(n), k2(n);
+    TmpBuf<uint32_t> v1(n), v2(n);
     LAUNCH((k_panel_keys<K>), n, trow, tcol, rowpos, n, cbits, k1.p, v1.p);
     K* kp = k1.p; K* ka = k2.p;
     uint32_t* vp = v1.p; uint32_t* va = v2.p;
     radix_sort_pairs<K>(kp, vp, ka, va, n, kbits, st);
 
-    DevBuf<int> hdist(n), hpanel(n), dc(n), pin(n), err(1);
+    TmpBuf<int> hdist(n), hpanel(n), dc(n), pin(n), err(1);
     VCSRMC_HIP(hipMemsetAsync(err.p, 0, sizeof(int), st));
     LAUNCH((k_panel_heads<K>), n, kp, n, cbits, hdist.p, hpanel.p, err.p);
     inclusive_sum<int, int>(hdist.p, dc.p, n, st);
@@ -662,14 +663,14 @@ static void build_exec_layout_k(DeviceFormat& F, const int* trow, const int* tco
     const int NP = read_scalar(pin.p + (n - 1), st);
     F.num_pairs = read_scalar(dc.p + (n - 1), st);
 
-    DevBuf<int> pstart(NP + 1), ppanel(NP), nch(NP), cbase(NP + 1), pmask(NP);
+    TmpBuf<int> pstart(NP + 1), ppanel(NP), nch(NP), cbase(NP + 1), pmask(NP);
     LAUNCH((k_panel_starts<K>), n, kp, hpanel.p, pin.p, n, cbits, pstart.p, ppanel.p);
     fill<int>(pstart.p + NP, 1, (int)n, st);
     LAUNCH(k_panel_chunks, NP, pstart.p, dc.p, NP, nch.p);
     exclusive_sum<int, int>(nch.p, cbase.p, NP, st);
     const int NC = read_scalar(cbase.p + NP, st);
     {
-        DevBuf<int> nmax(NP);
+        TmpBuf<int> nmax(NP);
         inclusive_max(nch.p, nmax.p, NP, st);
         F.max_panel_tiles = read_scalar(nmax.p + (NP - 1), st);
     }
@@ -680,12 +681,12 @@ static void build_exec_layout_k(DeviceFormat& F, const int* trow, const int* tco
     fill<int>(F.chunk_cols.p, (long long)NC * kChunkCols, -1, st);
     fill<int>(F.chunk_eptr.p + NC, 1, (int)n, st);
     {
-        DevBuf<unsigned char> rflag((size_t)num_panels_all * kPanelRows);
+        TmpBuf<unsigned char> rflag((size_t)num_panels_all * kPanelRows);
         fill<unsigned char>(rflag.p, (long long)num_panels_all * kPanelRows, 0, st);
         LAUNCH(k_row_flags, n, trow, rowpos, n, rflag.p);
         LAUNCH(k_panel_masks, NP, rflag.p, ppanel.p, NP, pmask.p);
     }
-    DevBuf<int> echunk(n);
+    TmpBuf<int> echunk(n);
     if (F.fp32)
         LAUNCH((k_panel_entries<K, true>), n, kp, vp, hdist.p, dc.p, pin.p, pstart.p, cbase.p, tcol,
                tval, n, F.entries.p, F.chunk_cols.p, F.chunk_eptr.p, echunk.p);
@@ -695,7 +696,7 @@ static void build_exec_layout_k(DeviceFormat& F, const int* trow, const int* tco
 
     // dense copies of well-filled tiles
     {
-        DevBuf<int> dflag(NC), didx(NC + 1);
+        TmpBuf<int> dflag(NC), didx(NC + 1);
         LAUNCH(k_dense_flags, NC, F.chunk_eptr.p, NC, dense_min(F.fp32, NP, NC), dflag.p);
         exclusive_sum<int, int>(dflag.p, didx.p, NC, st);
         const int ND = read_scalar(didx.p + NC, st);
@@ -718,15 +719,15 @@ static void build_exec_layout_k(DeviceFormat& F, const int* trow, const int* tco
     }
 
     // row steps of FP32 panels whose rows rarely share a column; their units count batches
-    DevBuf<int> nbat, rbase;
+    TmpBuf<int> nbat, rbase;
     int NB = 0;
     // (in the default mode only in formats whose launches take O tiles of 64 anyway: the
     // multiply kernel carries the row-step path only at that width)
     int rs_mode = F.fp32 ? fp32_row_steps() : 0;
     if (rs_mode == 1 && !fp32_narrow_o_tiles(n, NC, NP)) rs_mode = 0;
     if (rs_mode != 0) {
-        DevBuf<uint32_t> rsmask((size_t)NC * 4);
-        DevBuf<int> rscnt((size_t)NC * 4), rspre(((size_t)NC + 1) * 4);
+        TmpBuf<uint32_t> rsmask((size_t)NC * 4);
+        TmpBuf<int> rscnt((size_t)NC * 4), rspre(((size_t)NC + 1) * 4);
         nbat.alloc(NP);
         rbase.alloc(NP + 1);
         LAUNCH(k_row_step_masks, NC, F.chunk_eptr.p, F.entries.p, NC, rsmask.p, rscnt.p);
@@ -752,7 +753,7 @@ static void build_exec_layout_k(DeviceFormat& F, const int* trow, const int* tco
 
     const int light_max = light_tile_limit(NP);
     const int heavy_tiles = heavy_tile_limit(NC);
-    DevBuf<int> nu(NP), ubase(NP + 1), nheavy(NP), hbase(NP + 1), nsplit(NP), sbase(NP + 1);
+    TmpBuf<int> nu(NP), ubase(NP + 1), nheavy(NP), hbase(NP + 1), nsplit(NP), sbase(NP + 1);
     LAUNCH(k_units_per_panel, NP, nch.p, NP, light_max, heavy_tiles, nu.p, nheavy.p, nsplit.p);
     exclusive_sum<int, int>(nu.p, ubase.p, NP, st);
     exclusive_sum<int, int>(nheavy.p, hbase.p, NP, st);
@@ -761,8 +762,8 @@ static void build_exec_layout_k(DeviceFormat& F, const int* trow, const int* tco
     const int NH = read_scalar(hbase.p + NP, st);
     const int NS = read_scalar(sbase.p + NP, st);
     {
-        DevBuf<int4> raw(NU);
-        DevBuf<uint32_t> k1(NU), k2(NU), v1(NU), v2(NU);
+        TmpBuf<int4> raw(NU);
+        TmpBuf<uint32_t> k1(NU), k2(NU), v1(NU), v2(NU);
         const bool by_column = light_by_column(n, F.num_pairs);
         LAUNCH(k_make_units, NP, cbase.p, NB > 0 ? rbase.p : nullptr,
                NB > 0 ? nbat.p : nullptr, ubase.p, ppanel.p, pmask.p, nch.p, NP, light_max,
@@ -775,8 +776,8 @@ static void build_exec_layout_k(DeviceFormat& F, const int* trow, const int* tco
     // Light units are split into eight contiguous ranges of about equal tile count, one per XCD.
     {
         const int NL = NU - NH;
-        DevBuf<int> nt(NL > 0 ? NL : 1), cut(9);
-        DevBuf<long long> csum((size_t)NL + 1);
+        TmpBuf<int> nt(NL > 0 ? NL : 1), cut(9);
+        TmpBuf<long long> csum((size_t)NL + 1);
         LAUNCH(k_light_tiles, NL, F.units.p, NH, NL, nt.p);
         exclusive_sum<int, long long>(nt.p, csum.p, NL, st);
         hipLaunchKernelGGL(k_xcd_cuts, dim3(1), dim3(64), 0, st, csum.p, NL, cut.p);
@@ -864,7 +865,8 @@ static void build_exec_layout(DeviceFormat& F, const int* trow, const int* tcol,
                               long long n, hipStream_t st) {
     F.row_map.release();
     const int mode = row_grouping();
-    DevBuf<int> cpos, cmap;
+    TmpBuf<int> cpos;
+    DevBuf<int> cmap;
     const bool compact = mode != 0 && compact_rows(trow, n, F.M, st, cpos, cmap);
     build_layout_in_order(F, trow, tcol, tval, compact ? cpos.p : nullptr, n, st);
     if (compact) F.row_map = std::move(cmap);
@@ -882,7 +884,8 @@ static void build_exec_layout(DeviceFormat& F, const int* trow, const int* tcol,
         }
         if (64.0 * (double)n + 64.0 * (double)F.M > 0.5 * (double)free_b) return;
     }
-    DevBuf<int> rowpos, row_map;
+    TmpBuf<int> rowpos;
+    DevBuf<int> row_map;
     if (!group_rows(trow, tcol, n, F.M, F.N, st, rowpos, row_map)) return;
     DeviceFormat G;
     G.M = F.M;
@@ -904,9 +907,9 @@ static void build_groups_k(DeviceFormat& F, const int* d_col, const float* d_val
                            hipStream_t st) {
     const int segw = F.segw;
     const int kbits = 6 + bits_for((unsigned long long)(S > 0 ? S - 1 : 0));
-    DevBuf<K> k1(P), k2(P);
-    DevBuf<uint32_t> v1(P), v2(P);
-    DevBuf<int> seg_start(S + 1), gnum(S), gbase(S + 1);
+    TmpBuf<K> k1(P), k2(P);
+    TmpBuf<uint32_t> v1(P), v2(P);
+    TmpBuf<int> seg_start(S + 1), gnum(S), gbase(S + 1);
     LAUNCH((k_pair_keys<K>), P, pstart, d_col, P, segw, k1.p, v1.p);
     K* kp = k1.p; K* ka = k2.p;
     uint32_t* vp = v1.p; uint32_t* va = v2.p;
@@ -916,8 +919,8 @@ static void build_groups_k(DeviceFormat& F, const int* d_col, const float* d_val
     exclusive_sum<int, int>(gnum.p, gbase.p, S, st);
     const int G = read_scalar(gbase.p + S, st);
 
-    DevBuf<int> ghead(G), size16(G);
-    DevBuf<long long> gp64(G + 1);
+    TmpBuf<int> ghead(G), size16(G);
+    TmpBuf<long long> gp64(G + 1);
     F.group_depth.alloc(G);
     F.group_seg_base.alloc(G);
     F.group_rows.alloc((size_t)16 * G);
@@ -942,13 +945,13 @@ static void build_groups_k(DeviceFormat& F, const int* d_col, const float* d_val
 
     // Work items (src/vcsr_mc.cu:109-121).
     const int chunk = std::max(1, std::min(32, G / 4096));
-    DevBuf<int> inum(S), ibase(S + 1);
+    TmpBuf<int> inum(S), ibase(S + 1);
     LAUNCH(k_items_per_seg, S, gnum.p, S, chunk, inum.p);
     exclusive_sum<int, int>(inum.p, ibase.p, S, st);
     const int I = read_scalar(ibase.p + S, st);
     const int wmax = chunk * 16 * 64;  // work <= chunk groups x 16 lanes x depth <= 64
-    DevBuf<int> ib(I), ie(I);
-    DevBuf<uint32_t> ik1(I), ik2(I), ip1(I), ip2(I);
+    TmpBuf<int> ib(I), ie(I);
+    TmpBuf<uint32_t> ik1(I), ik2(I), ip1(I), ip2(I);
     LAUNCH(k_make_items, S, gbase.p, ibase.p, F.group_ptr.p, S, chunk, wmax, ib.p, ie.p, ik1.p,
            ip1.p);
     uint32_t *ikp = ik1.p, *ika = ik2.p, *ipp = ip1.p, *ipa = ip2.p;
@@ -959,6 +962,11 @@ static void build_groups_k(DeviceFormat& F, const int* d_col, const float* d_val
     F.G = G;
     F.nval = nval;
     F.nitems = I;
+}
+
+// About what a build's temporaries take at once.
+static size_t build_scratch(long long nnz, long long M) {
+    return (size_t)(64 * nnz + 64 * M);
 }
 
 void build_from_csr(DeviceFormat& F, const int* d_row_ptr, const int* d_col, const float* d_val,
@@ -977,8 +985,9 @@ void build_from_csr(DeviceFormat& F, const int* d_row_ptr, const int* d_col, con
     F.nnz = nnz;
     const int S = (int)(((long long)N + segw - 1) / segw);
     F.num_segments = S;
+    ScratchScope scratch(build_scratch(nnz, M));
 
-    DevBuf<int> err(1);
+    TmpBuf<int> err(1);
     VCSRMC_HIP(hipMemsetAsync(err.p, 0, sizeof(int), st));
     LAUNCH(k_check_row_ptr, (long long)M + 1, d_row_ptr, M, nnz, err.p);
     check_err(err.p, st);
@@ -996,20 +1005,20 @@ void build_from_csr(DeviceFormat& F, const int* d_row_ptr, const int* d_col, con
     }
 
     // Row of every nonzero.
-    DevBuf<int> row_of(nnz);
+    TmpBuf<int> row_of(nnz);
     {
-        DevBuf<int> head(nnz);
+        TmpBuf<int> head(nnz);
         fill<int>(head.p, nnz, (int)0x80000000, st);
         LAUNCH(k_mark_row_heads, M, d_row_ptr, M, head.p);
         inclusive_max(head.p, row_of.p, nnz, st);
     }
     // (segment, row) runs.
-    DevBuf<int> phead(nnz), pidx(nnz + 1);
+    TmpBuf<int> phead(nnz), pidx(nnz + 1);
     LAUNCH(k_pair_heads, nnz, d_row_ptr, d_col, row_of.p, nnz, N, segw, phead.p, err.p);
     check_err(err.p, st);
     exclusive_sum<int, int>(phead.p, pidx.p, nnz, st);
     const int P = read_scalar(pidx.p + nnz, st);
-    DevBuf<int> pstart(P + 1), prow(P);
+    TmpBuf<int> pstart(P + 1), prow(P);
     LAUNCH(k_emit_pairs, nnz, phead.p, pidx.p, row_of.p, nnz, pstart.p, prow.p);
     fill<int>(pstart.p + P, 1, nnz, st);
     phead.release();
@@ -1024,7 +1033,7 @@ void build_from_csr(DeviceFormat& F, const int* d_row_ptr, const int* d_col, con
     prow.release();
 
     // Execution layout from (row_of, col, val / scale).
-    DevBuf<float> sval(nnz);
+    TmpBuf<float> sval(nnz);
     LAUNCH(k_scale_values, nnz, d_val, sval.p, (long long)nnz, inv_scale);
     build_exec_layout(F, row_of.p, d_col, sval.p, nnz, st);
     VCSRMC_HIP(hipStreamSynchronize(st));
@@ -1131,22 +1140,23 @@ void build_from_host(DeviceFormat& F, const HostArrays& H, hipStream_t st) {
     upload_array(F.item_gbeg, H.item_gbeg, H.nitems, st);
     upload_array(F.item_gend, H.item_gend, H.nitems, st);
 
-    DevBuf<int> err(1);
+    ScratchScope scratch(build_scratch(H.nval, H.M));
+    TmpBuf<int> err(1);
     VCSRMC_HIP(hipMemsetAsync(err.p, 0, sizeof(int), st));
     LAUNCH(k_check_groups, (long long)H.G + 1, F.group_ptr.p, F.group_depth.p,
            F.group_seg_base.p, F.group_rows.p, H.G, H.nval, H.M, H.N, H.segw, err.p);
     check_err(err.p, st);
 
     const long long nval = H.nval;
-    DevBuf<int> flag(nval), pos(nval + 1);
+    TmpBuf<int> flag(nval), pos(nval + 1);
     LAUNCH(k_expand_flags, nval, F.group_ptr.p, F.group_seg_base.p, F.group_rows.p, F.lcol.p,
            H.G, nval, H.N, H.segw, flag.p, err.p);
     check_err(err.p, st);
     exclusive_sum<int, int>(flag.p, pos.p, nval, st);
     const int n = nval ? read_scalar(pos.p + nval, st) : 0;
     F.nnz = n;
-    DevBuf<int> trow(n), tcol(n);
-    DevBuf<float> tval(n);
+    TmpBuf<int> trow(n), tcol(n);
+    TmpBuf<float> tval(n);
     LAUNCH(k_expand_write, nval, F.group_ptr.p, F.group_seg_base.p, F.group_rows.p, F.lcol.p,
            F.val.p, flag.p, pos.p, H.G, nval, trow.p, tcol.p, tval.p);
     build_exec_layout(F, trow.p, tcol.p, tval.p, n, st);

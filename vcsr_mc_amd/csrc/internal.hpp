@@ -144,11 +144,11 @@ float device_absmax(const float* d_val, long long n, hipStream_t st);
 // (row, col) of n nonzeros: rowpos[row] = position, row_map[position] = row (-1 past the last
 // of M rows; M rounded up to 16 entries).  False when it found nothing to work with.
 bool group_rows(const int* trow, const int* tcol, long long n, int M, int N, hipStream_t st,
-                DevBuf<int>& rowpos, DevBuf<int>& row_map);
+                TmpBuf<int>& rowpos, DevBuf<int>& row_map);
 // The same maps for natural order with the rows that hold no nonzero moved after the others,
 // when they are at least an eighth of the rows (false otherwise): panels then hold 16 rows
 // with nonzeros instead of, on average, as many as the empty rows leave.
-bool compact_rows(const int* trow, long long n, int M, hipStream_t st, DevBuf<int>& rowpos,
+bool compact_rows(const int* trow, long long n, int M, hipStream_t st, TmpBuf<int>& rowpos,
                   DevBuf<int>& row_map);
 // Row order of the execution layout: 0 natural order, 1 empty rows moved last and rows grouped
 // where that saves tiles (the default; format_build.hip, build_exec_layout), 2 always grouped.

@@ -999,7 +999,7 @@ __global__ void k_mark_heads(const int* __restrict__ rp, int M, int* __restrict_
 
 // Row of every nonzero: each non-empty row marks its first slot, a running max fills the rest.
 void row_of_nonzeros(const int* rp, int M, int nnz, int* row_of, hipStream_t st) {
-    DevBuf<int> headmark(nnz);
+    TmpBuf<int> headmark(nnz);
     fill<int>(headmark.p, nnz, (int)0x80000000, st);
     RLAUNCH(k_mark_heads, M, rp, M, headmark.p);
     inclusive_max(headmark.p, row_of, nnz, st);
@@ -1008,8 +1008,8 @@ void row_of_nonzeros(const int* rp, int M, int nnz, int* row_of, hipStream_t st)
 // Work lists of the child-group sort, sized for the largest level (a range never holds fewer
 // than one element, so there are at most N ranges of each kind).
 struct SortJobs {
-    DevBuf<int4> big0, big1, small;
-    DevBuf<int> lpos, rpos, counts;  // counts: {big0, big1, small}
+    TmpBuf<int4> big0, big1, small;
+    TmpBuf<int> lpos, rpos, counts;  // counts: {big0, big1, small}
     explicit SortJobs(int N)
         : big0(N), big1(N), small(N), lpos(N), rpos(N), counts(3) {}
 };
@@ -1070,28 +1070,29 @@ void rcm_order_device(const int* rp, const int* col, int M, int N, int nnz, int*
         throw Error(VCSRMC_ERR_ARG, "null pointer");
     if (2ll * nnz >= (1ll << 31))
         throw Error(VCSRMC_ERR_OVERFLOW, "rcm ordering handles fewer than 2^30 nonzeros");
-    DevBuf<int> err(1);
+    ScratchScope scratch((size_t)(72ll * nnz + 160ll * N));
+    TmpBuf<int> err(1);
     check_csr(rp, col, M, N, nnz, err.p, st);
     if (N == 0) return;
 
     const int nb = std::max(1, bits_for((u64)N));  // holds 0..N
     // 1. adjacency
-    DevBuf<int> adj_u, adj;
-    DevBuf<long long> head((size_t)N + 1);
+    TmpBuf<int> adj_u, adj;
+    TmpBuf<long long> head((size_t)N + 1);
     long long E = 0;
     {
         const long long P = 2ll * nnz;
-        DevBuf<int> row_of(nnz);
+        TmpBuf<int> row_of(nnz);
         if (nnz) row_of_nonzeros(rp, M, nnz, row_of.p, st);
-        DevBuf<u64> k1(P), k2(P);
-        DevBuf<uint32_t> v1(P), v2(P);
+        TmpBuf<u64> k1(P), k2(P);
+        TmpBuf<uint32_t> v1(P), v2(P);
         RLAUNCH(k_adj_pairs, nnz, row_of.p, col, (long long)nnz, N, nb, k1.p);
         row_of.release();
         u64 *ka = k1.p, *kb = k2.p;
         uint32_t *va = v1.p, *vb = v2.p;
         radix_sort_pairs<u64>(ka, va, kb, vb, P, 2 * nb, st);
-        DevBuf<int> flag(P);
-        DevBuf<long long> pos(P + 1);
+        TmpBuf<int> flag(P);
+        TmpBuf<long long> pos(P + 1);
         RLAUNCH(k_unique_flags, P, ka, P, flag.p);
         exclusive_sum<int, long long>(flag.p, pos.p, P, st);
         E = P ? read_scalar(pos.p + P, st) : 0;
@@ -1102,11 +1103,11 @@ void rcm_order_device(const int* rp, const int* col, int M, int N, int nnz, int*
     RLAUNCH(k_heads, (long long)N + 1, adj_u.p, E, N, head.p);
 
     // 2. rank
-    DevBuf<uint32_t> order(N);
-    DevBuf<int> rank(N);
+    TmpBuf<uint32_t> order(N);
+    TmpBuf<int> rank(N);
     {
-        DevBuf<u64> k1(N), k2(N);
-        DevBuf<uint32_t> v2(N);
+        TmpBuf<u64> k1(N), k2(N);
+        TmpBuf<uint32_t> v2(N);
         RLAUNCH(k_rank_keys, N, head.p, N, nb, k1.p, order.p);
         u64 *ka = k1.p, *kb = k2.p;
         uint32_t *va = order.p, *vb = v2.p;
@@ -1130,9 +1131,9 @@ void rcm_order_device(const int* rp, const int* col, int M, int N, int nnz, int*
         lim_rounds > 0 ? lim_rounds : (long long)N * (bits_for((u64)N) + 2) + 1;
 
     // 3. components
-    DevBuf<int> comp(N);
+    TmpBuf<int> comp(N);
     {
-        DevBuf<int> changed(1);
+        TmpBuf<int> changed(1);
         RLAUNCH(k_cc_init, N, comp.p, N);
         for (long long round = 0;; ++round) {
             if (round >= max_rounds)
@@ -1147,25 +1148,25 @@ void rcm_order_device(const int* rp, const int* col, int M, int N, int nnz, int*
     adj_u.release();
 
     // 4. levels
-    DevBuf<int> lev(N), seq(N), claim(N), front(N), next(N), count(1);
+    TmpBuf<int> lev(N), seq(N), claim(N), front(N), next(N), count(1);
     fill<int>(lev.p, N, -1, st);
     fill<int>(claim.p, N, INT_MAX, st);
     int f = 0;
     {
-        DevBuf<int> flag(N);
-        DevBuf<long long> pos((size_t)N + 1);
+        TmpBuf<int> flag(N);
+        TmpBuf<long long> pos((size_t)N + 1);
         RLAUNCH(k_root_flags, N, order.p, comp.p, N, flag.p);
         exclusive_sum<int, long long>(flag.p, pos.p, N, st);
         f = (int)read_scalar(pos.p + N, st);
         RLAUNCH(k_root_list, N, order.p, flag.p, pos.p, N, front.p, lev.p, seq.p);
     }
-    DevBuf<long long> fdeg(N), fofs((size_t)N + 1);
-    DevBuf<u64> k1(N), k2(N);
-    DevBuf<uint32_t> v1(N), v2(N);
-    DevBuf<int> gflag(N), gstart(N);
-    DevBuf<long long> gpos((size_t)N + 1);
+    TmpBuf<long long> fdeg(N), fofs((size_t)N + 1);
+    TmpBuf<u64> k1(N), k2(N);
+    TmpBuf<uint32_t> v1(N), v2(N);
+    TmpBuf<int> gflag(N), gstart(N);
+    TmpBuf<long long> gpos((size_t)N + 1);
     SortJobs jobs(N);
-    DevBuf<int4> bfs_state(1);
+    TmpBuf<int4> bfs_state(1);
     int base = f, level = 1;
     while (f > 0 && base < N) {
         if (f <= kBfsCap) {  // run levels inside one work-group while they are small
@@ -1232,10 +1233,11 @@ void apply_column_permutation_device(const int* rp, int* col, float* val, int M,
     if ((B == nullptr) != (B_out == nullptr))
         throw Error(VCSRMC_ERR_ARG, "B and B_out must both be given or both be NULL");
     if (B && B == B_out) throw Error(VCSRMC_ERR_ARG, "B_out must not alias B");
-    DevBuf<int> err(1);
+    ScratchScope scratch((size_t)(36ll * nnz + 8ll * N));
+    TmpBuf<int> err(1);
     check_csr(rp, col, M, N, nnz, err.p, st);
     if (N > 0) {
-        DevBuf<int> seen(N);
+        TmpBuf<int> seen(N);
         VCSRMC_HIP(hipMemsetAsync(seen.p, 0, sizeof(int) * (size_t)N, st));
         RLAUNCH(k_perm_check, N, position, N, seen.p, err.p);
         raise_if(err.p, st);
@@ -1243,10 +1245,10 @@ void apply_column_permutation_device(const int* rp, int* col, float* val, int M,
     if (nnz > 0) {
         const int nb = std::max(1, bits_for((u64)N));
         const int mb = std::max(1, bits_for((u64)M));
-        DevBuf<int> row_of(nnz);
+        TmpBuf<int> row_of(nnz);
         row_of_nonzeros(rp, M, nnz, row_of.p, st);
-        DevBuf<u64> k1(nnz), k2(nnz);
-        DevBuf<uint32_t> v1(nnz), v2(nnz);
+        TmpBuf<u64> k1(nnz), k2(nnz);
+        TmpBuf<uint32_t> v1(nnz), v2(nnz);
         RLAUNCH(k_relabel_keys, nnz, row_of.p, col, position, (long long)nnz, nb, k1.p, v1.p);
         row_of.release();
         u64 *ka = k1.p, *kb = k2.p;
@@ -1254,7 +1256,7 @@ void apply_column_permutation_device(const int* rp, int* col, float* val, int M,
         radix_sort_pairs<u64>(ka, va, kb, vb, nnz, nb + mb, st);
         RLAUNCH(k_relabel_dups, nnz, ka, (long long)nnz, err.p);
         raise_if(err.p, st);
-        DevBuf<float> vcopy(nnz);
+        TmpBuf<float> vcopy(nnz);
         VCSRMC_HIP(hipMemcpyAsync(vcopy.p, val, sizeof(float) * (size_t)nnz,
                                   hipMemcpyDeviceToDevice, st));
         RLAUNCH(k_relabel_write, nnz, ka, va, vcopy.p, (long long)nnz, nb, col, val);

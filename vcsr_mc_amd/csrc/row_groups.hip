@@ -323,8 +323,8 @@ __global__ void k_positions(const uint32_t* __restrict__ order, int M, int P,
     }
 }
 
-void sort_keys(DevBuf<u64>& keys, DevBuf<u64>& alt, DevBuf<uint32_t>& pay,
-               DevBuf<uint32_t>& pay_alt, long long n, int bits, hipStream_t st) {
+void sort_keys(TmpBuf<u64>& keys, TmpBuf<u64>& alt, TmpBuf<uint32_t>& pay,
+               TmpBuf<uint32_t>& pay_alt, long long n, int bits, hipStream_t st) {
     u64 *k = keys.p, *ka = alt.p;
     uint32_t *v = pay.p, *va = pay_alt.p;
     radix_sort_pairs<u64>(k, v, ka, va, n, bits, st);
@@ -352,10 +352,10 @@ __global__ void k_compact_positions(const int* __restrict__ flag, const int* __r
 
 }  // namespace
 
-bool compact_rows(const int* trow, long long n, int M, hipStream_t st, DevBuf<int>& rowpos,
+bool compact_rows(const int* trow, long long n, int M, hipStream_t st, TmpBuf<int>& rowpos,
                   DevBuf<int>& row_map) {
     if (M < 1 || n < 1) return false;
-    DevBuf<int> flag(M), rank((size_t)M + 1);
+    TmpBuf<int> flag(M), rank((size_t)M + 1);
     fill<int>(flag.p, M, 0, st);
     hipLaunchKernelGGL(k_flag_rows, dim3(grid256(n)), dim3(256), 0, st, trow, n, flag.p);
     VCSRMC_HIP(hipGetLastError());
@@ -373,16 +373,16 @@ bool compact_rows(const int* trow, long long n, int M, hipStream_t st, DevBuf<in
 }
 
 bool group_rows(const int* trow, const int* tcol, long long n, int M, int N, hipStream_t st,
-                DevBuf<int>& rowpos, DevBuf<int>& row_map) {
+                TmpBuf<int>& rowpos, DevBuf<int>& row_map) {
     if (M < 2 * kPanelRows || N < 1 || n < 1) return false;
     const int rbits = bits_for((unsigned long long)(M - 1));
     const int cbits = bits_for((unsigned long long)(N - 1));
     const int hub = (int)std::max<long long>(32, std::min<long long>(1024, 4 * n / N));
 
     // Column degrees from the column-major order of the triples.
-    DevBuf<u64> keys(n), alt(n);
-    DevBuf<uint32_t> pay(n), pay_alt(n);
-    DevBuf<int> cptr((size_t)N + 1);
+    TmpBuf<u64> keys(n), alt(n);
+    TmpBuf<uint32_t> pay(n), pay_alt(n);
+    TmpBuf<int> cptr((size_t)N + 1);
     hipLaunchKernelGGL(k_col_major_keys, dim3(grid256(n)), dim3(256), 0, st, trow, tcol, n, rbits,
                        keys.p);
     VCSRMC_HIP(hipGetLastError());
@@ -394,7 +394,7 @@ bool group_rows(const int* trow, const int* tcol, long long n, int M, int N, hip
     // Level-0 cluster-column keys: the triples on columns of at most `hub` rows.
     long long np;
     {
-        DevBuf<int> keep(n), at((size_t)n + 1);
+        TmpBuf<int> keep(n), at((size_t)n + 1);
         hipLaunchKernelGGL(k_keep_flags, dim3(grid256(n)), dim3(256), 0, st, tcol, cptr.p, n, hub,
                            keep.p);
         VCSRMC_HIP(hipGetLastError());
@@ -408,15 +408,15 @@ bool group_rows(const int* trow, const int* tcol, long long n, int M, int N, hip
     sort_keys(keys, alt, pay, pay_alt, np, rbits + cbits, st);
 
     int nc = M;
-    DevBuf<int> rowcl(M), size(M), cmin(M);
+    TmpBuf<int> rowcl(M), size(M), cmin(M);
     hipLaunchKernelGGL(k_init_clusters, dim3(grid256(M)), dim3(256), 0, st, M, rowcl.p, size.p,
                        cmin.p);
     VCSRMC_HIP(hipGetLastError());
-    DevBuf<u64> rck(np), rca(np);
+    TmpBuf<u64> rck(np), rca(np);
     for (int level = 0; level < kLevels; ++level) {
         const int clbits = bits_for((unsigned long long)(nc - 1));
         // cluster -> columns (keys, sorted) and column -> clusters
-        DevBuf<int> cr_ptr((size_t)nc + 1), rc_ptr((size_t)N + 1);
+        TmpBuf<int> cr_ptr((size_t)nc + 1), rc_ptr((size_t)N + 1);
         hipLaunchKernelGGL(k_lower_bounds, dim3(grid256((long long)nc + 1)), dim3(256), 0, st,
                            keys.p, np, cbits, nc, cr_ptr.p);
         VCSRMC_HIP(hipGetLastError());
@@ -434,7 +434,7 @@ bool group_rows(const int* trow, const int* tcol, long long n, int M, int N, hip
         VCSRMC_HIP(hipGetLastError());
 
         const int maxsz = 2 << level;  // clusters of 2^level rows pair into 2^(level+1)
-        DevBuf<int> cand((size_t)nc * kCand), mate(nc), prop(nc);
+        TmpBuf<int> cand((size_t)nc * kCand), mate(nc), prop(nc);
         hipLaunchKernelGGL(k_score, dim3(grid_for(nc, 4)), dim3(256), 0, st, keys.p, cr_ptr.p,
                            rck.p, rc_ptr.p, cbits, clbits, size.p, cmin.p, nc, maxsz,
                            level == kLevels - 1, cand.p);
@@ -447,13 +447,13 @@ bool group_rows(const int* trow, const int* tcol, long long n, int M, int N, hip
             hipLaunchKernelGGL(k_accept, dim3(grid256(nc)), dim3(256), 0, st, prop.p, nc, mate.p);
             VCSRMC_HIP(hipGetLastError());
         }
-        DevBuf<int> isrep(nc), nid((size_t)nc + 1);
+        TmpBuf<int> isrep(nc), nid((size_t)nc + 1);
         hipLaunchKernelGGL(k_rep_flags, dim3(grid256(nc)), dim3(256), 0, st, mate.p, nc, isrep.p);
         VCSRMC_HIP(hipGetLastError());
         exclusive_sum<int, int>(isrep.p, nid.p, nc, st);
         const int nnc = read_scalar(nid.p + nc, st);
         if (nnc == nc) break;  // nothing merged at this level: none will at the next
-        DevBuf<int> newcl(nc), nsize(nnc), ncmin(nnc);
+        TmpBuf<int> newcl(nc), nsize(nnc), ncmin(nnc);
         hipLaunchKernelGGL(k_relabel, dim3(grid256(nc)), dim3(256), 0, st, mate.p, nid.p, size.p,
                            cmin.p, nc, newcl.p, nsize.p, ncmin.p);
         VCSRMC_HIP(hipGetLastError());
@@ -470,7 +470,7 @@ bool group_rows(const int* trow, const int* tcol, long long n, int M, int N, hip
         const int nclbits = bits_for((unsigned long long)(nnc - 1));
         sort_keys(keys, alt, pay, pay_alt, np, nclbits + cbits, st);
         {
-            DevBuf<int> head(np), at((size_t)np + 1);
+            TmpBuf<int> head(np), at((size_t)np + 1);
             hipLaunchKernelGGL(k_head_flags, dim3(grid256(np)), dim3(256), 0, st, keys.p, np,
                                head.p);
             VCSRMC_HIP(hipGetLastError());
@@ -487,12 +487,12 @@ bool group_rows(const int* trow, const int* tcol, long long n, int M, int N, hip
 
     // Rows by group (first row of the group), rows without nonzeros last.
     const int P = ((M + kPanelRows - 1) / kPanelRows) * kPanelRows;
-    DevBuf<unsigned char> has(M);
+    TmpBuf<unsigned char> has(M);
     fill<unsigned char>(has.p, M, 0, st);
     hipLaunchKernelGGL(k_has_nonzero, dim3(grid256(n)), dim3(256), 0, st, trow, n, has.p);
     VCSRMC_HIP(hipGetLastError());
-    DevBuf<u64> okey(M), oalt(M);
-    DevBuf<uint32_t> opay(M), opalt(M);
+    TmpBuf<u64> okey(M), oalt(M);
+    TmpBuf<uint32_t> opay(M), opalt(M);
     hipLaunchKernelGGL(k_order_keys, dim3(grid256(M)), dim3(256), 0, st, rowcl.p, cmin.p, has.p,
                        M, okey.p, opay.p);
     VCSRMC_HIP(hipGetLastError());
