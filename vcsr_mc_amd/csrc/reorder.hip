@@ -1085,12 +1085,10 @@ void rcm_order_device(const int* rp, const int* col, int M, int N, int nnz, int*
         TmpBuf<int> row_of(nnz);
         if (nnz) row_of_nonzeros(rp, M, nnz, row_of.p, st);
         TmpBuf<u64> k1(P), k2(P);
-        TmpBuf<uint32_t> v1(P), v2(P);
         RLAUNCH(k_adj_pairs, nnz, row_of.p, col, (long long)nnz, N, nb, k1.p);
         row_of.release();
         u64 *ka = k1.p, *kb = k2.p;
-        uint32_t *va = v1.p, *vb = v2.p;
-        radix_sort_pairs<u64>(ka, va, kb, vb, P, 2 * nb, st);
+        radix_sort_keys<u64>(ka, kb, P, 2 * nb, st);
         TmpBuf<int> flag(P);
         TmpBuf<long long> pos(P + 1);
         RLAUNCH(k_unique_flags, P, ka, P, flag.p);

@@ -299,14 +299,14 @@ __global__ void k_has_nonzero(const int* __restrict__ trow, long long n,
     if (i < n) has[trow[i]] = 1;
 }
 
-// Order key of row r: its group's first row (rows without nonzeros last), then r.
+// Order key of row r: its group's first row (rows without nonzeros last); the stable sort keeps
+// the rows of a group by index.
 __global__ void k_order_keys(const int* __restrict__ rowcl, const int* __restrict__ cmin,
-                             const unsigned char* __restrict__ has, int M, u64* __restrict__ key,
-                             uint32_t* __restrict__ pay) {
+                             const unsigned char* __restrict__ has, int M,
+                             uint32_t* __restrict__ key, uint32_t* __restrict__ pay) {
     const long long r = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= M) return;
-    const u64 first = has[r] ? (u64)cmin[rowcl[r]] : (u64)INT_MAX;
-    key[r] = (first << 32) | (u64)r;
+    key[r] = has[r] ? (uint32_t)cmin[rowcl[r]] : (uint32_t)M;
     pay[r] = (uint32_t)r;
 }
 
@@ -323,15 +323,10 @@ __global__ void k_positions(const uint32_t* __restrict__ order, int M, int P,
     }
 }
 
-void sort_keys(TmpBuf<u64>& keys, TmpBuf<u64>& alt, TmpBuf<uint32_t>& pay,
-               TmpBuf<uint32_t>& pay_alt, long long n, int bits, hipStream_t st) {
+void sort_keys(TmpBuf<u64>& keys, TmpBuf<u64>& alt, long long n, int bits, hipStream_t st) {
     u64 *k = keys.p, *ka = alt.p;
-    uint32_t *v = pay.p, *va = pay_alt.p;
-    radix_sort_pairs<u64>(k, v, ka, va, n, bits, st);
-    if (k != keys.p) {  // an odd number of passes: the result is in the alternate buffers
-        std::swap(keys, alt);
-        std::swap(pay, pay_alt);
-    }
+    radix_sort_keys<u64>(k, ka, n, bits, st);
+    if (k != keys.p) std::swap(keys, alt);  // an odd number of passes
 }
 
 __global__ void k_flag_rows(const int* __restrict__ trow, long long n, int* __restrict__ flag) {
@@ -381,12 +376,11 @@ bool group_rows(const int* trow, const int* tcol, long long n, int M, int N, hip
 
     // Column degrees from the column-major order of the triples.
     TmpBuf<u64> keys(n), alt(n);
-    TmpBuf<uint32_t> pay(n), pay_alt(n);
     TmpBuf<int> cptr((size_t)N + 1);
     hipLaunchKernelGGL(k_col_major_keys, dim3(grid256(n)), dim3(256), 0, st, trow, tcol, n, rbits,
                        keys.p);
     VCSRMC_HIP(hipGetLastError());
-    sort_keys(keys, alt, pay, pay_alt, n, cbits + rbits, st);
+    sort_keys(keys, alt, n, cbits + rbits, st);
     hipLaunchKernelGGL(k_lower_bounds, dim3(grid256((long long)N + 1)), dim3(256), 0, st, keys.p,
                        n, rbits, N, cptr.p);
     VCSRMC_HIP(hipGetLastError());
@@ -405,7 +399,7 @@ bool group_rows(const int* trow, const int* tcol, long long n, int M, int N, hip
         VCSRMC_HIP(hipGetLastError());
     }
     if (np == 0) return false;
-    sort_keys(keys, alt, pay, pay_alt, np, rbits + cbits, st);
+    sort_keys(keys, alt, np, rbits + cbits, st);
 
     int nc = M;
     TmpBuf<int> rowcl(M), size(M), cmin(M);
@@ -425,8 +419,7 @@ bool group_rows(const int* trow, const int* tcol, long long n, int M, int N, hip
         VCSRMC_HIP(hipGetLastError());
         {
             u64 *k = rck.p, *ka = rca.p;
-            uint32_t *v = pay.p, *va = pay_alt.p;
-            radix_sort_pairs<u64>(k, v, ka, va, np, cbits + clbits, st);
+            radix_sort_keys<u64>(k, ka, np, cbits + clbits, st);
             if (k != rck.p) std::swap(rck, rca);
         }
         hipLaunchKernelGGL(k_lower_bounds, dim3(grid256((long long)N + 1)), dim3(256), 0, st,
@@ -468,7 +461,7 @@ bool group_rows(const int* trow, const int* tcol, long long n, int M, int N, hip
         VCSRMC_HIP(hipGetLastError());
         std::swap(keys, alt);
         const int nclbits = bits_for((unsigned long long)(nnc - 1));
-        sort_keys(keys, alt, pay, pay_alt, np, nclbits + cbits, st);
+        sort_keys(keys, alt, np, nclbits + cbits, st);
         {
             TmpBuf<int> head(np), at((size_t)np + 1);
             hipLaunchKernelGGL(k_head_flags, dim3(grid256(np)), dim3(256), 0, st, keys.p, np,
@@ -491,15 +484,15 @@ bool group_rows(const int* trow, const int* tcol, long long n, int M, int N, hip
     fill<unsigned char>(has.p, M, 0, st);
     hipLaunchKernelGGL(k_has_nonzero, dim3(grid256(n)), dim3(256), 0, st, trow, n, has.p);
     VCSRMC_HIP(hipGetLastError());
-    TmpBuf<u64> okey(M), oalt(M);
-    TmpBuf<uint32_t> opay(M), opalt(M);
+    TmpBuf<uint32_t> okey(M), oalt(M), opay(M), opalt(M);
     hipLaunchKernelGGL(k_order_keys, dim3(grid256(M)), dim3(256), 0, st, rowcl.p, cmin.p, has.p,
                        M, okey.p, opay.p);
     VCSRMC_HIP(hipGetLastError());
-    sort_keys(okey, oalt, opay, opalt, M, 64, st);
+    uint32_t *ok = okey.p, *oka = oalt.p, *order = opay.p, *order_alt = opalt.p;
+    radix_sort_pairs<uint32_t>(ok, order, oka, order_alt, M, bits_for((unsigned long long)M), st);
     rowpos.alloc(M);
     row_map.alloc(P);
-    hipLaunchKernelGGL(k_positions, dim3(grid256(P)), dim3(256), 0, st, opay.p, M, P, rowpos.p,
+    hipLaunchKernelGGL(k_positions, dim3(grid256(P)), dim3(256), 0, st, order, M, P, rowpos.p,
                        row_map.p);
     VCSRMC_HIP(hipGetLastError());
     return true;
