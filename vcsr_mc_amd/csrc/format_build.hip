@@ -861,8 +861,8 @@ int fp32_row_steps() { return g_fp32_row_steps.load(std::memory_order_relaxed); 
 // 300 -> 316 / 251; 2D 5-point 1000^2 FP32 312 / 234 -> 297 / 196 (tiles halved); 3D 7-point
 // 100^3 FP32 390 / 328 -> 373 / 255; 27-point 16^3 (256 panels) within 2% either way.  Grouping
 // the excluded classes anyway saved 1-7% of their tiles and ran from 6% faster to 13% slower.
-static void build_exec_layout(DeviceFormat& F, const int* trow, const int* tcol, const float* tval,
-                              long long n, hipStream_t st) {
+static void build_exec_layout(DeviceFormat& F, const int* rp, const int* trow, const int* tcol,
+                              const float* tval, long long n, hipStream_t st) {
     F.row_map.release();
     const int mode = row_grouping();
     TmpBuf<int> cpos;
@@ -886,7 +886,7 @@ static void build_exec_layout(DeviceFormat& F, const int* trow, const int* tcol,
     }
     TmpBuf<int> rowpos;
     DevBuf<int> row_map;
-    if (!group_rows(trow, tcol, n, F.M, F.N, st, rowpos, row_map)) return;
+    if (!group_rows(rp, trow, tcol, n, F.M, F.N, st, rowpos, row_map)) return;
     DeviceFormat G;
     G.M = F.M;
     G.N = F.N;
@@ -1035,7 +1035,7 @@ void build_from_csr(DeviceFormat& F, const int* d_row_ptr, const int* d_col, con
     // Execution layout from (row_of, col, val / scale).
     TmpBuf<float> sval(nnz);
     LAUNCH(k_scale_values, nnz, d_val, sval.p, (long long)nnz, inv_scale);
-    build_exec_layout(F, row_of.p, d_col, sval.p, nnz, st);
+    build_exec_layout(F, d_row_ptr, row_of.p, d_col, sval.p, nnz, st);
     VCSRMC_HIP(hipStreamSynchronize(st));
     F.ready = true;
 }
@@ -1112,6 +1112,56 @@ __global__ void k_expand_write(const int* __restrict__ gp, const int* __restrict
     tval[i] = val[t];
 }
 
+template <typename K>
+__global__ void k_triple_keys(const int* __restrict__ trow, const int* __restrict__ tcol,
+                              long long n, int cbits, K* __restrict__ key,
+                              uint32_t* __restrict__ pay) {
+    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    key[i] = ((K)trow[i] << cbits) | (K)tcol[i];
+    pay[i] = (uint32_t)i;
+}
+
+template <typename K>
+__global__ void k_triple_gather(const K* __restrict__ key, const uint32_t* __restrict__ src,
+                                const float* __restrict__ tval, long long n, int cbits,
+                                int* __restrict__ row, int* __restrict__ col,
+                                float* __restrict__ val, int* __restrict__ err) {
+    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const K k = key[i];
+    if (i > 0 && key[i - 1] == k) atomicOr(err, kErrDuplicate);
+    row[i] = (int)(k >> cbits);
+    col[i] = (int)(k & (((K)1 << cbits) - 1));
+    val[i] = tval[src[i]];
+}
+
+// The triples in (row, column) order; refuses a coordinate given twice.
+template <typename K>
+static void sort_triples_k(TmpBuf<int>& trow, TmpBuf<int>& tcol, TmpBuf<float>& tval, long long n,
+                           int cbits, int bits, int* err, hipStream_t st) {
+    TmpBuf<K> k1(n), k2(n);
+    TmpBuf<uint32_t> v1(n), v2(n);
+    TmpBuf<float> val(n);
+    LAUNCH((k_triple_keys<K>), n, trow.p, tcol.p, n, cbits, k1.p, v1.p);
+    K *k = k1.p, *ka = k2.p;
+    uint32_t *v = v1.p, *va = v2.p;
+    radix_sort_pairs<K>(k, v, ka, va, n, bits, st);
+    LAUNCH((k_triple_gather<K>), n, k, v, tval.p, n, cbits, trow.p, tcol.p, val.p, err);
+    tval = std::move(val);
+}
+
+static void sort_triples(TmpBuf<int>& trow, TmpBuf<int>& tcol, TmpBuf<float>& tval, long long n,
+                         int M, int N, hipStream_t st) {
+    TmpBuf<int> err(1);
+    VCSRMC_HIP(hipMemsetAsync(err.p, 0, sizeof(int), st));
+    const int cbits = bits_for((unsigned long long)(N - 1));
+    const int bits = cbits + bits_for((unsigned long long)(M - 1));
+    if (bits <= 32) sort_triples_k<uint32_t>(trow, tcol, tval, n, cbits, bits, err.p, st);
+    else sort_triples_k<unsigned long long>(trow, tcol, tval, n, cbits, bits, err.p, st);
+    check_err(err.p, st);
+}
+
 template <typename T>
 static void upload_array(DevBuf<T>& d, const T* h, long long n, hipStream_t st) {
     d.alloc(n > 0 ? n : 0);
@@ -1155,11 +1205,15 @@ void build_from_host(DeviceFormat& F, const HostArrays& H, hipStream_t st) {
     exclusive_sum<int, int>(flag.p, pos.p, nval, st);
     const int n = nval ? read_scalar(pos.p + nval, st) : 0;
     F.nnz = n;
-    TmpBuf<int> trow(n), tcol(n);
+    TmpBuf<int> trow(n), tcol(n), rp((size_t)H.M + 1);
     TmpBuf<float> tval(n);
     LAUNCH(k_expand_write, nval, F.group_ptr.p, F.group_seg_base.p, F.group_rows.p, F.lcol.p,
            F.val.p, flag.p, pos.p, H.G, nval, trow.p, tcol.p, tval.p);
-    build_exec_layout(F, trow.p, tcol.p, tval.p, n, st);
+    if (n > 0) {
+        sort_triples(trow, tcol, tval, n, H.M, H.N, st);
+        key_ptr<int>(trow.p, n, H.M, rp.p, st);
+    }
+    build_exec_layout(F, rp.p, trow.p, tcol.p, tval.p, n, st);
     VCSRMC_HIP(hipStreamSynchronize(st));
     F.ready = true;
 }

@@ -469,25 +469,38 @@ __global__ __launch_bounds__(kSortThreads) void k_radix_scatter(
     }
 }
 
-// The digits of a sort by `bits` bits: passes of equal width, at most 8 bits each.
+// Passes of equal width, at most 8 bits each: the first reads (src, vsrc), the others what the
+// pass before wrote, in (a, va) and (b, vb) by turns.  Returns the sorted keys and payload.
 template <typename K, bool VAL>
-void radix_sort_impl(K*& k, uint32_t*& v, K*& k_alt, uint32_t*& v_alt, long long n, int bits,
-                     hipStream_t st) {
-    if (n <= 1 || bits <= 0) return;
+std::pair<K*, uint32_t*> radix_sort_impl(const K* src, const uint32_t* vsrc, K* a, uint32_t* va,
+                                         K* b, uint32_t* vb, long long n, int bits,
+                                         hipStream_t st) {
     const int passes = (bits + 7) / 8, width = (bits + passes - 1) / passes;
     const int ntiles = (int)((n + kSortTile - 1) / kSortTile);
     TmpBuf<int> hist((size_t)ntiles << width), offs(((size_t)ntiles << width) + 1);
     for (int shift = 0; shift < bits; shift += width) {
-        hipLaunchKernelGGL((k_radix_hist<K>), dim3(ntiles), dim3(kSortThreads), 0, st, k, n, shift,
-                           1 << width, hist.p, ntiles);
+        hipLaunchKernelGGL((k_radix_hist<K>), dim3(ntiles), dim3(kSortThreads), 0, st, src, n,
+                           shift, 1 << width, hist.p, ntiles);
         VCSRMC_HIP(hipGetLastError());
         exclusive_sum<int, int>(hist.p, offs.p, (long long)ntiles << width, st);
-        hipLaunchKernelGGL((k_radix_scatter<K, VAL>), dim3(ntiles), dim3(kSortThreads), 0, st, k,
-                           v, k_alt, v_alt, n, shift, width, offs.p, ntiles);
+        hipLaunchKernelGGL((k_radix_scatter<K, VAL>), dim3(ntiles), dim3(kSortThreads), 0, st, src,
+                           vsrc, a, va, n, shift, width, offs.p, ntiles);
         VCSRMC_HIP(hipGetLastError());
-        std::swap(k, k_alt);
-        if (VAL) std::swap(v, v_alt);
+        src = a;
+        vsrc = va;
+        std::swap(a, b);
+        std::swap(va, vb);
     }
+    return {b, vb};
+}
+
+// The n pairs of (src, vsrc), which stay as they are, sorted by the low `bits` (>= 1) bits of the
+// key into one of the two given pairs of arrays, the other being scratch.  n must be below 2^31.
+template <typename K>
+std::pair<K*, uint32_t*> radix_sort_pairs_from(const K* src, const uint32_t* vsrc, K* a,
+                                               uint32_t* va, K* b, uint32_t* vb, long long n,
+                                               int bits, hipStream_t st) {
+    return radix_sort_impl<K, true>(src, vsrc, a, va, b, vb, n, bits, st);
 }
 
 // Sorts n pairs by the low `bits` bits of the key.  The sorted pairs end up in (k, v); the
@@ -495,14 +508,20 @@ void radix_sort_impl(K*& k, uint32_t*& v, K*& k_alt, uint32_t*& v_alt, long long
 template <typename K>
 void radix_sort_pairs(K*& k, uint32_t*& v, K*& k_alt, uint32_t*& v_alt, long long n, int bits,
                       hipStream_t st) {
-    radix_sort_impl<K, true>(k, v, k_alt, v_alt, n, bits, st);
+    if (n <= 1 || bits <= 0) return;
+    const auto out = radix_sort_impl<K, true>(k, v, k_alt, v_alt, k, v, n, bits, st);
+    if (out.first != k) {
+        std::swap(k, k_alt);
+        std::swap(v, v_alt);
+    }
 }
 
 // The same for keys alone.
 template <typename K>
 void radix_sort_keys(K*& k, K*& k_alt, long long n, int bits, hipStream_t st) {
-    uint32_t *none = nullptr, *none_alt = nullptr;
-    radix_sort_impl<K, false>(k, none, k_alt, none_alt, n, bits, st);
+    if (n <= 1 || bits <= 0) return;
+    const auto out = radix_sort_impl<K, false>(k, nullptr, k_alt, nullptr, k, nullptr, n, bits, st);
+    if (out.first != k) std::swap(k, k_alt);
 }
 
 // ---- small kernels -----------------------------------------------------------------------
@@ -516,6 +535,40 @@ template <typename T>
 void fill(T* p, long long n, T value, hipStream_t st) {
     if (n <= 0) return;
     hipLaunchKernelGGL((k_fill<T>), dim3(grid_for(n, 256)), dim3(256), 0, st, p, n, value);
+    VCSRMC_HIP(hipGetLastError());
+}
+
+// ptr[v] = the first index of the ascending `keys` (each below count) that is >= v, for v in
+// [0, count]: every change of the key writes the values it passes, the whole wave where they are
+// many.
+__device__ __forceinline__ void key_ptr_write(int from, int to, int i, int* __restrict__ ptr) {
+    uint64_t wide = __ballot(to - from >= 64);
+    if (to - from < 64)
+        for (int v = from; v <= to; ++v) ptr[v] = i;
+    while (wide) {
+        const int l = (int)__builtin_ctzll(wide);
+        wide &= wide - 1;
+        const int f = __shfl(from, l), t = __shfl(to, l), x = __shfl(i, l);
+        for (int v = f + (int)(threadIdx.x & 63); v <= t; v += 64) ptr[v] = x;
+    }
+}
+
+template <typename K>
+__global__ __launch_bounds__(256) void k_key_ptr(const K* __restrict__ keys, long long n,
+                                                 int count, int* __restrict__ ptr) {
+    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    int from = 1, to = 0;  // nothing to write
+    if (i <= n) {
+        from = i == 0 ? 0 : (int)keys[i - 1] + 1;
+        to = i == n ? count : (int)keys[i];
+    }
+    key_ptr_write(from, to, (int)i, ptr);
+}
+
+template <typename K>
+void key_ptr(const K* keys, long long n, int count, int* ptr, hipStream_t st) {
+    hipLaunchKernelGGL((k_key_ptr<K>), dim3(grid_for(n + 1, 256)), dim3(256), 0, st, keys, n, count,
+                       ptr);
     VCSRMC_HIP(hipGetLastError());
 }
 

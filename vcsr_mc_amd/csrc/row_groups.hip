@@ -44,7 +44,8 @@ typedef unsigned long long u64;
 constexpr int kLevels = 4;            // 2^4 = kPanelRows rows per group
 constexpr int kRounds = 8;            // proposal rounds per level
 constexpr int kCand = 4;              // candidates kept per cluster and level
-constexpr int kTable = 1024;          // LDS hash table slots per wave (one cluster)
+constexpr int kTableBits = 10;
+constexpr int kTable = 1 << kTableBits;  // LDS hash table slots per wave (one cluster)
 constexpr int kProbes = 64;           // linear probes per insertion
 constexpr int kMaxCols = 512;         // clusters with more (non-hub) columns take no partner
 constexpr int kInsertsPerLane = 256;  // candidate insertions per lane and cluster
@@ -60,93 +61,111 @@ __device__ __forceinline__ unsigned mix32(unsigned x) {
     return x;
 }
 
-// keys[i] = col << shift | row for every triple.
-__global__ void k_col_major_keys(const int* __restrict__ trow, const int* __restrict__ tcol,
-                                 long long n, int shift, u64* __restrict__ key) {
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The largest of 64 values (and each lane's own value back): DPP scans, no LDS.
+__device__ __forceinline__ u64 wave_max_u64(u64 x) {
+    const int hi = (int)(unsigned)(x >> 32);  // below 2^31 (the count has 13 bits)
+    const int top = __builtin_amdgcn_readlane(wave_scan(hi, OpMax{}, INT_MIN), 63);
+    const int lo = hi == top ? (int)((unsigned)x ^ 0x80000000u) : INT_MIN;
+    const int low = __builtin_amdgcn_readlane(wave_scan(lo, OpMax{}, INT_MIN), 63);
+    return ((u64)(unsigned)top << 32) | ((unsigned)low ^ 0x80000000u);
+}
+
+__global__ void k_col_degrees(const int* __restrict__ col, long long n, int* __restrict__ deg) {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) key[i] = ((u64)tcol[i] << shift) | (u64)trow[i];
+    if (i < n) atomicAdd(&deg[col[i]], 1);
 }
 
-// ptr[v] = the first index of sorted `keys` whose key >> shift is >= v, for v in [0, count].
-__global__ void k_lower_bounds(const u64* __restrict__ keys, long long n, int shift, int count,
-                               int* __restrict__ ptr) {
-    const long long v = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (v > count) return;
-    long long lo = 0, hi = n;
-    while (lo < hi) {
-        const long long mid = (lo + hi) >> 1;
-        if ((long long)(keys[mid] >> shift) < v) lo = mid + 1;
-        else hi = mid;
-    }
-    ptr[v] = (int)lo;
+__global__ void k_any_hub(const int* __restrict__ deg, int N, int hub, int* __restrict__ any) {
+    const long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (c < N && deg[c] > hub) *any = 1;
 }
 
-// Level-0 cluster-column keys (row << cbits | col) of the triples whose column is not a hub.
-__global__ void k_keep_flags(const int* __restrict__ tcol, const int* __restrict__ cptr,
+// The entries whose column is not a hub.
+__global__ void k_keep_flags(const int* __restrict__ col, const int* __restrict__ deg,
                              long long n, int hub, int* __restrict__ keep) {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int c = tcol[i];
-    keep[i] = (cptr[c + 1] - cptr[c]) <= hub;
+    if (i < n) keep[i] = deg[col[i]] <= hub;
 }
 
-__global__ void k_keep_keys(const int* __restrict__ trow, const int* __restrict__ tcol,
-                            const int* __restrict__ keep, const int* __restrict__ at, long long n,
-                            int cbits, u64* __restrict__ key) {
+__global__ void k_keep_write(const int* __restrict__ row_of, const int* __restrict__ col,
+                             const int* __restrict__ keep, const int* __restrict__ at, long long n,
+                             uint32_t* __restrict__ kcol, uint32_t* __restrict__ krow) {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n && keep[i]) key[at[i]] = ((u64)trow[i] << cbits) | (u64)tcol[i];
+    if (i < n && keep[i]) {
+        kcol[at[i]] = (uint32_t)col[i];
+        krow[at[i]] = (uint32_t)row_of[i];
+    }
 }
 
-// Column-major copy of cluster-column keys: (cluster << cbits | col) -> (col << clbits | cluster).
-__global__ void k_transpose_keys(const u64* __restrict__ in, long long n, int cbits, int clbits,
-                                 u64* __restrict__ out) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const u64 k = in[i];
-    out[i] = ((k & ((1ull << cbits) - 1)) << clbits) | (k >> cbits);
+// ptr[v] = entries before row v that were kept (rp[v] of them existed).
+__global__ void k_keep_ptr(const int* __restrict__ rp, const int* __restrict__ at, int M,
+                           int* __restrict__ ptr) {
+    const long long v = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (v <= M) ptr[v] = at[rp[v]];
 }
 
 // One wave per cluster a: counts, in an LDS hash table, how many of a's columns each other
 // cluster b holds, then keeps the kCand best b with size(a) + size(b) <= maxsz (see the file
 // comment for the order).  cand[a * kCand + i] = b, or -1.
-__global__ __launch_bounds__(256) void k_score(const u64* __restrict__ crk,
+// Issue slots bound it: a 27-point stencil inserts 27 x 27 candidates a row and finds 125
+// clusters.  So a column's list is shared by as many lanes as its cluster's columns leave idle,
+// its entries are loaded four at a time ahead of the insertions, and the table is squeezed to its
+// filled slots before any of them is scored.  Scoring all 1024 slots, a lane a column and an
+// entry at a time, the four levels of the stencil 100^3 took 10.9 ms; now 4.4.
+__global__ __launch_bounds__(256) void k_score(const uint32_t* __restrict__ ccol,
                                                const int* __restrict__ cr_ptr,
-                                               const u64* __restrict__ rck,
-                                               const int* __restrict__ rc_ptr, int cbits,
-                                               int clbits, const int* __restrict__ size,
+                                               const uint32_t* __restrict__ rcl,
+                                               const int* __restrict__ rc_ptr,
+                                               const int* __restrict__ size,
                                                const int* __restrict__ cmin, int nc, int maxsz,
-                                               bool far, int* __restrict__ cand) {
-    __shared__ int tkey[4][kTable];
-    __shared__ int tcnt[4][kTable];
+                                               bool far, int4* __restrict__ cand) {
+    __shared__ __attribute__((aligned(16))) int tkey[4][kTable];
+    __shared__ __attribute__((aligned(16))) int tcnt[4][kTable];
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const long long a = (long long)blockIdx.x * 4 + w;
-    if (a >= nc) return;  // the whole wave
+    const long long wa = (long long)blockIdx.x * 4 + w;
+    if (wa >= nc) return;  // the whole wave
+    const int a = __builtin_amdgcn_readfirstlane((int)wa);
     int* K = tkey[w];
     int* Cn = tcnt[w];
-    for (int i = lane; i < kTable; i += 64) {
-        K[i] = -1;
-        Cn[i] = 0;
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     const int b0 = cr_ptr[a], b1 = cr_ptr[a + 1];
     const int sa = size[a];
-    const bool active = (b1 - b0) <= kMaxCols && sa < maxsz;
-    const u64 cmask = (1ull << cbits) - 1, lmask = (1ull << clbits) - 1;
-    if (active) {
-        int inserted = 0;
-        for (int ci = b0 + lane; ci < b1 && inserted < kInsertsPerLane; ci += 64) {
-            const int c = (int)(crk[ci] & cmask);
-            const int r1 = rc_ptr[c + 1];
-            for (int j = rc_ptr[c]; j < r1 && inserted < kInsertsPerLane; ++j) {
-                const int b = (int)(rck[j] & lmask);
-                if (b == (int)a) continue;
+    const int ncol = b1 - b0;
+    static_assert(kCand == 4, "candidates are stored as one int4");
+    if (ncol > kMaxCols || ncol == 0 || sa >= maxsz) {
+        if (lane == 0) cand[a] = make_int4(-1, -1, -1, -1);
+        return;
+    }
+    for (int i = lane * 4; i < kTable; i += 256) {
+        *reinterpret_cast<int4*>(K + i) = make_int4(-1, -1, -1, -1);
+        *reinterpret_cast<int4*>(Cn + i) = make_int4(0, 0, 0, 0);
+    }
+    wave_sync();
+    int sh = 0;  // 2^sh lanes share a column
+    while ((ncol << (sh + 1)) <= 64) ++sh;
+    const int S = 1 << sh;
+    int inserted = 0;
+    for (int ci = b0 + (lane >> sh); ci < b1 && inserted < kInsertsPerLane; ci += 64 >> sh) {
+        const int c = (int)ccol[ci];
+        const int r1 = rc_ptr[c + 1];
+        for (int j = rc_ptr[c] + (lane & (S - 1)); j < r1 && inserted < kInsertsPerLane;
+             j += 4 * S) {
+            int b[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) b[q] = j + q * S < r1 ? (int)rcl[j + q * S] : a;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                if (b[q] == a) continue;
                 ++inserted;
-                unsigned h = mix32((unsigned)b) & (kTable - 1);
+                unsigned h = ((unsigned)b[q] * 0x9e3779b1u) >> (32 - kTableBits);
                 for (int p = 0; p < kProbes; ++p) {
-                    const int prev = atomicCAS(&K[h], -1, b);
-                    if (prev == -1 || prev == b) {
+                    const int prev = atomicCAS(&K[h], -1, b[q]);
+                    if (prev == -1 || prev == b[q]) {
                         atomicAdd(&Cn[h], 1);
                         break;
                     }
@@ -155,62 +174,73 @@ __global__ __launch_bounds__(256) void k_score(const u64* __restrict__ crk,
             }
         }
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    // Score keys of this lane's slots: shared columns, phase, nearness, hash.
-    u64 score[kTable / 64];
-    const int ma = cmin[a];
-#pragma unroll
+    wave_sync();
+    // The filled slots, in slot order, to the table's front: slot group s goes to places at or
+    // before its own, which have been read.
+    int nd = 0;
+    const u64 below = lane ? (~0ull >> (64 - lane)) : 0ull;
     for (int s = 0; s < kTable / 64; ++s) {
-        const int slot = lane + 64 * s;
-        const int b = K[slot];
-        u64 key = 0;
-        if (active && b >= 0 && sa + size[b] <= maxsz) {
-            const int mb = cmin[b];
-            const int lo = min(ma, mb), d = max(ma, mb) - lo;  // d >= 1: distinct first rows
-            const u64 cnt = (u64)min(Cn[slot], 8191);
-            const u64 phase = ((lo / d) & 1) == 0;
-            const u64 near = far ? (u64)d : (u64)(0x7fffffff - d);
-            const u64 tie = mix32((unsigned)min((int)a, b) * 0x9e3779b9u ^ (unsigned)max((int)a, b)) &
-                            0x3ffffu;
-            key = (cnt << 50) | (phase << 49) | (near << 18) | tie;
+        const int k = K[lane + 64 * s], n = Cn[lane + 64 * s];
+        const u64 filled = __ballot(k >= 0);
+        wave_sync();
+        if (k >= 0) {
+            const int at = nd + __popcll(filled & below);
+            K[at] = k;
+            Cn[at] = n;
         }
-        score[s] = key;
+        nd += __popcll(filled);
+        wave_sync();
     }
-    // kCand rounds of a wave-wide maximum; the winner's lane clears that slot.
+    // Score keys: shared columns, phase, nearness, hash; each lane keeps its kCand best.
+    u64 best[kCand];
+    int who[kCand];
+#pragma unroll
+    for (int i = 0; i < kCand; ++i) {
+        best[i] = 0;
+        who[i] = -1;
+    }
+    const int ma = cmin[a];
+    for (int e = lane; e < nd; e += 64) {
+        int b = K[e];
+        if (sa + size[b] > maxsz) continue;
+        const int mb = cmin[b];
+        const int lo = min(ma, mb), d = max(ma, mb) - lo;  // d >= 1: distinct first rows
+        const u64 cnt = (u64)min(Cn[e], 8191);
+        const u64 phase = ((lo / d) & 1) == 0;
+        const u64 near = far ? (u64)d : (u64)(0x7fffffff - d);
+        const u64 tie =
+            mix32((unsigned)min(a, b) * 0x9e3779b9u ^ (unsigned)max(a, b)) & 0x3ffffu;
+        u64 key = (cnt << 50) | (phase << 49) | (near << 18) | tie;
+#pragma unroll
+        for (int i = 0; i < kCand; ++i) {
+            const bool up = key > best[i];
+            const u64 k = up ? best[i] : key;
+            const int x = up ? who[i] : b;
+            best[i] = up ? key : best[i];
+            who[i] = up ? b : who[i];
+            key = k;
+            b = x;
+        }
+    }
+    // kCand rounds of a wave-wide maximum; the lanes holding it move to their next.  Keys of two
+    // candidates tie only if their nearness, phase and 18-bit pair hash all agree, and then the
+    // lowest lane's candidate is kept and the other dropped.
+    int out[kCand];
+#pragma unroll
     for (int r = 0; r < kCand; ++r) {
-        u64 m = 0;
-        int ms = -1;
+        const u64 top = wave_max_u64(best[0]);
+        const u64 own = __ballot(best[0] == top);
+        out[r] = top ? __builtin_amdgcn_readlane(who[0], (int)__builtin_ctzll(own)) : -1;
+        if (best[0] == top) {
 #pragma unroll
-        for (int s = 0; s < kTable / 64; ++s)
-            if (score[s] > m) {
-                m = score[s];
-                ms = s;
+            for (int i = 0; i + 1 < kCand; ++i) {
+                best[i] = best[i + 1];
+                who[i] = who[i + 1];
             }
-        u64 best = m;
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-            const unsigned lo = __shfl_xor((unsigned)(best & 0xffffffffu), off);
-            const unsigned hi = __shfl_xor((unsigned)(best >> 32), off);
-            const u64 o = ((u64)hi << 32) | lo;
-            best = o > best ? o : best;
+            best[kCand - 1] = 0;
         }
-        int b = -1;
-        if (best != 0 && m == best && ms >= 0) {
-            // a lane holding the maximum; keys of two candidates tie only if their nearness,
-            // phase and 18-bit pair hash all agree, and then the lowest lane's candidate is kept
-            // and the other dropped
-            b = K[lane + 64 * ms];
-#pragma unroll
-            for (int s = 0; s < kTable / 64; ++s)
-                if (s == ms) score[s] = 0;
-        }
-        const unsigned long long own = __ballot(b >= 0);
-        int chosen = -1;
-        if (own) chosen = __shfl(b, (int)__builtin_ctzll(own));
-        if (lane == 0) cand[a * kCand + r] = chosen;
     }
+    if (lane == 0) cand[a] = make_int4(out[0], out[1], out[2], out[3]);
 }
 
 // A cluster still unmatched proposes to its first candidate that is unmatched too.
@@ -248,7 +278,7 @@ __global__ void k_rep_flags(const int* __restrict__ mate, int nc, int* __restric
 __global__ void k_relabel(const int* __restrict__ mate, const int* __restrict__ nid,
                           const int* __restrict__ size, const int* __restrict__ cmin, int nc,
                           int* __restrict__ newcl, int* __restrict__ nsize,
-                          int* __restrict__ ncmin) {
+                          int* __restrict__ ncmin, int2* __restrict__ parts) {
     const long long a = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (a >= nc) return;
     const int m = mate[a];
@@ -257,6 +287,7 @@ __global__ void k_relabel(const int* __restrict__ mate, const int* __restrict__ 
     if (rep == (int)a) {
         nsize[nid[a]] = size[a] + (m >= 0 ? size[m] : 0);
         ncmin[nid[a]] = m >= 0 ? min(cmin[a], cmin[m]) : cmin[a];
+        parts[nid[a]] = make_int2((int)a, m);
     }
 }
 
@@ -265,23 +296,85 @@ __global__ void k_relabel_rows(const int* __restrict__ newcl, int M, int* __rest
     if (r < M) rowcl[r] = newcl[rowcl[r]];
 }
 
-__global__ void k_relabel_keys(const u64* __restrict__ in, long long n, int cbits,
-                               const int* __restrict__ newcl, u64* __restrict__ out) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const u64 k = in[i];
-    out[i] = ((u64)newcl[k >> cbits] << cbits) | (k & ((1ull << cbits) - 1));
+// Elements of the ascending v[lo, hi) below x.
+__device__ __forceinline__ int below_in(const uint32_t* __restrict__ v, int lo, int hi,
+                                        uint32_t x) {
+    const int first = lo;
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (v[mid] < x) lo = mid + 1;
+        else hi = mid;
+    }
+    return lo - first;
 }
 
-__global__ void k_head_flags(const u64* __restrict__ k, long long n, int* __restrict__ head) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) head[i] = (i == 0) || k[i] != k[i - 1];
+// Column lists of the merged clusters, one wave each: the union of its parts' ascending lists, by
+// rank (an element's place is its index plus the other list's elements before it, less the common
+// ones before it), not by sorting all of them again.  k_union_sizes counts, k_union_write writes.
+__global__ __launch_bounds__(256) void k_union_sizes(const int2* __restrict__ parts,
+                                                     const int* __restrict__ ptr,
+                                                     const uint32_t* __restrict__ ccol, int nnc,
+                                                     int* __restrict__ len) {
+    const int x = (int)(((long long)blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+    const int lane = threadIdx.x & 63;
+    if (x >= nnc) return;  // the whole wave
+    const int2 p = parts[x];
+    const int a0 = ptr[p.x], a1 = ptr[p.x + 1];
+    int total = a1 - a0;
+    if (p.y >= 0) {
+        const int b0 = ptr[p.y], b1 = ptr[p.y + 1];
+        total += b1 - b0;
+        for (int j0 = b0; j0 < b1; j0 += 64) {
+            bool common = false;
+            if (j0 + lane < b1) {
+                const uint32_t c = ccol[j0 + lane];
+                const int at = a0 + below_in(ccol, a0, a1, c);
+                common = at < a1 && ccol[at] == c;
+            }
+            total -= __popcll(__ballot(common));
+        }
+    }
+    if (lane == 0) len[x] = total;
 }
 
-__global__ void k_compact_keys(const u64* __restrict__ in, const int* __restrict__ head,
-                               const int* __restrict__ at, long long n, u64* __restrict__ out) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n && head[i]) out[at[i]] = in[i];
+__global__ __launch_bounds__(256) void k_union_write(const int2* __restrict__ parts,
+                                                     const int* __restrict__ ptr,
+                                                     const uint32_t* __restrict__ ccol,
+                                                     const int* __restrict__ nptr, int nnc,
+                                                     uint32_t* __restrict__ ncol,
+                                                     uint32_t* __restrict__ ncl) {
+    const int x = (int)(((long long)blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+    const int lane = threadIdx.x & 63;
+    if (x >= nnc) return;  // the whole wave
+    const u64 below = lane ? (~0ull >> (64 - lane)) : 0ull;
+    const int2 p = parts[x];
+    const int out = nptr[x];
+#pragma unroll
+    for (int side = 0; side < 2; ++side) {
+        const int me = side ? p.y : p.x, other = side ? p.x : p.y;
+        if (me < 0) break;
+        const int a0 = ptr[me], a1 = ptr[me + 1];
+        const int b0 = other >= 0 ? ptr[other] : 0, b1 = other >= 0 ? ptr[other + 1] : 0;
+        int common_before = 0;
+        for (int i0 = a0; i0 < a1; i0 += 64) {
+            const int i = i0 + lane;
+            bool common = false;
+            int at = 0;
+            uint32_t c = 0;
+            if (i < a1) {
+                c = ccol[i];
+                at = below_in(ccol, b0, b1, c);
+                common = b0 + at < b1 && ccol[b0 + at] == c;
+            }
+            const u64 m = __ballot(common);
+            if (i < a1 && !(side && common)) {
+                const int dst = out + (i - a0) + at - common_before - __popcll(m & below);
+                ncol[dst] = c;
+                ncl[dst] = (uint32_t)x;
+            }
+            common_before += __popcll(m);
+        }
+    }
 }
 
 __global__ void k_init_clusters(int M, int* __restrict__ rowcl, int* __restrict__ size,
@@ -323,12 +416,6 @@ __global__ void k_positions(const uint32_t* __restrict__ order, int M, int P,
     }
 }
 
-void sort_keys(TmpBuf<u64>& keys, TmpBuf<u64>& alt, long long n, int bits, hipStream_t st) {
-    u64 *k = keys.p, *ka = alt.p;
-    radix_sort_keys<u64>(k, ka, n, bits, st);
-    if (k != keys.p) std::swap(keys, alt);  // an odd number of passes
-}
-
 __global__ void k_flag_rows(const int* __restrict__ trow, long long n, int* __restrict__ flag) {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) flag[trow[i]] = 1;
@@ -367,75 +454,76 @@ bool compact_rows(const int* trow, long long n, int M, hipStream_t st, TmpBuf<in
     return true;
 }
 
-bool group_rows(const int* trow, const int* tcol, long long n, int M, int N, hipStream_t st,
-                TmpBuf<int>& rowpos, DevBuf<int>& row_map) {
+bool group_rows(const int* rp, const int* row_of, const int* col, long long n, int M, int N,
+                hipStream_t st, TmpBuf<int>& rowpos, DevBuf<int>& row_map) {
     if (M < 2 * kPanelRows || N < 1 || n < 1) return false;
-    const int rbits = bits_for((unsigned long long)(M - 1));
     const int cbits = bits_for((unsigned long long)(N - 1));
     const int hub = (int)std::max<long long>(32, std::min<long long>(1024, 4 * n / N));
 
-    // Column degrees from the column-major order of the triples.
-    TmpBuf<u64> keys(n), alt(n);
-    TmpBuf<int> cptr((size_t)N + 1);
-    hipLaunchKernelGGL(k_col_major_keys, dim3(grid256(n)), dim3(256), 0, st, trow, tcol, n, rbits,
-                       keys.p);
-    VCSRMC_HIP(hipGetLastError());
-    sort_keys(keys, alt, n, cbits + rbits, st);
-    hipLaunchKernelGGL(k_lower_bounds, dim3(grid256((long long)N + 1)), dim3(256), 0, st, keys.p,
-                       n, rbits, N, cptr.p);
-    VCSRMC_HIP(hipGetLastError());
-
-    // Level-0 cluster-column keys: the triples on columns of at most `hub` rows.
-    long long np;
+    // Level-0 clusters are the rows, without the columns of more than `hub` rows.  A cluster's
+    // columns: cl_col (ascending) in [ptr[cluster], ptr[cluster + 1]), cl_of the cluster of each.
+    TmpBuf<uint32_t> cl_col, cl_of;
+    TmpBuf<int> cl_ptr;
+    const uint32_t *ccol = reinterpret_cast<const uint32_t*>(col),
+                   *cof = reinterpret_cast<const uint32_t*>(row_of);
+    const int* ptr = rp;
+    long long np = n;
     {
-        TmpBuf<int> keep(n), at((size_t)n + 1);
-        hipLaunchKernelGGL(k_keep_flags, dim3(grid256(n)), dim3(256), 0, st, tcol, cptr.p, n, hub,
-                           keep.p);
+        TmpBuf<int> deg((size_t)N + 1);
+        fill<int>(deg.p, (long long)N + 1, 0, st);
+        hipLaunchKernelGGL(k_col_degrees, dim3(grid256(n)), dim3(256), 0, st, col, n, deg.p);
         VCSRMC_HIP(hipGetLastError());
-        exclusive_sum<int, int>(keep.p, at.p, n, st);
-        np = read_scalar(at.p + n, st);
-        hipLaunchKernelGGL(k_keep_keys, dim3(grid256(n)), dim3(256), 0, st, trow, tcol, keep.p,
-                           at.p, n, cbits, keys.p);
+        hipLaunchKernelGGL(k_any_hub, dim3(grid256(N)), dim3(256), 0, st, deg.p, N, hub,
+                           deg.p + N);
         VCSRMC_HIP(hipGetLastError());
+        if (read_scalar(deg.p + N, st)) {
+            TmpBuf<int> keep(n), at((size_t)n + 1);
+            hipLaunchKernelGGL(k_keep_flags, dim3(grid256(n)), dim3(256), 0, st, col, deg.p, n,
+                               hub, keep.p);
+            VCSRMC_HIP(hipGetLastError());
+            exclusive_sum<int, int>(keep.p, at.p, n, st);
+            np = read_scalar(at.p + n, st);
+            if (np == 0) return false;
+            cl_col.alloc(np);
+            cl_of.alloc(np);
+            cl_ptr.alloc((size_t)M + 1);
+            hipLaunchKernelGGL(k_keep_write, dim3(grid256(n)), dim3(256), 0, st, row_of, col,
+                               keep.p, at.p, n, cl_col.p, cl_of.p);
+            VCSRMC_HIP(hipGetLastError());
+            hipLaunchKernelGGL(k_keep_ptr, dim3(grid256((long long)M + 1)), dim3(256), 0, st, rp,
+                               at.p, M, cl_ptr.p);
+            VCSRMC_HIP(hipGetLastError());
+            ccol = cl_col.p;
+            cof = cl_of.p;
+            ptr = cl_ptr.p;
+        }
     }
-    if (np == 0) return false;
-    sort_keys(keys, alt, np, rbits + cbits, st);
 
     int nc = M;
     TmpBuf<int> rowcl(M), size(M), cmin(M);
     hipLaunchKernelGGL(k_init_clusters, dim3(grid256(M)), dim3(256), 0, st, M, rowcl.p, size.p,
                        cmin.p);
     VCSRMC_HIP(hipGetLastError());
-    TmpBuf<u64> rck(np), rca(np);
     for (int level = 0; level < kLevels; ++level) {
-        const int clbits = bits_for((unsigned long long)(nc - 1));
-        // cluster -> columns (keys, sorted) and column -> clusters
-        TmpBuf<int> cr_ptr((size_t)nc + 1), rc_ptr((size_t)N + 1);
-        hipLaunchKernelGGL(k_lower_bounds, dim3(grid256((long long)nc + 1)), dim3(256), 0, st,
-                           keys.p, np, cbits, nc, cr_ptr.p);
-        VCSRMC_HIP(hipGetLastError());
-        hipLaunchKernelGGL(k_transpose_keys, dim3(grid256(np)), dim3(256), 0, st, keys.p, np,
-                           cbits, clbits, rck.p);
-        VCSRMC_HIP(hipGetLastError());
-        {
-            u64 *k = rck.p, *ka = rca.p;
-            radix_sort_keys<u64>(k, ka, np, cbits + clbits, st);
-            if (k != rck.p) std::swap(rck, rca);
-        }
-        hipLaunchKernelGGL(k_lower_bounds, dim3(grid256((long long)N + 1)), dim3(256), 0, st,
-                           rck.p, np, clbits, N, rc_ptr.p);
-        VCSRMC_HIP(hipGetLastError());
+        // column -> clusters, ascending: the entries stably sorted by column
+        TmpBuf<uint32_t> k1(np), k2(np), v1(np), v2(np);
+        TmpBuf<int> rc_ptr((size_t)N + 1);
+        const auto [scol, rcl] = radix_sort_pairs_from<uint32_t>(ccol, cof, k1.p, v1.p, k2.p, v2.p,
+                                                                 np, std::max(1, cbits), st);
+        key_ptr<uint32_t>(scol, np, N, rc_ptr.p, st);
 
         const int maxsz = 2 << level;  // clusters of 2^level rows pair into 2^(level+1)
-        TmpBuf<int> cand((size_t)nc * kCand), mate(nc), prop(nc);
-        hipLaunchKernelGGL(k_score, dim3(grid_for(nc, 4)), dim3(256), 0, st, keys.p, cr_ptr.p,
-                           rck.p, rc_ptr.p, cbits, clbits, size.p, cmin.p, nc, maxsz,
-                           level == kLevels - 1, cand.p);
+        TmpBuf<int4> cand(nc);
+        TmpBuf<int> mate(nc), prop(nc);
+        hipLaunchKernelGGL(k_score, dim3(grid_for(nc, 4)), dim3(256), 0, st, ccol, ptr, rcl,
+                           rc_ptr.p, size.p, cmin.p, nc, maxsz, level == kLevels - 1, cand.p);
         VCSRMC_HIP(hipGetLastError());
+        k1.release(); k2.release(); v1.release(); v2.release();
         fill<int>(mate.p, nc, -1, st);
+        const int* candidates = reinterpret_cast<const int*>(cand.p);
         for (int round = 0; round < kRounds; ++round) {
-            hipLaunchKernelGGL(k_propose, dim3(grid256(nc)), dim3(256), 0, st, cand.p, mate.p, nc,
-                               prop.p);
+            hipLaunchKernelGGL(k_propose, dim3(grid256(nc)), dim3(256), 0, st, candidates, mate.p,
+                               nc, prop.p);
             VCSRMC_HIP(hipGetLastError());
             hipLaunchKernelGGL(k_accept, dim3(grid256(nc)), dim3(256), 0, st, prop.p, nc, mate.p);
             VCSRMC_HIP(hipGetLastError());
@@ -447,32 +535,32 @@ bool group_rows(const int* trow, const int* tcol, long long n, int M, int N, hip
         const int nnc = read_scalar(nid.p + nc, st);
         if (nnc == nc) break;  // nothing merged at this level: none will at the next
         TmpBuf<int> newcl(nc), nsize(nnc), ncmin(nnc);
+        TmpBuf<int2> parts(nnc);
         hipLaunchKernelGGL(k_relabel, dim3(grid256(nc)), dim3(256), 0, st, mate.p, nid.p, size.p,
-                           cmin.p, nc, newcl.p, nsize.p, ncmin.p);
+                           cmin.p, nc, newcl.p, nsize.p, ncmin.p, parts.p);
         VCSRMC_HIP(hipGetLastError());
         hipLaunchKernelGGL(k_relabel_rows, dim3(grid256(M)), dim3(256), 0, st, newcl.p, M,
                            rowcl.p);
         VCSRMC_HIP(hipGetLastError());
         size = std::move(nsize);
         cmin = std::move(ncmin);
-        // the merged clusters' column sets: relabel, sort, drop repeats
-        hipLaunchKernelGGL(k_relabel_keys, dim3(grid256(np)), dim3(256), 0, st, keys.p, np, cbits,
-                           newcl.p, alt.p);
-        VCSRMC_HIP(hipGetLastError());
-        std::swap(keys, alt);
-        const int nclbits = bits_for((unsigned long long)(nnc - 1));
-        sort_keys(keys, alt, np, nclbits + cbits, st);
-        {
-            TmpBuf<int> head(np), at((size_t)np + 1);
-            hipLaunchKernelGGL(k_head_flags, dim3(grid256(np)), dim3(256), 0, st, keys.p, np,
-                               head.p);
+        if (level + 1 < kLevels) {
+            TmpBuf<int> len(nnc), nptr((size_t)nnc + 1);
+            hipLaunchKernelGGL(k_union_sizes, dim3(grid_for(nnc, 4)), dim3(256), 0, st, parts.p,
+                               ptr, ccol, nnc, len.p);
             VCSRMC_HIP(hipGetLastError());
-            exclusive_sum<int, int>(head.p, at.p, np, st);
-            const long long nu = read_scalar(at.p + np, st);
-            hipLaunchKernelGGL(k_compact_keys, dim3(grid256(np)), dim3(256), 0, st, keys.p, head.p,
-                               at.p, np, alt.p);
+            exclusive_sum<int, int>(len.p, nptr.p, nnc, st);
+            const long long nu = read_scalar(nptr.p + nnc, st);
+            TmpBuf<uint32_t> ncol(nu), ncl(nu);
+            hipLaunchKernelGGL(k_union_write, dim3(grid_for(nnc, 4)), dim3(256), 0, st, parts.p,
+                               ptr, ccol, nptr.p, nnc, ncol.p, ncl.p);
             VCSRMC_HIP(hipGetLastError());
-            std::swap(keys, alt);
+            cl_col = std::move(ncol);
+            cl_of = std::move(ncl);
+            cl_ptr = std::move(nptr);
+            ccol = cl_col.p;
+            cof = cl_of.p;
+            ptr = cl_ptr.p;
             np = nu;
         }
         nc = nnc;
@@ -482,7 +570,7 @@ bool group_rows(const int* trow, const int* tcol, long long n, int M, int N, hip
     const int P = ((M + kPanelRows - 1) / kPanelRows) * kPanelRows;
     TmpBuf<unsigned char> has(M);
     fill<unsigned char>(has.p, M, 0, st);
-    hipLaunchKernelGGL(k_has_nonzero, dim3(grid256(n)), dim3(256), 0, st, trow, n, has.p);
+    hipLaunchKernelGGL(k_has_nonzero, dim3(grid256(n)), dim3(256), 0, st, row_of, n, has.p);
     VCSRMC_HIP(hipGetLastError());
     TmpBuf<uint32_t> okey(M), oalt(M), opay(M), opalt(M);
     hipLaunchKernelGGL(k_order_keys, dim3(grid256(M)), dim3(256), 0, st, rowcl.p, cmin.p, has.p,
