@@ -17,6 +17,7 @@
 #include <climits>
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/vcsrmc.h"
@@ -260,121 +261,351 @@ __global__ void k_gather_items(const uint32_t* __restrict__ spay, const int* __r
     gend[i] = ie[spay[i]];
 }
 
-__global__ void k_scale_values(const float* __restrict__ v, float* __restrict__ out, long long n,
-                               float inv_scale) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] = v[i] * inv_scale;
-}
-
 // ------------------------------------------------------------------------------------------
-// Part 2: execution layout from triples (row, col, value already divided by the scale).
+// Part 2: execution layout from a CSR with ascending columns.
 // ------------------------------------------------------------------------------------------
-// Rows are placed at positions (rowpos[row], or the row itself in natural order); a panel is 16
-// consecutive positions.
-template <typename K>
-__global__ void k_panel_keys(const int* __restrict__ trow, const int* __restrict__ tcol,
-                             const int* __restrict__ rowpos, long long n, int cbits,
-                             K* __restrict__ key, uint32_t* __restrict__ pay) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int r = rowpos ? rowpos[trow[i]] : trow[i];
-    key[i] = ((K)(r >> 4) << (cbits + 4)) | ((K)tcol[i] << 4) | (K)(r & 15);
-    pay[i] = (uint32_t)i;
-}
-
-template <typename K>
-__global__ void k_panel_heads(const K* __restrict__ skey, long long n, int cbits,
-                              int* __restrict__ hdist, int* __restrict__ hpanel,
-                              int* __restrict__ err) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const K k = skey[i];
-    int hd = 1, hp = 1;
-    if (i > 0) {
-        const K prev = skey[i - 1];
-        if (prev == k) atomicOr(err, kErrDuplicate);
-        hd = (prev >> 4) != (k >> 4);
-        hp = (prev >> (cbits + 4)) != (k >> (cbits + 4));
+// Rows are placed at positions (row_map[position] = row, or the row itself in natural order); a
+// panel is 16 consecutive positions, its nonzeros (row, column) the rows' CSR runs.  `at` holds
+// the nonzeros before each position (natural order: the row pointer itself).
+struct Positions {
+    const int* rp;
+    const int* row_map;  // null: natural order
+    const int* at;       // with a row map: P + 1 entries, P = M rounded up to 16
+    int M;
+    __device__ __forceinline__ int begin(int p) const { return at ? at[p] : rp[min(p, M)]; }
+    // first nonzero of the row at position p (any value where the position holds none)
+    __device__ __forceinline__ int row_begin(int p) const {
+        if (!row_map) return rp[min(p, M)];
+        const int r = row_map[p];
+        return r < 0 ? 0 : rp[r];
     }
-    hdist[i] = hd;
-    hpanel[i] = hp;
+};
+
+__global__ void k_position_lens(const int* __restrict__ rp, const int* __restrict__ row_map, int P,
+                                int* __restrict__ len) {
+    const long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (p >= P) return;
+    const int r = row_map[p];
+    len[p] = r < 0 ? 0 : rp[r + 1] - rp[r];
 }
 
-template <typename K>
-__global__ void k_panel_starts(const K* __restrict__ skey, const int* __restrict__ hpanel,
-                               const int* __restrict__ pin, long long n, int cbits,
-                               int* __restrict__ pstart, int* __restrict__ ppanel) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    if (hpanel[i]) {
-        const int j = pin[i] - 1;
-        pstart[j] = (int)i;
-        ppanel[j] = (int)(skey[i] >> (cbits + 4));
-    }
-}
+// Panels by size, one thread each: the largest that one work-group sorts in LDS as a small
+// (kSortSmall) or a middle (kSortMid) one; the others are sorted through memory.  counts = {middle,
+// large}.  Also the panel's mask of non-empty rows, and its distinct columns set to 0.
+constexpr int kSortSmall = 1024, kSortMid = 8192;
 
-__global__ void k_panel_chunks(const int* __restrict__ pstart, const int* __restrict__ dc, int NP,
-                               int* __restrict__ nch) {
+__global__ void k_panel_classes(Positions pos, int panels, int* __restrict__ pmask,
+                                int* __restrict__ ndist, int* __restrict__ mid,
+                                int* __restrict__ big, int* __restrict__ big_size,
+                                int* __restrict__ counts) {
     const long long j = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= NP) return;
-    const int ndist = dc[pstart[j + 1] - 1] - dc[pstart[j]] + 1;
-    nch[j] = (ndist + kChunkCols - 1) / kChunkCols;
-}
-
-template <typename K, bool FP32>
-__global__ void k_panel_entries(const K* __restrict__ skey, const uint32_t* __restrict__ spay,
-                                const int* __restrict__ hdist, const int* __restrict__ dc,
-                                const int* __restrict__ pin, const int* __restrict__ pstart,
-                                const int* __restrict__ cbase, const int* __restrict__ tcol,
-                                const float* __restrict__ tval, long long n,
-                                uint32_t* __restrict__ entries, int* __restrict__ chunk_cols,
-                                int* __restrict__ chunk_eptr, int* __restrict__ echunk) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int j = pin[i] - 1;
-    const int lr = dc[i] - dc[pstart[j]];
-    const int c = cbase[j] + lr / kChunkCols;
-    const int k = lr % kChunkCols;
-    const int r16 = (int)(skey[i] & 15);
-    const uint32_t src = spay[i];
-    echunk[i] = c;
-    const float v = tval[src];
-    if constexpr (FP32) {
-        entries[2 * i] = (uint32_t)r16 | ((uint32_t)k << 4);
-        entries[2 * i + 1] = __float_as_uint(v);
-    } else {
-        const _Float16 h = (_Float16)v;  // v_cvt_f16_f32, round to nearest even
-        entries[i] = (uint32_t)__builtin_bit_cast(unsigned short, h) | ((uint32_t)r16 << 16) |
-                     ((uint32_t)k << 20);
+    if (j >= panels) return;
+    const int p0 = (int)j * kPanelRows;
+    int prev = pos.begin(p0), m = 0;
+    const int first = prev;
+    for (int r = 0; r < kPanelRows; ++r) {
+        const int next = pos.begin(p0 + r + 1);
+        m |= (int)(next > prev) << r;
+        prev = next;
     }
-    if (hdist[i]) {
-        // FP32 formats keep a tile's columns in K-step order: lane group g of the kernel reads
-        // columns 4 s + g (s = 0..7) as eight consecutive words.
-        const int slot = FP32 ? (k & 3) * 8 + (k >> 2) : k;
-        chunk_cols[(long long)c * kChunkCols + slot] = tcol[src];
-        if (k == 0) chunk_eptr[c] = (int)i;
-    }
-}
-
-// rflag[p] = 1 for every position whose row holds a nonzero (plain stores; every writer stores
-// the same 1).
-__global__ void k_row_flags(const int* __restrict__ trow, const int* __restrict__ rowpos,
-                            long long n, unsigned char* __restrict__ rflag) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) rflag[rowpos ? rowpos[trow[i]] : trow[i]] = 1;
-}
-
-// pmask[j] = the non-empty rows of panel j, from its 16 row flags (one 16-byte load).
-__global__ void k_panel_masks(const unsigned char* __restrict__ rflag,
-                              const int* __restrict__ ppanel, int NP, int* __restrict__ pmask) {
-    const long long j = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= NP) return;
-    const uint4 w = *reinterpret_cast<const uint4*>(rflag + (long long)ppanel[j] * kPanelRows);
-    const uint32_t words[4] = {w.x, w.y, w.z, w.w};
-    int m = 0;
-#pragma unroll
-    for (int b = 0; b < 16; ++b) m |= ((words[b >> 2] >> (8 * (b & 3))) & 1u) << b;
     pmask[j] = m;
+    ndist[j] = 0;
+    const int len = prev - first;
+    if (len > kSortMid) {
+        const int q = atomicAdd(&counts[1], 1);
+        big[q] = (int)j;
+        big_size[q] = len;
+    } else if (len > kSortSmall) {
+        mid[atomicAdd(&counts[0], 1)] = (int)j;
+    }
+}
+
+// The sorted value of a nonzero: the float's bits (FP32), or binary16 (round to nearest even) with
+// the row in the panel above it, as an FP16 entry holds them.
+template <bool FP32>
+__device__ __forceinline__ uint32_t entry_value(float v, int r16) {
+    if constexpr (FP32) return __float_as_uint(v);
+    const _Float16 h = (_Float16)v;
+    return (uint32_t)__builtin_bit_cast(unsigned short, h) | ((uint32_t)r16 << 16);
+}
+
+// Elements of the ascending v[lo, hi) below c (`or_equal`: at most c).
+template <typename T>
+__device__ __forceinline__ int rank_in(const T* v, int lo, int hi, uint32_t c, bool or_equal) {
+    const int first = lo;
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        const uint32_t x = (uint32_t)v[mid];
+        if (x < c || (or_equal && x == c)) lo = mid + 1;
+        else hi = mid;
+    }
+    return lo - first;
+}
+
+// Where the merge of two neighbouring runs of 2^s rows puts the element at index e of row r,
+// column c: its index plus the other run's elements before it (the lower rows' first among equal
+// columns).  off[r]: the panel's elements before row r.
+template <typename T, typename Off>
+__device__ __forceinline__ int merged_place(const T* cols, Off off, int s, int r, int e,
+                                            uint32_t c) {
+    const int g0 = (r >> (s + 1)) << (s + 1);
+    const int lo = off(g0), mid = off(g0 + (1 << s)), hi = off(g0 + (2 << s));
+    if (e < mid) return e + rank_in(cols, mid, hi, c, false);
+    return e - (mid - lo) + rank_in(cols, lo, mid, c, true);
+}
+
+// One panel per work-group: its nonzeros in (column, row) order, and its number of distinct
+// columns.  The 16 rows are sorted already, so four rounds of pairwise merges in LDS, by rank, do
+// it: 16 binary-search steps an element or so, where sorting (panel, column, row) keys of the
+// whole matrix took five passes of counting, scanning and scattering them, twice where rows are
+// grouped.  27-point stencil 100^3, both orders: the keys, sorts and scans 4.0 ms, this 0.77.
+template <int CAP, int T, bool FP32>
+__global__ __launch_bounds__(T) void k_panel_sort(Positions pos, const int* __restrict__ list,
+                                                  const int* __restrict__ col,
+                                                  const float* __restrict__ val, float inv_scale,
+                                                  uint32_t* __restrict__ scol,
+                                                  uint32_t* __restrict__ sval,
+                                                  unsigned char* __restrict__ srow,
+                                                  int* __restrict__ ndist) {
+    __shared__ uint32_t cols[2][CAP], from[2][CAP];  // from: row << 16 | index in row order
+    __shared__ int s_off[kPanelRows + 1], s_row[kPanelRows];
+    __shared__ int distinct;
+    const int t = threadIdx.x;
+    const int j = list ? list[blockIdx.x] : (int)blockIdx.x;
+    const int p0 = j * kPanelRows, first = pos.begin(p0);
+    if (t <= kPanelRows) s_off[t] = pos.begin(p0 + t) - first;
+    if (t < kPanelRows) s_row[t] = pos.row_begin(p0 + t);
+    if (t == 0) distinct = 0;
+    __syncthreads();
+    const int len = s_off[kPanelRows];
+    if (len == 0 || len > CAP) return;  // the whole work-group
+    for (int e = t; e < len; e += T) {
+        int r = 0;  // the last row that starts at or before e
+#pragma unroll
+        for (int step = 8; step > 0; step >>= 1)
+            if (s_off[r + step] <= e) r += step;
+        cols[0][e] = (uint32_t)col[s_row[r] + (e - s_off[r])];
+        from[0][e] = ((uint32_t)r << 16) | (uint32_t)e;
+    }
+    __syncthreads();
+    const auto off = [&](int r) { return s_off[r]; };
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+        const uint32_t* c0 = cols[s & 1];
+        const uint32_t* f0 = from[s & 1];
+        uint32_t* c1 = cols[(s + 1) & 1];
+        uint32_t* f1 = from[(s + 1) & 1];
+        for (int e = t; e < len; e += T) {
+            const uint32_t c = c0[e], f = f0[e];
+            const int dst = merged_place(c0, off, s, (int)(f >> 16), e, c);
+            c1[dst] = c;
+            f1[dst] = f;
+        }
+        __syncthreads();
+    }
+    int heads = 0;
+    for (int e = t; e < len; e += T) {
+        const uint32_t c = cols[0][e], f = from[0][e];
+        heads += e == 0 || cols[0][e - 1] != c;
+        const int r = (int)(f >> 16);
+        const float v = val[s_row[r] + ((int)(f & 0xffffu) - s_off[r])] * inv_scale;
+        scol[first + e] = c;
+        sval[first + e] = entry_value<FP32>(v, r);
+        if constexpr (FP32) srow[first + e] = (unsigned char)r;
+    }
+    heads = wave_last(wave_scan(heads, OpAdd{}, 0));
+    if ((t & 63) == 0) atomicAdd(&distinct, heads);
+    __syncthreads();
+    if (t == 0) ndist[j] = distinct;
+}
+
+// Large panels, laid one after another (bofs), a thread per element: load, four merge rounds
+// through memory, and the sorted elements out.  The large panel of element e: the last one that
+// starts at or before it.
+__device__ __forceinline__ int big_of(const int* __restrict__ bofs, int nbig, long long e) {
+    int lo = 0, hi = nbig - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (bofs[mid] <= e) lo = mid;
+        else hi = mid - 1;
+    }
+    return lo;
+}
+
+__global__ void k_big_load(Positions pos, const int* __restrict__ big, const int* __restrict__ bofs,
+                           int nbig, long long total, const int* __restrict__ col,
+                           uint32_t* __restrict__ bcol, uint32_t* __restrict__ bsrc,
+                           unsigned char* __restrict__ brow) {
+    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= total) return;
+    const int q = big_of(bofs, nbig, i), p0 = big[q] * kPanelRows, first = pos.begin(p0);
+    const int e = (int)(i - bofs[q]);
+    int r = 0;
+    for (int step = 8; step > 0; step >>= 1)
+        if (pos.begin(p0 + r + step) - first <= e) r += step;
+    const int src = pos.row_begin(p0 + r) + e - (pos.begin(p0 + r) - first);
+    bcol[i] = (uint32_t)col[src];
+    bsrc[i] = (uint32_t)src;
+    brow[i] = (unsigned char)r;
+}
+
+__global__ void k_big_merge(Positions pos, const int* __restrict__ big,
+                            const int* __restrict__ bofs, int nbig, long long total, int s,
+                            const uint32_t* __restrict__ bcol, const uint32_t* __restrict__ bsrc,
+                            const unsigned char* __restrict__ brow, uint32_t* __restrict__ ocol,
+                            uint32_t* __restrict__ osrc, unsigned char* __restrict__ orow) {
+    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= total) return;
+    const int q = big_of(bofs, nbig, i), p0 = big[q] * kPanelRows, first = pos.begin(p0);
+    const int base = bofs[q];
+    const auto off = [&](int r) { return pos.begin(p0 + r) - first; };
+    const uint32_t c = bcol[i];
+    const int r = brow[i];
+    const int dst = base + merged_place(bcol + base, off, s, r, (int)(i - base), c);
+    ocol[dst] = c;
+    osrc[dst] = bsrc[i];
+    orow[dst] = (unsigned char)r;
+}
+
+template <bool FP32>
+__global__ void k_big_store(Positions pos, const int* __restrict__ big,
+                            const int* __restrict__ bofs, int nbig, long long total,
+                            const uint32_t* __restrict__ bcol, const uint32_t* __restrict__ bsrc,
+                            const unsigned char* __restrict__ brow, const float* __restrict__ val,
+                            float inv_scale, uint32_t* __restrict__ scol,
+                            uint32_t* __restrict__ sval, unsigned char* __restrict__ srow,
+                            int* __restrict__ ndist) {
+    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    int q = -1;
+    bool head = false;
+    if (i < total) {
+        q = big_of(bofs, nbig, i);
+        const long long out = (long long)pos.begin(big[q] * kPanelRows) + (i - bofs[q]);
+        const uint32_t c = bcol[i];
+        head = i == bofs[q] || bcol[i - 1] != c;
+        const int r = brow[i];
+        scol[out] = c;
+        sval[out] = entry_value<FP32>(val[bsrc[i]] * inv_scale, r);
+        if constexpr (FP32) srow[out] = (unsigned char)r;
+    }
+    // one addition per wave where it holds one panel's elements
+    const int q0 = __builtin_amdgcn_readfirstlane(q);
+    if (__ballot(q != q0) == 0) {
+        const int heads = __popcll(__ballot(head));
+        if (q0 >= 0 && (threadIdx.x & 63) == 0) atomicAdd(&ndist[big[q0]], heads);
+    } else if (head) {
+        atomicAdd(&ndist[big[q]], 1);
+    }
+}
+
+// Tiles of every panel and whether it holds any; their totals in `totals` = {distinct (panel,
+// column) pairs, tiles, non-empty panels, tiles of the largest panel}, by one work-group.
+__global__ void k_panel_tiles(const int* __restrict__ ndist, int panels, int* __restrict__ nch,
+                              int* __restrict__ some) {
+    const long long j = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (j >= panels) return;
+    nch[j] = (ndist[j] + kChunkCols - 1) / kChunkCols;
+    some[j] = ndist[j] > 0;
+}
+
+__global__ __launch_bounds__(1024) void k_panel_totals(const int* __restrict__ ndist, int panels,
+                                                       int4* __restrict__ totals) {
+    __shared__ int part[4];
+    if (threadIdx.x < 4) part[threadIdx.x] = 0;
+    __syncthreads();
+    int pairs = 0, tiles = 0, some = 0, most = 0;
+    for (int j = threadIdx.x; j < panels; j += 1024) {
+        const int d = ndist[j], c = (d + kChunkCols - 1) / kChunkCols;
+        pairs += d;
+        tiles += c;
+        some += d > 0;
+        most = max(most, c);
+    }
+    atomicAdd(&part[0], pairs);
+    atomicAdd(&part[1], tiles);
+    atomicAdd(&part[2], some);
+    atomicMax(&part[3], most);
+    __syncthreads();
+    if (threadIdx.x == 0) *totals = make_int4(part[0], part[1], part[2], part[3]);
+}
+
+// The non-empty panels, in order: panel, first element, first tile, tiles, row mask.
+__global__ void k_panel_compact(Positions pos, const int* __restrict__ nch,
+                                const int* __restrict__ cbase_all, const int* __restrict__ pidx,
+                                const int* __restrict__ pmask_all, int panels, int NP, int NC,
+                                int n, int* __restrict__ ppanel, int* __restrict__ pstart,
+                                int* __restrict__ cbase, int* __restrict__ pch,
+                                int* __restrict__ pmask, int* __restrict__ chunk_eptr) {
+    const long long j = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (j == 0) {
+        pstart[NP] = n;
+        cbase[NP] = NC;
+        chunk_eptr[NC] = n;
+    }
+    if (j >= panels || nch[j] == 0) return;
+    const int i = pidx[j];
+    ppanel[i] = (int)j;
+    pstart[i] = pos.begin((int)j * kPanelRows);
+    cbase[i] = cbase_all[j];
+    pch[i] = nch[j];
+    pmask[i] = pmask_all[j];
+}
+
+// Tiles of one panel per work-group, from its sorted nonzeros: the running number of distinct
+// columns gives each nonzero its tile and column in it.
+template <bool FP32>
+__global__ __launch_bounds__(256) void k_panel_fill(
+    const int* __restrict__ pstart, const int* __restrict__ cbase,
+    const uint32_t* __restrict__ scol, const uint32_t* __restrict__ sval,
+    const unsigned char* __restrict__ srow, uint32_t* __restrict__ entries,
+    int* __restrict__ chunk_cols, int* __restrict__ chunk_eptr) {
+    __shared__ int whead[2][4];
+    const int j = blockIdx.x, t = threadIdx.x, w = t >> 6, lane = t & 63;
+    const int p0 = pstart[j], p1 = pstart[j + 1], c0 = cbase[j];
+    const uint64_t upto = ~0ull >> (63 - lane);
+    int run = 0, phase = 0;  // distinct columns before this round's nonzeros
+    for (int i0 = p0; i0 < p1; i0 += 256, phase ^= 1) {
+        const int i = i0 + t;
+        uint32_t c = 0;
+        bool head = false;
+        if (i < p1) {
+            c = scol[i];
+            head = i == p0 || scol[i - 1] != c;
+        }
+        const uint64_t m = __ballot(head);
+        if (lane == 0) whead[phase][w] = __popcll(m);
+        __syncthreads();
+        int before = run, all = 0;
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+            const int h = whead[phase][x];
+            if (x < w) before += h;
+            all += h;
+        }
+        run += all;
+        if (i < p1) {
+            const int lr = before + __popcll(m & upto) - 1;
+            const int tile = c0 + lr / kChunkCols, k = lr % kChunkCols;
+            if constexpr (FP32) {
+                *reinterpret_cast<uint2*>(entries + 2 * (long long)i) =
+                    make_uint2((uint32_t)srow[i] | ((uint32_t)k << 4), sval[i]);
+            } else {
+                entries[i] = sval[i] | ((uint32_t)k << 20);
+            }
+            if (head) {
+                // FP32 formats keep a tile's columns in K-step order: lane group g of the kernel
+                // reads columns 4 s + g (s = 0..7) as eight consecutive words.
+                const int slot = FP32 ? (k & 3) * 8 + (k >> 2) : k;
+                chunk_cols[(long long)tile * kChunkCols + slot] = (int)c;
+                if (k == 0) chunk_eptr[tile] = i;
+            }
+        }
+    }
+    // the last tile's unused columns
+    if (run % kChunkCols != 0 && t >= run % kChunkCols && t < kChunkCols) {
+        const int slot = FP32 ? (t & 3) * 8 + (t >> 2) : t;
+        chunk_cols[(long long)(c0 + run / kChunkCols) * kChunkCols + slot] = -1;
+    }
 }
 
 __global__ void k_dense_flags(const int* __restrict__ eptr, int NC, int dmin,
@@ -400,23 +631,46 @@ __global__ void k_dense_index(const int* __restrict__ flag, const int* __restric
     if (c < NC) chunk_dense[c] = flag[c] ? idx[c] : -1;
 }
 
+// One wave per tile: its dense copy, put together in LDS and written whole.
 template <bool FP32>
-__global__ void k_dense_fill(const uint32_t* __restrict__ entries,
-                             const int* __restrict__ echunk, const int* __restrict__ chunk_dense,
-                             long long n, _Float16* __restrict__ a16, float* __restrict__ a32) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int d = chunk_dense[echunk[i]];
+__global__ __launch_bounds__(256) void k_dense_fill(const uint32_t* __restrict__ entries,
+                                                    const int* __restrict__ eptr,
+                                                    const int* __restrict__ chunk_dense, int NC,
+                                                    _Float16* __restrict__ a16,
+                                                    float* __restrict__ a32) {
+    typedef typename std::conditional<FP32, float, _Float16>::type T;
+    __shared__ __attribute__((aligned(16))) T tile[4][512];
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const long long c = (long long)blockIdx.x * 4 + w;
+    if (c >= NC) return;  // the whole wave
+    const int d = chunk_dense[c];
     if (d < 0) return;
-    if constexpr (FP32) {
-        const uint32_t w = entries[2 * i];
-        const int r = w & 15, k = (w >> 4) & 31;
-        a32[(long long)d * 512 + (k & 3) * 128 + r * 8 + (k >> 2)] = __uint_as_float(entries[2 * i + 1]);
-    } else {
-        const uint32_t w = entries[i];
-        const int r = (w >> 16) & 15, k = (w >> 20) & 31;
-        a16[(long long)d * 512 + r * 32 + k] = __builtin_bit_cast(_Float16, (unsigned short)(w & 0xffffu));
+    constexpr int V = 512 * sizeof(T) / (64 * 16);  // 16-byte pieces a lane
+    uint4* mine = reinterpret_cast<uint4*>(tile[w]);
+#pragma unroll
+    for (int q = 0; q < V; ++q) mine[lane + 64 * q] = make_uint4(0, 0, 0, 0);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    for (int e = eptr[c] + lane; e < eptr[c + 1]; e += 64) {
+        if constexpr (FP32) {
+            const uint2 x = *reinterpret_cast<const uint2*>(entries + 2 * (long long)e);
+            const int r = x.x & 15, k = (x.x >> 4) & 31;
+            tile[w][(k & 3) * 128 + r * 8 + (k >> 2)] = __uint_as_float(x.y);
+        } else {
+            const uint32_t x = entries[e];
+            const int r = (x >> 16) & 15, k = (x >> 20) & 31;
+            tile[w][r * 32 + k] = __builtin_bit_cast(_Float16, (unsigned short)(x & 0xffffu));
+        }
     }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    uint4* out;
+    if constexpr (FP32) out = reinterpret_cast<uint4*>(a32 + (long long)d * 512);
+    else out = reinterpret_cast<uint4*>(a16 + (long long)d * 512);
+#pragma unroll
+    for (int q = 0; q < V; ++q) out[lane + 64 * q] = mine[lane + 64 * q];
 }
 
 // Row steps of FP32 panels (the layout is described with DeviceFormat).  rsmask[4c + g] = the
@@ -638,61 +892,113 @@ static int heavy_tile_limit(int num_chunks) {
 // to 2.5%, and leaves grids, stencils and R-MAT within 1%.
 static bool light_by_column(long long nnz, long long num_pairs) { return nnz >= 4 * num_pairs; }
 
-template <typename K>
-static void build_exec_layout_k(DeviceFormat& F, const int* trow, const int* tcol,
-                                const float* tval, const int* rowpos, long long n,
-                                hipStream_t st) {
-    const int num_panels_all = (F.M + kPanelRows - 1) / kPanelRows;
-    const int cbits = bits_for(F.N > 0 ? (unsigned long long)(F.N - 1) : 0ull);
-    const int pbits = bits_for(num_panels_all > 0 ? (unsigned long long)(num_panels_all - 1) : 0ull);
-    const int kbits = pbits + cbits + 4;
+// The nonzeros of every panel in (column, row) order, panels in order.
+struct SortedNonzeros {
+    TmpBuf<uint32_t> col, val;
+    TmpBuf<unsigned char> row;  // FP32 formats (FP16 ones keep it in val)
+    SortedNonzeros(long long n, bool fp32) : col(n), val(n), row(fp32 ? n : 0) {}
+};
 
-    TmpBuf<K> k1(n), k2(n);
-    TmpBuf<uint32_t> v1(n), v2(n);
-    LAUNCH((k_panel_keys<K>), n, trow, tcol, rowpos, n, cbits, k1.p, v1.p);
-    K* kp = k1.p; K* ka = k2.p;
-    uint32_t* vp = v1.p; uint32_t* va = v2.p;
-    radix_sort_pairs<K>(kp, vp, ka, va, n, kbits, st);
+// What sorting a row order's panels found.
+struct PanelSet {
+    int panels = 0;  // with empty ones
+    const int* row_map = nullptr;
+    TmpBuf<int> at, pmask, ndist;
+    int pairs = 0, NC = 0, NP = 0, max_tiles = 0;
+    Positions positions(const int* rp, int M) const { return Positions{rp, row_map, at.p, M}; }
+};
 
-    TmpBuf<int> hdist(n), hpanel(n), dc(n), pin(n), err(1);
-    VCSRMC_HIP(hipMemsetAsync(err.p, 0, sizeof(int), st));
-    LAUNCH((k_panel_heads<K>), n, kp, n, cbits, hdist.p, hpanel.p, err.p);
-    inclusive_sum<int, int>(hdist.p, dc.p, n, st);
-    inclusive_sum<int, int>(hpanel.p, pin.p, n, st);
-    check_err(err.p, st);
-    const int NP = read_scalar(pin.p + (n - 1), st);
-    F.num_pairs = read_scalar(dc.p + (n - 1), st);
-
-    TmpBuf<int> pstart(NP + 1), ppanel(NP), nch(NP), cbase(NP + 1), pmask(NP);
-    LAUNCH((k_panel_starts<K>), n, kp, hpanel.p, pin.p, n, cbits, pstart.p, ppanel.p);
-    fill<int>(pstart.p + NP, 1, (int)n, st);
-    LAUNCH(k_panel_chunks, NP, pstart.p, dc.p, NP, nch.p);
-    exclusive_sum<int, int>(nch.p, cbase.p, NP, st);
-    const int NC = read_scalar(cbase.p + NP, st);
-    {
-        TmpBuf<int> nmax(NP);
-        inclusive_max(nch.p, nmax.p, NP, st);
-        F.max_panel_tiles = read_scalar(nmax.p + (NP - 1), st);
+template <bool FP32>
+static PanelSet sort_panels(int M, const int* rp, const int* row_map, const int* col,
+                            const float* val, float inv_scale, SortedNonzeros& S, hipStream_t st) {
+    PanelSet P;
+    P.panels = (M + kPanelRows - 1) / kPanelRows;
+    P.row_map = row_map;
+    if (row_map) {
+        const int npos = P.panels * kPanelRows;
+        TmpBuf<int> len(npos);
+        P.at.alloc((size_t)npos + 1);
+        LAUNCH(k_position_lens, npos, rp, row_map, npos, len.p);
+        exclusive_sum<int, int>(len.p, P.at.p, npos, st);
     }
+    const Positions pos = P.positions(rp, M);
+    P.pmask.alloc(P.panels);
+    P.ndist.alloc(P.panels);
+    TmpBuf<int> mid(P.panels), big(P.panels), bsize(P.panels), counts(2);
+    fill<int>(counts.p, 2, 0, st);
+    LAUNCH(k_panel_classes, P.panels, pos, P.panels, P.pmask.p, P.ndist.p, mid.p, big.p, bsize.p,
+           counts.p);
+    hipLaunchKernelGGL((k_panel_sort<kSortSmall, 256, FP32>), dim3((unsigned)P.panels), dim3(256),
+                       0, st, pos, (const int*)nullptr, col, val, inv_scale, S.col.p, S.val.p,
+                       S.row.p, P.ndist.p);
+    VCSRMC_HIP(hipGetLastError());
+    int nsort[2];
+    VCSRMC_HIP(hipMemcpyAsync(nsort, counts.p, sizeof nsort, hipMemcpyDeviceToHost, st));
+    VCSRMC_HIP(hipStreamSynchronize(st));
+    if (nsort[0] > 0) {
+        hipLaunchKernelGGL((k_panel_sort<kSortMid, 1024, FP32>), dim3((unsigned)nsort[0]),
+                           dim3(1024), 0, st, pos, (const int*)mid.p, col, val, inv_scale, S.col.p,
+                           S.val.p, S.row.p, P.ndist.p);
+        VCSRMC_HIP(hipGetLastError());
+    }
+    if (nsort[1] > 0) {
+        const int nbig = nsort[1];
+        TmpBuf<int> bofs((size_t)nbig + 1);
+        exclusive_sum<int, int>(bsize.p, bofs.p, nbig, st);
+        const long long total = read_scalar(bofs.p + nbig, st);
+        TmpBuf<uint32_t> c0(total), c1(total), s0(total), s1(total);
+        TmpBuf<unsigned char> r0(total), r1(total);
+        LAUNCH(k_big_load, total, pos, big.p, bofs.p, nbig, total, col, c0.p, s0.p, r0.p);
+        for (int s = 0; s < 4; ++s) {
+            LAUNCH(k_big_merge, total, pos, big.p, bofs.p, nbig, total, s, c0.p, s0.p, r0.p, c1.p,
+                   s1.p, r1.p);
+            std::swap(c0, c1);
+            std::swap(s0, s1);
+            std::swap(r0, r1);
+        }
+        LAUNCH((k_big_store<FP32>), total, pos, big.p, bofs.p, nbig, total, c0.p, s0.p, r0.p, val,
+               inv_scale, S.col.p, S.val.p, S.row.p, P.ndist.p);
+    }
+    TmpBuf<int4> totals(1);
+    hipLaunchKernelGGL(k_panel_totals, dim3(1), dim3(1024), 0, st, P.ndist.p, P.panels, totals.p);
+    VCSRMC_HIP(hipGetLastError());
+    const int4 T = read_scalar(totals.p, st);
+    P.pairs = T.x;
+    P.NC = T.y;
+    P.NP = T.z;
+    P.max_tiles = T.w;
+    return P;
+}
 
-    F.chunk_eptr.alloc(NC + 1);
+// The execution layout of the sorted panels.
+static void fill_layout(DeviceFormat& F, const PanelSet& S, const SortedNonzeros& nz,
+                        const int* rp, long long n, hipStream_t st) {
+    const int NP = S.NP, NC = S.NC;
+    F.num_pairs = S.pairs;
+    F.max_panel_tiles = S.max_tiles;
+    F.chunk_eptr.alloc((size_t)NC + 1);
     F.chunk_cols.alloc((size_t)NC * kChunkCols);
     F.entries.alloc(F.fp32 ? 2 * n : n);
-    fill<int>(F.chunk_cols.p, (long long)NC * kChunkCols, -1, st);
-    fill<int>(F.chunk_eptr.p + NC, 1, (int)n, st);
+    TmpBuf<int> pstart((size_t)NP + 1), ppanel(NP), nch(NP), cbase((size_t)NP + 1), pmask(NP);
     {
-        TmpBuf<unsigned char> rflag((size_t)num_panels_all * kPanelRows);
-        fill<unsigned char>(rflag.p, (long long)num_panels_all * kPanelRows, 0, st);
-        LAUNCH(k_row_flags, n, trow, rowpos, n, rflag.p);
-        LAUNCH(k_panel_masks, NP, rflag.p, ppanel.p, NP, pmask.p);
+        TmpBuf<int> all(S.panels), some(S.panels), cbase_all((size_t)S.panels + 1),
+            pidx((size_t)S.panels + 1);
+        LAUNCH(k_panel_tiles, S.panels, S.ndist.p, S.panels, all.p, some.p);
+        exclusive_sum<int, int>(all.p, cbase_all.p, S.panels, st);
+        exclusive_sum<int, int>(some.p, pidx.p, S.panels, st);
+        LAUNCH(k_panel_compact, S.panels, S.positions(rp, F.M), all.p, cbase_all.p, pidx.p,
+               S.pmask.p, S.panels, NP, NC, (int)n, ppanel.p, pstart.p, cbase.p, nch.p, pmask.p,
+               F.chunk_eptr.p);
     }
-    TmpBuf<int> echunk(n);
     if (F.fp32)
-        LAUNCH((k_panel_entries<K, true>), n, kp, vp, hdist.p, dc.p, pin.p, pstart.p, cbase.p, tcol,
-               tval, n, F.entries.p, F.chunk_cols.p, F.chunk_eptr.p, echunk.p);
+        hipLaunchKernelGGL((k_panel_fill<true>), dim3((unsigned)NP), dim3(256), 0, st, pstart.p,
+                           cbase.p, nz.col.p, nz.val.p, nz.row.p, F.entries.p, F.chunk_cols.p,
+                           F.chunk_eptr.p);
     else
-        LAUNCH((k_panel_entries<K, false>), n, kp, vp, hdist.p, dc.p, pin.p, pstart.p, cbase.p,
-               tcol, tval, n, F.entries.p, F.chunk_cols.p, F.chunk_eptr.p, echunk.p);
+        hipLaunchKernelGGL((k_panel_fill<false>), dim3((unsigned)NP), dim3(256), 0, st, pstart.p,
+                           cbase.p, nz.col.p, nz.val.p, nz.row.p, F.entries.p, F.chunk_cols.p,
+                           F.chunk_eptr.p);
+    VCSRMC_HIP(hipGetLastError());
 
     // dense copies of well-filled tiles
     {
@@ -706,15 +1012,16 @@ static void build_exec_layout_k(DeviceFormat& F, const int* trow, const int* tco
         if (ND > 0) {
             if (F.fp32) {
                 F.dense_a32.alloc((size_t)ND * 512);
-                VCSRMC_HIP(hipMemsetAsync(F.dense_a32.p, 0, sizeof(float) * 512 * (size_t)ND, st));
-                LAUNCH((k_dense_fill<true>), n, F.entries.p, echunk.p, F.chunk_dense.p, n,
-                       (_Float16*)nullptr, F.dense_a32.p);
+                hipLaunchKernelGGL((k_dense_fill<true>), dim3(grid_for(NC, 4)), dim3(256), 0, st,
+                                   F.entries.p, F.chunk_eptr.p, F.chunk_dense.p, NC,
+                                   (_Float16*)nullptr, F.dense_a32.p);
             } else {
                 F.dense_a16.alloc((size_t)ND * 512);
-                VCSRMC_HIP(hipMemsetAsync(F.dense_a16.p, 0, sizeof(_Float16) * 512 * (size_t)ND, st));
-                LAUNCH((k_dense_fill<false>), n, F.entries.p, echunk.p, F.chunk_dense.p, n,
-                       F.dense_a16.p, (float*)nullptr);
+                hipLaunchKernelGGL((k_dense_fill<false>), dim3(grid_for(NC, 4)), dim3(256), 0, st,
+                                   F.entries.p, F.chunk_eptr.p, F.chunk_dense.p, NC,
+                                   F.dense_a16.p, (float*)nullptr);
             }
+            VCSRMC_HIP(hipGetLastError());
         }
     }
 
@@ -794,48 +1101,6 @@ static void build_exec_layout_k(DeviceFormat& F, const int* trow, const int* tco
     F.heavy_tiles = heavy_tiles;
 }
 
-static void build_layout_in_order(DeviceFormat& F, const int* trow, const int* tcol,
-                                  const float* tval, const int* rowpos, long long n,
-                                  hipStream_t st) {
-    F.num_panels = F.num_chunks = F.num_units = F.num_dense = F.max_panel_tiles = 0;
-    F.num_row_step_batches = 0;
-    F.num_pairs = 0;
-    if (n == 0) return;
-    const int num_panels_all = (F.M + kPanelRows - 1) / kPanelRows;
-    const int cbits = bits_for(F.N > 0 ? (unsigned long long)(F.N - 1) : 0ull);
-    const int pbits = bits_for(num_panels_all > 0 ? (unsigned long long)(num_panels_all - 1) : 0ull);
-    if (pbits + cbits + 4 <= 32)
-        build_exec_layout_k<uint32_t>(F, trow, tcol, tval, rowpos, n, st);
-    else
-        build_exec_layout_k<unsigned long long>(F, trow, tcol, tval, rowpos, n, st);
-}
-
-// Moves the execution layout (not the format arrays) between two formats of the same matrix.
-static void swap_layout(DeviceFormat& a, DeviceFormat& b) {
-    std::swap(a.num_panels, b.num_panels);
-    std::swap(a.num_chunks, b.num_chunks);
-    std::swap(a.num_units, b.num_units);
-    std::swap(a.num_heavy, b.num_heavy);
-    std::swap(a.light_max, b.light_max);
-    std::swap(a.heavy_tiles, b.heavy_tiles);
-    std::swap(a.num_split_panels, b.num_split_panels);
-    std::swap(a.max_panel_tiles, b.max_panel_tiles);
-    std::swap(a.num_pairs, b.num_pairs);
-    std::swap(a.xcd_start, b.xcd_start);
-    std::swap(a.units, b.units);
-    std::swap(a.row_map, b.row_map);
-    std::swap(a.chunk_eptr, b.chunk_eptr);
-    std::swap(a.chunk_cols, b.chunk_cols);
-    std::swap(a.entries, b.entries);
-    std::swap(a.num_dense, b.num_dense);
-    std::swap(a.chunk_dense, b.chunk_dense);
-    std::swap(a.dense_a16, b.dense_a16);
-    std::swap(a.dense_a32, b.dense_a32);
-    std::swap(a.num_row_step_batches, b.num_row_step_batches);
-    std::swap(a.rs_cols, b.rs_cols);
-    std::swap(a.rs_vals, b.rs_vals);
-}
-
 // 0 off, 1 when it pays (the default), 2 always; read once by each build.
 static std::atomic<int> g_row_grouping{1};
 void set_row_grouping(int mode) { g_row_grouping.store(mode, std::memory_order_relaxed); }
@@ -861,41 +1126,49 @@ int fp32_row_steps() { return g_fp32_row_steps.load(std::memory_order_relaxed); 
 // 300 -> 316 / 251; 2D 5-point 1000^2 FP32 312 / 234 -> 297 / 196 (tiles halved); 3D 7-point
 // 100^3 FP32 390 / 328 -> 373 / 255; 27-point 16^3 (256 panels) within 2% either way.  Grouping
 // the excluded classes anyway saved 1-7% of their tiles and ran from 6% faster to 13% slower.
-static void build_exec_layout(DeviceFormat& F, const int* rp, const int* trow, const int* tcol,
-                              const float* tval, long long n, hipStream_t st) {
-    F.row_map.release();
+template <bool FP32>
+static void build_exec_layout_t(DeviceFormat& F, const int* rp, const int* row_of, const int* col,
+                                const float* val, float inv_scale, long long n, hipStream_t st) {
     const int mode = row_grouping();
-    TmpBuf<int> cpos;
-    DevBuf<int> cmap;
-    const bool compact = mode != 0 && compact_rows(trow, n, F.M, st, cpos, cmap);
-    build_layout_in_order(F, trow, tcol, tval, compact ? cpos.p : nullptr, n, st);
-    if (compact) F.row_map = std::move(cmap);
-    if (mode == 0 || F.num_chunks == 0) return;
-    const long long NC = F.num_chunks;
-    if (mode == 1) {
-        if (!(10 * n >= 13 * F.num_pairs && n < 256 * NC)) return;
-        // Grouping is an optimisation here: it is skipped, natural order kept, unless its buffers
-        // (at most ~64 bytes per nonzero and per row, for the sorts and a second layout) fit
-        // in half the free device memory.
-        size_t free_b = 0, total_b = 0;
-        if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) {
-            (void)hipGetLastError();
-            return;
-        }
-        if (64.0 * (double)n + 64.0 * (double)F.M > 0.5 * (double)free_b) return;
-    }
-    TmpBuf<int> rowpos;
+    SortedNonzeros nz(n, FP32);
     DevBuf<int> row_map;
-    if (!group_rows(rp, trow, tcol, n, F.M, F.N, st, rowpos, row_map)) return;
-    DeviceFormat G;
-    G.M = F.M;
-    G.N = F.N;
-    G.fp32 = F.fp32;
-    G.nnz = F.nnz;
-    build_layout_in_order(G, trow, tcol, tval, rowpos.p, n, st);
-    if (mode == 1 && 10LL * G.num_chunks > 9LL * NC) return;
-    G.row_map = std::move(row_map);
-    swap_layout(F, G);
+    if (mode != 0) compact_rows(rp, F.M, st, row_map);
+    PanelSet S = sort_panels<FP32>(F.M, rp, row_map.p, col, val, inv_scale, nz, st);
+    bool group = mode == 2;
+    if (mode == 1 && 10 * n >= 13LL * S.pairs && n < 256LL * S.NC) {
+        // Grouping is an optimisation here: it is skipped, natural order kept, unless its buffers
+        // (at most ~64 bytes per nonzero and per row, for the lists and their sorts) fit in half
+        // the free device memory.
+        size_t free_b = 0, total_b = 0;
+        if (hipMemGetInfo(&free_b, &total_b) == hipSuccess)
+            group = 64.0 * (double)n + 64.0 * (double)F.M <= 0.5 * (double)free_b;
+        else
+            (void)hipGetLastError();
+    }
+    DevBuf<int> groups;
+    if (group && group_rows(rp, row_of, col, n, F.M, F.N, st, groups)) {
+        PanelSet G = sort_panels<FP32>(F.M, rp, groups.p, col, val, inv_scale, nz, st);
+        if (mode == 2 || 10LL * G.NC <= 9LL * S.NC) {
+            S = std::move(G);
+            row_map = std::move(groups);
+        } else {
+            S = sort_panels<FP32>(F.M, rp, row_map.p, col, val, inv_scale, nz, st);
+        }
+    }
+    fill_layout(F, S, nz, rp, n, st);
+    F.row_map = std::move(row_map);
+}
+
+// From a CSR with ascending columns and the row of each nonzero.
+static void build_exec_layout(DeviceFormat& F, const int* rp, const int* row_of, const int* col,
+                              const float* val, float inv_scale, long long n, hipStream_t st) {
+    F.row_map.release();
+    F.num_panels = F.num_chunks = F.num_units = F.num_dense = F.max_panel_tiles = 0;
+    F.num_row_step_batches = 0;
+    F.num_pairs = 0;
+    if (n == 0) return;
+    if (F.fp32) build_exec_layout_t<true>(F, rp, row_of, col, val, inv_scale, n, st);
+    else build_exec_layout_t<false>(F, rp, row_of, col, val, inv_scale, n, st);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1032,10 +1305,7 @@ void build_from_csr(DeviceFormat& F, const int* d_row_ptr, const int* d_col, con
     pstart.release();
     prow.release();
 
-    // Execution layout from (row_of, col, val / scale).
-    TmpBuf<float> sval(nnz);
-    LAUNCH(k_scale_values, nnz, d_val, sval.p, (long long)nnz, inv_scale);
-    build_exec_layout(F, d_row_ptr, row_of.p, d_col, sval.p, nnz, st);
+    build_exec_layout(F, d_row_ptr, row_of.p, d_col, d_val, inv_scale, nnz, st);
     VCSRMC_HIP(hipStreamSynchronize(st));
     F.ready = true;
 }
@@ -1213,7 +1483,7 @@ void build_from_host(DeviceFormat& F, const HostArrays& H, hipStream_t st) {
         sort_triples(trow, tcol, tval, n, H.M, H.N, st);
         key_ptr<int>(trow.p, n, H.M, rp.p, st);
     }
-    build_exec_layout(F, rp.p, trow.p, tcol.p, tval.p, n, st);
+    build_exec_layout(F, rp.p, trow.p, tcol.p, tval.p, 1.0f, n, st);
     VCSRMC_HIP(hipStreamSynchronize(st));
     F.ready = true;
 }

@@ -141,15 +141,14 @@ float half_scale_from_amax(float amax);
 float device_absmax(const float* d_val, long long n, hipStream_t st);
 
 // A row order that groups rows sharing columns into 16-row panels (row_groups.hip), from a CSR
-// of n nonzeros with ascending columns and the row of each: rowpos[row] = position, row_map[position] = row (-1 past the last
-// of M rows; M rounded up to 16 entries).  False when it found nothing to work with.
+// of n nonzeros with ascending columns and the row of each: row_map[position] = row (-1 past the
+// last of M rows; M rounded up to 16 entries).  False when it found nothing to work with.
 bool group_rows(const int* rp, const int* row_of, const int* col, long long n, int M, int N,
-                hipStream_t st, TmpBuf<int>& rowpos, DevBuf<int>& row_map);
-// The same maps for natural order with the rows that hold no nonzero moved after the others,
-// when they are at least an eighth of the rows (false otherwise): panels then hold 16 rows
-// with nonzeros instead of, on average, as many as the empty rows leave.
-bool compact_rows(const int* trow, long long n, int M, hipStream_t st, TmpBuf<int>& rowpos,
-                  DevBuf<int>& row_map);
+                hipStream_t st, DevBuf<int>& row_map);
+// The same map for natural order with the rows that hold no nonzero moved after the others,
+// when they are at least an eighth of the rows (false, and no map, otherwise): panels then hold 16
+// rows with nonzeros instead of, on average, as many as the empty rows leave.
+bool compact_rows(const int* rp, int M, hipStream_t st, DevBuf<int>& row_map);
 // Row order of the execution layout: 0 natural order, 1 empty rows moved last and rows grouped
 // where that saves tiles (the default; format_build.hip, build_exec_layout), 2 always grouped.
 // Read by later builds.

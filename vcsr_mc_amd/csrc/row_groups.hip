@@ -386,76 +386,58 @@ __global__ void k_init_clusters(int M, int* __restrict__ rowcl, int* __restrict_
     cmin[r] = (int)r;
 }
 
-__global__ void k_has_nonzero(const int* __restrict__ trow, long long n,
-                              unsigned char* __restrict__ has) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) has[trow[i]] = 1;
-}
-
 // Order key of row r: its group's first row (rows without nonzeros last); the stable sort keeps
 // the rows of a group by index.
 __global__ void k_order_keys(const int* __restrict__ rowcl, const int* __restrict__ cmin,
-                             const unsigned char* __restrict__ has, int M,
+                             const int* __restrict__ rp, int M,
                              uint32_t* __restrict__ key, uint32_t* __restrict__ pay) {
     const long long r = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= M) return;
-    key[r] = has[r] ? (uint32_t)cmin[rowcl[r]] : (uint32_t)M;
+    key[r] = rp[r + 1] > rp[r] ? (uint32_t)cmin[rowcl[r]] : (uint32_t)M;
     pay[r] = (uint32_t)r;
 }
 
 __global__ void k_positions(const uint32_t* __restrict__ order, int M, int P,
-                            int* __restrict__ rowpos, int* __restrict__ row_map) {
+                            int* __restrict__ row_map) {
     const long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= P) return;
-    if (p < M) {
-        const int r = (int)order[p];
-        row_map[p] = r;
-        rowpos[r] = (int)p;
-    } else {
-        row_map[p] = -1;
-    }
+    if (p < P) row_map[p] = p < M ? (int)order[p] : -1;
 }
 
-__global__ void k_flag_rows(const int* __restrict__ trow, long long n, int* __restrict__ flag) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) flag[trow[i]] = 1;
+__global__ void k_flag_rows(const int* __restrict__ rp, int M, int* __restrict__ flag) {
+    const long long r = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (r < M) flag[r] = rp[r + 1] > rp[r];
 }
 
 // Rows with nonzeros keep their order at positions 0..NE-1, the others follow in order.
 __global__ void k_compact_positions(const int* __restrict__ flag, const int* __restrict__ rank,
-                                    int M, int NE, int* __restrict__ rowpos,
-                                    int* __restrict__ row_map) {
+                                    int M, int NE, int* __restrict__ row_map) {
     const long long r = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= M) return;
     const int p = flag[r] ? rank[r] : NE + ((int)r - rank[r]);
-    rowpos[r] = p;
     row_map[p] = (int)r;
 }
 
 }  // namespace
 
-bool compact_rows(const int* trow, long long n, int M, hipStream_t st, TmpBuf<int>& rowpos,
-                  DevBuf<int>& row_map) {
-    if (M < 1 || n < 1) return false;
+bool compact_rows(const int* rp, int M, hipStream_t st, DevBuf<int>& row_map) {
+    if (M < 1) return false;
     TmpBuf<int> flag(M), rank((size_t)M + 1);
-    fill<int>(flag.p, M, 0, st);
-    hipLaunchKernelGGL(k_flag_rows, dim3(grid256(n)), dim3(256), 0, st, trow, n, flag.p);
+    hipLaunchKernelGGL(k_flag_rows, dim3(grid256(M)), dim3(256), 0, st, rp, M, flag.p);
     VCSRMC_HIP(hipGetLastError());
     exclusive_sum<int, int>(flag.p, rank.p, M, st);
     const int NE = read_scalar(rank.p + M, st);
     if (8LL * (M - NE) < M) return false;
     const int P = ((M + kPanelRows - 1) / kPanelRows) * kPanelRows;
-    rowpos.alloc(M);
     row_map.alloc(P);
     fill<int>(row_map.p, P, -1, st);
     hipLaunchKernelGGL(k_compact_positions, dim3(grid256(M)), dim3(256), 0, st, flag.p, rank.p, M,
-                       NE, rowpos.p, row_map.p);
+                       NE, row_map.p);
     VCSRMC_HIP(hipGetLastError());
     return true;
 }
 
 bool group_rows(const int* rp, const int* row_of, const int* col, long long n, int M, int N,
-                hipStream_t st, TmpBuf<int>& rowpos, DevBuf<int>& row_map) {
+                hipStream_t st, DevBuf<int>& row_map) {
     if (M < 2 * kPanelRows || N < 1 || n < 1) return false;
     const int cbits = bits_for((unsigned long long)(N - 1));
     const int hub = (int)std::max<long long>(32, std::min<long long>(1024, 4 * n / N));
@@ -568,20 +550,14 @@ bool group_rows(const int* rp, const int* row_of, const int* col, long long n, i
 
     // Rows by group (first row of the group), rows without nonzeros last.
     const int P = ((M + kPanelRows - 1) / kPanelRows) * kPanelRows;
-    TmpBuf<unsigned char> has(M);
-    fill<unsigned char>(has.p, M, 0, st);
-    hipLaunchKernelGGL(k_has_nonzero, dim3(grid256(n)), dim3(256), 0, st, row_of, n, has.p);
-    VCSRMC_HIP(hipGetLastError());
     TmpBuf<uint32_t> okey(M), oalt(M), opay(M), opalt(M);
-    hipLaunchKernelGGL(k_order_keys, dim3(grid256(M)), dim3(256), 0, st, rowcl.p, cmin.p, has.p,
-                       M, okey.p, opay.p);
+    hipLaunchKernelGGL(k_order_keys, dim3(grid256(M)), dim3(256), 0, st, rowcl.p, cmin.p, rp, M,
+                       okey.p, opay.p);
     VCSRMC_HIP(hipGetLastError());
     uint32_t *ok = okey.p, *oka = oalt.p, *order = opay.p, *order_alt = opalt.p;
     radix_sort_pairs<uint32_t>(ok, order, oka, order_alt, M, bits_for((unsigned long long)M), st);
-    rowpos.alloc(M);
     row_map.alloc(P);
-    hipLaunchKernelGGL(k_positions, dim3(grid256(P)), dim3(256), 0, st, order, M, P, rowpos.p,
-                       row_map.p);
+    hipLaunchKernelGGL(k_positions, dim3(grid256(P)), dim3(256), 0, st, order, M, P, row_map.p);
     VCSRMC_HIP(hipGetLastError());
     return true;
 }
