@@ -972,22 +972,111 @@ __global__ void k_relabel_dups(const u64* __restrict__ key, long long nnz,
     if (i > 0 && i < nnz && key[i - 1] == key[i]) atomicOr(err, kDupCol);
 }
 
-__global__ void k_relabel_write(const u64* __restrict__ key, const uint32_t* __restrict__ src,
-                                const float* __restrict__ vin, long long nnz, int nb,
-                                int* __restrict__ col, float* __restrict__ vout) {
+__global__ void k_relabel_gather(const u64* __restrict__ key, const uint32_t* __restrict__ src,
+                                 const float* __restrict__ vin, long long nnz, int nb,
+                                 int* __restrict__ cout, float* __restrict__ vout) {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nnz) return;
-    col[i] = (int)(key[i] & ((1ull << nb) - 1));
+    cout[i] = (int)(key[i] & ((1ull << nb) - 1));
     vout[i] = vin[src[i]];
 }
 
-// B_out[position[r], :] = B[r, :]; one thread per element, rows of O consecutive floats.
+// Rows relabelled and sorted by new column on their own, since they do not move: up to 64
+// nonzeros by one wave, each lane counting the row's columns below its own; longer ones, up to
+// kRowSortMax, are listed and sorted by a work-group in LDS (bitonic).  A radix sort of (row, column)
+// keys of the whole matrix, which rows beyond that still take, moved 12 bytes a nonzero five times.
+// 27-point mesh 64^3, 6.9 M nonzeros: 95 us, ordering and relabelling 14.3 -> 13.8 ms.
+constexpr int kRowSortMax = 4096;
+
+__global__ void k_longest_row(const int* __restrict__ rp, int M, int* __restrict__ longest) {
+    const long long r = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    const int len = r < M ? rp[r + 1] - rp[r] : 0;
+    const int m = wave_last(wave_scan(len, OpMax{}, INT_MIN));
+    if ((threadIdx.x & 63) == 0 && m > *longest) atomicMax(longest, m);
+}
+
+__global__ __launch_bounds__(256) void k_relabel_rows(
+    const int* __restrict__ rp, const int* __restrict__ col, const float* __restrict__ val,
+    const int* __restrict__ position, int M, int* __restrict__ cout, float* __restrict__ vout,
+    int* __restrict__ listed, int* __restrict__ nlisted, int* __restrict__ err) {
+    const long long r = ((long long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+    const int lane = threadIdx.x & 63;
+    if (r >= M) return;  // the whole wave
+    const int a = __builtin_amdgcn_readfirstlane(rp[r]);
+    const int len = __builtin_amdgcn_readfirstlane(rp[r + 1]) - a;
+    if (len > 64) {
+        if (lane == 0) listed[atomicAdd(nlisted, 1)] = (int)r;
+        return;
+    }
+    int c = INT_MAX;
+    float v = 0.0f;
+    if (lane < len) {
+        c = position[col[a + lane]];
+        v = val[a + lane];
+    }
+    int rank = 0, same = 0;
+    for (int i = 0; i < len; ++i) {
+        const int x = __builtin_amdgcn_readlane(c, i);
+        rank += x < c;
+        same += x == c;
+    }
+    if (lane < len) {
+        if (same > 1) atomicOr(err, kDupCol);  // nothing of this is kept then
+        cout[a + rank] = c;
+        vout[a + rank] = v;
+    }
+}
+
+__global__ __launch_bounds__(256) void k_relabel_listed(
+    const int* __restrict__ rp, const int* __restrict__ col, const float* __restrict__ val,
+    const int* __restrict__ position, const int* __restrict__ listed,
+    const int* __restrict__ nlisted, int* __restrict__ cout, float* __restrict__ vout,
+    int* __restrict__ err) {
+    __shared__ u64 key[kRowSortMax];  // new column << 32 | index in the row
+    const int t = threadIdx.x, n = *nlisted;
+    for (int q = blockIdx.x; q < n; q += gridDim.x) {
+        const int r = listed[q], a = rp[r], len = rp[r + 1] - a;
+        int size = 128;
+        while (size < len) size *= 2;
+        __syncthreads();
+        for (int i = t; i < size; i += 256)
+            key[i] = i < len ? (u64)(uint32_t)position[col[a + i]] << 32 | (uint32_t)i : ~0ull;
+        for (int k = 2; k <= size; k *= 2)
+            for (int j = k / 2; j > 0; j /= 2) {
+                __syncthreads();
+                for (int p = t; p < size / 2; p += 256) {
+                    const int i = 2 * p - (p & (j - 1)), o = i + j;
+                    const u64 x = key[i], y = key[o];
+                    if ((x > y) == ((i & k) == 0)) {
+                        key[i] = y;
+                        key[o] = x;
+                    }
+                }
+            }
+        __syncthreads();
+        for (int i = t; i < len; i += 256) {
+            const u64 x = key[i];
+            if (i > 0 && (uint32_t)(key[i - 1] >> 32) == (uint32_t)(x >> 32))
+                atomicOr(err, kDupCol);
+            cout[a + i] = (int)(x >> 32);
+            vout[a + i] = val[a + (int)(uint32_t)x];
+        }
+    }
+}
+
+// B_out[position[r], :] = B[r, :]; one thread per V consecutive floats of a row of W * V.
+template <int V>
 __global__ void k_permute_rows(const float* __restrict__ B, const int* __restrict__ position,
-                               int N, int O, float* __restrict__ Bout) {
+                               long long n, unsigned W, float* __restrict__ Bout) {
+    typedef float vec __attribute__((ext_vector_type(V)));
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (long long)N * O) return;
-    const long long r = i / O, k = i - r * O;
-    Bout[(long long)position[r] * O + k] = B[i];
+    if (i >= n) return;
+    long long r;
+    if (n <= 0xffffffffll) r = (unsigned)i / W;
+    else r = i / W;
+    const long long k = i - r * W;
+    reinterpret_cast<vec*>(Bout)[(long long)position[r] * W + k] =
+        reinterpret_cast<const vec*>(B)[i];
 }
 
 __global__ void k_mark_heads(const int* __restrict__ rp, int M, int* __restrict__ head) {
@@ -1231,36 +1320,57 @@ void apply_column_permutation_device(const int* rp, int* col, float* val, int M,
     if ((B == nullptr) != (B_out == nullptr))
         throw Error(VCSRMC_ERR_ARG, "B and B_out must both be given or both be NULL");
     if (B && B == B_out) throw Error(VCSRMC_ERR_ARG, "B_out must not alias B");
-    ScratchScope scratch((size_t)(36ll * nnz + 8ll * N));
-    TmpBuf<int> err(1);
-    check_csr(rp, col, M, N, nnz, err.p, st);
-    if (N > 0) {
-        TmpBuf<int> seen(N);
-        VCSRMC_HIP(hipMemsetAsync(seen.p, 0, sizeof(int) * (size_t)N, st));
-        RLAUNCH(k_perm_check, N, position, N, seen.p, err.p);
-        raise_if(err.p, st);
-    }
+    ScratchScope scratch((size_t)(36ll * nnz + 8ll * N + 4ll * M));
+    // every check of the input at once: {errors, longest row}
+    TmpBuf<int> err(2), seen(N);
+    fill<int>(err.p, 2, 0, st);
+    RLAUNCH(k_check_rp, (long long)M + 1, rp, M, nnz, err.p);
+    RLAUNCH(k_longest_row, M, rp, M, err.p + 1);
+    RLAUNCH(k_check_cols, (long long)nnz, col, (long long)nnz, N, err.p);
+    fill<int>(seen.p, N, 0, st);
+    RLAUNCH(k_perm_check, N, position, N, seen.p, err.p);
+    raise_if(err.p, st);
     if (nnz > 0) {
-        const int nb = std::max(1, bits_for((u64)N));
-        const int mb = std::max(1, bits_for((u64)M));
-        TmpBuf<int> row_of(nnz);
-        row_of_nonzeros(rp, M, nnz, row_of.p, st);
-        TmpBuf<u64> k1(nnz), k2(nnz);
-        TmpBuf<uint32_t> v1(nnz), v2(nnz);
-        RLAUNCH(k_relabel_keys, nnz, row_of.p, col, position, (long long)nnz, nb, k1.p, v1.p);
-        row_of.release();
-        u64 *ka = k1.p, *kb = k2.p;
-        uint32_t *va = v1.p, *vb = v2.p;
-        radix_sort_pairs<u64>(ka, va, kb, vb, nnz, nb + mb, st);
-        RLAUNCH(k_relabel_dups, nnz, ka, (long long)nnz, err.p);
+        const int longest = read_scalar(err.p + 1, st);
+        TmpBuf<int> ncol(nnz);
+        TmpBuf<float> nval(nnz);
+        if (longest <= kRowSortMax) {
+            TmpBuf<int> listed(longest > 64 ? M : 0), nlisted(1);
+            fill<int>(nlisted.p, 1, 0, st);
+            RLAUNCH(k_relabel_rows, 64ll * M, rp, col, val, position, M, ncol.p, nval.p, listed.p,
+                    nlisted.p, err.p);
+            if (longest > 64) {
+                hipLaunchKernelGGL(k_relabel_listed, dim3(2048), dim3(256), 0, st, rp, col, val,
+                                   position, listed.p, nlisted.p, ncol.p, nval.p, err.p);
+                VCSRMC_HIP(hipGetLastError());
+            }
+        } else {
+            const int nb = std::max(1, bits_for((u64)N));
+            const int mb = std::max(1, bits_for((u64)M));
+            TmpBuf<int> row_of(nnz);
+            row_of_nonzeros(rp, M, nnz, row_of.p, st);
+            TmpBuf<u64> k1(nnz), k2(nnz);
+            TmpBuf<uint32_t> v1(nnz), v2(nnz);
+            RLAUNCH(k_relabel_keys, nnz, row_of.p, col, position, (long long)nnz, nb, k1.p, v1.p);
+            row_of.release();
+            u64 *ka = k1.p, *kb = k2.p;
+            uint32_t *va = v1.p, *vb = v2.p;
+            radix_sort_pairs<u64>(ka, va, kb, vb, nnz, nb + mb, st);
+            RLAUNCH(k_relabel_dups, nnz, ka, (long long)nnz, err.p);
+            RLAUNCH(k_relabel_gather, nnz, ka, va, val, (long long)nnz, nb, ncol.p, nval.p);
+        }
         raise_if(err.p, st);
-        TmpBuf<float> vcopy(nnz);
-        VCSRMC_HIP(hipMemcpyAsync(vcopy.p, val, sizeof(float) * (size_t)nnz,
+        VCSRMC_HIP(hipMemcpyAsync(col, ncol.p, sizeof(int) * (size_t)nnz, hipMemcpyDeviceToDevice,
+                                  st));
+        VCSRMC_HIP(hipMemcpyAsync(val, nval.p, sizeof(float) * (size_t)nnz,
                                   hipMemcpyDeviceToDevice, st));
-        RLAUNCH(k_relabel_write, nnz, ka, va, vcopy.p, (long long)nnz, nb, col, val);
     }
-    if (B && N > 0 && O > 0)
-        RLAUNCH(k_permute_rows, (long long)N * O, B, position, N, O, B_out);
+    if (B && N > 0 && O > 0) {
+        const bool wide = O % 4 == 0 && ((uintptr_t)B | (uintptr_t)B_out) % 16 == 0;
+        const long long n = wide ? (long long)N * (O / 4) : (long long)N * O;
+        if (wide) RLAUNCH((k_permute_rows<4>), n, B, position, n, (unsigned)(O / 4), B_out);
+        else RLAUNCH((k_permute_rows<1>), n, B, position, n, (unsigned)O, B_out);
+    }
     VCSRMC_HIP(hipStreamSynchronize(st));
 }
 
