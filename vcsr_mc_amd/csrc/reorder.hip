@@ -18,12 +18,10 @@
 //      inside one parent's children as the reference orders them: ascending id, then
 //      std::sort by degree (reorder.hpp:67-69), whose steps (libstdc++ introsort) are carried
 //      out exactly, since equal degrees make the result depend on them.  Levels of up to 8192
-//      frontier edges run inside one work-group, many at a time (k_bfs_levels; groups above 64
-//      elements partitioned by the work-group, pieces finished by one thread each); larger
-//      levels take several kernels: claims, a radix sort by (parent index, id), and the group
-//      sorts (large groups a partition step at a time by work-groups, pieces of up to 256
-//      elements by one wave each in LDS, with wave-wide partition steps).
-//   5. order: vertices sorted by (component rank, level, index in level) give the
+//      frontier edges run inside one work-group, many at a time (k_bfs_levels); larger ones take
+//      four kernels each over the frontier's edges (k_level_claim, _count, _place, _sort), with
+//      their sizes kept on the device, so that several levels are enqueued at a time.
+//   5. order: vertices sorted by (component rank, place in the walk) give the
 //      Cuthill-McKee order; position = N - 1 - that index (reorder.hpp:72-76).
 #include <algorithm>
 #include <atomic>
@@ -89,52 +87,42 @@ void check_csr(const int* rp, const int* col, int M, int N, int nnz, int* d_err,
 // ---- 1. adjacency ------------------------------------------------------------------------
 // Nonzero (r, c) contributes r -> c and c -> r when r < N; a row r >= N has no vertex of its
 // own and makes c its own neighbour (twice, merged by the deduplication).
+template <typename K>
 __global__ void k_adj_pairs(const int* __restrict__ row_of, const int* __restrict__ col,
-                            long long nnz, int N, int nb, u64* __restrict__ key) {
+                            long long nnz, int N, int nb, K* __restrict__ key) {
+    typedef K pair __attribute__((ext_vector_type(2)));
     const long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= nnz) return;
     const int r = row_of[p], c = col[p];
     const bool own = r < N;
-    key[2 * p] = own ? ((u64)r << nb | (u64)c) : ((u64)c << nb | (u64)c);
-    key[2 * p + 1] = (u64)c << nb | (u64)(own ? r : c);
+    const K first = own ? ((K)r << nb | (K)c) : ((K)c << nb | (K)c);
+    *reinterpret_cast<pair*>(key + 2 * p) = pair{first, (K)c << nb | (K)(own ? r : c)};
 }
 
-__global__ void k_unique_flags(const u64* __restrict__ key, long long n, int* __restrict__ flag) {
+template <typename K>
+__global__ void k_unique_flags(const K* __restrict__ key, long long n, int* __restrict__ flag) {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) flag[i] = (i == 0 || key[i] != key[i - 1]) ? 1 : 0;
 }
 
-__global__ void k_unique_write(const u64* __restrict__ key, const int* __restrict__ flag,
-                               const long long* __restrict__ pos, long long n, int nb,
-                               int* __restrict__ adj_u, int* __restrict__ adj) {
+template <typename K>
+__global__ void k_unique_write(const K* __restrict__ key, const int* __restrict__ pos, long long n,
+                               int nb, int* __restrict__ adj_u, int* __restrict__ adj) {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n || !flag[i]) return;
-    const u64 k = key[i];
-    const long long p = pos[i];
+    if (i >= n || pos[i + 1] == pos[i]) return;
+    const K k = key[i];
+    const int p = pos[i];
     adj_u[p] = (int)(k >> nb);
-    adj[p] = (int)(k & ((1ull << nb) - 1));
-}
-
-// head[v] = first adjacency entry of vertex v (lower bound in the sorted adj_u), v in [0, N].
-__global__ void k_heads(const int* __restrict__ adj_u, long long E, int N,
-                        long long* __restrict__ head) {
-    const long long v = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (v > N) return;
-    long long lo = 0, hi = E;
-    while (lo < hi) {
-        const long long mid = (lo + hi) >> 1;
-        if (adj_u[mid] < v) lo = mid + 1;
-        else hi = mid;
-    }
-    head[v] = lo;
+    adj[p] = (int)(k & (((K)1 << nb) - 1));
 }
 
 // ---- 2. rank -----------------------------------------------------------------------------
-__global__ void k_rank_keys(const long long* __restrict__ head, int N, int nb,
-                            u64* __restrict__ key, uint32_t* __restrict__ val) {
+// Degrees; the stable sort keeps vertices of one degree by id.
+__global__ void k_rank_keys(const int* __restrict__ head, int N, uint32_t* __restrict__ key,
+                            uint32_t* __restrict__ val) {
     const long long v = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (v >= N) return;
-    key[v] = (u64)(head[v + 1] - head[v]) << nb | (u64)v;
+    key[v] = (uint32_t)(head[v + 1] - head[v]);
     val[v] = (uint32_t)v;
 }
 
@@ -189,84 +177,14 @@ __global__ void k_root_flags(const uint32_t* __restrict__ order, const int* __re
 }
 
 __global__ void k_root_list(const uint32_t* __restrict__ order, const int* __restrict__ flag,
-                            const long long* __restrict__ pos, int N, int* __restrict__ front,
-                            int* __restrict__ lev, int* __restrict__ seq) {
+                            const int* __restrict__ pos, int N, int* __restrict__ walk,
+                            int* __restrict__ seq) {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= N || !flag[i]) return;
     const int v = (int)order[i];
-    const int p = (int)pos[i];
-    front[p] = v;
-    lev[v] = 0;
+    const int p = pos[i];
+    walk[p] = v;
     seq[v] = p;
-}
-
-__global__ void k_front_degree(const int* __restrict__ front, int f,
-                               const long long* __restrict__ head, long long* __restrict__ fdeg) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < f) {
-        const int v = front[i];
-        fdeg[i] = head[v + 1] - head[v];
-    }
-}
-
-// One thread per (frontier vertex, neighbour) edge.  An unvisited neighbour keeps the smallest
-// frontier index that reaches it; the thread that claims it first appends it to `next`
-// (wave-aggregated counter).  The order of `next` is fixed afterwards by a sort.
-__global__ void k_claim(const int* __restrict__ front, const long long* __restrict__ fofs, int f,
-                        long long Ef, const long long* __restrict__ head,
-                        const int* __restrict__ adj, const int* __restrict__ lev,
-                        int* __restrict__ claim, int* __restrict__ next,
-                        int* __restrict__ count) {
-    const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    bool first = false;
-    int u = 0;
-    if (e < Ef) {
-        int lo = 0, hi = f;  // largest i with fofs[i] <= e
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (fofs[mid] <= e) lo = mid;
-            else hi = mid;
-        }
-        const int v = front[lo];
-        u = adj[head[v] + (e - fofs[lo])];
-        if (lev[u] < 0) first = atomicMin(&claim[u], lo) == INT_MAX;
-    }
-    const u64 m = __ballot(first);
-    if (m == 0) return;
-    const int leader = __ffsll((long long)m) - 1;
-    int base = 0;
-    if (lane_id() == leader) base = atomicAdd(count, __popcll(m));
-    base = __shfl(base, leader);
-    if (first) {
-        const u64 below = lane_id() ? (~0ull >> (64 - lane_id())) : 0ull;
-        next[base + __popcll(m & below)] = u;
-    }
-}
-
-__global__ void k_next_keys(const int* __restrict__ next, int n, const int* __restrict__ claim,
-                            int nb, u64* __restrict__ key, uint32_t* __restrict__ val) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int u = next[i];
-    key[i] = (u64)claim[u] << nb | (u64)u;
-    val[i] = (uint32_t)u;
-}
-
-__global__ void k_group_flags(const u64* __restrict__ key, int n, int nb, int* __restrict__ flag) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) flag[i] = (i == 0 || (key[i] >> nb) != (key[i - 1] >> nb)) ? 1 : 0;
-}
-
-// Children in (parent, ascending id) order, packed as degree << 32 | id for the group sort.
-__global__ void k_group_pack(const int* __restrict__ flag, const long long* __restrict__ pos,
-                             const uint32_t* __restrict__ val, int n,
-                             const long long* __restrict__ head, int* __restrict__ gstart,
-                             u64* __restrict__ packed) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    if (flag[i]) gstart[pos[i]] = (int)i;
-    const uint32_t u = val[i];
-    packed[i] = (u64)(head[u + 1] - head[u]) << 32 | (u64)u;
 }
 
 // std::sort(first, last, [](a, b) { return degree[a] < degree[b]; }) with the steps of GCC 11's
@@ -398,261 +316,29 @@ __device__ __forceinline__ int lg_floor(int n) {
     return lg;
 }
 
-// Ranges of at most this many elements are sorted by one thread; larger ones are partitioned by
-// a work-group first.
-constexpr int kSortSmall = 256;
-
-// One job per child group: (begin, end, partition depth 2 floor(lg n)).
-__global__ void k_group_jobs(const int* __restrict__ gstart, int ngroups, int n,
-                             int4* __restrict__ big, int* __restrict__ nbig,
-                             int4* __restrict__ small, int* __restrict__ nsmall) {
-    const long long g = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= ngroups) return;
-    const int b = gstart[g], e = g + 1 < ngroups ? gstart[g + 1] : n;
-    if (e - b <= 1) return;
-    const int4 job = make_int4(b, e, 2 * lg_floor(e - b), 0);
-    if (e - b > kSortSmall) big[atomicAdd(nbig, 1)] = job;
-    else small[atomicAdd(nsmall, 1)] = job;
-}
-
-// One wave per piece of at most kSortSmall elements, in LDS.  The wave runs the library's
-// introsort loop with wave-wide partition steps (wave_partition_lds) and marks the pieces it
-// leaves (at most 16 elements, or depth exhausted); then each lane finishes the pieces it finds:
-// the insertion pass, or a heapsort.  As in k_bfs_levels, every lane keeps its own identical
-// copy of the range stack, so no branch taken by one lane alone steers the loop.
-constexpr int kSmallSortWaves = 4;
-constexpr unsigned char kPieceNone = 255, kPieceEnd = 254, kPieceHeap = 253;
-
 __device__ __forceinline__ void wave_lds_fence() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// One step of the introsort loop on s[lo, hi) (hi - lo > 16, depth > 0) by one wave: the
-// computation of k_partition_pass on 64 lanes.  lpos and rpos hold the pair positions
-// (K <= (hi - lo) / 2).  Returns the cut in every lane.
-__device__ int wave_partition_lds(u64* s, int lo, int hi, int* lpos, int* rpos, int* lnext) {
-    const int lane = threadIdx.x & 63;
-    if (lane == 0) {
-        ls_median_to_first(s, lo, lo + 1, lo + (hi - lo) / 2, hi - 1);
-        *lnext = INT_MAX;
-    }
-    wave_lds_fence();
-    const uint32_t kp = skey(s[lo]);
-    const int first = lo + 1, n = hi - first;
-    const int per = (n + 63) / 64;
-    const int b0 = min(first + lane * per, hi), b1 = min(b0 + per, hi);
-    int cge = 0, cle = 0;
-    for (int p = b0; p < b1; ++p) {
-        const uint32_t k = skey(s[p]);
-        cge += !(k < kp);
-        cle += !(kp < k);
-    }
-    const int ge_incl = wave_scan(cge, OpAdd{}, 0), le_all = wave_scan(cle, OpAdd{}, 0);
-    const int ge_before = ge_incl - cge, le_before = le_all - cle;
-    const int LE = __builtin_amdgcn_readlane(le_all, 63);
-    int kc = 0;
-    {
-        int rank = ge_before, le_incl = le_before;
-        for (int p = b0; p < b1; ++p) {
-            const uint32_t k = skey(s[p]);
-            le_incl += !(kp < k);
-            if (!(k < kp)) {
-                ++rank;
-                kc += (LE - le_incl >= rank);
-            }
-        }
-    }
-    const int K = __builtin_amdgcn_readlane(wave_scan(kc, OpAdd{}, 0), 63);
-    {
-        int rank = ge_before, le_excl = le_before;
-        for (int p = b0; p < b1; ++p) {
-            const uint32_t k = skey(s[p]);
-            if (!(k < kp)) {
-                ++rank;
-                if (rank <= K) lpos[rank - 1] = p;
-                else if (rank == K + 1) *lnext = p;
-            }
-            if (!(kp < k)) {
-                const int rr = LE - le_excl;
-                if (rr <= K) rpos[rr - 1] = p;
-                ++le_excl;
-            }
-        }
-    }
-    wave_lds_fence();
-    for (int r = lane; r < K; r += 64) {
-        const int x = lpos[r], y = rpos[r];
-        const u64 ax = s[x], ay = s[y];
-        s[x] = ay;
-        s[y] = ax;
-    }
-    wave_lds_fence();
-    return K == 0 ? *lnext : min(*lnext, rpos[K - 1]);
-}
-
-__global__ __launch_bounds__(64 * kSmallSortWaves) void k_small_sort(
-    const int4* __restrict__ jobs, int njobs, u64* __restrict__ a) {
-    __shared__ u64 piece[kSmallSortWaves][kSortSmall];
-    __shared__ unsigned char marks[kSmallSortWaves][kSortSmall + 4];
-    __shared__ int pairs[kSmallSortWaves][kSortSmall];  // lpos, then rpos
-    __shared__ int lnext[kSmallSortWaves];
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const long long j = (long long)blockIdx.x * kSmallSortWaves + w;
-    if (j >= njobs) return;  // the same for every lane of the wave
-    const int4 job = jobs[j];
-    const int n = job.y - job.x;  // at most kSortSmall
-    if (n <= 1) return;
-    u64* s = piece[w];
-    unsigned char* mark = marks[w];
-    for (int i = lane; i < n; i += 64) s[i] = a[job.x + i];
-    for (int i = lane; i < n; i += 64) mark[i] = kPieceNone;
-    if (lane == 0) mark[n] = kPieceEnd;
-    wave_lds_fence();
-    int4 stk[64];  // depth <= 2 floor(lg n) < 63 for n < 2^31
-    int sp = 1;
-    stk[0] = make_int4(0, n, job.z, 0);
-    while (sp > 0) {
-        const int4 r = stk[sp - 1];
-        if (r.y - r.x <= 16 || r.z == 0) {
-            mark[r.x] = r.y - r.x > 16 ? kPieceHeap : (unsigned char)r.z;
-            --sp;
-        } else {
-            const int cut = wave_partition_lds(s, r.x, r.y, pairs[w], pairs[w] + kSortSmall / 2,
-                                               &lnext[w]);
-            stk[sp - 1] = make_int4(cut, r.y, r.z - 1, 0);
-            stk[sp] = make_int4(r.x, cut, r.z - 1, 0);
-            ++sp;
-        }
-    }
-    wave_lds_fence();
-    for (int i = lane; i < n; i += 64) {
-        const int m = mark[i];
-        if (m <= kPieceHeap) {
-            int e = i + 1;
-            while (mark[e] == kPieceNone) ++e;
-            if (m == kPieceHeap) ls_heapsort(s, i, e);
-            else if (e - i > 1) ls_sort_range(s, i, e, m);
-        }
-    }
-    wave_lds_fence();
-    for (int i = lane; i < n; i += 64) a[job.x + i] = s[i];
-}
-
-// One step of the introsort loop on a large range, by a whole work-group, with the same result
-// as the library's sequential step.  After the median of three is moved to a[lo], the Hoare
-// scans over a[lo+1, hi) stop, from the left, at elements whose key is not below the pivot's
-// (l_1 < l_2 < ...) and, from the right, at elements whose key is not above it
-// (r_1 > r_2 > ...); the k-th swap exchanges a[l_k] and a[r_k] while l_k < r_k, so K = the
-// number of left stops x with at least rank(x) right stops after x; the cut is l_1 when K = 0,
-// else min(l_{K+1}, r_K).  Both parts continue with depth - 1; a range at depth 0 is heapsorted.
-__global__ __launch_bounds__(256) void k_partition_pass(
-    const int4* __restrict__ jobs, int4* __restrict__ next, int* __restrict__ nnext,
-    int4* __restrict__ small, int* __restrict__ nsmall, u64* a, int* __restrict__ lpos,
-    int* __restrict__ rpos) {
-    __shared__ int wsum[4];
-    __shared__ int sh_lnext;
-    const int4 job = jobs[blockIdx.x];
-    const int lo = job.x, hi = job.y, depth = job.z;
-    const int t = threadIdx.x;
-    if (depth == 0) {
-        if (t == 0) ls_heapsort(a, lo, hi);  // sorted: the insertion pass would change nothing
-        return;
-    }
-    if (t == 0) {
-        ls_median_to_first(a, lo, lo + 1, lo + (hi - lo) / 2, hi - 1);
-        sh_lnext = INT_MAX;
-    }
-    __syncthreads();
-    const uint32_t kp = skey(a[lo]);
-    const int first = lo + 1, n = hi - first;
-    const int per = (n + 255) / 256;
-    const int b0 = min(first + t * per, hi), b1 = min(b0 + per, hi);
-    int cge = 0, cle = 0;
-    for (int p = b0; p < b1; ++p) {
-        const uint32_t k = skey(a[p]);
-        cge += !(k < kp);
-        cle += !(kp < k);
-    }
-    int GE, LE;
-    const int ge_before = block_scan_256(cge, OpAdd{}, 0, wsum, GE) - cge;
-    const int le_before = block_scan_256(cle, OpAdd{}, 0, wsum, LE) - cle;
-    (void)GE;
-    // K: left stops x (rank r) with LE - (right stops at or before x) >= r.
-    int kc = 0;
-    {
-        int rank = ge_before, le_incl = le_before;
-        for (int p = b0; p < b1; ++p) {
-            const uint32_t k = skey(a[p]);
-            le_incl += !(kp < k);
-            if (!(k < kp)) {
-                ++rank;
-                kc += (LE - le_incl >= rank);
-            }
-        }
-    }
-    int K;
-    block_scan_256(kc, OpAdd{}, 0, wsum, K);
-    // Pair positions: lpos[lo + r - 1] = l_r, rpos[lo + r - 1] = r_r for r <= K; and l_{K+1}.
-    {
-        int rank = ge_before, le_excl = le_before;
-        for (int p = b0; p < b1; ++p) {
-            const uint32_t k = skey(a[p]);
-            if (!(k < kp)) {
-                ++rank;
-                if (rank <= K) lpos[lo + rank - 1] = p;
-                else if (rank == K + 1) sh_lnext = p;
-            }
-            if (!(kp < k)) {
-                const int rr = LE - le_excl;  // right stops in [p, hi)
-                if (rr <= K) rpos[lo + rr - 1] = p;
-                ++le_excl;
-            }
-        }
-    }
-    __syncthreads();
-    for (int r = t; r < K; r += 256) {
-        const int x = lpos[lo + r], y = rpos[lo + r];
-        const u64 ax = a[x], ay = a[y];
-        a[x] = ay;
-        a[y] = ax;
-    }
-    if (t == 0) {
-        const int cut = K == 0 ? sh_lnext : min(sh_lnext, rpos[lo + K - 1]);
-        const int d = depth - 1;
-        const int4 left = make_int4(lo, cut, d, 0), right = make_int4(cut, hi, d, 0);
-        if (cut - lo > kSortSmall) next[atomicAdd(nnext, 1)] = left;
-        else small[atomicAdd(nsmall, 1)] = left;
-        if (hi - cut > kSortSmall) next[atomicAdd(nnext, 1)] = right;
-        else small[atomicAdd(nsmall, 1)] = right;
-    }
-}
-
-__global__ void k_level_write(const u64* __restrict__ packed, int n, int level, int base,
-                              int* __restrict__ front, int* __restrict__ lev,
-                              int* __restrict__ seq) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int u = (int)(uint32_t)packed[i];
-    front[i] = u;
-    lev[u] = level;
-    seq[u] = base + (int)i;
-}
-
-// ---- 4b. small levels in one work-group ---------------------------------------------------
+// The walk.  walk[i] = the vertex of place i, seq[v] = v's place or -1; a level's frontier is the
+// last f vertices placed.  state = {frontier size, vertices placed, level, finished}.  A vertex
+// reached from several frontier vertices belongs to the one of the lowest place: claim[u] = the
+// smallest place of a frontier vertex adjacent to u, taken only while u has no place, so
+// claim[u] == place tells a parent its children, in every later kernel of the level.
+//
+// ---- 4a. small levels in one work-group ---------------------------------------------------
 // While a level has at most kBfsCap frontier vertices and frontier edges, one work-group runs
-// level after level with no host round trip: each frontier edge claims its neighbour (atomic
-// minimum of the frontier index, as k_claim), then an edge holds a child when its frontier
-// vertex won the claim.  Frontier vertices are in level order and each adjacency list is in
-// ascending id, so an exclusive scan over the edges places the children in (parent index,
-// ascending id) order directly; each parent's children are then sorted by degree with
-// std::sort's steps in LDS: groups of up to kBfsSortSmall by their parent's thread, larger ones
-// (the children of hub vertices) partitioned by the whole work-group, a step at a time as
-// k_partition_pass does, and the pieces finished by one thread each.  Thread t owns a contiguous run of up to
+// level after level with no host round trip: each frontier edge claims its neighbour, then an
+// edge holds a child when its frontier vertex won the claim.  Frontier vertices are in level order
+// and each adjacency list is in ascending id, so an exclusive scan over the edges places the
+// children in (parent index, ascending id) order directly; each parent's children are then sorted
+// by degree with std::sort's steps in LDS: groups of up to kBfsSortSmall by their parent's thread,
+// larger ones (the children of hub vertices) partitioned by the whole work-group, a step at a
+// time, and the pieces finished by one thread each.  Thread t owns a contiguous run of up to
 // kBfsPer vertices or edges, so each phase needs one block scan.  The work-group stops at the
-// first level that does not fit (state.w = 0: the frontier is left in front[]) or when the walk
-// ends (state.w = 1).  state = {frontier size, vertices placed, level, finished}.
+// first level that does not fit (state.w = 0) or when the walk ends (state.w = 1).
 constexpr int kBfsThreads = 1024;
 constexpr int kBfsPer = 8;
 constexpr int kBfsCap = kBfsThreads * kBfsPer;
@@ -679,72 +365,200 @@ __device__ __forceinline__ int block_scan_int(int x, int* wsum /* LDS[NW] */, in
     return before + incl;
 }
 
-// One step of the introsort loop on a[lo, hi) (depth > 0) by the whole work-group, with the
-// library's result: k_partition_pass's computation on an LDS range.  lpos and rpos hold the
-// pair positions relative to the range (K <= (hi - lo) / 2, as the pairs are disjoint).
-// Returns the cut (the same value in every thread).
 template <int NW>
-__device__ int block_partition_lds(u64* a, int lo, int hi, int* lpos, int* rpos, int* wsum,
-                                   int* lnext) {
-    const int t = threadIdx.x;
+__device__ __forceinline__ void team_sync() {
+    if constexpr (NW == 1) wave_lds_fence();
+    else __syncthreads();
+}
+
+// One step of the introsort loop on a[lo, hi) (depth > 0), in LDS or memory, by NW waves (one: a
+// wave on its own; more: the whole work-group), with the same result as the library's sequential
+// step.  After the median of three is moved to a[lo], the Hoare scans over a[lo+1, hi) stop, from
+// the left, at elements whose key is not below the pivot's (l_1 < l_2 < ...) and, from the right,
+// at elements whose key is not above it (r_1 > r_2 > ...); the k-th swap exchanges a[l_k] and
+// a[r_k] while l_k < r_k, so K = the number of left stops x with at least rank(x) right stops
+// after x; the cut is l_1 when K = 0, else min(l_{K+1}, r_K).  Both parts continue with depth - 1;
+// a range at depth 0 is heapsorted.  Each wave counts and ranks a run of its own by ballots.
+// lpos and rpos hold the pair positions (K <= (hi - lo) / 2, as the pairs are disjoint); part (NW
+// entries) and lnext are LDS of the team.  Returns the cut (the same value in every thread).
+template <int NW>
+__device__ int partition_step(u64* a, int lo, int hi, int* lpos, int* rpos, int2* part,
+                              int* lnext) {
+    const int lane = threadIdx.x & 63, w = NW == 1 ? 0 : (int)(threadIdx.x >> 6);
+    const int t = NW == 1 ? lane : (int)threadIdx.x;
     if (t == 0) {
         ls_median_to_first(a, lo, lo + 1, lo + (hi - lo) / 2, hi - 1);
         *lnext = INT_MAX;
     }
-    __syncthreads();
+    team_sync<NW>();
     const uint32_t kp = skey(a[lo]);
     const int first = lo + 1, n = hi - first;
-    const int per = (n + kBfsThreads - 1) / kBfsThreads;
-    const int b0 = min(first + t * per, hi), b1 = min(b0 + per, hi);
+    const int per = ((n + NW - 1) / NW + 63) / 64 * 64;
+    const int b0 = min(first + w * per, hi), b1 = min(b0 + per, hi);
+    const u64 below = lane ? (~0ull >> (64 - lane)) : 0ull;
+    // masks of the left and right stops among the 64 elements at p
+    const auto stops = [&](int p, u64& ge, u64& le) {
+        const bool in = p + lane < b1;
+        const uint32_t k = in ? skey(a[p + lane]) : 0u;
+        ge = __ballot(in && !(k < kp));
+        le = __ballot(in && !(kp < k));
+    };
+    u64 ge, le;
     int cge = 0, cle = 0;
-    for (int p = b0; p < b1; ++p) {
-        const uint32_t k = skey(a[p]);
-        cge += !(k < kp);
-        cle += !(kp < k);
+    for (int p = b0; p < b1; p += 64) {
+        stops(p, ge, le);
+        cge += __popcll(ge);
+        cle += __popcll(le);
     }
-    int GE, LE;
-    const int ge_before = block_scan_int<NW>(cge, wsum, GE) - cge;
-    const int le_before = block_scan_int<NW>(cle, wsum, LE) - cle;
-    int kc = 0;
+    int ge_before = 0, le_before = 0, LE = cle;
+    if constexpr (NW > 1) {
+        if (lane == 0) part[w] = make_int2(cge, cle);
+        __syncthreads();
+        LE = 0;
+        for (int i = 0; i < NW; ++i) {
+            const int2 x = part[i];
+            ge_before += i < w ? x.x : 0;
+            le_before += i < w ? x.y : 0;
+            LE += x.y;
+        }
+        __syncthreads();
+    }
+    int K = 0;
     {
-        int rank = ge_before, le_incl = le_before;
-        for (int p = b0; p < b1; ++p) {
-            const uint32_t k = skey(a[p]);
-            le_incl += !(kp < k);
-            if (!(k < kp)) {
-                ++rank;
-                kc += (LE - le_incl >= rank);
-            }
+        int g = ge_before, l = le_before;
+        for (int p = b0; p < b1; p += 64) {
+            stops(p, ge, le);
+            const int rank = g + __popcll(ge & below) + 1;
+            const int le_incl = l + __popcll(le & below) + (int)((le >> lane) & 1);
+            K += __popcll(__ballot(((ge >> lane) & 1) && LE - le_incl >= rank));
+            g += __popcll(ge);
+            l += __popcll(le);
         }
     }
-    int K;
-    block_scan_int<NW>(kc, wsum, K);
+    if constexpr (NW > 1) {
+        if (lane == 0) part[w].x = K;
+        __syncthreads();
+        K = 0;
+        for (int i = 0; i < NW; ++i) K += part[i].x;
+    }
     {
-        int rank = ge_before, le_excl = le_before;
-        for (int p = b0; p < b1; ++p) {
-            const uint32_t k = skey(a[p]);
-            if (!(k < kp)) {
-                ++rank;
-                if (rank <= K) lpos[rank - 1] = p;
-                else if (rank == K + 1) *lnext = p;
+        int g = ge_before, l = le_before;
+        for (int p = b0; p < b1; p += 64) {
+            stops(p, ge, le);
+            if ((ge >> lane) & 1) {
+                const int rank = g + __popcll(ge & below) + 1;
+                if (rank <= K) lpos[rank - 1] = p + lane;
+                else if (rank == K + 1) *lnext = p + lane;
             }
-            if (!(kp < k)) {
-                const int rr = LE - le_excl;
-                if (rr <= K) rpos[rr - 1] = p;
-                ++le_excl;
+            if ((le >> lane) & 1) {
+                const int rr = LE - (l + __popcll(le & below));
+                if (rr <= K) rpos[rr - 1] = p + lane;
             }
+            g += __popcll(ge);
+            l += __popcll(le);
         }
     }
-    __syncthreads();
-    for (int r = t; r < K; r += kBfsThreads) {
+    team_sync<NW>();
+    for (int r = t; r < K; r += 64 * NW) {
         const int x = lpos[r], y = rpos[r];
         const u64 ax = a[x], ay = a[y];
         a[x] = ay;
         a[y] = ax;
     }
     const int cut = K == 0 ? *lnext : min(*lnext, rpos[K - 1]);
-    __syncthreads();
+    team_sync<NW>();
     return cut;
+}
+
+// The partition steps of std::sort on a[lo, hi) from partition depth `depth`: leaf(lo, hi, depth)
+// for every piece of at most `stop` elements, or of any size with the depth used up.
+// Every thread runs the same stack of ranges (lo, hi, depth) in its own registers: its control flow
+// depends only on values all threads share (the ranges and the cuts), and no branch taken by one
+// thread alone decides what the others do next (with the stack in LDS and thread 0 alone updating
+// it, the compiler moved that update out of the loop for thread 0, and the other threads never saw
+// it).
+template <int NW, typename Leaf>
+__device__ void partition_range(u64* a, int lo, int hi, int depth, int stop, int* lpos, int* rpos,
+                                int2* part, int* lnext, Leaf&& leaf) {
+    int4 stk[64];  // depth <= 2 floor(lg n) <= 62 for n < 2^31
+    int sp = 1;
+    stk[0] = make_int4(lo, hi, depth, 0);
+    while (sp > 0) {
+        const int4 r = stk[sp - 1];
+        if (r.y - r.x <= stop || r.z == 0) {
+            leaf(r.x, r.y, r.z);
+            --sp;
+        } else {
+            const int cut = partition_step<NW>(a, r.x, r.y, lpos, rpos, part, lnext);
+            stk[sp - 1] = make_int4(cut, r.y, r.z - 1, 0);
+            stk[sp] = make_int4(r.x, cut, r.z - 1, 0);
+            ++sp;
+        }
+    }
+}
+
+// Sorting a group in LDS takes three widths: the work-group partitions ranges down to kWavePiece
+// elements, each wave partitions pieces that start in its part of the array down to kBfsSortSmall,
+// and one thread finishes each of those.  mark[i] (one byte an element) says what starts at i: the
+// partition depth a piece continues from, or one of the marks above.
+constexpr int kWavePiece = 512;
+
+template <int NW>
+__device__ void mark_group(u64* a, int lo, int hi, int depth, unsigned char* mark, int* lpos,
+                           int* rpos, int2* part, int* lnext) {
+    partition_range<NW>(a, lo, hi, depth, kWavePiece, lpos, rpos, part, lnext,
+                        [&](int x, int y, int d) {
+                            mark[x] = y - x > kWavePiece ? kMarkHeap : (unsigned char)d;
+                        });
+}
+
+// Pieces of a[0, n) (n <= kBfsCap) above kBfsSortSmall elements partitioned by waves; lnext: one
+// LDS word a wave.  Each wave notes the pieces that start in its part before any wave marks more.
+template <int NW>
+__device__ void wave_pieces(u64* a, int n, unsigned char* mark, int* lpos, int* rpos, int* lnext) {
+    constexpr int P = kBfsCap / NW / 64;
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, base = w * P * 64;
+    u64 starts[P];
+#pragma unroll
+    for (int k = 0; k < P; ++k) {
+        const int i = base + 64 * k + lane;
+        starts[k] = __ballot(i < n && mark[i] < kMarkHeap);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < P; ++k) {
+        while (starts[k]) {
+            const int lo = base + 64 * k + (int)__builtin_ctzll(starts[k]);
+            starts[k] &= starts[k] - 1;
+            int hi = lo + 1;  // the next mark, or n
+            for (;;) {
+                const u64 m = __ballot(hi + lane >= n || mark[hi + lane] != kMarkNone);
+                if (m) {
+                    hi += (int)__builtin_ctzll(m);
+                    break;
+                }
+                hi += 64;
+            }
+            if (hi - lo <= kBfsSortSmall) continue;
+            partition_range<1>(a, lo, hi, (int)mark[lo], kBfsSortSmall, lpos + lo / 2,
+                               rpos + lo / 2, nullptr, lnext + w, [&](int x, int y, int d) {
+                                   mark[x] = y - x > kBfsSortSmall ? kMarkHeap : (unsigned char)d;
+                               });
+        }
+    }
+    __syncthreads();
+}
+
+// Finishes the marked pieces of a[lo, hi): std::sort's insertion pass, or its heapsort.
+__device__ void finish_pieces(u64* a, int lo, int hi, const unsigned char* mark) {
+    for (int i = lo + (int)threadIdx.x; i < hi; i += kBfsThreads) {
+        const int m = mark[i];
+        if (m > kMarkHeap) continue;
+        int e = i + 1;
+        while (e < hi && mark[e] == kMarkNone) ++e;  // the group's end is marked
+        if (m == kMarkHeap) ls_heapsort(a, i, e);    // depth exhausted
+        else if (e - i > 1) ls_sort_range(a, i, e, m);
+    }
 }
 
 // A walk of N vertices has at most N levels after the roots; the loop runs to `max_level` at
@@ -752,24 +566,25 @@ __device__ int block_partition_lds(u64* a, int lo, int hi, int* lpos, int* rpos,
 constexpr int kBfsOverrun = 2;
 
 __global__ __launch_bounds__(kBfsThreads) void k_bfs_levels(
-    int* __restrict__ front, const long long* __restrict__ head, const int* __restrict__ adj,
-    int* __restrict__ lev, int* __restrict__ seq, int* claim, int N, long long max_level,
-    int4* __restrict__ state) {
+    int* __restrict__ walk, const int* __restrict__ head, const int* __restrict__ adj,
+    int* __restrict__ seq, int* claim, int N, long long max_level, int4* __restrict__ state) {
     constexpr int NW = kBfsThreads / 64;
     __shared__ int s_ofs[kBfsCap + 1];    // edge offset of each frontier vertex
     __shared__ int s_fx[kBfsCap + 1];     // the frontier; then children before each edge
     __shared__ u64 s_packed[kBfsCap];     // degree << 32 | id of the next level
     __shared__ int s_wsum[NW];
     __shared__ int2 s_big[kBfsMaxBig];  // child groups larger than kBfsSortSmall
-    __shared__ int s_nbig, s_lnext;
+    __shared__ int s_nbig, s_lnext[NW];
+    __shared__ int2 s_part[NW];
     int* const s_front = s_fx;
     int* const s_ex = s_fx;
     unsigned char* const s_mark = reinterpret_cast<unsigned char*>(s_fx);  // during the sort
     const int t = threadIdx.x;
     const int4 s0 = *state;
     int f = s0.x, base = s0.y, level = s0.z;
-    bool finished = false, moved = false, overrun = false;
-    for (int i = t; i < f; i += kBfsThreads) s_front[i] = front[i];
+    if (s0.w || f > kBfsCap) return;
+    bool finished = false, overrun = false;
+    for (int i = t; i < f; i += kBfsThreads) s_front[i] = walk[base - f + i];
     // `level` is the same in every thread: the bound ends the loop for all of them at once.
     for (;;) {
         __syncthreads();
@@ -791,7 +606,7 @@ __global__ __launch_bounds__(kBfsThreads) void k_bfs_levels(
             deg[i] = 0;
             if (v0 + i < v1) {
                 const int v = s_front[v0 + i];
-                deg[i] = (int)min(head[v + 1] - head[v], (long long)kBfsCap + 1);
+                deg[i] = min(head[v + 1] - head[v], kBfsCap + 1);
                 dsum += deg[i];
             }
         }
@@ -830,10 +645,10 @@ __global__ __launch_bounds__(kBfsThreads) void k_bfs_levels(
                     while (s_ofs[lo + 1] <= e) ++lo;
                     const int v = s_front[lo];
                     const int u = adj[head[v] + (e - s_ofs[lo])];
-                    if (lev[u] < 0) {
-                        atomicMin(&claim[u], lo);
+                    if (seq[u] < 0) {
+                        los[i] = base - f + lo;
+                        atomicMin(&claim[u], los[i]);
                         us[i] = u;
-                        los[i] = lo;
                     }
                 }
             }
@@ -877,68 +692,337 @@ __global__ __launch_bounds__(kBfsThreads) void k_bfs_levels(
             for (int i = t; i <= n; i += kBfsThreads) s_mark[i] = kMarkNone;
             __syncthreads();
             for (int g = t; g < nbig; g += kBfsThreads) s_mark[s_big[g].y] = kMarkGroupEnd;
-            // Every thread runs the same stack of ranges (lo, hi, depth) in its own registers:
-            // its control flow depends only on values all threads share (the ranges and the
-            // cuts), and no branch taken by one thread alone decides what the others do next
-            // (with the stack in LDS and thread 0 alone updating it, the compiler moved that
-            // update out of the loop for thread 0, and the other threads never saw it).
             for (int g = 0; g < nbig; ++g) {
                 __syncthreads();
                 const int2 gr = s_big[g];
-                int4 stk[2 * 13 + 2];  // depth 2 floor(lg n) <= 26 for n <= kBfsCap
-                int sp = 1;
-                stk[0] = make_int4(gr.x, gr.y, 2 * lg_floor(gr.y - gr.x), 0);
-                while (sp > 0) {
-                    const int4 r = stk[sp - 1];
-                    if (r.y - r.x <= kBfsSortSmall || r.z == 0) {
-                        // a piece to finish after the loop, by the thread that finds its mark
-                        s_mark[r.x] = r.y - r.x > kBfsSortSmall ? kMarkHeap : (unsigned char)r.z;
-                        --sp;
-                    } else {
-                        const int cut = block_partition_lds<NW>(
-                            s_packed, r.x, r.y, s_ofs, s_ofs + kBfsCap / 2, s_wsum, &s_lnext);
-                        stk[sp - 1] = make_int4(cut, r.y, r.z - 1, 0);
-                        stk[sp] = make_int4(r.x, cut, r.z - 1, 0);
-                        ++sp;
-                    }
-                }
+                mark_group<NW>(s_packed, gr.x, gr.y, 2 * lg_floor(gr.y - gr.x), s_mark, s_ofs,
+                               s_ofs + kBfsCap / 2, s_part, s_lnext);
             }
             __syncthreads();
-            for (int i = t; i < n; i += kBfsThreads) {
-                const int m = s_mark[i];
-                if (m <= kMarkHeap) {
-                    int e = i + 1;
-                    while (e < n && s_mark[e] == kMarkNone) ++e;  // the group's end is marked
-                    if (m == kMarkHeap) ls_heapsort(s_packed, i, e);  // depth exhausted
-                    else if (e - i > 1) ls_sort_range(s_packed, i, e, m);
-                }
-            }
+            wave_pieces<NW>(s_packed, n, s_mark, s_ofs, s_ofs + kBfsCap / 2, s_lnext);
+            finish_pieces(s_packed, 0, n, s_mark);
         }
         __syncthreads();
         for (int i = t; i < n; i += kBfsThreads) {
             const int w = (int)(uint32_t)s_packed[i];
             s_front[i] = w;
-            lev[w] = level;
+            walk[base + i] = w;
             seq[w] = base + i;
         }
         base += n;
         f = n;
         ++level;
-        moved = true;
     }
-    if (moved)
-        for (int i = t; i < f; i += kBfsThreads) front[i] = s_front[i];
     if (t == 0) *state = make_int4(f, base, level, overrun ? kBfsOverrun : finished ? 1 : 0);
 }
 
+// ---- 4b. a level of any size, four kernels over its edges ----------------------------------
+// Work-groups own contiguous runs of frontier vertices (level_run), waves eight of them at a time:
+// the wave's lanes go over the eight adjacency lists end to end (WaveEdges), so a hub's list is
+// spread over the lanes and short lists share a round.  An edge's place among its work-group's
+// edges is then also its children's order: (parent, ascending id).
+// With sizes known to the host a level took ~20 kernels (a radix sort of (parent, id) keys, scans,
+// sorts of the groups) and four host round trips: the ordering of a 27-point mesh 64^3 in random
+// numbering, 53 levels above 8192 edges, 14.3 -> 3.6 ms, its relabelling included.
+constexpr int kLevelBlocks = 1024, kLevelWaves = 4, kLevelVerts = 8;
+constexpr int kLevelStage = 512;  // children a wave sorts in LDS at a time
+
+__device__ __forceinline__ bool level_over(const int4& s, long long max_level) {
+    return s.w || s.x == 0 || s.z > max_level;
+}
+
+// The frontier vertices [x, y) of this work-group.
+__device__ __forceinline__ int2 level_run(int f) {
+    constexpr int step = kLevelWaves * kLevelVerts;
+    const int per = ((f + kLevelBlocks - 1) / kLevelBlocks + step - 1) / step * step;
+    const long long b = (long long)blockIdx.x * per;
+    return make_int2((int)min(b, (long long)f), (int)min(b + per, (long long)f));
+}
+
+// The edges of frontier vertices v0 .. v1 - 1 (at most kLevelVerts), end to end.  Lanes past the
+// last vertex hold excl = total, so vertex() never picks them for e < total; of equal excl the last
+// holds the edge, the lists before it being empty.
+struct WaveEdges {
+    int begin, excl, total;  // lane i < 8: its vertex's list, and the edges before it
+    __device__ __forceinline__ WaveEdges(const int* walk, const int* head, int at, int v0, int v1) {
+        const int lane = threadIdx.x & 63;
+        int deg = 0;
+        begin = 0;
+        if (v0 + lane < v1) {
+            const int v = walk[at + v0 + lane];
+            begin = head[v];
+            deg = head[v + 1] - begin;
+        }
+        const int incl = wave_scan(deg, OpAdd{}, 0);
+        excl = incl - deg;
+        total = wave_last(incl);
+    }
+    // The vertex (0 .. 7) of edge e < total, and the edge's index in adj: every lane together.
+    __device__ __forceinline__ int vertex(int e, int& index) const {
+        int v = 0;
+#pragma unroll
+        for (int step = kLevelVerts / 2; step > 0; step >>= 1)
+            if (__shfl(excl, v + step) <= e) v += step;
+        index = __shfl(begin, v) + e - __shfl(excl, v);
+        return v;
+    }
+    // f(neighbour, vertex, whether the lane holds an edge) for 64 edges at a time, in order.  The
+    // loop waits for memory: U rounds' neighbours, and what `also` loads for each, are in flight
+    // at once (eight rounds where a hub makes the lists long).
+    template <int U, typename Also, typename F>
+    __device__ __forceinline__ void rounds(const int* adj, Also&& also, F&& f) const {
+        const int lane = threadIdx.x & 63;
+        for (int e0 = 0; e0 < total; e0 += 64 * U) {
+            int u[U], v[U], x[U];
+#pragma unroll
+            for (int q = 0; q < U; ++q) {
+                int index;
+                v[q] = vertex(min(e0 + 64 * q + lane, total - 1), index);
+                u[q] = adj[index];
+            }
+#pragma unroll
+            for (int q = 0; q < U; ++q) x[q] = also(u[q]);
+#pragma unroll
+            for (int q = 0; q < U; ++q)
+                if (e0 + 64 * q < total) f(u[q], v[q], x[q], e0 + 64 * q + lane < total);
+        }
+    }
+    template <typename Also, typename F>
+    __device__ __forceinline__ void each(const int* adj, Also&& also, F&& f) const {
+        if (total <= 512) rounds<4>(adj, also, f);
+        else rounds<8>(adj, also, f);
+    }
+};
+
+__global__ __launch_bounds__(64 * kLevelWaves) void k_level_claim(
+    const int* __restrict__ walk, const int* __restrict__ head, const int* __restrict__ adj,
+    const int* __restrict__ seq, int* claim, const int4* __restrict__ state, long long max_level,
+    int* __restrict__ njobs) {
+    const int4 s = *state;
+    if (blockIdx.x == 0 && threadIdx.x < 2) njobs[threadIdx.x] = 0;
+    if (level_over(s, max_level)) return;
+    const int2 run = level_run(s.x);
+    const int at = s.y - s.x, w = threadIdx.x >> 6;
+    for (int v0 = run.x + w * kLevelVerts; v0 < run.y; v0 += kLevelWaves * kLevelVerts) {
+        const WaveEdges E(walk, head, at, v0, min(v0 + kLevelVerts, run.y));
+        E.each(adj, [&](int u) { return seq[u]; },
+               [&](int u, int v, int place, bool edge) {
+                   if (edge && place < 0) atomicMin(&claim[u], at + v0 + v);
+               });
+    }
+}
+
+// Children of each work-group's run.
+__global__ __launch_bounds__(64 * kLevelWaves) void k_level_count(
+    const int* __restrict__ walk, const int* __restrict__ head, const int* __restrict__ adj,
+    const int* __restrict__ claim, const int4* __restrict__ state, long long max_level,
+    int* __restrict__ block_children) {
+    __shared__ int total;
+    const int4 s = *state;
+    if (level_over(s, max_level)) return;
+    if (threadIdx.x == 0) total = 0;
+    __syncthreads();
+    const int2 run = level_run(s.x);
+    const int at = s.y - s.x, w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    int n = 0;
+    for (int v0 = run.x + w * kLevelVerts; v0 < run.y; v0 += kLevelWaves * kLevelVerts) {
+        const WaveEdges E(walk, head, at, v0, min(v0 + kLevelVerts, run.y));
+        E.each(adj, [&](int u) { return claim[u]; },
+               [&](int, int v, int place, bool edge) {
+                   n += __popcll(__ballot(edge && place == at + v0 + v));
+               });
+    }
+    if (lane == 0 && n) atomicAdd(&total, n);
+    __syncthreads();
+    if (threadIdx.x == 0) block_children[blockIdx.x] = total;
+}
+
+// Places the children: packed degree << 32 | id in child[], in (parent, ascending id) order.  A
+// wave's children are staged in LDS, where each vertex's are sorted by one lane, and take their
+// places; vertices with more than kBfsSortSmall children, and all of a wave with more than
+// kLevelStage, become jobs {begin, end, partition depth} for k_level_sort.  The next state goes to `next`.
+__global__ __launch_bounds__(64 * kLevelWaves) void k_level_place(
+    int* walk, const int* __restrict__ head, const int* __restrict__ adj, int* seq,
+    const int* __restrict__ claim, const int4* __restrict__ state, int4* __restrict__ next,
+    long long max_level, const int* __restrict__ block_children, u64* __restrict__ child,
+    int4* __restrict__ jobs, int* __restrict__ njobs) {
+    __shared__ u64 s_stage[kLevelWaves][kLevelStage];
+    __shared__ int s_cnt[kLevelWaves][kLevelVerts];
+    __shared__ int s_round[2][kLevelWaves];
+    __shared__ int s_before, s_all;
+    const int4 s = *state;
+    if (level_over(s, max_level)) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) *next = make_int4(s.x, s.y, s.z, s.w | (s.x == 0));
+        return;
+    }
+    const int t = threadIdx.x, w = t >> 6, lane = t & 63;
+    if (t == 0) s_before = s_all = 0;
+    __syncthreads();
+    {
+        int before = 0, all = 0;
+        for (int b = t; b < kLevelBlocks; b += 64 * kLevelWaves) {
+            const int c = block_children[b];
+            all += c;
+            if (b < (int)blockIdx.x) before += c;
+        }
+        before = wave_last(wave_scan(before, OpAdd{}, 0));
+        all = wave_last(wave_scan(all, OpAdd{}, 0));
+        if (lane == 0) {
+            atomicAdd(&s_before, before);
+            atomicAdd(&s_all, all);
+        }
+    }
+    __syncthreads();
+    if (blockIdx.x == 0 && t == 0)
+        *next = make_int4(s_all, s.y + s_all, s.z + 1, s_all == 0);
+    const int2 run = level_run(s.x);
+    const int at = s.y - s.x;
+    int out = s_before, phase = 0;  // children before this round's vertices
+    const u64 below = lane ? (~0ull >> (64 - lane)) : 0ull;
+    for (int r0 = run.x; r0 < run.y; r0 += kLevelWaves * kLevelVerts, phase ^= 1) {
+        const int v0 = min(r0 + w * kLevelVerts, run.y), v1 = min(v0 + kLevelVerts, run.y);
+        const WaveEdges E(walk, head, at, v0, v1);
+        if (lane < kLevelVerts) s_cnt[w][lane] = 0;
+        wave_lds_fence();
+        // the wave's children, staged as far as they fit
+        int n = 0;
+        E.each(adj, [&](int u) { return claim[u]; },
+               [&](int u, int v, int place, bool edge) {
+                   const bool mine = edge && place == at + v0 + v;
+                   const u64 m = __ballot(mine);
+                   if (mine) {
+                       atomicAdd(&s_cnt[w][v], 1);
+                       const int p = n + __popcll(m & below);
+                       if (p < kLevelStage)
+                           s_stage[w][p] =
+                               (u64)(uint32_t)(head[u + 1] - head[u]) << 32 | (uint32_t)u;
+                   }
+                   n += __popcll(m);
+               });
+        if (lane == 0) s_round[phase][w] = n;
+        __syncthreads();
+        int mine_at = out, round = 0;
+        for (int x = 0; x < kLevelWaves; ++x) {
+            if (x < w) mine_at += s_round[phase][x];
+            round += s_round[phase][x];
+        }
+        out += round;
+        const int cnt = lane < kLevelVerts ? s_cnt[w][lane] : 0;
+        const int first = wave_scan(cnt, OpAdd{}, 0) - cnt;  // lane i < 8: its children's start
+        if (n <= kLevelStage) {
+            if (cnt > kBfsSortSmall)
+                jobs[atomicAdd(njobs, 1)] =
+                    make_int4(mine_at + first, mine_at + first + cnt, 2 * lg_floor(cnt), 0);
+            else if (cnt > 1)
+                ls_sort_range(s_stage[w], first, first + cnt, 2 * lg_floor(cnt));
+            wave_lds_fence();
+            for (int p0 = 0; p0 < n; p0 += 64) {
+                const int p = p0 + lane;
+                // the vertex of child p: is its group a job?
+                int v = 0;
+#pragma unroll
+                for (int step = kLevelVerts / 2; step > 0; step >>= 1)
+                    if (__shfl(first, v + step) <= min(p, n - 1)) v += step;
+                const bool job = __shfl(cnt, v) > kBfsSortSmall;
+                if (p < n) {
+                    const u64 c = s_stage[w][p];
+                    if (job) {
+                        child[mine_at + p] = c;
+                    } else {
+                        const int u = (int)(uint32_t)c;
+                        walk[s.y + mine_at + p] = u;
+                        seq[u] = s.y + mine_at + p;
+                    }
+                }
+            }
+        } else {
+            if (cnt > 0)
+                jobs[atomicAdd(njobs, 1)] =
+                    make_int4(mine_at + first, mine_at + first + cnt, 2 * lg_floor(cnt), 0);
+            int k = 0;
+            E.each(adj, [&](int u) { return claim[u]; },
+                   [&](int u, int v, int place, bool edge) {
+                       const bool mine = edge && place == at + v0 + v;
+                       const u64 m = __ballot(mine);
+                       if (mine)
+                           child[mine_at + k + __popcll(m & below)] =
+                               (u64)(uint32_t)(head[u + 1] - head[u]) << 32 | (uint32_t)u;
+                       k += __popcll(m);
+                   });
+        }
+        wave_lds_fence();
+    }
+}
+
+// Groups of more than kBfsCap children, one work-group each, partitioned in memory (lpos, rpos at
+// the group's own places) down to that size: the pieces join the jobs at jobs[njobs[0] ..], their
+// number in njobs[1].
+__global__ __launch_bounds__(kBfsThreads) void k_level_split(int4* jobs, int* njobs, u64* child,
+                                                             int* lpos, int* rpos) {
+    constexpr int NW = kBfsThreads / 64;
+    __shared__ int2 s_part[NW];
+    __shared__ int s_lnext;
+    const int n = njobs[0];
+    for (int q = blockIdx.x; q < n; q += gridDim.x) {
+        const int4 job = jobs[q];
+        if (job.y - job.x <= kBfsCap) continue;
+        __syncthreads();
+        partition_range<NW>(child, job.x, job.y, job.z, kBfsCap, lpos + job.x, rpos + job.x,
+                            s_part, &s_lnext, [&](int x, int y, int d) {
+                                if (threadIdx.x == 0)
+                                    jobs[n + atomicAdd(&njobs[1], 1)] = make_int4(x, y, d, 0);
+                            });
+    }
+}
+
+// The groups k_level_place left, and the pieces of those k_level_split took: one work-group each,
+// in LDS; a piece beyond it has its depth used up and is heapsorted.
+__global__ __launch_bounds__(kBfsThreads) void k_level_sort(
+    const int4* __restrict__ jobs, const int* __restrict__ njobs, const int4* __restrict__ state,
+    u64* child, int* __restrict__ walk, int* __restrict__ seq) {
+    constexpr int NW = kBfsThreads / 64;
+    __shared__ u64 s_child[kBfsCap];
+    __shared__ int s_lpos[kBfsCap / 2], s_rpos[kBfsCap / 2];
+    __shared__ unsigned char s_mark[kBfsCap + 4];
+    __shared__ int2 s_part[NW];
+    __shared__ int s_lnext[NW];
+    const int t = threadIdx.x, groups = njobs[0], all = groups + njobs[1];
+    const int base = state->y;  // vertices placed before this level
+    for (int q = blockIdx.x; q < all; q += gridDim.x) {
+        const int4 job = jobs[q];
+        const int n = job.y - job.x;
+        u64* a = s_child;
+        __syncthreads();
+        if (n <= kBfsCap) {
+            for (int i = t; i < n; i += kBfsThreads) {
+                s_child[i] = child[job.x + i];
+                s_mark[i] = kMarkNone;
+            }
+            __syncthreads();
+            mark_group<NW>(s_child, 0, n, job.z, s_mark, s_lpos, s_rpos, s_part, s_lnext);
+            __syncthreads();
+            wave_pieces<NW>(s_child, n, s_mark, s_lpos, s_rpos, s_lnext);
+            finish_pieces(s_child, 0, n, s_mark);
+        } else {
+            if (q < groups) continue;  // its pieces follow
+            a = child + job.x;
+            if (t == 0) ls_heapsort(a, 0, n);
+        }
+        __syncthreads();
+        for (int i = t; i < n; i += kBfsThreads) {
+            const int u = (int)(uint32_t)a[i];
+            walk[base + job.x + i] = u;
+            seq[u] = base + job.x + i;
+        }
+    }
+}
+
 // ---- 5. order ----------------------------------------------------------------------------
-__global__ void k_order_keys(const int* __restrict__ comp, const int* __restrict__ rank,
-                             const int* __restrict__ seq, int N, int nb, u64* __restrict__ key,
-                             uint32_t* __restrict__ val) {
-    const long long v = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= N) return;
-    key[v] = (u64)rank[comp[v]] << nb | (u64)seq[v];
-    val[v] = (uint32_t)v;
+// The component of place i's vertex: its root's place, roots being placed in rank order.
+__global__ void k_order_keys(const int* __restrict__ walk, const int* __restrict__ comp,
+                             const int* __restrict__ seq, int N, uint32_t* __restrict__ key) {
+    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < N) key[i] = (uint32_t)seq[comp[walk[i]]];
 }
 
 __global__ void k_positions(const uint32_t* __restrict__ order, int N, int* __restrict__ position) {
@@ -1094,51 +1178,27 @@ void row_of_nonzeros(const int* rp, int M, int nnz, int* row_of, hipStream_t st)
     inclusive_max(headmark.p, row_of, nnz, st);
 }
 
-// Work lists of the child-group sort, sized for the largest level (a range never holds fewer
-// than one element, so there are at most N ranges of each kind).
-struct SortJobs {
-    TmpBuf<int4> big0, big1, small;
-    TmpBuf<int> lpos, rpos, counts;  // counts: {big0, big1, small}
-    explicit SortJobs(int N)
-        : big0(N), big1(N), small(N), lpos(N), rpos(N), counts(3) {}
-};
-
-// Each child group of one level sorted by degree with std::sort's steps: large ranges are
-// partitioned a step at a time by work-groups until every piece holds at most kSortSmall
-// elements (or reached heapsort), then one thread per piece finishes it.
-void sort_groups(const int* gstart, int ngroups, int n, u64* packed, SortJobs& J, hipStream_t st) {
-    VCSRMC_HIP(hipMemsetAsync(J.counts.p, 0, sizeof(int) * 3, st));
-    RLAUNCH(k_group_jobs, ngroups, gstart, ngroups, n, J.big0.p, J.counts.p, J.small.p,
-            J.counts.p + 2);
-    int4* cur = J.big0.p;
-    int4* nxt = J.big1.p;
-    int* ccur = J.counts.p;
-    int* cnxt = J.counts.p + 1;
-    int counts[3];
-    VCSRMC_HIP(hipMemcpyAsync(counts, J.counts.p, sizeof(counts), hipMemcpyDeviceToHost, st));
-    VCSRMC_HIP(hipStreamSynchronize(st));
-    int nbig = counts[0], nsmall = counts[2];
-    const bool passes = nbig > 0;
-    // Every pass lowers the depth of the ranges it keeps, which starts at 2 floor(lg n) < 63:
-    // more passes than that means a broken partition step, reported instead of looping.
-    int pass = 0;
-    while (nbig > 0) {
-        if (++pass > 64) throw Error(VCSRMC_ERR_STATE, "RCM child sort did not converge");
-        VCSRMC_HIP(hipMemsetAsync(cnxt, 0, sizeof(int), st));
-        hipLaunchKernelGGL(k_partition_pass, dim3(nbig), dim3(256), 0, st, cur, nxt, cnxt,
-                           J.small.p, J.counts.p + 2, packed, J.lpos.p, J.rpos.p);
-        VCSRMC_HIP(hipGetLastError());
-        nbig = read_scalar(cnxt, st);
-        std::swap(cur, nxt);
-        std::swap(ccur, cnxt);
-    }
-    if (passes) nsmall = read_scalar(J.counts.p + 2, st);
-    if (nsmall > 0) {
-        hipLaunchKernelGGL(k_small_sort, dim3((unsigned)((nsmall + kSmallSortWaves - 1) /
-                                                          kSmallSortWaves)),
-                           dim3(64 * kSmallSortWaves), 0, st, J.small.p, nsmall, packed);
-        VCSRMC_HIP(hipGetLastError());
-    }
+// The distinct (vertex, neighbour) pairs in order; returns their number.
+template <typename K>
+long long adjacency(const int* rp, const int* col, int M, int N, int nnz, int nb,
+                    TmpBuf<int>& adj_u, TmpBuf<int>& adj, hipStream_t st) {
+    const long long P = 2ll * nnz;
+    if (P == 0) return 0;
+    TmpBuf<int> row_of(nnz);
+    row_of_nonzeros(rp, M, nnz, row_of.p, st);
+    TmpBuf<K> k1(P), k2(P);
+    RLAUNCH((k_adj_pairs<K>), nnz, row_of.p, col, (long long)nnz, N, nb, k1.p);
+    row_of.release();
+    K *ka = k1.p, *kb = k2.p;
+    radix_sort_keys<K>(ka, kb, P, 2 * nb, st);
+    TmpBuf<int> flag(P), pos(P + 1);
+    RLAUNCH((k_unique_flags<K>), P, ka, P, flag.p);
+    exclusive_sum<int, int>(flag.p, pos.p, P, st);
+    const long long E = read_scalar(pos.p + P, st);
+    adj_u.alloc(E);
+    adj.alloc(E);
+    RLAUNCH((k_unique_write<K>), P, ka, pos.p, P, nb, adj_u.p, adj.p);
+    return E;
 }
 
 // Iteration limits of the ordering's loops; 0 selects the proven maxima (see rcm_order_device).
@@ -1166,44 +1226,21 @@ void rcm_order_device(const int* rp, const int* col, int M, int N, int nnz, int*
 
     const int nb = std::max(1, bits_for((u64)N));  // holds 0..N
     // 1. adjacency
-    TmpBuf<int> adj_u, adj;
-    TmpBuf<long long> head((size_t)N + 1);
-    long long E = 0;
-    {
-        const long long P = 2ll * nnz;
-        TmpBuf<int> row_of(nnz);
-        if (nnz) row_of_nonzeros(rp, M, nnz, row_of.p, st);
-        TmpBuf<u64> k1(P), k2(P);
-        RLAUNCH(k_adj_pairs, nnz, row_of.p, col, (long long)nnz, N, nb, k1.p);
-        row_of.release();
-        u64 *ka = k1.p, *kb = k2.p;
-        radix_sort_keys<u64>(ka, kb, P, 2 * nb, st);
-        TmpBuf<int> flag(P);
-        TmpBuf<long long> pos(P + 1);
-        RLAUNCH(k_unique_flags, P, ka, P, flag.p);
-        exclusive_sum<int, long long>(flag.p, pos.p, P, st);
-        E = P ? read_scalar(pos.p + P, st) : 0;
-        adj_u.alloc(E);
-        adj.alloc(E);
-        RLAUNCH(k_unique_write, P, ka, flag.p, pos.p, P, nb, adj_u.p, adj.p);
-    }
-    RLAUNCH(k_heads, (long long)N + 1, adj_u.p, E, N, head.p);
+    TmpBuf<int> adj_u, adj, head((size_t)N + 1);
+    const long long E = 2 * nb <= 32
+                            ? adjacency<uint32_t>(rp, col, M, N, nnz, nb, adj_u, adj, st)
+                            : adjacency<u64>(rp, col, M, N, nnz, nb, adj_u, adj, st);
+    key_ptr<int>(adj_u.p, E, N, head.p, st);
 
     // 2. rank
-    TmpBuf<uint32_t> order(N);
+    TmpBuf<uint32_t> k1(N), k2(N), v1(N), v2(N);
+    uint32_t *ka = k1.p, *kb = k2.p, *va = v1.p, *vb = v2.p;
     TmpBuf<int> rank(N);
-    {
-        TmpBuf<u64> k1(N), k2(N);
-        TmpBuf<uint32_t> v2(N);
-        RLAUNCH(k_rank_keys, N, head.p, N, nb, k1.p, order.p);
-        u64 *ka = k1.p, *kb = k2.p;
-        uint32_t *va = order.p, *vb = v2.p;
-        radix_sort_pairs<u64>(ka, va, kb, vb, N, 2 * nb, st);
-        if (va != order.p)
-            VCSRMC_HIP(hipMemcpyAsync(order.p, va, sizeof(uint32_t) * (size_t)N,
-                                      hipMemcpyDeviceToDevice, st));
-        RLAUNCH(k_scatter_rank, N, order.p, N, rank.p);
-    }
+    RLAUNCH(k_rank_keys, N, head.p, N, ka, va);
+    radix_sort_pairs<uint32_t>(ka, va, kb, vb, N, nb, st);  // a degree is at most N
+    const uint32_t* order = va;
+    const int max_degree = (int)read_scalar(ka + (N - 1), st);
+    RLAUNCH(k_scatter_rank, N, order, N, rank.p);
 
     // Proven maxima of the loops below.  Levels: every level but the last places at least one
     // vertex, so level <= N.  Component rounds: a round changes something or ends the loop;
@@ -1217,97 +1254,102 @@ void rcm_order_device(const int* rp, const int* col, int M, int N, int nnz, int*
     const long long max_rounds =
         lim_rounds > 0 ? lim_rounds : (long long)N * (bits_for((u64)N) + 2) + 1;
 
-    // 3. components
+    // 3. components.  Rounds are enqueued a few at a time, each with its own flag; rounds after
+    // one that changed nothing change nothing either.
     TmpBuf<int> comp(N);
     {
-        TmpBuf<int> changed(1);
+        constexpr int kBatch = 4;
+        TmpBuf<int> changed(kBatch);
         RLAUNCH(k_cc_init, N, comp.p, N);
-        for (long long round = 0;; ++round) {
+        for (long long round = 0;;) {
             if (round >= max_rounds)
                 throw Error(VCSRMC_ERR_STATE, "rcm ordering: connected components did not settle "
                                               "within " + std::to_string(max_rounds) + " rounds");
-            fill<int>(changed.p, 1, 0, st);
-            RLAUNCH(k_cc_hook, E, adj_u.p, adj.p, E, rank.p, comp.p, changed.p);
-            RLAUNCH(k_cc_jump, N, comp.p, N, changed.p);
-            if (!read_scalar(changed.p, st)) break;
+            const int batch = (int)std::min<long long>(kBatch, max_rounds - round);
+            fill<int>(changed.p, kBatch, 0, st);
+            for (int i = 0; i < batch; ++i) {
+                RLAUNCH(k_cc_hook, E, adj_u.p, adj.p, E, rank.p, comp.p, changed.p + i);
+                RLAUNCH(k_cc_jump, N, comp.p, N, changed.p + i);
+            }
+            int flags[kBatch];
+            VCSRMC_HIP(hipMemcpyAsync(flags, changed.p, sizeof flags, hipMemcpyDeviceToHost, st));
+            VCSRMC_HIP(hipStreamSynchronize(st));
+            if (std::find(flags, flags + batch, 0) != flags + batch) break;
+            round += batch;
         }
     }
     adj_u.release();
 
     // 4. levels
-    TmpBuf<int> lev(N), seq(N), claim(N), front(N), next(N), count(1);
-    fill<int>(lev.p, N, -1, st);
+    TmpBuf<int> seq(N), claim(N), walk(N);
+    fill<int>(seq.p, N, -1, st);
     fill<int>(claim.p, N, INT_MAX, st);
-    int f = 0;
+    TmpBuf<int4> state(2);
+    int roots = 0;
     {
-        TmpBuf<int> flag(N);
-        TmpBuf<long long> pos((size_t)N + 1);
-        RLAUNCH(k_root_flags, N, order.p, comp.p, N, flag.p);
-        exclusive_sum<int, long long>(flag.p, pos.p, N, st);
-        f = (int)read_scalar(pos.p + N, st);
-        RLAUNCH(k_root_list, N, order.p, flag.p, pos.p, N, front.p, lev.p, seq.p);
+        TmpBuf<int> flag(N), pos((size_t)N + 1);
+        RLAUNCH(k_root_flags, N, order, comp.p, N, flag.p);
+        exclusive_sum<int, int>(flag.p, pos.p, N, st);
+        roots = read_scalar(pos.p + N, st);
+        RLAUNCH(k_root_list, N, order, flag.p, pos.p, N, walk.p, seq.p);
     }
-    TmpBuf<long long> fdeg(N), fofs((size_t)N + 1);
-    TmpBuf<u64> k1(N), k2(N);
-    TmpBuf<uint32_t> v1(N), v2(N);
-    TmpBuf<int> gflag(N), gstart(N);
-    TmpBuf<long long> gpos((size_t)N + 1);
-    SortJobs jobs(N);
-    TmpBuf<int4> bfs_state(1);
-    int base = f, level = 1;
-    while (f > 0 && base < N) {
-        if (f <= kBfsCap) {  // run levels inside one work-group while they are small
-            const int4 s0 = make_int4(f, base, level, 0);
-            VCSRMC_HIP(hipMemcpyAsync(bfs_state.p, &s0, sizeof(s0), hipMemcpyHostToDevice, st));
-            hipLaunchKernelGGL(k_bfs_levels, dim3(1), dim3(kBfsThreads), 0, st, front.p, head.p,
-                               adj.p, lev.p, seq.p, claim.p, N, max_level, bfs_state.p);
+    TmpBuf<u64> child(N);
+    // A group or piece holds at least one child and there are at most N of each.  Without a vertex
+    // of more than kBfsSortSmall neighbours no group becomes a job (nor do eight fill more than
+    // kLevelStage), and none needs splitting without one of more than kBfsCap.
+    static_assert(kLevelVerts * kBfsSortSmall <= kLevelStage, "small groups always fit");
+    const bool sorts = max_degree > kBfsSortSmall, splits = max_degree > kBfsCap;
+    TmpBuf<int4> jobs(sorts ? 2 * (size_t)N : 0);
+    TmpBuf<int> njobs(2), lpos(splits ? N : 0), rpos(splits ? N : 0), children(kLevelBlocks);
+    int4 s = make_int4(roots, roots, 1, 0);
+    VCSRMC_HIP(hipMemcpyAsync(state.p, &s, sizeof s, hipMemcpyHostToDevice, st));
+    int cur = 0;
+    for (int batch = 1; s.y < N && !s.w && s.z <= max_level; batch = std::min(2 * batch, 16)) {
+        // levels inside one work-group while they are small, then `batch` of any size
+        hipLaunchKernelGGL(k_bfs_levels, dim3(1), dim3(kBfsThreads), 0, st, walk.p, head.p, adj.p,
+                           seq.p, claim.p, N, max_level, state.p + cur);
+        VCSRMC_HIP(hipGetLastError());
+        for (int i = 0; i < batch; ++i, cur ^= 1) {
+            const dim3 grid(kLevelBlocks), block(64 * kLevelWaves);
+            const int4* now = state.p + cur;
+            hipLaunchKernelGGL(k_level_claim, grid, block, 0, st, walk.p, head.p, adj.p, seq.p,
+                               claim.p, now, max_level, njobs.p);
             VCSRMC_HIP(hipGetLastError());
-            const int4 s1 = read_scalar(bfs_state.p, st);
-            f = s1.x;
-            base = s1.y;
-            level = s1.z;
-            if (s1.w || f == 0 || base >= N) break;  // finished, or overran max_level
+            hipLaunchKernelGGL(k_level_count, grid, block, 0, st, walk.p, head.p, adj.p, claim.p,
+                               now, max_level, children.p);
+            VCSRMC_HIP(hipGetLastError());
+            hipLaunchKernelGGL(k_level_place, grid, block, 0, st, walk.p, head.p, adj.p, seq.p,
+                               claim.p, now, state.p + (cur ^ 1), max_level, children.p, child.p,
+                               jobs.p, njobs.p);
+            VCSRMC_HIP(hipGetLastError());
+            if (splits) {
+                hipLaunchKernelGGL(k_level_split, dim3(256), dim3(kBfsThreads), 0, st, jobs.p,
+                                   njobs.p, child.p, lpos.p, rpos.p);
+                VCSRMC_HIP(hipGetLastError());
+            }
+            if (sorts) {
+                hipLaunchKernelGGL(k_level_sort, dim3(256), dim3(kBfsThreads), 0, st, jobs.p,
+                                   njobs.p, now, child.p, walk.p, seq.p);
+                VCSRMC_HIP(hipGetLastError());
+            }
         }
-        if (level > max_level) break;
-        // a level whose frontier or edge count exceeds one work-group
-        RLAUNCH(k_front_degree, f, front.p, f, head.p, fdeg.p);
-        exclusive_sum<long long, long long>(fdeg.p, fofs.p, f, st);
-        const long long Ef = read_scalar(fofs.p + f, st);
-        if (Ef == 0) break;
-        VCSRMC_HIP(hipMemsetAsync(count.p, 0, sizeof(int), st));
-        RLAUNCH(k_claim, Ef, front.p, fofs.p, f, Ef, head.p, adj.p, lev.p, claim.p, next.p,
-                count.p);
-        const int n = read_scalar(count.p, st);
-        if (n == 0) break;
-        const int cb = std::max(1, bits_for((u64)(f - 1)));
-        RLAUNCH(k_next_keys, n, next.p, n, claim.p, nb, k1.p, v1.p);
-        u64 *ka = k1.p, *kb = k2.p;
-        uint32_t *va = v1.p, *vb = v2.p;
-        radix_sort_pairs<u64>(ka, va, kb, vb, n, nb + cb, st);
-        RLAUNCH(k_group_flags, n, ka, n, nb, gflag.p);
-        exclusive_sum<int, long long>(gflag.p, gpos.p, n, st);
-        const int ngroups = (int)read_scalar(gpos.p + n, st);
-        u64* packed = kb;  // free half of the key double buffer
-        RLAUNCH(k_group_pack, n, gflag.p, gpos.p, va, n, head.p, gstart.p, packed);
-        sort_groups(gstart.p, ngroups, n, packed, jobs, st);
-        RLAUNCH(k_level_write, n, packed, n, level, base, front.p, lev.p, seq.p);
-        base += n;
-        f = n;
-        ++level;
+        s = read_scalar(state.p + cur, st);
     }
-    if (level > max_level)
-        throw Error(VCSRMC_ERR_STATE, "rcm ordering: the breadth-first walk passed " +
-                                          std::to_string(max_level) + " levels");
-    if (base != N) throw Error(VCSRMC_ERR_STATE, "rcm ordering left vertices unvisited");
+    if (s.y != N) {
+        if (s.w == kBfsOverrun || s.z > max_level)
+            throw Error(VCSRMC_ERR_STATE, "rcm ordering: the breadth-first walk passed " +
+                                              std::to_string(max_level) + " levels");
+        throw Error(VCSRMC_ERR_STATE, "rcm ordering left vertices unvisited");
+    }
 
-    // 5. order
-    {
-        RLAUNCH(k_order_keys, N, comp.p, rank.p, seq.p, N, nb, k1.p, v1.p);
-        u64 *ka = k1.p, *kb = k2.p;
-        uint32_t *va = v1.p, *vb = v2.p;
-        radix_sort_pairs<u64>(ka, va, kb, vb, N, 2 * nb, st);
-        RLAUNCH(k_positions, N, va, N, position);
+    // 5. order: the walk, its components one after another
+    const uint32_t* last = reinterpret_cast<const uint32_t*>(walk.p);
+    if (roots > 1) {
+        RLAUNCH(k_order_keys, N, walk.p, comp.p, seq.p, N, k1.p);
+        last = radix_sort_pairs_from<uint32_t>(k1.p, last, k2.p, v1.p, k1.p, v2.p, N,
+                                               bits_for((u64)(roots - 1)), st).second;
     }
+    RLAUNCH(k_positions, N, last, N, position);
     VCSRMC_HIP(hipStreamSynchronize(st));
 }
 
