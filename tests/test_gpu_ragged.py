@@ -46,3 +46,35 @@ def test_ragged_widths(orc, O, fp32, half_b, tileK):
             ok, worst, row = row_l1_parity(C[touched], want[touched], bound[touched], tau)
             assert ok, f"shift {shift} add {add} row {row}: error / bound = {worst:.3g}"
             assert C[~touched].tobytes() == C0[~touched].tobytes()
+
+
+@pytest.mark.parametrize("fp32,half_b", [(True, False), (False, True)])
+@pytest.mark.parametrize("N", [1 << 24, (1 << 24) + 1])
+@pytest.mark.parametrize("O", [7, 8])
+def test_row_numbers_around_24_bits(O, N, fp32, half_b):
+    """B of 2^24 rows, the last that 24-bit row numbers reach, and of one more (64-bit addresses):
+    rows that use B's first and last rows, with padding in every tile.  The sums of at most 40
+    products are checked against 64 bits: 40 roundings of 2^-24 (FP32) or inputs of 11 bits."""
+    import torch
+    rng = np.random.default_rng(O + N % 7)
+    M = 70
+    cols = [np.unique(np.concatenate([rng.integers(0, N, int(rng.integers(0, 38))), [0, N - 1]]))
+            for _ in range(M)]
+    rp = np.zeros(M + 1, np.int32)
+    rp[1:] = np.cumsum([len(x) for x in cols])
+    c = np.concatenate(cols).astype(np.int32)
+    v = rng.uniform(-1, 1, c.size).astype(np.float32)
+    say("24-bit rows", O, N, fp32)
+    B = torch.rand((N, O), device="cuda", dtype=torch.float32) - 0.5
+    B = B.half() if half_b else B
+    row = torch.repeat_interleave(torch.arange(M, device="cuda"), dev(np.diff(rp)).long())
+    P = dev(v).double()[:, None] * B[dev(c).long()].double()
+    want = torch.zeros((M, O), device="cuda", dtype=torch.float64).index_add_(0, row, P)
+    bound = torch.zeros_like(want).index_add_(0, row, P.abs()).sum(1)
+    with vm.DeviceFormat.from_device_csr(dev(rp), dev(c), dev(v), M, N, fp32, 32) as f:
+        C = torch.zeros((M, O), device="cuda")
+        f.spmm(B, C)
+        torch.cuda.synchronize()
+    err = (C.double() - want).abs().sum(1)
+    assert bool((err <= (40 * 2.0 ** -24 if fp32 else 2e-3) * bound + 1e-30).all()), \
+        float((err / bound).max())

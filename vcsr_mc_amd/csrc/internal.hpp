@@ -58,7 +58,8 @@ struct XcdSplit {
 //                     order of the panels' first columns for blocks; XCD x runs the range
 //                     starting at xcd_start[x], cut for equal tile counts).
 //   chunk_eptr[c]   = first entry of chunk c (chunk_eptr[num_chunks] = nnz)
-//   chunk_cols[32c+k] = column of the chunk's k-th distinct column, -1 past the end (FP32
+//   chunk_cols[32c+k] = column of the chunk's k-th distinct column, the complement
+//                   (negative) of one of the chunk's columns past the end (FP32
 //                   formats: slot (k & 3) * 8 + (k >> 2), the order the FP32 kernel's lanes read)
 //   entries[e]      FP16 format: f16 value | row-in-panel << 16 | k << 20
 //                   FP32 format: two words per entry, entries[2e] = row-in-panel | k << 4 and
@@ -68,7 +69,7 @@ struct XcdSplit {
 //                   blocks are the panel's 4 row groups (rows 4g..4g+3) x 4 groups of output
 //                   columns.  At each step every row group g takes its own next column: the
 //                   row group's distinct columns in ascending order, one per step, padded with
-//                   -1 after the last; a panel has as many steps as its busiest row group has
+//                   the last one's complement (-1 where there is none); a panel has as many steps as its busiest row group has
 //                   columns, rounded up to 8.  rs_cols[32b + 8g + t] = the column of step t of
 //                   batch b for row group g (the slots the tile path's lane group g reads), and
 //                   rs_vals[128b + 32g + 8x + t] = the value of row 4g + x at that column (0 if

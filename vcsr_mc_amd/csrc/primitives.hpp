@@ -79,10 +79,15 @@ public:
                 if (r.size == 0) b.free.erase(b.free.begin() + i);
                 return p;
             }
-        const size_t size = std::max(bytes, blocks_.empty() ? std::max(first_, kBlock) : kBlock);
+        size_t size = std::max(bytes, blocks_.empty() ? std::max(first_, kBlock) : kBlock);
         blocks_.reserve(blocks_.size() + 1);
         char* p = nullptr;
         hipError_t e = hipMalloc((void**)&p, size);
+        if (e != hipSuccess && size > bytes) {  // memory is short: only what is asked for
+            (void)hipGetLastError();
+            size = bytes;
+            e = hipMalloc((void**)&p, size);
+        }
         if (e != hipSuccess) {
             (void)hipGetLastError();
             throw_hip(e, "hipMalloc", __FILE__, __LINE__);

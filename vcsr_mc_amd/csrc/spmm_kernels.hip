@@ -63,9 +63,9 @@ struct BRows {
     vec_t r[8];
 };
 
-// Zeros read in place of a B row by padding columns.  Never written; not `const`, so that it lives
-// in the global address space like B and the loads stay global loads (a constant-space operand
-// would turn them into flat loads, which also count against the LDS wait counter).
+// Zeros read in place of C where there is none to add to.  Never written; not `const`, so that it
+// lives in the global address space like C and the loads stay global loads (a constant-space
+// operand would turn them into flat loads, which also count against the LDS wait counter).
 __device__ __attribute__((aligned(16))) float kZeroRow[16];
 
 // The first of the VEC output columns a lane multiplies: c0, or O - VEC where that is lower (O >=
@@ -79,25 +79,64 @@ __device__ __attribute__((aligned(16))) float kZeroRow[16];
 template <int VEC>
 __device__ __forceinline__ int lane_column(int c0, int O) { return min(c0, O - VEC); }
 
-// Every load is issued unconditionally (padding columns read kZeroRow): the number of loads in
-// flight is then the same on every path, which lets the compiler wait for exactly the older loads
-// it needs, and no select is needed after a load.  Rows of a ragged O, or of an unaligned B, start
-// at any element: the same one load at element alignment (global loads need no more on gfx950).
+// Address of the B elements a lane reads for a column slot: element c0 of the column's row, from a
+// base all lanes share.  Padding slots hold the complement (negative) of a column that the tile (or
+// row-step group) holds, and its row is read in their place, against zeros of A: products that
+// every row of the tile without that column forms anyway, so nothing is added to any row, whatever
+// B holds there, and no slot needs a test of its own.  All lanes read a padding row's one element
+// `cpad`, the first of the launch's O tile: one address, of a line the tile reads anyway (reading
+// the whole row again cost R-MAT scale 22, 3% of its slots padding, 2%).
+// Offsets take 32 bits (one 24-bit multiply-add, and loads that add them to a scalar base) unless
+// the operand or the layout needs more (WIDE; fits_32 below).  In 64 bits, with a select of a row
+// of zeros for padding, a row took two quarter-rate multiplies and a dozen other instructions, 130
+// of the 180 of an FP16 tile.  Before -> now: power-law 10,000^2 with 12 per row FP16 O = 64
+// 8.4 -> 6.8 us, FP32 O = 128 14.6 -> 11.9; R-MAT scale 18 FP32 O = 16 44 -> 38; uniform 50,000^2
+// FP16 O = 16 9.0 -> 7.7.
+template <typename TB, bool WIDE>
+__device__ __forceinline__ const TB* b_address(const TB* __restrict__ B, int slot, long long ld,
+                                               int c0, int cpad) {
+    const int pad = slot >> 31, col = slot ^ pad;
+    if constexpr (WIDE) return B + (long long)col * ld + (pad ? cpad : c0);
+    const uint32_t row_bytes = (uint32_t)ld * (uint32_t)sizeof(TB);
+    // pad ? cpad : c0, as the one bit-field insert that the compiler makes a compare and a select of
+    uint32_t at;
+    asm("v_bfi_b32 %0, %1, %2, %3"
+        : "=v"(at)
+        : "v"(pad), "s"((uint32_t)cpad * (uint32_t)sizeof(TB)),
+          "v"((uint32_t)c0 * (uint32_t)sizeof(TB)));
+    const uint32_t off = __umul24((uint32_t)col, row_bytes) + at;
+    return reinterpret_cast<const TB*>(reinterpret_cast<const char*>(B) + off);
+}
+
+// A pause of 16 cycles after each load of a B row, in launches whose B comes from beyond the
+// last-level cache (FAR, the launches that read C non-temporally).  A wave that issues its eight
+// rows back to back there ends up slower: R-MAT scale 22 FP16 2480 us, with the pause 2440; scale 19
+// FP32 at O = 256 859 -> 835; stencil 100^3 and blocks within 0.5% (64 cycles: scale 20 472 -> 496).
+__device__ __forceinline__ void space_loads() {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_nop 15");
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// Every load is issued unconditionally: the number of loads in flight is then the same on every
+// path, which lets the compiler wait for exactly the older loads it needs, and no select is needed
+// after a load.  Rows of a ragged O, or of an unaligned B, start at any element: the same one load
+// at element alignment (global loads need no more on gfx950).
 // Measured against a load per element: FP16 power-law 100,000^2 with 12 per row, C = A.B, O = 100
 // 142 -> 36 us, 33 45 -> 24, 130 281 -> 65; FP32 the same, O = 130 180 -> 106; FP32 27-point
 // stencil 60^3, C += A.B, O = 100 246 -> 71.
-template <int VEC, typename TB, bool ALIGNED>
+template <int VEC, typename TB, bool ALIGNED, bool WIDE, bool FAR>
 __device__ __forceinline__ void load_b_rows(const TB* __restrict__ B, const int (&cols)[8],
-                                            long long ld, int c0, BRows<VEC, TB>& R) {
+                                            long long ld, int c0, int cpad,
+                                            BRows<VEC, TB>& R) {
     typedef typename BRows<VEC, TB>::vec_t vec_t;
     typedef vec_t vec_any __attribute__((aligned(sizeof(TB))));
-    const TB* zero = reinterpret_cast<const TB*>(kZeroRow);
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-        const int col = cols[i];
-        const TB* src = col >= 0 ? B + (long long)col * ld + c0 : zero;
+        const TB* src = b_address<TB, WIDE>(B, cols[i], ld, c0, cpad);
         if constexpr (ALIGNED) R.r[i] = *reinterpret_cast<const vec_t*>(src);
         else R.r[i] = *reinterpret_cast<const vec_any*>(src);
+        if constexpr (FAR) space_loads();
     }
 }
 
@@ -320,23 +359,39 @@ static_assert(kDenseMin <= 3 * 64, "a sparse tile must fit three entries per lan
 
 // A state of an FP16 tile in four words per lane: the dense operand (8 halves), or this lane's
 // entries eb + lane, eb + 64 + lane, eb + 128 + lane (addresses clamped into the tile, so the
-// four loads are always issued; the scatter skips the ones past ee).
+// four loads are always issued; the scatter skips the ones past ee).  Either way the words are at
+// 32-bit offsets from one base.
+template <bool WIDE>
 __device__ __forceinline__ uint4 load_a16(const TileMeta& m, int lane, int a_off,
                                           const uint32_t* __restrict__ entries,
                                           const _Float16* __restrict__ dense_a) {
-    const uint32_t *p0, *p1, *p2, *p3;
-    if (m.d >= 0) {
-        const uint32_t* base =
-            reinterpret_cast<const uint32_t*>(dense_a + (long long)m.d * 512 + a_off);
-        p0 = base; p1 = base + 1; p2 = base + 2; p3 = base + 3;
+    const bool dense = m.d >= 0;
+    if constexpr (WIDE) {
+        const uint32_t *p0, *p1, *p2, *p3;
+        if (dense) {
+            const uint32_t* base =
+                reinterpret_cast<const uint32_t*>(dense_a + (long long)m.d * 512 + a_off);
+            p0 = base; p1 = base + 1; p2 = base + 2; p3 = base + 3;
+        } else {
+            const int last = m.ee - 1;
+            p0 = entries + min(m.eb + lane, last);
+            p1 = entries + min(m.eb + 64 + lane, last);
+            p2 = entries + min(m.eb + 128 + lane, last);
+            p3 = p2;
+        }
+        return uint4{*p0, *p1, *p2, *p3};
     } else {
-        const int last = m.ee - 1;
-        p0 = entries + min(m.eb + lane, last);
-        p1 = entries + min(m.eb + 64 + lane, last);
-        p2 = entries + min(m.eb + 128 + lane, last);
-        p3 = p2;
+        const char* base = dense ? reinterpret_cast<const char*>(dense_a + (long long)m.d * 512)
+                                 : reinterpret_cast<const char*>(entries + m.eb);
+        const int last = m.ee - m.eb - 1;
+        const uint32_t at = (uint32_t)a_off * 2;
+        const uint32_t o0 = dense ? at : 4u * (uint32_t)min(lane, last);
+        const uint32_t o1 = dense ? at + 4 : 4u * (uint32_t)min(64 + lane, last);
+        const uint32_t o2 = dense ? at + 8 : 4u * (uint32_t)min(128 + lane, last);
+        const uint32_t o3 = dense ? at + 12 : o2;
+        const auto word = [&](uint32_t o) { return *reinterpret_cast<const uint32_t*>(base + o); };
+        return uint4{word(o0), word(o1), word(o2), word(o3)};
     }
-    return uint4{*p0, *p1, *p2, *p3};
 }
 
 // Schedule of a 4-wave work-group.  Work-groups are dealt to the 8 XCDs round robin (the grid's
@@ -403,9 +458,9 @@ __device__ __forceinline__ void mma_tile_f16(const TileMeta& m, const uint4& st,
 //   * column indices are loaded before the B rows and A state they lead to, so waiting for
 //     them does not wait for those;
 //   * every iteration issues the same loads (column indices past the last tile are clamped).
-template <int TK, typename TB, bool ALIGNED, typename Pre>
+template <int TK, typename TB, bool ALIGNED, bool WIDE, bool FAR, typename Pre>
 __device__ __forceinline__ void tiles_f16(int first, int end, int W, int lane, int n, int g,
-                                          int c0, long long OL,
+                                          int c0, int cpad, long long OL,
                                           const int* __restrict__ chunk_eptr,
                                           const int* __restrict__ chunk_cols,
                                           const int* __restrict__ chunk_dense,
@@ -426,23 +481,23 @@ __device__ __forceinline__ void tiles_f16(int first, int end, int W, int lane, i
     const int c1 = min(c + W, last);
     load_cols8(chunk_cols, c1, g, colsB);
     TileMeta mB = tile_meta(c1, chunk_dense, chunk_eptr);
-    load_b_rows<VEC, TB, ALIGNED>(B, colsA, OL, c0, RA);
-    uint4 sA = load_a16(mA, lane, a_off, entries, dense_a);
+    load_b_rows<VEC, TB, ALIGNED, WIDE, FAR>(B, colsA, OL, c0, cpad, RA);
+    uint4 sA = load_a16<WIDE>(mA, lane, a_off, entries, dense_a);
     uint4 sB;
     // Invariant at the top: tile c in A (B rows, A state, metadata), the column indices and
     // metadata of tile c + W in B; at least three tiles c, c + W, c + 2 W remain.
     for (; c + W < last; c += 2 * W) {
         load_cols8(chunk_cols, c + 2 * W, g, colsA);
         const TileMeta mA2 = tile_meta(c + 2 * W, chunk_dense, chunk_eptr);
-        load_b_rows<VEC, TB, ALIGNED>(B, colsB, OL, c0, RB);
-        sB = load_a16(mB, lane, a_off, entries, dense_a);
+        load_b_rows<VEC, TB, ALIGNED, WIDE, FAR>(B, colsB, OL, c0, cpad, RB);
+        sB = load_a16<WIDE>(mB, lane, a_off, entries, dense_a);
         mma_tile_f16<VEC, TB>(mA, sA, lane, Aw, my_a, RA, acc);
 
         const int c3 = min(c + 3 * W, last);
         load_cols8(chunk_cols, c3, g, colsB);
         const TileMeta mB2 = tile_meta(c3, chunk_dense, chunk_eptr);
-        load_b_rows<VEC, TB, ALIGNED>(B, colsA, OL, c0, RA);
-        sA = load_a16(mA2, lane, a_off, entries, dense_a);
+        load_b_rows<VEC, TB, ALIGNED, WIDE, FAR>(B, colsA, OL, c0, cpad, RA);
+        sA = load_a16<WIDE>(mA2, lane, a_off, entries, dense_a);
         mma_tile_f16<VEC, TB>(mB, sB, lane, Aw, my_a, RB, acc);
         mA = mA2;
         mB = mB2;
@@ -451,8 +506,8 @@ __device__ __forceinline__ void tiles_f16(int first, int end, int W, int lane, i
     // free (see read_c_ahead); with two tiles left, after them (holding both buffers and the C
     // values at once would spill registers).
     if (c < last) {  // two tiles left: c and c + W = last
-        load_b_rows<VEC, TB, ALIGNED>(B, colsB, OL, c0, RB);
-        sB = load_a16(mB, lane, a_off, entries, dense_a);
+        load_b_rows<VEC, TB, ALIGNED, WIDE, FAR>(B, colsB, OL, c0, cpad, RB);
+        sB = load_a16<WIDE>(mB, lane, a_off, entries, dense_a);
         mma_tile_f16<VEC, TB>(mA, sA, lane, Aw, my_a, RA, acc);
         mma_tile_f16<VEC, TB>(mB, sB, lane, Aw, my_a, RB, acc);
         pre();
@@ -467,7 +522,7 @@ __device__ __forceinline__ void tiles_f16(int first, int end, int W, int lane, i
 template <typename TB>
 constexpr int f16_min_waves() { return sizeof(TB) == 2 ? 3 : 2; }
 
-template <int TK, typename TB, bool ALIGNED, bool ACC, bool MAPPED, bool NTC>
+template <int TK, typename TB, bool ALIGNED, bool WIDE, bool ACC, bool MAPPED, bool NTC>
 __global__ __launch_bounds__(64 * kWaves, (f16_min_waves<TB>())) void k_spmm_f16(
     const int4* __restrict__ units, const int* __restrict__ rmap, int num_heavy, XcdSplit xs,
     const int* __restrict__ chunk_eptr, const int* __restrict__ chunk_cols,
@@ -495,6 +550,7 @@ __global__ __launch_bounds__(64 * kWaves, (f16_min_waves<TB>())) void k_spmm_f16
     const TB* Bt = tiled_n > 0 ? B + (long long)(k0 / TK) * tiled_n * TK : B;
     const long long ldb = tiled_n > 0 ? TK : O;
     const int cb = tiled_n > 0 ? VEC * n : lane_column<VEC>(c0, O);
+    const int cpad = tiled_n > 0 ? 0 : min(k0, O - VEC);
     floatx4 acc[VEC];
 #pragma unroll
     for (int q = 0; q < VEC; ++q) acc[q] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -503,13 +559,13 @@ __global__ __launch_bounds__(64 * kWaves, (f16_min_waves<TB>())) void k_spmm_f16
     if (heavy) {
         CAhead<TK, kWaves> ca;
         read_c_ahead<TK, kWaves, NTC>(ca, U, pr, k0, O, ACC, C);
-        tiles_f16<TK, TB, ALIGNED>(U.y + wave, U.z, kWaves, lane, n, g, cb, ldb,
+        tiles_f16<TK, TB, ALIGNED, WIDE, NTC>(U.y + wave, U.z, kWaves, lane, n, g, cb, cpad, ldb,
                                    chunk_eptr, chunk_cols, chunk_dense, entries, dense_a, Bt,
                                    As[wave], acc, [] {});
         merge_into_c<TK, kWaves, ALIGNED, ACC>(acc, scale, U, pr, k0, O, C, P, ca);
     } else {
         CAhead<TK, 1> ca;
-        tiles_f16<TK, TB, ALIGNED>(U.y, U.z, 1, lane, n, g, cb, ldb, chunk_eptr,
+        tiles_f16<TK, TB, ALIGNED, WIDE, NTC>(U.y, U.z, 1, lane, n, g, cb, cpad, ldb, chunk_eptr,
                                    chunk_cols, chunk_dense, entries, dense_a, Bt, As[wave], acc,
                                    [&] { read_c_ahead<TK, 1, NTC>(ca, U, pr, k0, O, ACC, C); });
         merge_into_c<TK, 1, ALIGNED, ACC>(acc, scale, U, pr, k0, O, C, P, ca);
@@ -528,18 +584,19 @@ struct FRows {
 
 // Half a tile of B rows (K steps s0 .. s0 + 3 of the lane's column group): row s holds the VEC
 // output columns c0 .. c0 + VEC - 1 of B row cols[s0 + s].  Loads are unconditional like
-// load_b_rows (padding reads kZeroRow).
-template <int VEC, bool ALIGNED>
+// load_b_rows.
+template <int VEC, bool ALIGNED, bool WIDE, bool FAR>
 __device__ __forceinline__ void load_b_half_f32(const float* __restrict__ B, const int (&cols)[8],
-                                                int s0, long long ld, int c0, FRows<VEC>& R) {
+                                                int s0, long long ld, int c0, int cpad,
+                                                FRows<VEC>& R) {
     typedef typename FRows<VEC>::vec_t vec_t;
     typedef vec_t vec_any __attribute__((aligned(4)));
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
-        const int col = cols[s0 + s];
-        const float* src = col >= 0 ? B + (long long)col * ld + c0 : kZeroRow;
+        const float* src = b_address<float, WIDE>(B, cols[s0 + s], ld, c0, cpad);
         if constexpr (ALIGNED) R.r[s] = *reinterpret_cast<const vec_t*>(src);
         else R.r[s] = *reinterpret_cast<const vec_any*>(src);
+        if constexpr (FAR) space_loads();
     }
 }
 
@@ -663,9 +720,9 @@ __device__ __forceinline__ void a_operand_f32(const TileMeta& m, const AState32&
 // RS: the unit's work items are row-step batches instead (column slots in chunk_cols = rs_cols,
 // A values in dense_a = rs_vals, 128 per batch, this lane's eight at 32 g + 8 (lane & 3)), with
 // the same loads of columns and B rows and mfma_half_rs as the product.
-template <int TK, bool ALIGNED, bool RS, typename Pre>
+template <int TK, bool ALIGNED, bool WIDE, bool FAR, bool RS, typename Pre>
 __device__ __forceinline__ void tiles_f32(int first, int end, int W, int lane, int n, int g,
-                                          int c0, long long OL,
+                                          int c0, int cpad, long long OL,
                                           const int* __restrict__ chunk_eptr,
                                           const int* __restrict__ chunk_cols,
                                           const int* __restrict__ chunk_dense,
@@ -718,24 +775,24 @@ __device__ __forceinline__ void tiles_f32(int first, int end, int W, int lane, i
     const int c1 = min(c + W, last);
     load_cols8(chunk_cols, c1, g, colsB);
     TileMeta mB = meta(c1);
-    load_b_half_f32<VEC, ALIGNED>(B, colsA, 0, OL, c0, X);
+    load_b_half_f32<VEC, ALIGNED, WIDE, FAR>(B, colsA, 0, OL, c0, cpad, X);
     AState32 sA = load_a(mA), sB;
     for (; c + W < last; c += 2 * W) {
-        load_b_half_f32<VEC, ALIGNED>(B, colsA, 4, OL, c0, Y);
+        load_b_half_f32<VEC, ALIGNED, WIDE, FAR>(B, colsA, 4, OL, c0, cpad, Y);
         operand(mA, sA, a);
         mma(a, 0, colsA, X);
 
-        load_b_half_f32<VEC, ALIGNED>(B, colsB, 0, OL, c0, X);
+        load_b_half_f32<VEC, ALIGNED, WIDE, FAR>(B, colsB, 0, OL, c0, cpad, X);
         sB = load_a(mB);
         mma(a, 4, colsA, Y);
         load_cols8(chunk_cols, c + 2 * W, g, colsA);
         const TileMeta mA2 = meta(c + 2 * W);
 
-        load_b_half_f32<VEC, ALIGNED>(B, colsB, 4, OL, c0, Y);
+        load_b_half_f32<VEC, ALIGNED, WIDE, FAR>(B, colsB, 4, OL, c0, cpad, Y);
         operand(mB, sB, a);
         mma(a, 0, colsB, X);
 
-        load_b_half_f32<VEC, ALIGNED>(B, colsA, 0, OL, c0, X);
+        load_b_half_f32<VEC, ALIGNED, WIDE, FAR>(B, colsA, 0, OL, c0, cpad, X);
         sA = load_a(mA2);
         mma(a, 4, colsB, Y);
         const int c3 = min(c + 3 * W, last);
@@ -743,15 +800,15 @@ __device__ __forceinline__ void tiles_f32(int first, int end, int W, int lane, i
         mB = meta(c3);
         mA = mA2;
     }
-    load_b_half_f32<VEC, ALIGNED>(B, colsA, 4, OL, c0, Y);
+    load_b_half_f32<VEC, ALIGNED, WIDE, FAR>(B, colsA, 4, OL, c0, cpad, Y);
     operand(mA, sA, a);
     mma(a, 0, colsA, X);
     // `pre` runs before the last half tile is multiplied, once X is free (see read_c_ahead).
     if (c < last) {  // two tiles left: c and c + W = last
-        load_b_half_f32<VEC, ALIGNED>(B, colsB, 0, OL, c0, X);
+        load_b_half_f32<VEC, ALIGNED, WIDE, FAR>(B, colsB, 0, OL, c0, cpad, X);
         sB = load_a(mB);
         mma(a, 4, colsA, Y);
-        load_b_half_f32<VEC, ALIGNED>(B, colsB, 4, OL, c0, Y);
+        load_b_half_f32<VEC, ALIGNED, WIDE, FAR>(B, colsB, 4, OL, c0, cpad, Y);
         operand(mB, sB, a);
         mma(a, 0, colsB, X);
         pre();
@@ -762,7 +819,7 @@ __device__ __forceinline__ void tiles_f32(int first, int end, int W, int lane, i
     }
 }
 
-template <int TK, bool ALIGNED, bool ACC, bool MAPPED, bool NTC>
+template <int TK, bool ALIGNED, bool WIDE, bool ACC, bool MAPPED, bool NTC>
 __global__ __launch_bounds__(64 * kWaves, 3) void k_spmm_f32(
     const int4* __restrict__ units, const int* __restrict__ rmap, int num_heavy, XcdSplit xs,
     const int* __restrict__ chunk_eptr, const int* __restrict__ chunk_cols,
@@ -781,7 +838,7 @@ __global__ __launch_bounds__(64 * kWaves, 3) void k_spmm_f32(
     const int4 U = units[u];
     const PanelRows<MAPPED> pr = panel_rows<MAPPED>(U, rmap);
     const int k0 = ((blockIdx.y << (3 - xs.lgp)) + ot) * TK;
-    const int c0 = lane_column<VEC>(k0 + VEC * n, O);
+    const int c0 = lane_column<VEC>(k0 + VEC * n, O), cpad = min(k0, O - VEC);
     floatx4 acc[VEC];
 #pragma unroll
     for (int q = 0; q < VEC; ++q) acc[q] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -793,13 +850,13 @@ __global__ __launch_bounds__(64 * kWaves, 3) void k_spmm_f32(
     auto run = [&](int first, int W, auto&& pre) {
         if constexpr (TK <= 64) {
             if (rs) {
-                tiles_f32<TK, ALIGNED, true>(first, U.z, W, lane, n, g, c0, (long long)O,
+                tiles_f32<TK, ALIGNED, WIDE, NTC, true>(first, U.z, W, lane, n, g, c0, cpad, (long long)O,
                                              chunk_eptr, rs_cols, chunk_dense, entries, rs_vals,
                                              B, At[wave], acc, pre);
                 return;
             }
         }
-        tiles_f32<TK, ALIGNED, false>(first, U.z, W, lane, n, g, c0, (long long)O,
+        tiles_f32<TK, ALIGNED, WIDE, NTC, false>(first, U.z, W, lane, n, g, c0, cpad, (long long)O,
                                       chunk_eptr, chunk_cols, chunk_dense, entries, dense_a, B,
                                       At[wave], acc, pre);
     };
@@ -815,9 +872,16 @@ __global__ __launch_bounds__(64 * kWaves, 3) void k_spmm_f32(
     }
 }
 
+// The operand and the layout within what 32-bit offsets reach: B's rows and their bytes in 24 bits
+// each, and B within 4 GB.
+static bool fits_32(const DeviceFormat& F, bool b_f16, int O) {
+    const long long row_bytes = (long long)O * (b_f16 ? 2 : 4);
+    return F.N <= (1 << 24) && row_bytes < (1 << 24) && F.N * row_bytes <= 0xffffffffll;
+}
+
 // NTC: C read ahead with non-temporal loads (accumulating launches whose C and B exceed the
 // last-level cache, see load_c4); only the aligned variants take it.
-template <int TK, bool ACC, bool MAPPED, bool NTC>
+template <int TK, bool ACC, bool MAPPED, bool NTC, bool WIDE>
 static void launch_tk_mode(const DeviceFormat& F, const void* dB, bool b_f16, bool b_tiled, int O,
                            float* dC, hipStream_t st) {
     constexpr int VEC = TK / 16;
@@ -854,10 +918,10 @@ static void launch_tk_mode(const DeviceFormat& F, const void* dB, bool b_f16, bo
         const int* rsc = F.rs_cols.p;
         const float* rsv = F.rs_vals.p;
         if (aligned)
-            hipLaunchKernelGGL((k_spmm_f32<TK, true, ACC, MAPPED, NTC>), grid, block, 0, st, U, rmap,
+            hipLaunchKernelGGL((k_spmm_f32<TK, true, WIDE, ACC, MAPPED, NTC>), grid, block, 0, st, U, rmap,
                                NH, xs, eptr, cols, dense, ent, F.dense_a32.p, rsc, rsv, B, O, dC);
         else
-            hipLaunchKernelGGL((k_spmm_f32<TK, false, ACC, MAPPED, false>), grid, block, 0, st, U, rmap,
+            hipLaunchKernelGGL((k_spmm_f32<TK, false, WIDE, ACC, MAPPED, false>), grid, block, 0, st, U, rmap,
                                NH, xs, eptr, cols, dense, ent, F.dense_a32.p, rsc, rsv, B, O, dC);
     } else if (b_f16) {
         const _Float16* B = static_cast<const _Float16*>(dB);
@@ -866,21 +930,21 @@ static void launch_tk_mode(const DeviceFormat& F, const void* dB, bool b_f16, bo
             throw Error(VCSRMC_ERR_STATE, "O-tile-major B needs full O tiles");
         const int tiled_n = b_tiled ? F.N : 0;
         if (aligned)
-            hipLaunchKernelGGL((k_spmm_f16<TK, _Float16, true, ACC, MAPPED, NTC>), grid, block, 0, st,
+            hipLaunchKernelGGL((k_spmm_f16<TK, _Float16, true, WIDE, ACC, MAPPED, NTC>), grid, block, 0, st,
                                U, rmap, NH, xs, eptr, cols, dense, ent, F.dense_a16.p, B, O,
                                tiled_n, F.scale, dC);
         else
-            hipLaunchKernelGGL((k_spmm_f16<TK, _Float16, false, ACC, MAPPED, false>), grid, block, 0, st,
+            hipLaunchKernelGGL((k_spmm_f16<TK, _Float16, false, WIDE, ACC, MAPPED, false>), grid, block, 0, st,
                                U, rmap, NH, xs, eptr, cols, dense, ent, F.dense_a16.p, B, O,
                                tiled_n, F.scale, dC);
     } else if constexpr (TK <= 64) {
         const float* B = static_cast<const float*>(dB);
         if (aligned)
-            hipLaunchKernelGGL((k_spmm_f16<TK, float, true, ACC, MAPPED, NTC>), grid, block, 0, st, U,
+            hipLaunchKernelGGL((k_spmm_f16<TK, float, true, WIDE, ACC, MAPPED, NTC>), grid, block, 0, st, U,
                                rmap, NH, xs, eptr, cols, dense, ent, F.dense_a16.p, B, O, 0,
                                F.scale, dC);
         else
-            hipLaunchKernelGGL((k_spmm_f16<TK, float, false, ACC, MAPPED, false>), grid, block, 0, st, U,
+            hipLaunchKernelGGL((k_spmm_f16<TK, float, false, WIDE, ACC, MAPPED, false>), grid, block, 0, st, U,
                                rmap, NH, xs, eptr, cols, dense, ent, F.dense_a16.p, B, O, 0,
                                F.scale, dC);
     } else {
@@ -890,20 +954,29 @@ static void launch_tk_mode(const DeviceFormat& F, const void* dB, bool b_f16, bo
     VCSRMC_HIP(hipGetLastError());
 }
 
+template <int TK, bool WIDE>
+static void launch_tk_wide(const DeviceFormat& F, const void* dB, bool b_f16, bool b_tiled, int O,
+                           float* dC, bool accumulate, bool nt_c, hipStream_t st) {
+    const bool mapped = F.row_map.n > 0;
+    if (accumulate && nt_c) {
+        if (mapped) launch_tk_mode<TK, true, true, true, WIDE>(F, dB, b_f16, b_tiled, O, dC, st);
+        else launch_tk_mode<TK, true, false, true, WIDE>(F, dB, b_f16, b_tiled, O, dC, st);
+    } else if (accumulate) {
+        if (mapped) launch_tk_mode<TK, true, true, false, WIDE>(F, dB, b_f16, b_tiled, O, dC, st);
+        else launch_tk_mode<TK, true, false, false, WIDE>(F, dB, b_f16, b_tiled, O, dC, st);
+    } else {
+        if (mapped) launch_tk_mode<TK, false, true, false, WIDE>(F, dB, b_f16, b_tiled, O, dC, st);
+        else launch_tk_mode<TK, false, false, false, WIDE>(F, dB, b_f16, b_tiled, O, dC, st);
+    }
+}
+
 template <int TK>
 static void launch_tk(const DeviceFormat& F, const void* dB, bool b_f16, bool b_tiled, int O,
                       float* dC, bool accumulate, bool nt_c, hipStream_t st) {
-    const bool mapped = F.row_map.n > 0;
-    if (accumulate && nt_c) {
-        if (mapped) launch_tk_mode<TK, true, true, true>(F, dB, b_f16, b_tiled, O, dC, st);
-        else launch_tk_mode<TK, true, false, true>(F, dB, b_f16, b_tiled, O, dC, st);
-    } else if (accumulate) {
-        if (mapped) launch_tk_mode<TK, true, true, false>(F, dB, b_f16, b_tiled, O, dC, st);
-        else launch_tk_mode<TK, true, false, false>(F, dB, b_f16, b_tiled, O, dC, st);
-    } else {
-        if (mapped) launch_tk_mode<TK, false, true, false>(F, dB, b_f16, b_tiled, O, dC, st);
-        else launch_tk_mode<TK, false, false, false>(F, dB, b_f16, b_tiled, O, dC, st);
-    }
+    if (fits_32(F, b_f16, O))
+        launch_tk_wide<TK, false>(F, dB, b_f16, b_tiled, O, dC, accumulate, nt_c, st);
+    else
+        launch_tk_wide<TK, true>(F, dB, b_f16, b_tiled, O, dC, accumulate, nt_c, st);
 }
 
 // Before an overwriting launch (C = A.B), the rows of every split panel are set to zero: their
