@@ -94,3 +94,37 @@ def test_handles_on_threads(orc):
             assert info_s == info_c, i
             for k, (a, b) in enumerate(zip(outs_s, outs_c)):
                 assert np.array_equal(a, b), (rep, i, k)
+
+
+def test_scratch_kept_between_calls_is_bounded():
+    """Scratch blocks of finished builds serve later ones: builds of growing sizes, with a refused
+    one between them, multiply as the first did, and leave at most 2 GiB (and the runtime's own
+    granules) held once the formats are closed."""
+    import torch
+    say("kept scratch")
+    rng = np.random.default_rng(77)
+    rp, c, v = random_csr(rng, 3000, 2500, nnz_per_row=9)
+    B = rng.uniform(-1, 1, (2500, 48)).astype(np.float32)
+    d = lambda a: torch.from_numpy(a).cuda()
+    dB, first = d(B), None
+    torch.cuda.synchronize()
+    free0 = torch.cuda.mem_get_info()[0]
+    for k in range(6):
+        n = 200000 << k  # rows of one nonzero each, in a column of its own
+        ones = torch.ones(n, device="cuda")
+        seq = torch.arange(n + 1, device="cuda", dtype=torch.int32)
+        with vm.DeviceFormat.from_device_csr(seq, seq[:n], ones, n, n, True, 32) as big:
+            assert big.info()["nnz"] == n
+        with pytest.raises(vm.VCSRMCError):
+            vm.DeviceFormat.from_device_csr(seq, torch.zeros_like(seq[:n]) - 1, ones, n, n, True, 32)
+        del ones, seq
+        with vm.DeviceFormat.from_device_csr(d(rp), d(c), d(v), 3000, 2500, True, 32) as f:
+            C = torch.zeros((3000, 48), device="cuda")
+            f.spmm(dB, C)
+            torch.cuda.synchronize()
+        first = C if first is None else first
+        assert torch.equal(C, first)
+    del C, first
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    assert free0 - torch.cuda.mem_get_info()[0] <= (2 << 30) + (256 << 20)

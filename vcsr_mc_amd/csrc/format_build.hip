@@ -65,6 +65,7 @@ float device_absmax(const float* d_val, long long n, hipStream_t st) {
         VCSRMC_HIP(hipGetLastError());
     }
     const unsigned b = read_scalar(bits.p, st);
+    scratch.idle();
     float a;
     std::memcpy(&a, &b, sizeof a);
     return a;
@@ -1325,6 +1326,7 @@ void build_from_csr(DeviceFormat& F, const int* d_row_ptr, const int* d_col, con
 
     build_exec_layout(F, d_row_ptr, row_of.p, d_col, d_val, inv_scale, nnz, st);
     VCSRMC_HIP(hipStreamSynchronize(st));
+    scratch.idle();
     F.ready = true;
 }
 
@@ -1503,6 +1505,7 @@ void build_from_host(DeviceFormat& F, const HostArrays& H, hipStream_t st) {
     }
     build_exec_layout(F, rp.p, trow.p, tcol.p, tval.p, 1.0f, n, st);
     VCSRMC_HIP(hipStreamSynchronize(st));
+    scratch.idle();
     F.ready = true;
 }
 

@@ -1351,6 +1351,7 @@ void rcm_order_device(const int* rp, const int* col, int M, int N, int nnz, int*
     }
     RLAUNCH(k_positions, N, last, N, position);
     VCSRMC_HIP(hipStreamSynchronize(st));
+    scratch.idle();
 }
 
 void apply_column_permutation_device(const int* rp, int* col, float* val, int M, int N, int nnz,
@@ -1414,6 +1415,7 @@ void apply_column_permutation_device(const int* rp, int* col, float* val, int M,
         else RLAUNCH((k_permute_rows<1>), n, B, position, n, (unsigned)O, B_out);
     }
     VCSRMC_HIP(hipStreamSynchronize(st));
+    scratch.idle();
 }
 
 }  // namespace vcsrmc
