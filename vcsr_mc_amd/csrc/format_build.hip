@@ -602,10 +602,10 @@ __global__ __launch_bounds__(256) void k_panel_fill(
             }
         }
     }
-    // the last tile's unused columns: the complement of its last one
+    // the last tile's unused columns
     if (run % kChunkCols != 0 && t >= run % kChunkCols && t < kChunkCols) {
         const int slot = FP32 ? (t & 3) * 8 + (t >> 2) : t;
-        chunk_cols[(long long)(c0 + run / kChunkCols) * kChunkCols + slot] = ~(int)scol[p1 - 1];
+        chunk_cols[(long long)(c0 + run / kChunkCols) * kChunkCols + slot] = kPadSlot;
     }
 }
 
@@ -744,22 +744,6 @@ __global__ void k_row_step_fill(const int* __restrict__ cbase, const int* __rest
         rs_cols[32 * b + 8 * g + t] = chunk_cols[c * kChunkCols + (k & 3) * 8 + (k >> 2)];
         rs_vals[128 * b + 32 * g + 8 * x + t] = __uint_as_float(entries[2 * (long long)e + 1]);
     }
-}
-
-// The unused steps of a panel's row groups, one thread per panel and group: the complement of the
-// group's last column (-1, column 0's, where its rows hold none and none of them is written).
-__global__ void k_row_step_pad(const int* __restrict__ cbase, const int* __restrict__ rbase,
-                               const int* __restrict__ nbat, const int* __restrict__ rspre, int NP,
-                               int NC, int* __restrict__ rs_cols) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int j = (int)(i >> 2), g = (int)(i & 3);
-    if (j >= NP || nbat[j] == 0) return;
-    const int* pre = rspre + g * ((long long)NC + 1);
-    const int used = pre[cbase[j + 1]] - pre[cbase[j]];
-    if (used == 0) return;
-    int* cols = rs_cols + 32ll * rbase[j] + 8 * g;  // step s at 32 (s / 8) + s % 8
-    const int pad = ~cols[32 * ((used - 1) / 8) + (used - 1) % 8];
-    for (int s = used; s < 8 * nbat[j]; ++s) cols[32 * (s / 8) + s % 8] = pad;
 }
 
 __global__ void k_pick_work(const int* __restrict__ nbat, int NP, int* __restrict__ nch) {
@@ -1065,12 +1049,10 @@ static void fill_layout(DeviceFormat& F, const PanelSet& S, const SortedNonzeros
         if (NB > 0) {
             F.rs_cols.alloc((size_t)NB * kChunkCols);
             F.rs_vals.alloc((size_t)NB * 128);
-            fill<int>(F.rs_cols.p, (long long)NB * kChunkCols, -1, st);
+            fill<int>(F.rs_cols.p, (long long)NB * kChunkCols, kPadSlot, st);
             fill<float>(F.rs_vals.p, (long long)NB * 128, 0.0f, st);
             LAUNCH(k_row_step_fill, NC, cbase.p, rbase.p, nbat.p, rsmask.p, rspre.p,
                    F.chunk_eptr.p, F.entries.p, F.chunk_cols.p, NP, NC, F.rs_cols.p, F.rs_vals.p);
-            LAUNCH(k_row_step_pad, 4ll * NP, cbase.p, rbase.p, nbat.p, rspre.p, NP, NC,
-                   F.rs_cols.p);
             // a panel's work items: its batches where it takes row steps, else its tiles
             LAUNCH(k_pick_work, NP, nbat.p, NP, nch.p);
         }

@@ -32,6 +32,8 @@ constexpr int kUnitRowSteps = 1 << 18;    // the unit runs row-step batches, not
 // (as numerator / denominator), in the default mode (format_build.hip, k_row_step_batches).
 constexpr int kRowStepRatioNum = 3, kRowStepRatioDen = 2;
 constexpr int kWaves = 4;
+// Column slots that hold no column (chunk_cols, rs_cols): the multiply kernels read zeros there.
+constexpr int kPadSlot = -(1 << 24);
 
 // Light-unit ranges per XCD, passed to the multiply kernels by value.
 struct XcdSplit {
@@ -58,8 +60,7 @@ struct XcdSplit {
 //                     order of the panels' first columns for blocks; XCD x runs the range
 //                     starting at xcd_start[x], cut for equal tile counts).
 //   chunk_eptr[c]   = first entry of chunk c (chunk_eptr[num_chunks] = nnz)
-//   chunk_cols[32c+k] = column of the chunk's k-th distinct column, the complement
-//                   (negative) of one of the chunk's columns past the end (FP32
+//   chunk_cols[32c+k] = column of the chunk's k-th distinct column, kPadSlot past the end (FP32
 //                   formats: slot (k & 3) * 8 + (k >> 2), the order the FP32 kernel's lanes read)
 //   entries[e]      FP16 format: f16 value | row-in-panel << 16 | k << 20
 //                   FP32 format: two words per entry, entries[2e] = row-in-panel | k << 4 and
@@ -68,9 +69,9 @@ struct XcdSplit {
 //                   a unit runs batches of 8 steps of v_mfma_f32_4x4x1_16b_f32, whose 16
 //                   blocks are the panel's 4 row groups (rows 4g..4g+3) x 4 groups of output
 //                   columns.  At each step every row group g takes its own next column: the
-//                   row group's distinct columns in ascending order, one per step, padded with
-//                   the last one's complement (-1 where there is none); a panel has as many steps as its busiest row group has
-//                   columns, rounded up to 8.  rs_cols[32b + 8g + t] = the column of step t of
+//                   row group's distinct columns in ascending order, one per step, then
+//                   kPadSlot; a panel has as many steps as its busiest row group has columns,
+//                   rounded up to 8.  rs_cols[32b + 8g + t] = the column of step t of
 //                   batch b for row group g (the slots the tile path's lane group g reads), and
 //                   rs_vals[128b + 32g + 8x + t] = the value of row 4g + x at that column (0 if
 //                   the row does not hold it), so a lane reads its eight A values with two

@@ -54,6 +54,11 @@ constexpr int kApitch = 40;  // FP16 A tile row pitch in halves (80 B: conflict-
 constexpr int kApitch32 = 12;
 constexpr int kAgroup32 = 16 * kApitch32;
 
+// What 32-bit offsets reach of B; a padding slot, read as an offset, is past it, and its low 24 bits
+// are zero.
+constexpr uint32_t kBufferBytes = 0xff000000u;
+static_assert((uint32_t)kPadSlot >= kBufferBytes && (kPadSlot & 0xffffff) == 0, "see load_b_row");
+
 // Raw B values of the 8 tile rows a lane feeds into the MFMA B operand, one vector of VEC
 // consecutive output columns per row (kept in the storage type until use, so a prefetched load
 // is never waited for early by a conversion).
@@ -61,9 +66,30 @@ template <int VEC, typename TB>
 struct BRows {
     typedef TB vec_t __attribute__((ext_vector_type(VEC)));
     vec_t r[8];
+    // The MFMA B operand of output column q.
+    __device__ __forceinline__ half8 operand(int q) const {
+        return half8{(_Float16)r[0][q], (_Float16)r[1][q], (_Float16)r[2][q], (_Float16)r[3][q],
+                     (_Float16)r[4][q], (_Float16)r[5][q], (_Float16)r[6][q], (_Float16)r[7][q]};
+    }
 };
 
-// Zeros read in place of C where there is none to add to.  Never written; not `const`, so that it
+// Pairs of halves, as the words they are loaded as (as vectors of two the compiler puts the rows in
+// memory).
+template <>
+struct BRows<2, _Float16> {
+    typedef uint32_t vec_t;
+    uint32_t r[8];
+    __device__ __forceinline__ half8 operand(int q) const {
+        const uint32_t pick = q ? 0x07060302u : 0x05040100u;
+        return __builtin_bit_cast(half8, uint4{__builtin_amdgcn_perm(r[1], r[0], pick),
+                                               __builtin_amdgcn_perm(r[3], r[2], pick),
+                                               __builtin_amdgcn_perm(r[5], r[4], pick),
+                                               __builtin_amdgcn_perm(r[7], r[6], pick)});
+    }
+};
+
+// Zeros read in place of C where there is none to add to (and of B by the 64-bit variants' padding
+// slots).  Never written; not `const`, so that it
 // lives in the global address space like C and the loads stay global loads (a constant-space
 // operand would turn them into flat loads, which also count against the LDS wait counter).
 __device__ __attribute__((aligned(16))) float kZeroRow[16];
@@ -79,33 +105,52 @@ __device__ __attribute__((aligned(16))) float kZeroRow[16];
 template <int VEC>
 __device__ __forceinline__ int lane_column(int c0, int O) { return min(c0, O - VEC); }
 
-// Address of the B elements a lane reads for a column slot: element c0 of the column's row, from a
-// base all lanes share.  Padding slots hold the complement (negative) of a column that the tile (or
-// row-step group) holds, and its row is read in their place, against zeros of A: products that
-// every row of the tile without that column forms anyway, so nothing is added to any row, whatever
-// B holds there, and no slot needs a test of its own.  All lanes read a padding row's one element
-// `cpad`, the first of the launch's O tile: one address, of a line the tile reads anyway (reading
-// the whole row again cost R-MAT scale 22, 3% of its slots padding, 2%).
-// Offsets take 32 bits (one 24-bit multiply-add, and loads that add them to a scalar base) unless
-// the operand or the layout needs more (WIDE; fits_32 below).  In 64 bits, with a select of a row
-// of zeros for padding, a row took two quarter-rate multiplies and a dozen other instructions, 130
-// of the 180 of an FP16 tile.  Before -> now: power-law 10,000^2 with 12 per row FP16 O = 64
-// 8.4 -> 6.8 us, FP32 O = 128 14.6 -> 11.9; R-MAT scale 18 FP32 O = 16 44 -> 38; uniform 50,000^2
-// FP16 O = 16 9.0 -> 7.7.
-template <typename TB, bool WIDE>
-__device__ __forceinline__ const TB* b_address(const TB* __restrict__ B, int slot, long long ld,
-                                               int c0, int cpad) {
-    const int pad = slot >> 31, col = slot ^ pad;
-    if constexpr (WIDE) return B + (long long)col * ld + (pad ? cpad : c0);
-    const uint32_t row_bytes = (uint32_t)ld * (uint32_t)sizeof(TB);
-    // pad ? cpad : c0, as the one bit-field insert that the compiler makes a compare and a select of
-    uint32_t at;
-    asm("v_bfi_b32 %0, %1, %2, %3"
-        : "=v"(at)
-        : "v"(pad), "s"((uint32_t)cpad * (uint32_t)sizeof(TB)),
-          "v"((uint32_t)c0 * (uint32_t)sizeof(TB)));
-    const uint32_t off = __umul24((uint32_t)col, row_bytes) + at;
-    return reinterpret_cast<const TB*>(reinterpret_cast<const char*>(B) + off);
+// The VEC elements of B a lane reads for a column slot: those from element c0 on of the column's
+// row, or zeros for a padding slot (kPadSlot), whatever B holds: a padding slot's products are with
+// zeros of A, and against an Inf or NaN of B they would reach rows and output columns that have no
+// part in it.
+// A buffer load does both: its 32-bit offset from B takes one 24-bit multiply-add and a maximum that
+// puts a padding slot's past the buffer's end, where a load returns zeros and fetches nothing.  An
+// operand or layout that needs more than that (WIDE; fits_32 below) takes 64-bit addresses and a
+// select of a row of zeros: two quarter-rate multiplies and a dozen other instructions a row, 130 of
+// the 180 of an FP16 tile.  64-bit addresses for every launch -> now: power-law 10,000^2 with 12 per
+// row FP16 O = 64 8.3 -> 6.7 us, FP32 O = 128 15.4 -> 12.9; R-MAT scale 18 FP32 O = 16 45 -> 37;
+// uniform 50,000^2 with 16 per row FP16 O = 16 9.5 -> 8.0.  (Zeros selected after the load instead,
+// behind a count of the last tile's padding: power-law 36,692^2 FP16 15.2 -> 15.7 us.)
+template <int VEC, typename TB, bool ALIGNED, bool WIDE>
+__device__ __forceinline__ auto load_b_row(const TB* __restrict__ B, int slot, long long ld,
+                                           int c0) {
+    typedef TB vec_t __attribute__((ext_vector_type(VEC)));
+    typedef vec_t vec_any __attribute__((aligned(sizeof(TB))));
+    if constexpr (WIDE) {
+        const TB* src = slot >= 0 ? B + (long long)slot * ld + c0
+                                  : reinterpret_cast<const TB*>(kZeroRow);
+        if constexpr (ALIGNED) return *reinterpret_cast<const vec_t*>(src);
+        else return (vec_t)*reinterpret_cast<const vec_any*>(src);
+    } else {
+        // a raw buffer of 32-bit data, no stride; a column's offset is never below its number
+        const __amdgpu_buffer_rsrc_t buf =
+            __builtin_amdgcn_make_buffer_rsrc(const_cast<TB*>(B), 0, kBufferBytes, 0x27000);
+        const uint32_t row_bytes = (uint32_t)ld * (uint32_t)sizeof(TB);
+        const uint32_t at = (uint32_t)c0 * (uint32_t)sizeof(TB);
+        const uint32_t off = max(__umul24((uint32_t)slot, row_bytes) + at, (uint32_t)slot);
+        if constexpr (sizeof(vec_t) == 2)
+            return __builtin_bit_cast(vec_t, __builtin_amdgcn_raw_buffer_load_b16(buf, off, 0, 0));
+        else if constexpr (sizeof(vec_t) == 4)
+            return __builtin_bit_cast(vec_t, __builtin_amdgcn_raw_buffer_load_b32(buf, off, 0, 0));
+        else if constexpr (sizeof(vec_t) == 8)
+            return __builtin_bit_cast(vec_t, __builtin_amdgcn_raw_buffer_load_b64(buf, off, 0, 0));
+        else if constexpr (sizeof(vec_t) == 16)
+            return __builtin_bit_cast(vec_t, __builtin_amdgcn_raw_buffer_load_b128(buf, off, 0, 0));
+        else {
+            typedef uint32_t words __attribute__((ext_vector_type(4)));
+            struct {
+                words lo, hi;
+            } v = {__builtin_amdgcn_raw_buffer_load_b128(buf, off, 0, 0),
+                   __builtin_amdgcn_raw_buffer_load_b128(buf, off + 16, 0, 0)};
+            return __builtin_bit_cast(vec_t, v);
+        }
+    }
 }
 
 // A pause of 16 cycles after each load of a B row, in launches whose B comes from beyond the
@@ -121,21 +166,17 @@ __device__ __forceinline__ void space_loads() {
 // Every load is issued unconditionally: the number of loads in flight is then the same on every
 // path, which lets the compiler wait for exactly the older loads it needs, and no select is needed
 // after a load.  Rows of a ragged O, or of an unaligned B, start at any element: the same one load
-// at element alignment (global loads need no more on gfx950).
+// at element alignment (loads need no more on gfx950).
 // Measured against a load per element: FP16 power-law 100,000^2 with 12 per row, C = A.B, O = 100
 // 142 -> 36 us, 33 45 -> 24, 130 281 -> 65; FP32 the same, O = 130 180 -> 106; FP32 27-point
 // stencil 60^3, C += A.B, O = 100 246 -> 71.
 template <int VEC, typename TB, bool ALIGNED, bool WIDE, bool FAR>
 __device__ __forceinline__ void load_b_rows(const TB* __restrict__ B, const int (&cols)[8],
-                                            long long ld, int c0, int cpad,
-                                            BRows<VEC, TB>& R) {
-    typedef typename BRows<VEC, TB>::vec_t vec_t;
-    typedef vec_t vec_any __attribute__((aligned(sizeof(TB))));
+                                            long long ld, int c0, BRows<VEC, TB>& R) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-        const TB* src = b_address<TB, WIDE>(B, cols[i], ld, c0, cpad);
-        if constexpr (ALIGNED) R.r[i] = *reinterpret_cast<const vec_t*>(src);
-        else R.r[i] = *reinterpret_cast<const vec_any*>(src);
+        R.r[i] = __builtin_bit_cast(typename BRows<VEC, TB>::vec_t,
+                                    load_b_row<VEC, TB, ALIGNED, WIDE>(B, cols[i], ld, c0));
         if constexpr (FAR) space_loads();
     }
 }
@@ -442,9 +483,7 @@ __device__ __forceinline__ void mma_tile_f16(const TileMeta& m, const uint4& st,
     }
 #pragma unroll
     for (int q = 0; q < VEC; ++q) {
-        const half8 b = half8{(_Float16)R.r[0][q], (_Float16)R.r[1][q], (_Float16)R.r[2][q],
-                              (_Float16)R.r[3][q], (_Float16)R.r[4][q], (_Float16)R.r[5][q],
-                              (_Float16)R.r[6][q], (_Float16)R.r[7][q]};
+        const half8 b = R.operand(q);
         acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, acc[q], 0, 0, 0);
     }
 }
@@ -460,7 +499,7 @@ __device__ __forceinline__ void mma_tile_f16(const TileMeta& m, const uint4& st,
 //   * every iteration issues the same loads (column indices past the last tile are clamped).
 template <int TK, typename TB, bool ALIGNED, bool WIDE, bool FAR, typename Pre>
 __device__ __forceinline__ void tiles_f16(int first, int end, int W, int lane, int n, int g,
-                                          int c0, int cpad, long long OL,
+                                          int c0, long long OL,
                                           const int* __restrict__ chunk_eptr,
                                           const int* __restrict__ chunk_cols,
                                           const int* __restrict__ chunk_dense,
@@ -481,7 +520,7 @@ __device__ __forceinline__ void tiles_f16(int first, int end, int W, int lane, i
     const int c1 = min(c + W, last);
     load_cols8(chunk_cols, c1, g, colsB);
     TileMeta mB = tile_meta(c1, chunk_dense, chunk_eptr);
-    load_b_rows<VEC, TB, ALIGNED, WIDE, FAR>(B, colsA, OL, c0, cpad, RA);
+    load_b_rows<VEC, TB, ALIGNED, WIDE, FAR>(B, colsA, OL, c0, RA);
     uint4 sA = load_a16<WIDE>(mA, lane, a_off, entries, dense_a);
     uint4 sB;
     // Invariant at the top: tile c in A (B rows, A state, metadata), the column indices and
@@ -489,14 +528,14 @@ __device__ __forceinline__ void tiles_f16(int first, int end, int W, int lane, i
     for (; c + W < last; c += 2 * W) {
         load_cols8(chunk_cols, c + 2 * W, g, colsA);
         const TileMeta mA2 = tile_meta(c + 2 * W, chunk_dense, chunk_eptr);
-        load_b_rows<VEC, TB, ALIGNED, WIDE, FAR>(B, colsB, OL, c0, cpad, RB);
+        load_b_rows<VEC, TB, ALIGNED, WIDE, FAR>(B, colsB, OL, c0, RB);
         sB = load_a16<WIDE>(mB, lane, a_off, entries, dense_a);
         mma_tile_f16<VEC, TB>(mA, sA, lane, Aw, my_a, RA, acc);
 
         const int c3 = min(c + 3 * W, last);
         load_cols8(chunk_cols, c3, g, colsB);
         const TileMeta mB2 = tile_meta(c3, chunk_dense, chunk_eptr);
-        load_b_rows<VEC, TB, ALIGNED, WIDE, FAR>(B, colsA, OL, c0, cpad, RA);
+        load_b_rows<VEC, TB, ALIGNED, WIDE, FAR>(B, colsA, OL, c0, RA);
         sA = load_a16<WIDE>(mA2, lane, a_off, entries, dense_a);
         mma_tile_f16<VEC, TB>(mB, sB, lane, Aw, my_a, RB, acc);
         mA = mA2;
@@ -506,7 +545,7 @@ __device__ __forceinline__ void tiles_f16(int first, int end, int W, int lane, i
     // free (see read_c_ahead); with two tiles left, after them (holding both buffers and the C
     // values at once would spill registers).
     if (c < last) {  // two tiles left: c and c + W = last
-        load_b_rows<VEC, TB, ALIGNED, WIDE, FAR>(B, colsB, OL, c0, cpad, RB);
+        load_b_rows<VEC, TB, ALIGNED, WIDE, FAR>(B, colsB, OL, c0, RB);
         sB = load_a16<WIDE>(mB, lane, a_off, entries, dense_a);
         mma_tile_f16<VEC, TB>(mA, sA, lane, Aw, my_a, RA, acc);
         mma_tile_f16<VEC, TB>(mB, sB, lane, Aw, my_a, RB, acc);
@@ -550,7 +589,6 @@ __global__ __launch_bounds__(64 * kWaves, (f16_min_waves<TB>())) void k_spmm_f16
     const TB* Bt = tiled_n > 0 ? B + (long long)(k0 / TK) * tiled_n * TK : B;
     const long long ldb = tiled_n > 0 ? TK : O;
     const int cb = tiled_n > 0 ? VEC * n : lane_column<VEC>(c0, O);
-    const int cpad = tiled_n > 0 ? 0 : min(k0, O - VEC);
     floatx4 acc[VEC];
 #pragma unroll
     for (int q = 0; q < VEC; ++q) acc[q] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -559,13 +597,13 @@ __global__ __launch_bounds__(64 * kWaves, (f16_min_waves<TB>())) void k_spmm_f16
     if (heavy) {
         CAhead<TK, kWaves> ca;
         read_c_ahead<TK, kWaves, NTC>(ca, U, pr, k0, O, ACC, C);
-        tiles_f16<TK, TB, ALIGNED, WIDE, NTC>(U.y + wave, U.z, kWaves, lane, n, g, cb, cpad, ldb,
+        tiles_f16<TK, TB, ALIGNED, WIDE, NTC>(U.y + wave, U.z, kWaves, lane, n, g, cb, ldb,
                                    chunk_eptr, chunk_cols, chunk_dense, entries, dense_a, Bt,
                                    As[wave], acc, [] {});
         merge_into_c<TK, kWaves, ALIGNED, ACC>(acc, scale, U, pr, k0, O, C, P, ca);
     } else {
         CAhead<TK, 1> ca;
-        tiles_f16<TK, TB, ALIGNED, WIDE, NTC>(U.y, U.z, 1, lane, n, g, cb, cpad, ldb, chunk_eptr,
+        tiles_f16<TK, TB, ALIGNED, WIDE, NTC>(U.y, U.z, 1, lane, n, g, cb, ldb, chunk_eptr,
                                    chunk_cols, chunk_dense, entries, dense_a, Bt, As[wave], acc,
                                    [&] { read_c_ahead<TK, 1, NTC>(ca, U, pr, k0, O, ACC, C); });
         merge_into_c<TK, 1, ALIGNED, ACC>(acc, scale, U, pr, k0, O, C, P, ca);
@@ -587,15 +625,10 @@ struct FRows {
 // load_b_rows.
 template <int VEC, bool ALIGNED, bool WIDE, bool FAR>
 __device__ __forceinline__ void load_b_half_f32(const float* __restrict__ B, const int (&cols)[8],
-                                                int s0, long long ld, int c0, int cpad,
-                                                FRows<VEC>& R) {
-    typedef typename FRows<VEC>::vec_t vec_t;
-    typedef vec_t vec_any __attribute__((aligned(4)));
+                                                int s0, long long ld, int c0, FRows<VEC>& R) {
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
-        const float* src = b_address<float, WIDE>(B, cols[s0 + s], ld, c0, cpad);
-        if constexpr (ALIGNED) R.r[s] = *reinterpret_cast<const vec_t*>(src);
-        else R.r[s] = *reinterpret_cast<const vec_any*>(src);
+        R.r[s] = load_b_row<VEC, float, ALIGNED, WIDE>(B, cols[s0 + s], ld, c0);
         if constexpr (FAR) space_loads();
     }
 }
@@ -722,7 +755,7 @@ __device__ __forceinline__ void a_operand_f32(const TileMeta& m, const AState32&
 // the same loads of columns and B rows and mfma_half_rs as the product.
 template <int TK, bool ALIGNED, bool WIDE, bool FAR, bool RS, typename Pre>
 __device__ __forceinline__ void tiles_f32(int first, int end, int W, int lane, int n, int g,
-                                          int c0, int cpad, long long OL,
+                                          int c0, long long OL,
                                           const int* __restrict__ chunk_eptr,
                                           const int* __restrict__ chunk_cols,
                                           const int* __restrict__ chunk_dense,
@@ -775,24 +808,24 @@ __device__ __forceinline__ void tiles_f32(int first, int end, int W, int lane, i
     const int c1 = min(c + W, last);
     load_cols8(chunk_cols, c1, g, colsB);
     TileMeta mB = meta(c1);
-    load_b_half_f32<VEC, ALIGNED, WIDE, FAR>(B, colsA, 0, OL, c0, cpad, X);
+    load_b_half_f32<VEC, ALIGNED, WIDE, FAR>(B, colsA, 0, OL, c0, X);
     AState32 sA = load_a(mA), sB;
     for (; c + W < last; c += 2 * W) {
-        load_b_half_f32<VEC, ALIGNED, WIDE, FAR>(B, colsA, 4, OL, c0, cpad, Y);
+        load_b_half_f32<VEC, ALIGNED, WIDE, FAR>(B, colsA, 4, OL, c0, Y);
         operand(mA, sA, a);
         mma(a, 0, colsA, X);
 
-        load_b_half_f32<VEC, ALIGNED, WIDE, FAR>(B, colsB, 0, OL, c0, cpad, X);
+        load_b_half_f32<VEC, ALIGNED, WIDE, FAR>(B, colsB, 0, OL, c0, X);
         sB = load_a(mB);
         mma(a, 4, colsA, Y);
         load_cols8(chunk_cols, c + 2 * W, g, colsA);
         const TileMeta mA2 = meta(c + 2 * W);
 
-        load_b_half_f32<VEC, ALIGNED, WIDE, FAR>(B, colsB, 4, OL, c0, cpad, Y);
+        load_b_half_f32<VEC, ALIGNED, WIDE, FAR>(B, colsB, 4, OL, c0, Y);
         operand(mB, sB, a);
         mma(a, 0, colsB, X);
 
-        load_b_half_f32<VEC, ALIGNED, WIDE, FAR>(B, colsA, 0, OL, c0, cpad, X);
+        load_b_half_f32<VEC, ALIGNED, WIDE, FAR>(B, colsA, 0, OL, c0, X);
         sA = load_a(mA2);
         mma(a, 4, colsB, Y);
         const int c3 = min(c + 3 * W, last);
@@ -800,15 +833,15 @@ __device__ __forceinline__ void tiles_f32(int first, int end, int W, int lane, i
         mB = meta(c3);
         mA = mA2;
     }
-    load_b_half_f32<VEC, ALIGNED, WIDE, FAR>(B, colsA, 4, OL, c0, cpad, Y);
+    load_b_half_f32<VEC, ALIGNED, WIDE, FAR>(B, colsA, 4, OL, c0, Y);
     operand(mA, sA, a);
     mma(a, 0, colsA, X);
     // `pre` runs before the last half tile is multiplied, once X is free (see read_c_ahead).
     if (c < last) {  // two tiles left: c and c + W = last
-        load_b_half_f32<VEC, ALIGNED, WIDE, FAR>(B, colsB, 0, OL, c0, cpad, X);
+        load_b_half_f32<VEC, ALIGNED, WIDE, FAR>(B, colsB, 0, OL, c0, X);
         sB = load_a(mB);
         mma(a, 4, colsA, Y);
-        load_b_half_f32<VEC, ALIGNED, WIDE, FAR>(B, colsB, 4, OL, c0, cpad, Y);
+        load_b_half_f32<VEC, ALIGNED, WIDE, FAR>(B, colsB, 4, OL, c0, Y);
         operand(mB, sB, a);
         mma(a, 0, colsB, X);
         pre();
@@ -838,7 +871,7 @@ __global__ __launch_bounds__(64 * kWaves, 3) void k_spmm_f32(
     const int4 U = units[u];
     const PanelRows<MAPPED> pr = panel_rows<MAPPED>(U, rmap);
     const int k0 = ((blockIdx.y << (3 - xs.lgp)) + ot) * TK;
-    const int c0 = lane_column<VEC>(k0 + VEC * n, O), cpad = min(k0, O - VEC);
+    const int c0 = lane_column<VEC>(k0 + VEC * n, O);
     floatx4 acc[VEC];
 #pragma unroll
     for (int q = 0; q < VEC; ++q) acc[q] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -850,13 +883,13 @@ __global__ __launch_bounds__(64 * kWaves, 3) void k_spmm_f32(
     auto run = [&](int first, int W, auto&& pre) {
         if constexpr (TK <= 64) {
             if (rs) {
-                tiles_f32<TK, ALIGNED, WIDE, NTC, true>(first, U.z, W, lane, n, g, c0, cpad, (long long)O,
+                tiles_f32<TK, ALIGNED, WIDE, NTC, true>(first, U.z, W, lane, n, g, c0, (long long)O,
                                              chunk_eptr, rs_cols, chunk_dense, entries, rs_vals,
                                              B, At[wave], acc, pre);
                 return;
             }
         }
-        tiles_f32<TK, ALIGNED, WIDE, NTC, false>(first, U.z, W, lane, n, g, c0, cpad, (long long)O,
+        tiles_f32<TK, ALIGNED, WIDE, NTC, false>(first, U.z, W, lane, n, g, c0, (long long)O,
                                       chunk_eptr, chunk_cols, chunk_dense, entries, dense_a, B,
                                       At[wave], acc, pre);
     };
@@ -873,10 +906,10 @@ __global__ __launch_bounds__(64 * kWaves, 3) void k_spmm_f32(
 }
 
 // The operand and the layout within what 32-bit offsets reach: B's rows and their bytes in 24 bits
-// each, and B within 4 GB.
+// each, and B within the buffer.
 static bool fits_32(const DeviceFormat& F, bool b_f16, int O) {
     const long long row_bytes = (long long)O * (b_f16 ? 2 : 4);
-    return F.N <= (1 << 24) && row_bytes < (1 << 24) && F.N * row_bytes <= 0xffffffffll;
+    return F.N <= (1 << 24) && row_bytes < (1 << 24) && F.N * row_bytes <= (long long)kBufferBytes;
 }
 
 // NTC: C read ahead with non-temporal loads (accumulating launches whose C and B exceed the
