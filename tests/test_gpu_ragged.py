@@ -78,3 +78,41 @@ def test_row_numbers_around_24_bits(O, N, fp32, half_b):
     err = (C.double() - want).abs().sum(1)
     assert bool((err <= (40 * 2.0 ** -24 if fp32 else 2e-3) * bound + 1e-30).all()), \
         float((err / bound).max())
+
+
+@pytest.mark.parametrize("more", [0, 1])
+@pytest.mark.parametrize("fp32,O", [(True, 256), (True, 65), (False, 128), (False, 137)])
+def test_operands_around_the_32_bit_reach(fp32, O, more):
+    """The largest B that 32-bit offsets reach (0xff000000 bytes, fewer than 2^24 rows) and one row
+    more (64-bit addresses): rows that use its first and last rows and the ones around byte 2^31, an
+    Inf in the row after a used one.  Bound as in test_row_numbers_around_24_bits."""
+    import torch
+    row_bytes = O * (4 if fp32 else 2)
+    N = 0xff000000 // row_bytes + more
+    if N > 1 << 24:
+        N = (1 << 24) + more
+    rng = np.random.default_rng(O + more)
+    M, half = 70, 2 ** 31 // row_bytes
+    edge = [0, half - 1, half, half + 1, N - 1]
+    cols = [np.unique(np.concatenate([rng.integers(0, N - 2, int(rng.integers(0, 30))), edge]))
+            for _ in range(M)]
+    rp = np.zeros(M + 1, np.int32)
+    rp[1:] = np.cumsum([len(x) for x in cols])
+    c = np.concatenate(cols).astype(np.int32)
+    v = rng.uniform(-1, 1, c.size).astype(np.float32)
+    say("32-bit reach", fp32, O, N)
+    B = torch.empty((N, O), device="cuda", dtype=torch.float32 if fp32 else torch.float16)
+    B.uniform_(-0.5, 0.5)
+    free = np.setdiff1d(np.array([1, half + 2, N - 2]), c)
+    B[torch.from_numpy(free).cuda()] = float("inf")
+    row = torch.repeat_interleave(torch.arange(M, device="cuda"), dev(np.diff(rp)).long())
+    P = dev(v).double()[:, None] * B[dev(c).long()].double()
+    want = torch.zeros((M, O), device="cuda", dtype=torch.float64).index_add_(0, row, P)
+    bound = torch.zeros_like(want).index_add_(0, row, P.abs()).sum(1)
+    with vm.DeviceFormat.from_device_csr(dev(rp), dev(c), dev(v), M, N, fp32, 32) as f:
+        C = torch.zeros((M, O), device="cuda")
+        f.spmm(B, C)
+        torch.cuda.synchronize()
+    err = (C.double() - want).abs().sum(1)
+    assert bool((err <= (40 * 2.0 ** -24 if fp32 else 2e-3) * bound + 1e-30).all()), \
+        float((err / bound).max())
