@@ -362,7 +362,7 @@ __device__ __forceinline__ int merged_place(const T* cols, Off off, int s, int r
 // grouped.  27-point stencil 100^3, both orders: the keys, sorts and scans 4.0 ms, this 0.77.
 template <int CAP, int T, bool FP32>
 __global__ __launch_bounds__(T) void k_panel_sort(Positions pos, const int* __restrict__ list,
-                                                  const int* __restrict__ col,
+                                                  int count, const int* __restrict__ col,
                                                   const float* __restrict__ val, float inv_scale,
                                                   uint32_t* __restrict__ scol,
                                                   uint32_t* __restrict__ sval,
@@ -372,7 +372,9 @@ __global__ __launch_bounds__(T) void k_panel_sort(Positions pos, const int* __re
     __shared__ int s_off[kPanelRows + 1], s_row[kPanelRows];
     __shared__ int distinct;
     const int t = threadIdx.x;
-    const int j = list ? list[blockIdx.x] : (int)blockIdx.x;
+    const long long group = group_index();
+    if (group >= count) return;  // the whole work-group
+    const int j = list ? list[group] : (int)group;
     const int p0 = j * kPanelRows, first = pos.begin(p0);
     if (t <= kPanelRows) s_off[t] = pos.begin(p0 + t) - first;
     if (t < kPanelRows) s_row[t] = pos.row_begin(p0 + t);
@@ -556,12 +558,14 @@ __global__ void k_panel_compact(Positions pos, const int* __restrict__ nch,
 // columns gives each nonzero its tile and column in it.
 template <bool FP32>
 __global__ __launch_bounds__(256) void k_panel_fill(
-    const int* __restrict__ pstart, const int* __restrict__ cbase,
+    const int* __restrict__ pstart, const int* __restrict__ cbase, int NP,
     const uint32_t* __restrict__ scol, const uint32_t* __restrict__ sval,
     const unsigned char* __restrict__ srow, uint32_t* __restrict__ entries,
     int* __restrict__ chunk_cols, int* __restrict__ chunk_eptr) {
     __shared__ int whead[2][4];
-    const int j = blockIdx.x, t = threadIdx.x, w = t >> 6, lane = t & 63;
+    const long long j = group_index();
+    if (j >= NP) return;  // the whole work-group
+    const int t = threadIdx.x, w = t >> 6, lane = t & 63;
     const int p0 = pstart[j], p1 = pstart[j + 1], c0 = cbase[j];
     const uint64_t upto = ~0ull >> (63 - lane);
     int run = 0, phase = 0;  // distinct columns before this round's nonzeros
@@ -642,7 +646,7 @@ __global__ __launch_bounds__(256) void k_dense_fill(const uint32_t* __restrict__
     typedef typename std::conditional<FP32, float, _Float16>::type T;
     __shared__ __attribute__((aligned(16))) T tile[4][512];
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const long long c = (long long)blockIdx.x * 4 + w;
+    const long long c = group_index() * 4 + w;
     if (c >= NC) return;  // the whole wave
     const int d = chunk_dense[c];
     if (d < 0) return;
@@ -929,16 +933,16 @@ static PanelSet sort_panels(int M, const int* rp, const int* row_map, const int*
     fill<int>(counts.p, 2, 0, st);
     LAUNCH(k_panel_classes, P.panels, pos, P.panels, P.pmask.p, P.ndist.p, mid.p, big.p, bsize.p,
            counts.p);
-    hipLaunchKernelGGL((k_panel_sort<kSortSmall, 256, FP32>), dim3((unsigned)P.panels), dim3(256),
-                       0, st, pos, (const int*)nullptr, col, val, inv_scale, S.col.p, S.val.p,
+    hipLaunchKernelGGL((k_panel_sort<kSortSmall, 256, FP32>), grid_of(P.panels), dim3(256), 0, st,
+                       pos, (const int*)nullptr, P.panels, col, val, inv_scale, S.col.p, S.val.p,
                        S.row.p, P.ndist.p);
     VCSRMC_HIP(hipGetLastError());
     int nsort[2];
     VCSRMC_HIP(hipMemcpyAsync(nsort, counts.p, sizeof nsort, hipMemcpyDeviceToHost, st));
     VCSRMC_HIP(hipStreamSynchronize(st));
     if (nsort[0] > 0) {
-        hipLaunchKernelGGL((k_panel_sort<kSortMid, 1024, FP32>), dim3((unsigned)nsort[0]),
-                           dim3(1024), 0, st, pos, (const int*)mid.p, col, val, inv_scale, S.col.p,
+        hipLaunchKernelGGL((k_panel_sort<kSortMid, 1024, FP32>), grid_of(nsort[0]), dim3(1024), 0,
+                           st, pos, (const int*)mid.p, nsort[0], col, val, inv_scale, S.col.p,
                            S.val.p, S.row.p, P.ndist.p);
         VCSRMC_HIP(hipGetLastError());
     }
@@ -992,12 +996,12 @@ static void fill_layout(DeviceFormat& F, const PanelSet& S, const SortedNonzeros
                F.chunk_eptr.p);
     }
     if (F.fp32)
-        hipLaunchKernelGGL((k_panel_fill<true>), dim3((unsigned)NP), dim3(256), 0, st, pstart.p,
-                           cbase.p, nz.col.p, nz.val.p, nz.row.p, F.entries.p, F.chunk_cols.p,
+        hipLaunchKernelGGL((k_panel_fill<true>), grid_of(NP), dim3(256), 0, st, pstart.p, cbase.p,
+                           NP, nz.col.p, nz.val.p, nz.row.p, F.entries.p, F.chunk_cols.p,
                            F.chunk_eptr.p);
     else
-        hipLaunchKernelGGL((k_panel_fill<false>), dim3((unsigned)NP), dim3(256), 0, st, pstart.p,
-                           cbase.p, nz.col.p, nz.val.p, nz.row.p, F.entries.p, F.chunk_cols.p,
+        hipLaunchKernelGGL((k_panel_fill<false>), grid_of(NP), dim3(256), 0, st, pstart.p, cbase.p,
+                           NP, nz.col.p, nz.val.p, nz.row.p, F.entries.p, F.chunk_cols.p,
                            F.chunk_eptr.p);
     VCSRMC_HIP(hipGetLastError());
 
@@ -1013,12 +1017,12 @@ static void fill_layout(DeviceFormat& F, const PanelSet& S, const SortedNonzeros
         if (ND > 0) {
             if (F.fp32) {
                 F.dense_a32.alloc((size_t)ND * 512);
-                hipLaunchKernelGGL((k_dense_fill<true>), dim3(grid_for(NC, 4)), dim3(256), 0, st,
+                hipLaunchKernelGGL((k_dense_fill<true>), grid_of(((long long)NC + 3) / 4), dim3(256), 0, st,
                                    F.entries.p, F.chunk_eptr.p, F.chunk_dense.p, NC,
                                    (_Float16*)nullptr, F.dense_a32.p);
             } else {
                 F.dense_a16.alloc((size_t)ND * 512);
-                hipLaunchKernelGGL((k_dense_fill<false>), dim3(grid_for(NC, 4)), dim3(256), 0, st,
+                hipLaunchKernelGGL((k_dense_fill<false>), grid_of(((long long)NC + 3) / 4), dim3(256), 0, st,
                                    F.entries.p, F.chunk_eptr.p, F.chunk_dense.p, NC,
                                    F.dense_a16.p, (float*)nullptr);
             }

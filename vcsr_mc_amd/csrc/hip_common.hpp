@@ -122,4 +122,15 @@ inline unsigned grid_for(long long n, int per_block) {
     return (unsigned)((n + per_block - 1) / per_block);
 }
 
+// A launch of one work-group (or wave) per item: HIP takes fewer than 2^32 work-items in a dimension
+// of the grid, so more than kGridRow work-groups continue in y.  group_index() may exceed the last.
+constexpr long long kGridRow = 1ll << 21;
+inline dim3 grid_of(long long groups) {
+    const long long x = groups < kGridRow ? groups : kGridRow;
+    return dim3((unsigned)x, (unsigned)((groups + x - 1) / x));
+}
+__device__ __forceinline__ long long group_index() {
+    return (long long)blockIdx.y * gridDim.x + blockIdx.x;
+}
+
 }  // namespace vcsrmc

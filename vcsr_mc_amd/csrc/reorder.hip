@@ -1083,7 +1083,7 @@ __global__ __launch_bounds__(256) void k_relabel_rows(
     const int* __restrict__ rp, const int* __restrict__ col, const float* __restrict__ val,
     const int* __restrict__ position, int M, int* __restrict__ cout, float* __restrict__ vout,
     int* __restrict__ listed, int* __restrict__ nlisted, int* __restrict__ err) {
-    const long long r = ((long long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+    const long long r = group_index() * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     if (r >= M) return;  // the whole wave
     const int a = __builtin_amdgcn_readfirstlane(rp[r]);
@@ -1380,8 +1380,9 @@ void apply_column_permutation_device(const int* rp, int* col, float* val, int M,
         if (longest <= kRowSortMax) {
             TmpBuf<int> listed(longest > 64 ? M : 0), nlisted(1);
             fill<int>(nlisted.p, 1, 0, st);
-            RLAUNCH(k_relabel_rows, 64ll * M, rp, col, val, position, M, ncol.p, nval.p, listed.p,
-                    nlisted.p, err.p);
+            hipLaunchKernelGGL(k_relabel_rows, grid_of(((long long)M + 3) / 4), dim3(256), 0, st, rp,
+                               col, val, position, M, ncol.p, nval.p, listed.p, nlisted.p, err.p);
+            VCSRMC_HIP(hipGetLastError());
             if (longest > 64) {
                 hipLaunchKernelGGL(k_relabel_listed, dim3(2048), dim3(256), 0, st, rp, col, val,
                                    position, listed.p, nlisted.p, ncol.p, nval.p, err.p);

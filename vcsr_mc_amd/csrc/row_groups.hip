@@ -51,6 +51,7 @@ constexpr int kMaxCols = 512;         // clusters with more (non-hub) columns ta
 constexpr int kInsertsPerLane = 256;  // candidate insertions per lane and cluster
 
 inline unsigned grid256(long long n) { return grid_for(n, 256); }
+inline dim3 waves_of(long long n) { return grid_of((n + 3) / 4); }  // four in a work-group
 
 __device__ __forceinline__ unsigned mix32(unsigned x) {
     x ^= x >> 16;
@@ -128,7 +129,7 @@ __global__ __launch_bounds__(256) void k_score(const uint32_t* __restrict__ ccol
     __shared__ __attribute__((aligned(16))) int tkey[4][kTable];
     __shared__ __attribute__((aligned(16))) int tcnt[4][kTable];
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const long long wa = (long long)blockIdx.x * 4 + w;
+    const long long wa = group_index() * 4 + w;
     if (wa >= nc) return;  // the whole wave
     const int a = __builtin_amdgcn_readfirstlane((int)wa);
     int* K = tkey[w];
@@ -315,9 +316,9 @@ __global__ __launch_bounds__(256) void k_union_sizes(const int2* __restrict__ pa
                                                      const int* __restrict__ ptr,
                                                      const uint32_t* __restrict__ ccol, int nnc,
                                                      int* __restrict__ len) {
-    const int x = (int)(((long long)blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-    const int lane = threadIdx.x & 63;
-    if (x >= nnc) return;  // the whole wave
+    const long long wx = group_index() * 4 + (threadIdx.x >> 6);
+    if (wx >= nnc) return;  // the whole wave
+    const int x = (int)wx, lane = threadIdx.x & 63;
     const int2 p = parts[x];
     const int a0 = ptr[p.x], a1 = ptr[p.x + 1];
     int total = a1 - a0;
@@ -343,9 +344,9 @@ __global__ __launch_bounds__(256) void k_union_write(const int2* __restrict__ pa
                                                      const int* __restrict__ nptr, int nnc,
                                                      uint32_t* __restrict__ ncol,
                                                      uint32_t* __restrict__ ncl) {
-    const int x = (int)(((long long)blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-    const int lane = threadIdx.x & 63;
-    if (x >= nnc) return;  // the whole wave
+    const long long wx = group_index() * 4 + (threadIdx.x >> 6);
+    if (wx >= nnc) return;  // the whole wave
+    const int x = (int)wx, lane = threadIdx.x & 63;
     const u64 below = lane ? (~0ull >> (64 - lane)) : 0ull;
     const int2 p = parts[x];
     const int out = nptr[x];
@@ -497,7 +498,7 @@ bool group_rows(const int* rp, const int* row_of, const int* col, long long n, i
         const int maxsz = 2 << level;  // clusters of 2^level rows pair into 2^(level+1)
         TmpBuf<int4> cand(nc);
         TmpBuf<int> mate(nc), prop(nc);
-        hipLaunchKernelGGL(k_score, dim3(grid_for(nc, 4)), dim3(256), 0, st, ccol, ptr, rcl,
+        hipLaunchKernelGGL(k_score, waves_of(nc), dim3(256), 0, st, ccol, ptr, rcl,
                            rc_ptr.p, size.p, cmin.p, nc, maxsz, level == kLevels - 1, cand.p);
         VCSRMC_HIP(hipGetLastError());
         k1.release(); k2.release(); v1.release(); v2.release();
@@ -528,13 +529,13 @@ bool group_rows(const int* rp, const int* row_of, const int* col, long long n, i
         cmin = std::move(ncmin);
         if (level + 1 < kLevels) {
             TmpBuf<int> len(nnc), nptr((size_t)nnc + 1);
-            hipLaunchKernelGGL(k_union_sizes, dim3(grid_for(nnc, 4)), dim3(256), 0, st, parts.p,
+            hipLaunchKernelGGL(k_union_sizes, waves_of(nnc), dim3(256), 0, st, parts.p,
                                ptr, ccol, nnc, len.p);
             VCSRMC_HIP(hipGetLastError());
             exclusive_sum<int, int>(len.p, nptr.p, nnc, st);
             const long long nu = read_scalar(nptr.p + nnc, st);
             TmpBuf<uint32_t> ncol(nu), ncl(nu);
-            hipLaunchKernelGGL(k_union_write, dim3(grid_for(nnc, 4)), dim3(256), 0, st, parts.p,
+            hipLaunchKernelGGL(k_union_write, waves_of(nnc), dim3(256), 0, st, parts.p,
                                ptr, ccol, nptr.p, nnc, ncol.p, ncl.p);
             VCSRMC_HIP(hipGetLastError());
             cl_col = std::move(ncol);
