@@ -20,10 +20,11 @@ def _rows(torch, M, nnz, N, g):
     return rp, (key - r * N).int(), r
 
 
-@pytest.mark.parametrize("M,nnz", [((1 << 26) + 5, 200000), ((1 << 26) + 5, 1 << 26),
-                                   ((1 << 28) + 9, 200000)])
+@pytest.mark.parametrize("M,nnz", [((1 << 26) + 5, 200000), ((1 << 26) + 5, 1 << 28),
+                                   ((1 << 28) + 9, 200000), (1 << 20, 200000),
+                                   ((1 << 20) + 1, 1 << 21), ((1 << 20) + 1, (1 << 21) + 6000)])
 def test_relabel_rows(M, nnz):
-    """Columns relabelled and rows sorted again, few nonzeros and about one a row."""
+    """Columns relabelled and rows sorted again, each row on its own or all by one sort."""
     import torch
     say("relabel", M, nnz)
     g = torch.Generator(device="cuda")

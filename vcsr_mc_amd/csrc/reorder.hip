@@ -1070,13 +1070,30 @@ __global__ void k_relabel_gather(const u64* __restrict__ key, const uint32_t* __
 // kRowSortMax, are listed and sorted by a work-group in LDS (bitonic).  A radix sort of (row, column)
 // keys of the whole matrix, which rows beyond that still take, moved 12 bytes a nonzero five times.
 // 27-point mesh 64^3, 6.9 M nonzeros: 95 us, ordering and relabelling 14.3 -> 13.8 ms.
+// A wave a row costs 0.19 ns a row, nonzeros or not, the keys about 0.09 ns a nonzero and 0.1 ms for
+// their launches: many rows of fewer than two nonzeros on average take the keys.  Rows alone / keys,
+// us, the checks included: 1 M rows of 0.3 M nonzeros 284 / 307, of 1 M 336 / 332, of 4 M 385 / 502;
+// 10 M rows of 1 M 1365 / 392, of 10 M 2100 / 968; 50 M rows of 1 M 3790 / 556; 3 M rows of 30 M
+// 1226 / 2690.
+constexpr int kRowsAlone = 1 << 20;  // up to this many rows never take the keys for being short
 constexpr int kRowSortMax = 4096;
 
-__global__ void k_longest_row(const int* __restrict__ rp, int M, int* __restrict__ longest) {
-    const long long r = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int len = r < M ? rp[r + 1] - rp[r] : 0;
-    const int m = wave_last(wave_scan(len, OpMax{}, INT_MIN));
-    if ((threadIdx.x & 63) == 0 && m > *longest) atomicMax(longest, m);
+// One atomic a work-group, of which a launch has at most kLongestBlocks: one a wave took 17 ns a wave
+// (relabelling 10 M rows of 1 M nonzeros 2.7 -> 1.4 ms).
+constexpr unsigned kLongestBlocks = 1024;
+
+__global__ __launch_bounds__(256) void k_longest_row(const int* __restrict__ rp, int M,
+                                                     int* __restrict__ longest) {
+    __shared__ int most;
+    if (threadIdx.x == 0) most = 0;
+    __syncthreads();
+    int m = 0;
+    for (long long r = (long long)blockIdx.x * 256 + threadIdx.x; r < M; r += 256ll * gridDim.x)
+        m = max(m, rp[r + 1] - rp[r]);
+    m = wave_last(wave_scan(m, OpMax{}, 0));
+    if ((threadIdx.x & 63) == 0) atomicMax(&most, m);
+    __syncthreads();
+    if (threadIdx.x == 0 && most > 0) atomicMax(longest, most);
 }
 
 __global__ __launch_bounds__(256) void k_relabel_rows(
@@ -1368,7 +1385,11 @@ void apply_column_permutation_device(const int* rp, int* col, float* val, int M,
     TmpBuf<int> err(2), seen(N);
     fill<int>(err.p, 2, 0, st);
     RLAUNCH(k_check_rp, (long long)M + 1, rp, M, nnz, err.p);
-    RLAUNCH(k_longest_row, M, rp, M, err.p + 1);
+    if (M > 0) {
+        hipLaunchKernelGGL(k_longest_row, dim3(std::min(nblk(M), kLongestBlocks)), dim3(256), 0, st,
+                           rp, M, err.p + 1);
+        VCSRMC_HIP(hipGetLastError());
+    }
     RLAUNCH(k_check_cols, (long long)nnz, col, (long long)nnz, N, err.p);
     fill<int>(seen.p, N, 0, st);
     RLAUNCH(k_perm_check, N, position, N, seen.p, err.p);
@@ -1377,7 +1398,7 @@ void apply_column_permutation_device(const int* rp, int* col, float* val, int M,
         const int longest = read_scalar(err.p + 1, st);
         TmpBuf<int> ncol(nnz);
         TmpBuf<float> nval(nnz);
-        if (longest <= kRowSortMax) {
+        if (longest <= kRowSortMax && (M <= kRowsAlone || 2ll * M <= nnz)) {
             TmpBuf<int> listed(longest > 64 ? M : 0), nlisted(1);
             fill<int>(nlisted.p, 1, 0, st);
             hipLaunchKernelGGL(k_relabel_rows, grid_of(((long long)M + 3) / 4), dim3(256), 0, st, rp,
