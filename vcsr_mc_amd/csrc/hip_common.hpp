@@ -1,27 +1,13 @@
-// hip_common.hpp -- error plumbing and wave64 helpers shared by the VCSR-MC HIP sources.
+// hip_common.hpp -- wave64 helpers shared by the VCSR-MC HIP sources.
 // Target: gfx950 (CDNA4), 64-lane wavefronts.
 #pragma once
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
-#include <stdexcept>
-#include <string>
+
+#include "hip_error.hpp"
 
 namespace vcsrmc {
-
-// Internal error: carries a C-ABI status code; converted to a return value at the ABI.
-struct Error : std::runtime_error {
-    int status;
-    Error(int s, const std::string& m) : std::runtime_error(m), status(s) {}
-};
-
-[[noreturn]] void throw_hip(hipError_t e, const char* what, const char* file, int line);
-
-#define VCSRMC_HIP(call)                                                        \
-    do {                                                                        \
-        const hipError_t e_ = (call);                                           \
-        if (e_ != hipSuccess) ::vcsrmc::throw_hip(e_, #call, __FILE__, __LINE__); \
-    } while (0)
 
 constexpr int kWave = 64;
 

@@ -8,6 +8,7 @@
 #include "../../include/reorder.hpp"
 #include "../../include/vcsr_formats.hpp"
 #include "../../include/vcsrmc.h"
+#include "device_memory.hpp"
 
 namespace {
 
@@ -35,13 +36,13 @@ template <typename T>
 struct Dev {
     T* p = nullptr;
     explicit Dev(const std::vector<T>& h) {
-        hip_check(hipMalloc((void**)&p, sizeof(T) * (h.size() ? h.size() : 1)), "hipMalloc");
+        hip_check(vcsrmc::device_malloc((void**)&p, sizeof(T) * (h.size() ? h.size() : 1)), "hipMalloc");
         if (!h.empty())
             hip_check(hipMemcpy(p, h.data(), sizeof(T) * h.size(), hipMemcpyHostToDevice),
                       "hipMemcpy");
     }
     explicit Dev(size_t n) {
-        hip_check(hipMalloc((void**)&p, sizeof(T) * (n ? n : 1)), "hipMalloc");
+        hip_check(vcsrmc::device_malloc((void**)&p, sizeof(T) * (n ? n : 1)), "hipMalloc");
     }
     ~Dev() { if (p) (void)hipFree(p); }
     void to_host(std::vector<T>& h) const {
