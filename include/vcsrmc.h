@@ -10,8 +10,9 @@
  * Threads: a handle holds all of its format's state, so different handles may be used from
  * different host threads at the same time; one handle must not be used by two threads at once
  * (its FP16 copy of an FP32 B is allocated on first use).  State shared by all handles is the
- * row-grouping mode and the RCM limits (atomics, read once per call) and the per-device
- * scratch of vcsrmc_spmm_noalloc (see there).  The C++ drop-in keeps the reference's single
+ * row-grouping mode and the RCM limits (atomics, read once per call), the per-device scratch
+ * of vcsrmc_spmm_noalloc (see there) and the device memory kept between calls
+ * (vcsrmc_release_scratch).  The C++ drop-in keeps the reference's single
  * library-global format and is not re-entrant, like the reference (src/vcsr_mc.cu:126-131).
  *
  * Each entry point names the reference interface it replaces (MuuSeoTia/VCSR_MC,
@@ -70,6 +71,13 @@ int vcsrmc_create(vcsrmc_t *out);
 /* Frees the device copies and the handle.  Replaces destroy_vcsr_mc_device
  * (include/vcsr_formats.hpp:26, src/vcsr_mc.cu:397-404). */
 int vcsrmc_destroy(vcsrmc_t h);
+
+/* Device memory that finished calls left for later ones goes back to the driver.  Builds, uploads
+ * and the reordering calls keep the scratch of a call that has ended, at most 2 GiB per process:
+ * a block is given back once 16 such calls have not used it, and all of them when an allocation of
+ * the library finds memory short.  Other allocators of the process see that memory as taken: call
+ * this when no build follows.  Any thread may, at any time; no counterpart in the reference. */
+int vcsrmc_release_scratch(void);
 
 /* FP16 range scale of the values of a device array (src/vcsr_mc.cu:14-22, evaluated as the
  * reference binary does: it is built with -ffast-math, CMakeLists.txt:24-27, so amax / 60000

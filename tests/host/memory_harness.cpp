@@ -130,6 +130,37 @@ static void unused_blocks_of_the_call_are_given_back() {
     CHECK(out_of_memory([] { TmpBuf<char> t(GB); }));
 }
 
+// A block stays for 16 calls that do not take it, however many blocks those use.
+static void blocks_age_by_calls() {
+    start(64 * GB);
+    call(100 * MB);
+    const uintptr_t block = card::live.begin()->first;
+    for (int i = 0; i < 17; ++i) {
+        CHECK(card::live.count(block) == 1);
+        ScratchScope scratch(200 * MB);
+        TmpBuf<char> a(200 * MB), b(220 * MB), c(240 * MB);
+        scratch.idle();
+    }
+    CHECK(card::live.count(block) == 0);
+}
+
+// At most 2 GiB are kept, the youngest; a call that asks for a word takes and leaves a word.
+static void kept_memory_is_bounded() {
+    start(64 * GB);
+    for (size_t size = 100 * MB; size < 3 * GB; size += 300 * MB) {
+        call(size);
+        CHECK(card::used <= 2 * GB);
+    }
+    start(64 * GB);
+    {
+        ScratchScope scratch(0);
+        TmpBuf<unsigned> word(1);
+        CHECK(card::used <= 4096);
+        scratch.idle();
+    }
+    CHECK(card::used <= 4096);
+}
+
 // Ranges in use at the same time never overlap, lie in live blocks, and all goes back.
 static void ranges_are_apart() {
     start(64 * GB);
@@ -196,6 +227,8 @@ int main(int argc, char** argv) {
     const std::pair<const char*, void (*)()> checks[] = {
         {"kept_blocks_are_given_back", kept_blocks_are_given_back},
         {"unused_blocks_of_the_call_are_given_back", unused_blocks_of_the_call_are_given_back},
+        {"blocks_age_by_calls", blocks_age_by_calls},
+        {"kept_memory_is_bounded", kept_memory_is_bounded},
         {"ranges_are_apart", ranges_are_apart},
         {"failed_calls_keep_nothing", failed_calls_keep_nothing},
         {"threads", threads},

@@ -98,6 +98,7 @@ def lib():
         L.vcsrmc_spmm_noalloc.argtypes = [vp, vp, C.c_int, C.c_int, C.c_int, vp, C.c_int, vp]
         L.vcsrmc_rcm_order.argtypes = [vp, vp, C.c_int, C.c_int, C.c_int, vp, vp]
         L.vcsrmc_set_rcm_limits.argtypes = [C.c_longlong, C.c_longlong]
+        L.vcsrmc_release_scratch.argtypes = []
         L.vcsrmc_set_row_grouping.argtypes = [C.c_int]
         L.vcsrmc_set_fp32_row_steps.argtypes = [C.c_int]
         L.vcsrmc_get_row_map.argtypes = [vp, vp, C.c_longlong, C.POINTER(C.c_longlong)]
@@ -114,7 +115,7 @@ def lib():
                   "vcsrmc_spmm_ex", "vcsrmc_spmm_noalloc", "vcsrmc_rcm_order",
                   "vcsrmc_set_rcm_limits", "vcsrmc_set_row_grouping", "vcsrmc_get_row_map",
                   "vcsrmc_apply_column_permutation", "vcsrmc_set_fp32_row_steps",
-                  "vcsrmc_get_units", "vcsrmc_traffic_floor"):
+                  "vcsrmc_get_units", "vcsrmc_traffic_floor", "vcsrmc_release_scratch"):
             getattr(L, f).restype = C.c_int
         _lib_handle = L
     return _lib_handle
@@ -420,6 +421,12 @@ class DeviceFormat:
 
 # ---- the reference's free functions (global single format, src/vcsr_mc.cu:126-131) ---------
 _global = {"fmt": None, "uploaded": False}
+
+
+def release_scratch() -> None:
+    """Gives the device memory that finished builds, uploads and reorderings left for later ones (at
+    most 2 GiB) back to the driver."""
+    _check(lib().vcsrmc_release_scratch(), "vcsrmc_release_scratch")
 
 
 def half_scale(csr: CSR) -> float:

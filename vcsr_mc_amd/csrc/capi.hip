@@ -114,6 +114,10 @@ int vcsrmc_destroy(vcsrmc_t h) {
     });
 }
 
+int vcsrmc_release_scratch(void) {
+    return guarded([] { vcsrmc::BlockCache::instance().give_back_all(); });
+}
+
 int vcsrmc_half_scale(const float* d_val, long long nnz, float* scale, void* stream) {
     return guarded([&] {
         need(scale != nullptr && nnz >= 0 && (nnz == 0 || d_val != nullptr), "bad argument");

@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <cstddef>
 #include <mutex>
+#include <new>
 #include <utility>
 #include <vector>
 
@@ -63,8 +64,10 @@ struct DevBuf {
 // or stream: the driver clears memory that is freed, and a program that builds or orders one matrix
 // after another frees faster than that (builds of the stencil in a row: 14 ms at first, 34 once no
 // cleared memory is left; orderings of a 64^3 mesh 3.6, then 17).  The cache holds at most
-// kMaxBytes, gives back a block that the last kIdleCalls calls did not take, and all of them when any
-// allocation of the library finds memory short (device_malloc).  A call that ends in an error frees its blocks (hipFree waits for the device).
+// kMaxBytes, gives back a block that the last kIdleCalls calls with scratch did not take, and all of
+// them when any allocation of the library finds memory short (device_malloc) or the caller asks for it
+// (vcsrmc_release_scratch): a program that builds once and then multiplies makes no later call that
+// would give them back.  A call that ends in an error frees its blocks (hipFree waits for the device).
 class BlockCache {
 public:
     static BlockCache& instance() {
@@ -86,16 +89,17 @@ public:
         kept_.erase(kept_.begin() + best);
         return p;
     }
-    void give(int device, char* p, size_t size) {
+    // The blocks of one call.
+    void give(int device, const std::vector<std::pair<char*, size_t>>& blocks) noexcept {
         std::vector<char*> out;
-        {
+        try {
             std::lock_guard<std::mutex> lock(m_);
+            out.reserve(kept_.size() + blocks.size());
+            kept_.reserve(kept_.size() + blocks.size());
             ++calls_;
-            if (size <= kMaxBytes) {
+            for (const auto& [p, size] : blocks) {
                 kept_.push_back(Kept{device, p, size, calls_});
                 total_ += size;
-            } else {
-                out.push_back(p);
             }
             for (size_t i = 0; i < kept_.size();)  // oldest first
                 if (total_ > kMaxBytes || calls_ - kept_[i].call > kIdleCalls) {
@@ -105,6 +109,8 @@ public:
                 } else {
                     ++i;
                 }
+        } catch (const std::bad_alloc&) {  // of the two reserves: nothing was kept
+            for (const auto& b : blocks) (void)hipFree(b.first);
         }
         for (char* q : out) (void)hipFree(q);
     }
@@ -141,14 +147,22 @@ public:
     Arena(const Arena&) = delete;
     Arena& operator=(const Arena&) = delete;
     ~Arena() {
-        for (Block& b : blocks_)
-            if (idle_) BlockCache::instance().give(device_, b.p, b.size);
-            else (void)hipFree(b.p);
+        if (idle_ && !blocks_.empty()) {
+            try {
+                std::vector<std::pair<char*, size_t>> all;
+                for (const Block& b : blocks_) all.emplace_back(b.p, b.size);
+                BlockCache::instance().give(device_, all);
+                return;
+            } catch (const std::bad_alloc&) {
+            }
+        }
+        for (Block& b : blocks_) (void)hipFree(b.p);
     }
     // The call has waited for its stream: nothing on the device uses the blocks any more.
     void idle() { idle_ = true; }
-    // The size of the first block; later ones are as large as what asks for them, or kBlock.
-    void reserve(size_t bytes) { first_ = bytes; }
+    // The size of the first block (0: as large as what asks for it); later ones are as large as what
+    // asks for them, or kBlock.
+    void reserve(size_t bytes) { first_ = bytes ? std::max(bytes, kBlock) : 0; }
     void* take(size_t bytes) {
         bytes = (bytes + kAlign - 1) / kAlign * kAlign;
         for (Block& b : blocks_)
@@ -161,7 +175,7 @@ public:
                 if (r.size == 0) b.free.erase(b.free.begin() + i);
                 return p;
             }
-        size_t size = std::max(bytes, blocks_.empty() ? std::max(first_, kBlock) : kBlock);
+        size_t size = std::max(bytes, blocks_.empty() ? first_ : kBlock);
         blocks_.reserve(blocks_.size() + 1);
         if (device_ < 0) VCSRMC_HIP(hipGetDevice(&device_));
         char* p = BlockCache::instance().take(device_, size, size);
