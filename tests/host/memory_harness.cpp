@@ -130,6 +130,41 @@ static void unused_blocks_of_the_call_are_given_back() {
     CHECK(out_of_memory([] { TmpBuf<char> t(GB); }));
 }
 
+// What a call can use does not depend on what it has reserved or what earlier calls left.
+static void available_counts_idle_memory() {
+    start(64 * GB);
+    call(GB);
+    ScratchScope scratch(2 * GB);
+    CHECK(tl_arena->available() == 64 * GB);
+    TmpBuf<char> a(512 * MB);
+    CHECK(tl_arena->available() == 64 * GB - 512 * MB);
+    DevBuf<char> format(GB);
+    {
+        TmpBuf<char> b(8 * GB);
+        CHECK(tl_arena->available() == 64 * GB - 512 * MB - 9 * GB);
+    }
+    CHECK(tl_arena->available() == 64 * GB - 512 * MB - GB);
+}
+
+// Scratch is reserved ahead only where there is room for what lasts; else it grows as asked for.
+static void large_reserves_need_room() {
+    start(64 * GB);
+    {
+        ScratchScope scratch(12 * GB);
+        TmpBuf<char> a(MB);
+        CHECK(card::used == 12 * GB);
+    }
+    CHECK(card::used == 0);
+    {
+        DevBuf<char> others(40 * GB);
+        ScratchScope scratch(12 * GB);
+        TmpBuf<char> a(MB), b(GB);
+        CHECK(card::used < 42 * GB);
+        DevBuf<char> format(22 * GB);
+    }
+    CHECK(card::used == 0);
+}
+
 // A block stays for 16 calls that do not take it, however many blocks those use.
 static void blocks_age_by_calls() {
     start(64 * GB);
@@ -227,6 +262,8 @@ int main(int argc, char** argv) {
     const std::pair<const char*, void (*)()> checks[] = {
         {"kept_blocks_are_given_back", kept_blocks_are_given_back},
         {"unused_blocks_of_the_call_are_given_back", unused_blocks_of_the_call_are_given_back},
+        {"available_counts_idle_memory", available_counts_idle_memory},
+        {"large_reserves_need_room", large_reserves_need_room},
         {"blocks_age_by_calls", blocks_age_by_calls},
         {"kept_memory_is_bounded", kept_memory_is_bounded},
         {"ranges_are_apart", ranges_are_apart},

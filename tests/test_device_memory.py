@@ -21,7 +21,8 @@ def harness(tmp_path_factory):
 
 
 @pytest.mark.parametrize("check", [
-    "kept_blocks_are_given_back", "unused_blocks_of_the_call_are_given_back", "blocks_age_by_calls",
+    "kept_blocks_are_given_back", "unused_blocks_of_the_call_are_given_back", "available_counts_idle_memory",
+    "large_reserves_need_room", "blocks_age_by_calls",
     "kept_memory_is_bounded", "ranges_are_apart", "failed_calls_keep_nothing", "threads"])
 def test_device_memory(harness, check):
     r = subprocess.run([harness, check], capture_output=True, text=True, timeout=120)

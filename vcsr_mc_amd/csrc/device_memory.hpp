@@ -114,6 +114,12 @@ public:
         }
         for (char* q : out) (void)hipFree(q);
     }
+    size_t kept(int device) {
+        std::lock_guard<std::mutex> lock(m_);
+        size_t bytes = 0;
+        for (const Kept& k : kept_) bytes += k.device == device ? k.size : 0;
+        return bytes;
+    }
     // Whether there were any.
     bool give_back_all() {
         std::vector<Kept> out;
@@ -161,8 +167,26 @@ public:
     // The call has waited for its stream: nothing on the device uses the blocks any more.
     void idle() { idle_ = true; }
     // The size of the first block (0: as large as what asks for it); later ones are as large as what
-    // asks for them, or kBlock.
-    void reserve(size_t bytes) { first_ = bytes ? std::max(bytes, kBlock) : 0; }
+    // asks for them, or kBlock.  A large one is not reserved ahead unless four times as much is
+    // free: what a call makes to last, a format, has to find room beside it.
+    void reserve(size_t bytes) {
+        first_ = bytes ? std::max(bytes, kBlock) : 0;
+        if (first_ > kLargeReserve && first_ > available() / 4) first_ = kBlock;
+    }
+    // Free memory of the current device for temporaries of this call: the driver's, what is kept from
+    // earlier calls, and what this call holds and does not use.
+    size_t available() {
+        int device = 0;
+        size_t bytes = 0, total = 0;
+        if (hipGetDevice(&device) != hipSuccess || hipMemGetInfo(&bytes, &total) != hipSuccess) {
+            (void)hipGetLastError();
+            return 0;
+        }
+        bytes += BlockCache::instance().kept(device);
+        for (const Block& b : blocks_)
+            for (const Range& r : b.free) bytes += r.size;
+        return bytes;
+    }
     void* take(size_t bytes) {
         bytes = (bytes + kAlign - 1) / kAlign * kAlign;
         for (Block& b : blocks_)
@@ -228,7 +252,7 @@ public:
     }
 
 private:
-    static constexpr size_t kAlign = 256, kBlock = (size_t)32 << 20;
+    static constexpr size_t kAlign = 256, kBlock = (size_t)32 << 20, kLargeReserve = (size_t)1 << 30;
     struct Range {
         size_t at, size;
     };

@@ -1185,12 +1185,9 @@ static void build_exec_layout_t(DeviceFormat& F, const int* rp, const int* row_o
     if (mode == 1 && 10 * n >= 13LL * S.pairs && n < 256LL * S.NC) {
         // Grouping is an optimisation here: it is skipped, natural order kept, unless its buffers
         // (at most ~64 bytes per nonzero and per row, for the lists and their sorts) fit in half
-        // the free device memory.
-        size_t free_b = 0, total_b = 0;
-        if (hipMemGetInfo(&free_b, &total_b) == hipSuccess)
-            group = 64.0 * (double)n + 64.0 * (double)F.M <= 0.5 * (double)free_b;
-        else
-            (void)hipGetLastError();
+        // the device memory that this call can use.  What it has reserved for them, and what earlier
+        // calls left, is free: the order depends on neither.
+        group = 64.0 * (double)n + 64.0 * (double)F.M <= 0.5 * (double)tl_arena->available();
     }
     DevBuf<int> groups;
     if (group && group_rows(rp, row_of, col, n, F.M, F.N, st, groups)) {

@@ -1380,7 +1380,10 @@ void apply_column_permutation_device(const int* rp, int* col, float* val, int M,
     if ((B == nullptr) != (B_out == nullptr))
         throw Error(VCSRMC_ERR_ARG, "B and B_out must both be given or both be NULL");
     if (B && B == B_out) throw Error(VCSRMC_ERR_ARG, "B_out must not alias B");
-    ScratchScope scratch((size_t)(36ll * nnz + 8ll * N + 4ll * M));
+    // rows on their own: columns and values; else keys and payloads too (rows beyond kRowSortMax,
+    // which are not known yet, ask for those when they come to it)
+    const bool rows_alone = M <= kRowsAlone || 2ll * M <= nnz;
+    ScratchScope scratch((size_t)((rows_alone ? 8ll : 36ll) * nnz + 8ll * N + 4ll * M));
     // every check of the input at once: {errors, longest row}
     TmpBuf<int> err(2), seen(N);
     fill<int>(err.p, 2, 0, st);
@@ -1398,7 +1401,7 @@ void apply_column_permutation_device(const int* rp, int* col, float* val, int M,
         const int longest = read_scalar(err.p + 1, st);
         TmpBuf<int> ncol(nnz);
         TmpBuf<float> nval(nnz);
-        if (longest <= kRowSortMax && (M <= kRowsAlone || 2ll * M <= nnz)) {
+        if (longest <= kRowSortMax && rows_alone) {
             TmpBuf<int> listed(longest > 64 ? M : 0), nlisted(1);
             fill<int>(nlisted.p, 1, 0, st);
             hipLaunchKernelGGL(k_relabel_rows, grid_of(((long long)M + 3) / 4), dim3(256), 0, st, rp,

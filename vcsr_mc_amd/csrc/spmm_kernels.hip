@@ -153,10 +153,13 @@ __device__ __forceinline__ auto load_b_row(const TB* __restrict__ B, int slot, l
     }
 }
 
-// A pause of 16 cycles after each load of a B row, in launches whose B comes from beyond the
-// last-level cache (FAR, the launches that read C non-temporally).  A wave that issues its eight
-// rows back to back there ends up slower: R-MAT scale 22 FP16 2480 us, with the pause 2440; scale 19
-// FP32 at O = 256 859 -> 835; stencil 100^3 and blocks within 0.5% (64 cycles: scale 20 472 -> 496).
+// A pause of 16 cycles after each load of a B row (FAR), in the launches that read C non-temporally:
+// those that accumulate, are aligned, and whose B and C together exceed the last-level cache.  A wave
+// that issues its eight rows back to back ends up slower where they come from beyond that cache.
+// With the pause / without, us: R-MAT scale 22 FP16 2430 / 2491, scale 20 FP16 O = 256 946 / 953,
+// scale 19 FP32 O = 256 817 / 822, stencil 100^3 401 / 403, blocks FP32 250.7 / 250.5, FP16 160.6 /
+// 159.9 (64 cycles, scale 20: 472 -> 496).  Launches of those sizes that overwrite C, or are ragged,
+// go without.
 __device__ __forceinline__ void space_loads() {
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("s_nop 15");
