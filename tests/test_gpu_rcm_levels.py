@@ -1,6 +1,7 @@
 """Sizes where the ordering's walk and the relabelling change paths: levels above one work-group's
 8192 edges, children sorted by a lane (up to 64), in LDS and in memory (8192), a wave's children
-beyond its 512 staged, and rows sorted by a wave (64), by a work-group (4096) or by keys."""
+beyond its 512 staged, adjacency lists cut into segments of 512 (with a vertex of more than 2048
+neighbours), and rows sorted by a wave (64), by a work-group (4096) or by keys."""
 import numpy as np
 import pytest
 
@@ -17,6 +18,9 @@ pytestmark = pytest.mark.gpu
     (1, 8190, 8191, 8192, 8193, 8194, 2),
     tuple([0, 70, 0, 600, 3] * 40),
     (60000, 66, 5),
+    (2045, 2046, 2047, 2048, 511, 512, 513, 1),
+    (2049, 1023, 1024, 1025, 510, 0, 64, 65, 4095, 4096, 4097),
+    tuple([2500, 0, 1, 700] * 12),
 ])
 def test_hub_levels(orc, sizes):
     """A centre joined to hubs with the given numbers of leaves, the leaves with 0 to 5 pendant
@@ -40,6 +44,28 @@ def test_hub_levels(orc, sizes):
     e = e[rng.permutation(len(e))]
     rp, col = csr_from_edges(n, n, [tuple(x) for x in e])
     say("hub levels", sizes[:4], n, col.size)
+    assert np.array_equal(gpu_rcm(rp, col, n, n), orc.rcm_order(rp, col, n, n))
+
+
+@pytest.mark.parametrize("hubs,n,spread", [(1, 70000, 1), (4, 40000, 1), (30, 20000, 40),
+                                           (3, 100000, 2000), (200, 30000, 7)])
+def test_shared_hubs(orc, hubs, n, spread):
+    """Hubs joined to most vertices, which all compete for them: lists cut into segments, groups split
+    in several passes and, with degrees that lie far apart (`spread`), in parts of unlike sizes."""
+    rng = np.random.default_rng(hubs * 7 + spread)
+    e = []
+    for k in range(hubs):
+        leaves = rng.choice(n, int(n * rng.uniform(0.3, 1.0)), replace=False)
+        e.append(np.stack([np.full(leaves.size, k), leaves], 1))
+    # edges among the leaves, their number falling off steeply from vertex to vertex
+    k = np.minimum(spread, (spread / (1 + rng.permutation(n) % 997)).astype(np.int64))
+    src = np.repeat(np.arange(n), k)
+    e.append(np.stack([src, rng.integers(0, n, src.size)], 1))
+    e = np.concatenate(e)
+    key = np.unique(rng.permutation(n)[e] @ np.array([n, 1]))
+    rp = np.searchsorted(key, n * np.arange(n + 1)).astype(np.int32)
+    col = (key % n).astype(np.int32)
+    say("shared hubs", hubs, n, spread, col.size)
     assert np.array_equal(gpu_rcm(rp, col, n, n), orc.rcm_order(rp, col, n, n))
 
 

@@ -28,6 +28,7 @@
 #include <climits>
 #include <cstdint>
 #include <string>
+#include <type_traits>
 
 #include "../../include/vcsrmc.h"
 #include "internal.hpp"
@@ -718,14 +719,30 @@ __global__ __launch_bounds__(kBfsThreads) void k_bfs_levels(
 
 // ---- 4b. a level of any size, four kernels over its edges ----------------------------------
 // Work-groups own contiguous runs of frontier vertices (level_run), waves eight of them at a time:
-// the wave's lanes go over the eight adjacency lists end to end (WaveEdges), so a hub's list is
-// spread over the lanes and short lists share a round.  An edge's place among its work-group's
-// edges is then also its children's order: (parent, ascending id).
+// the wave's lanes go over the eight adjacency lists end to end (WaveEdges), so short lists share a
+// round.  An edge's place among its work-group's edges is then also its children's order: (parent,
+// ascending id).
+// In a graph with a vertex of more than kHubDegree neighbours (HUBS) the lists are cut into segments
+// of kSegment edges first, two more kernels a level, and the waves take eight segments at a time: the
+// order of segments is the order of edges.  With a hub's list on one wave, ordering four hubs joined
+// to 1 M vertices each took 72.6 ms, now 5.1 (20 kernels a level, as below, 23.5); 20 hubs of 0.1 M
+// neighbours 26.9, now 5.4; R-MAT scale 18 4.3, now 2.4.
 // With sizes known to the host a level took ~20 kernels (a radix sort of (parent, id) keys, scans,
 // sorts of the groups) and four host round trips: the ordering of a 27-point mesh 64^3 in random
 // numbering, 53 levels above 8192 edges, 14.3 -> 3.6 ms, its relabelling included.
 constexpr int kLevelBlocks = 1024, kLevelWaves = 4, kLevelVerts = 8;
 constexpr int kLevelStage = 512;  // children a wave sorts in LDS at a time
+constexpr int kHubDegree = 2048, kSegment = 512;
+
+// Counters of a level: {child groups left to k_level_sort, pieces of the split ones, segments,
+// ranges left by every split pass}.
+enum : int { kGroups, kPieces, kSegments, kRanges };
+constexpr int kSplitPasses = 24;
+constexpr int kCounters = kRanges + kSplitPasses;
+
+// A segment: the place of its vertex, its first edge and edges, and -1, or (of a vertex cut into
+// several) 4 times its job, plus kFirstSegment and kLastSegment.
+enum : int { kFirstSegment = 1, kLastSegment = 2 };
 
 __device__ __forceinline__ bool level_over(const int4& s, long long max_level) {
     return s.w || s.x == 0 || s.z > max_level;
@@ -739,25 +756,43 @@ __device__ __forceinline__ int2 level_run(int f) {
     return make_int2((int)min(b, (long long)f), (int)min(b + per, (long long)f));
 }
 
-// The edges of frontier vertices v0 .. v1 - 1 (at most kLevelVerts), end to end.  Lanes past the
-// last vertex hold excl = total, so vertex() never picks them for e < total; of equal excl the last
-// holds the edge, the lists before it being empty.
+// The edges of frontier items v0 .. v1 - 1 (at most kLevelVerts vertices, or HUBS: segments), end to
+// end.  Lanes past the last item hold excl = total, so vertex() never picks them for e < total; of
+// equal excl the last holds the edge, the lists before it being empty.
+template <bool HUBS>
 struct WaveEdges {
-    int begin, excl, total;  // lane i < 8: its vertex's list, and the edges before it
-    __device__ __forceinline__ WaveEdges(const int* walk, const int* head, int at, int v0, int v1) {
+    int begin, excl, total;  // lane i < 8: its item's list, and the edges before it
+    int place, part;         // lane i < 8: its vertex's place, its segment's last word
+    __device__ __forceinline__ WaveEdges(const int* walk, const int* head, const int4* segs, int at,
+                                         int v0, int v1) {
         const int lane = threadIdx.x & 63;
         int deg = 0;
         begin = 0;
+        place = at + v0 + lane;
+        part = -1;
         if (v0 + lane < v1) {
-            const int v = walk[at + v0 + lane];
-            begin = head[v];
-            deg = head[v + 1] - begin;
+            if constexpr (HUBS) {
+                const int4 g = segs[v0 + lane];
+                place = g.x;
+                begin = g.y;
+                deg = g.z;
+                part = g.w;
+            } else {
+                const int v = walk[place];
+                begin = head[v];
+                deg = head[v + 1] - begin;
+            }
         }
         const int incl = wave_scan(deg, OpAdd{}, 0);
         excl = incl - deg;
         total = wave_last(incl);
     }
-    // The vertex (0 .. 7) of edge e < total, and the edge's index in adj: every lane together.
+    // The place of item v's vertex: every lane together.
+    __device__ __forceinline__ int parent(int v) const {
+        if constexpr (HUBS) return __shfl(place, v);
+        else return place - (int)(threadIdx.x & 63) + v;
+    }
+    // The item (0 .. 7) of edge e < total, and the edge's index in adj: every lane together.
     __device__ __forceinline__ int vertex(int e, int& index) const {
         int v = 0;
 #pragma unroll
@@ -766,9 +801,9 @@ struct WaveEdges {
         index = __shfl(begin, v) + e - __shfl(excl, v);
         return v;
     }
-    // f(neighbour, vertex, whether the lane holds an edge) for 64 edges at a time, in order.  The
-    // loop waits for memory: U rounds' neighbours, and what `also` loads for each, are in flight
-    // at once (eight rounds where a hub makes the lists long).
+    // f(neighbour, item, also's value, whether the lane holds an edge) for 64 edges at a time, in
+    // order, all lanes together.  The loop waits for memory: U rounds' neighbours, and what `also`
+    // loads for each, are in flight at once (eight rounds where the lists are long).
     template <int U, typename Also, typename F>
     __device__ __forceinline__ void rounds(const int* adj, Also&& also, F&& f) const {
         const int lane = threadIdx.x & 63;
@@ -794,42 +829,128 @@ struct WaveEdges {
     }
 };
 
+// Segments of each work-group's run of frontier vertices.
+__global__ __launch_bounds__(256) void k_level_seg_count(
+    const int* __restrict__ walk, const int* __restrict__ head, const int4* __restrict__ state,
+    long long max_level, int* __restrict__ block_segs, int* __restrict__ counters) {
+    __shared__ int total;
+    const int4 s = *state;
+    if (blockIdx.x == 0 && threadIdx.x < kCounters) counters[threadIdx.x] = 0;
+    if (level_over(s, max_level)) return;
+    if (threadIdx.x == 0) total = 0;
+    __syncthreads();
+    const int2 run = level_run(s.x);
+    int n = 0;
+    for (int i = run.x + (int)threadIdx.x; i < run.y; i += 256) {
+        const int v = walk[s.y - s.x + i];
+        n += (head[v + 1] - head[v] + kSegment - 1) / kSegment;
+    }
+    n = wave_last(wave_scan(n, OpAdd{}, 0));
+    if ((threadIdx.x & 63) == 0 && n) atomicAdd(&total, n);
+    __syncthreads();
+    if (threadIdx.x == 0) block_segs[blockIdx.x] = total;
+}
+
+// The sums of `counts` over the work-groups before this one and over all, by 256 threads.
+__device__ __forceinline__ void block_sums(const int* __restrict__ counts, int& before, int& all,
+                                           int* part /* LDS[2] */) {
+    if (threadIdx.x < 2) part[threadIdx.x] = 0;
+    __syncthreads();
+    int b = 0, a = 0;
+    for (int i = threadIdx.x; i < kLevelBlocks; i += 256) {
+        const int c = counts[i];
+        a += c;
+        if (i < (int)blockIdx.x) b += c;
+    }
+    b = wave_last(wave_scan(b, OpAdd{}, 0));
+    a = wave_last(wave_scan(a, OpAdd{}, 0));
+    if ((threadIdx.x & 63) == 0) {
+        atomicAdd(&part[0], b);
+        atomicAdd(&part[1], a);
+    }
+    __syncthreads();
+    before = part[0];
+    all = part[1];
+}
+
+// The segments, in order.  A vertex of several gets a job of its own here; k_level_place fills in
+// where its children begin and end.
+__global__ __launch_bounds__(256) void k_level_seg_write(
+    const int* __restrict__ walk, const int* __restrict__ head, const int4* __restrict__ state,
+    long long max_level, const int* __restrict__ block_segs, int4* __restrict__ segs,
+    int4* __restrict__ jobs, int* __restrict__ counters) {
+    __shared__ int part[2], wsum[4];
+    const int4 s = *state;
+    if (level_over(s, max_level)) return;
+    int out, all;
+    block_sums(block_segs, out, all, part);
+    if (blockIdx.x == 0 && threadIdx.x == 0) counters[kSegments] = all;
+    const int2 run = level_run(s.x);
+    for (int i0 = run.x; i0 < run.y; i0 += 256) {
+        const int i = i0 + (int)threadIdx.x, place = s.y - s.x + i;
+        int begin = 0, deg = 0;
+        if (i < run.y) {
+            const int v = walk[place];
+            begin = head[v];
+            deg = head[v + 1] - begin;
+        }
+        const int n = (deg + kSegment - 1) / kSegment;
+        int sum;
+        const int at = out + block_scan_256(n, OpAdd{}, 0, wsum, sum) - n;
+        if (n == 1) segs[at] = make_int4(place, begin, deg, -1);
+        if (n > 1) {
+            const int job = atomicAdd(&counters[kGroups], 1);
+            jobs[job] = make_int4(0, 0, -1, 0);
+            for (int k = 0; k < n; ++k)
+                segs[at + k] =
+                    make_int4(place, begin + k * kSegment, min(kSegment, deg - k * kSegment),
+                              4 * job + (k == 0 ? kFirstSegment : 0) + (k == n - 1 ? kLastSegment : 0));
+        }
+        out += sum;
+        __syncthreads();
+    }
+}
+
+template <bool HUBS>
 __global__ __launch_bounds__(64 * kLevelWaves) void k_level_claim(
     const int* __restrict__ walk, const int* __restrict__ head, const int* __restrict__ adj,
-    const int* __restrict__ seq, int* claim, const int4* __restrict__ state, long long max_level,
-    int* __restrict__ njobs) {
+    const int4* __restrict__ segs, const int* __restrict__ seq, int* claim,
+    const int4* __restrict__ state, long long max_level, int* __restrict__ counters) {
     const int4 s = *state;
-    if (blockIdx.x == 0 && threadIdx.x < 2) njobs[threadIdx.x] = 0;
+    if (!HUBS && blockIdx.x == 0 && threadIdx.x < kCounters) counters[threadIdx.x] = 0;
     if (level_over(s, max_level)) return;
-    const int2 run = level_run(s.x);
+    const int2 run = level_run(HUBS ? counters[kSegments] : s.x);
     const int at = s.y - s.x, w = threadIdx.x >> 6;
     for (int v0 = run.x + w * kLevelVerts; v0 < run.y; v0 += kLevelWaves * kLevelVerts) {
-        const WaveEdges E(walk, head, at, v0, min(v0 + kLevelVerts, run.y));
+        const WaveEdges<HUBS> E(walk, head, segs, at, v0, min(v0 + kLevelVerts, run.y));
         E.each(adj, [&](int u) { return seq[u]; },
-               [&](int u, int v, int place, bool edge) {
-                   if (edge && place < 0) atomicMin(&claim[u], at + v0 + v);
+               [&](int u, int v, int placed, bool edge) {
+                   const int parent = E.parent(v);
+                   if (edge && placed < 0) atomicMin(&claim[u], parent);
                });
     }
 }
 
 // Children of each work-group's run.
+template <bool HUBS>
 __global__ __launch_bounds__(64 * kLevelWaves) void k_level_count(
     const int* __restrict__ walk, const int* __restrict__ head, const int* __restrict__ adj,
-    const int* __restrict__ claim, const int4* __restrict__ state, long long max_level,
-    int* __restrict__ block_children) {
+    const int4* __restrict__ segs, const int* __restrict__ claim, const int4* __restrict__ state,
+    long long max_level, int* __restrict__ block_children, const int* __restrict__ counters) {
     __shared__ int total;
     const int4 s = *state;
     if (level_over(s, max_level)) return;
     if (threadIdx.x == 0) total = 0;
     __syncthreads();
-    const int2 run = level_run(s.x);
+    const int2 run = level_run(HUBS ? counters[kSegments] : s.x);
     const int at = s.y - s.x, w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     int n = 0;
     for (int v0 = run.x + w * kLevelVerts; v0 < run.y; v0 += kLevelWaves * kLevelVerts) {
-        const WaveEdges E(walk, head, at, v0, min(v0 + kLevelVerts, run.y));
+        const WaveEdges<HUBS> E(walk, head, segs, at, v0, min(v0 + kLevelVerts, run.y));
         E.each(adj, [&](int u) { return claim[u]; },
-               [&](int, int v, int place, bool edge) {
-                   n += __popcll(__ballot(edge && place == at + v0 + v));
+               [&](int, int v, int parent, bool edge) {
+                   const bool mine = parent == E.parent(v) && edge;
+                   n += __popcll(__ballot(mine));
                });
     }
     if (lane == 0 && n) atomicAdd(&total, n);
@@ -840,55 +961,41 @@ __global__ __launch_bounds__(64 * kLevelWaves) void k_level_count(
 // Places the children: packed degree << 32 | id in child[], in (parent, ascending id) order.  A
 // wave's children are staged in LDS, where each vertex's are sorted by one lane, and take their
 // places; vertices with more than kBfsSortSmall children, and all of a wave with more than
-// kLevelStage, become jobs {begin, end, partition depth} for k_level_sort.  The next state goes to `next`.
+// kLevelStage, become jobs {begin, end, partition depth} for k_level_sort, as those of several
+// segments are already (depth -1: from the size).  The next state goes to `next`.
+template <bool HUBS>
 __global__ __launch_bounds__(64 * kLevelWaves) void k_level_place(
-    int* walk, const int* __restrict__ head, const int* __restrict__ adj, int* seq,
-    const int* __restrict__ claim, const int4* __restrict__ state, int4* __restrict__ next,
-    long long max_level, const int* __restrict__ block_children, u64* __restrict__ child,
-    int4* __restrict__ jobs, int* __restrict__ njobs) {
+    int* walk, const int* __restrict__ head, const int* __restrict__ adj,
+    const int4* __restrict__ segs, int* seq, const int* __restrict__ claim,
+    const int4* __restrict__ state, int4* __restrict__ next, long long max_level,
+    const int* __restrict__ block_children, u64* __restrict__ child, int4* __restrict__ jobs,
+    int* __restrict__ counters) {
     __shared__ u64 s_stage[kLevelWaves][kLevelStage];
     __shared__ int s_cnt[kLevelWaves][kLevelVerts];
     __shared__ int s_round[2][kLevelWaves];
-    __shared__ int s_before, s_all;
+    __shared__ int s_part[2];
     const int4 s = *state;
     if (level_over(s, max_level)) {
         if (blockIdx.x == 0 && threadIdx.x == 0) *next = make_int4(s.x, s.y, s.z, s.w | (s.x == 0));
         return;
     }
     const int t = threadIdx.x, w = t >> 6, lane = t & 63;
-    if (t == 0) s_before = s_all = 0;
-    __syncthreads();
-    {
-        int before = 0, all = 0;
-        for (int b = t; b < kLevelBlocks; b += 64 * kLevelWaves) {
-            const int c = block_children[b];
-            all += c;
-            if (b < (int)blockIdx.x) before += c;
-        }
-        before = wave_last(wave_scan(before, OpAdd{}, 0));
-        all = wave_last(wave_scan(all, OpAdd{}, 0));
-        if (lane == 0) {
-            atomicAdd(&s_before, before);
-            atomicAdd(&s_all, all);
-        }
-    }
-    __syncthreads();
-    if (blockIdx.x == 0 && t == 0)
-        *next = make_int4(s_all, s.y + s_all, s.z + 1, s_all == 0);
-    const int2 run = level_run(s.x);
+    int out, all, phase = 0;  // out: children before this round's items
+    block_sums(block_children, out, all, s_part);
+    if (blockIdx.x == 0 && t == 0) *next = make_int4(all, s.y + all, s.z + 1, all == 0);
+    const int2 run = level_run(HUBS ? counters[kSegments] : s.x);
     const int at = s.y - s.x;
-    int out = s_before, phase = 0;  // children before this round's vertices
     const u64 below = lane ? (~0ull >> (64 - lane)) : 0ull;
     for (int r0 = run.x; r0 < run.y; r0 += kLevelWaves * kLevelVerts, phase ^= 1) {
         const int v0 = min(r0 + w * kLevelVerts, run.y), v1 = min(v0 + kLevelVerts, run.y);
-        const WaveEdges E(walk, head, at, v0, v1);
+        const WaveEdges<HUBS> E(walk, head, segs, at, v0, v1);
         if (lane < kLevelVerts) s_cnt[w][lane] = 0;
         wave_lds_fence();
         // the wave's children, staged as far as they fit
         int n = 0;
         E.each(adj, [&](int u) { return claim[u]; },
-               [&](int u, int v, int place, bool edge) {
-                   const bool mine = edge && place == at + v0 + v;
+               [&](int u, int v, int parent, bool edge) {
+                   const bool mine = parent == E.parent(v) && edge;
                    const u64 m = __ballot(mine);
                    if (mine) {
                        atomicAdd(&s_cnt[w][v], 1);
@@ -909,21 +1016,28 @@ __global__ __launch_bounds__(64 * kLevelWaves) void k_level_place(
         out += round;
         const int cnt = lane < kLevelVerts ? s_cnt[w][lane] : 0;
         const int first = wave_scan(cnt, OpAdd{}, 0) - cnt;  // lane i < 8: its children's start
+        const bool part = HUBS && E.part >= 0;  // of a vertex that has its job
+        if (part) {
+            int* const job = reinterpret_cast<int*>(jobs + (E.part >> 2));
+            if (E.part & kFirstSegment) job[0] = mine_at + first;
+            if (E.part & kLastSegment) job[1] = mine_at + first + cnt;
+        }
+        const bool sorts = !part && cnt > (n <= kLevelStage ? kBfsSortSmall : 0);
+        if (sorts)
+            jobs[atomicAdd(&counters[kGroups], 1)] =
+                make_int4(mine_at + first, mine_at + first + cnt, 2 * lg_floor(cnt), 0);
         if (n <= kLevelStage) {
-            if (cnt > kBfsSortSmall)
-                jobs[atomicAdd(njobs, 1)] =
-                    make_int4(mine_at + first, mine_at + first + cnt, 2 * lg_floor(cnt), 0);
-            else if (cnt > 1)
+            if (!part && !sorts && cnt > 1)
                 ls_sort_range(s_stage[w], first, first + cnt, 2 * lg_floor(cnt));
             wave_lds_fence();
             for (int p0 = 0; p0 < n; p0 += 64) {
                 const int p = p0 + lane;
-                // the vertex of child p: is its group a job?
+                // the item of child p: is its group a job?
                 int v = 0;
 #pragma unroll
                 for (int step = kLevelVerts / 2; step > 0; step >>= 1)
                     if (__shfl(first, v + step) <= min(p, n - 1)) v += step;
-                const bool job = __shfl(cnt, v) > kBfsSortSmall;
+                const bool job = __shfl((int)(part || sorts), v);
                 if (p < n) {
                     const u64 c = s_stage[w][p];
                     if (job) {
@@ -936,13 +1050,10 @@ __global__ __launch_bounds__(64 * kLevelWaves) void k_level_place(
                 }
             }
         } else {
-            if (cnt > 0)
-                jobs[atomicAdd(njobs, 1)] =
-                    make_int4(mine_at + first, mine_at + first + cnt, 2 * lg_floor(cnt), 0);
             int k = 0;
             E.each(adj, [&](int u) { return claim[u]; },
-                   [&](int u, int v, int place, bool edge) {
-                       const bool mine = edge && place == at + v0 + v;
+                   [&](int u, int v, int parent, bool edge) {
+                       const bool mine = parent == E.parent(v) && edge;
                        const u64 m = __ballot(mine);
                        if (mine)
                            child[mine_at + k + __popcll(m & below)] =
@@ -954,39 +1065,77 @@ __global__ __launch_bounds__(64 * kLevelWaves) void k_level_place(
     }
 }
 
-// Groups of more than kBfsCap children, one work-group each, partitioned in memory (lpos, rpos at
-// the group's own places) down to that size: the pieces join the jobs at jobs[njobs[0] ..], their
-// number in njobs[1].
-__global__ __launch_bounds__(kBfsThreads) void k_level_split(int4* jobs, int* njobs, u64* child,
+// Partition depth of a job or range: the library's for its size where it is not known yet.
+__device__ __forceinline__ int job_depth(const int4& job) {
+    return job.z < 0 ? 2 * lg_floor(max(job.y - job.x, 1)) : job.z;
+}
+
+// A range of a group is done with once it fits k_level_sort, or its depth is used up: a piece, which
+// joins the jobs after the groups.
+__device__ __forceinline__ bool range_done(int lo, int hi, int depth) {
+    return hi - lo <= kBfsCap || depth == 0;
+}
+
+__device__ __forceinline__ void add_piece(int4* jobs, int* counters, int lo, int hi, int depth) {
+    jobs[counters[kGroups] + atomicAdd(&counters[kPieces], 1)] = make_int4(lo, hi, depth, 0);
+}
+
+// Groups of more than kBfsCap children: one partition step of every range, a work-group each, in
+// memory (lpos, rpos at the range's own places).  The ranges of pass 0 are the jobs; what is not done
+// with goes to the next pass.  One work-group from start to end took 9.3 ms for 1 M children of equal
+// degree, parts side by side take 3.
+__global__ __launch_bounds__(kBfsThreads) void k_level_split_pass(
+    const int4* src, int pass, int4* __restrict__ dst, int4* jobs, int* counters, u64* child,
+    int* lpos, int* rpos) {
+    constexpr int NW = kBfsThreads / 64;
+    __shared__ int2 s_part[NW];
+    __shared__ int s_lnext;
+    const int n = pass == 0 ? counters[kGroups] : counters[kRanges + pass - 1];
+    for (int q = blockIdx.x; q < n; q += gridDim.x) {
+        const int4 job = src[q];
+        if (job.y - job.x <= kBfsCap) continue;
+        __syncthreads();
+        const int depth = job_depth(job) - 1;
+        const int cut = partition_step<NW>(child, job.x, job.y, lpos + job.x, rpos + job.x, s_part,
+                                           &s_lnext);
+        if (threadIdx.x < 2) {
+            const int lo = threadIdx.x ? cut : job.x, hi = threadIdx.x ? job.y : cut;
+            if (range_done(lo, hi, depth)) add_piece(jobs, counters, lo, hi, depth);
+            else dst[atomicAdd(&counters[kRanges + pass], 1)] = make_int4(lo, hi, depth, 0);
+        }
+    }
+}
+
+// The ranges that the passes left (parts of unlike sizes), each to its end in one work-group.
+__global__ __launch_bounds__(kBfsThreads) void k_level_split(const int4* __restrict__ src, int passes,
+                                                             int4* jobs, int* counters, u64* child,
                                                              int* lpos, int* rpos) {
     constexpr int NW = kBfsThreads / 64;
     __shared__ int2 s_part[NW];
     __shared__ int s_lnext;
-    const int n = njobs[0];
+    const int n = counters[kRanges + passes - 1];
     for (int q = blockIdx.x; q < n; q += gridDim.x) {
-        const int4 job = jobs[q];
-        if (job.y - job.x <= kBfsCap) continue;
+        const int4 job = src[q];
         __syncthreads();
         partition_range<NW>(child, job.x, job.y, job.z, kBfsCap, lpos + job.x, rpos + job.x,
                             s_part, &s_lnext, [&](int x, int y, int d) {
-                                if (threadIdx.x == 0)
-                                    jobs[n + atomicAdd(&njobs[1], 1)] = make_int4(x, y, d, 0);
+                                if (threadIdx.x == 0) add_piece(jobs, counters, x, y, d);
                             });
     }
 }
 
-// The groups k_level_place left, and the pieces of those k_level_split took: one work-group each,
+// The groups k_level_place left, and the pieces of those that were split: one work-group each,
 // in LDS; a piece beyond it has its depth used up and is heapsorted.
 __global__ __launch_bounds__(kBfsThreads) void k_level_sort(
-    const int4* __restrict__ jobs, const int* __restrict__ njobs, const int4* __restrict__ state,
-    u64* child, int* __restrict__ walk, int* __restrict__ seq) {
+    const int4* __restrict__ jobs, const int* __restrict__ counters,
+    const int4* __restrict__ state, u64* child, int* __restrict__ walk, int* __restrict__ seq) {
     constexpr int NW = kBfsThreads / 64;
     __shared__ u64 s_child[kBfsCap];
     __shared__ int s_lpos[kBfsCap / 2], s_rpos[kBfsCap / 2];
     __shared__ unsigned char s_mark[kBfsCap + 4];
     __shared__ int2 s_part[NW];
     __shared__ int s_lnext[NW];
-    const int t = threadIdx.x, groups = njobs[0], all = groups + njobs[1];
+    const int t = threadIdx.x, groups = counters[kGroups], all = groups + counters[kPieces];
     const int base = state->y;  // vertices placed before this level
     for (int q = blockIdx.x; q < all; q += gridDim.x) {
         const int4 job = jobs[q];
@@ -999,7 +1148,7 @@ __global__ __launch_bounds__(kBfsThreads) void k_level_sort(
                 s_mark[i] = kMarkNone;
             }
             __syncthreads();
-            mark_group<NW>(s_child, 0, n, job.z, s_mark, s_lpos, s_rpos, s_part, s_lnext);
+            mark_group<NW>(s_child, 0, n, job_depth(job), s_mark, s_lpos, s_rpos, s_part, s_lnext);
             __syncthreads();
             wave_pieces<NW>(s_child, n, s_mark, s_lpos, s_rpos, s_lnext);
             finish_pieces(s_child, 0, n, s_mark);
@@ -1315,38 +1464,68 @@ void rcm_order_device(const int* rp, const int* col, int M, int N, int nnz, int*
     // of more than kBfsSortSmall neighbours no group becomes a job (nor do eight fill more than
     // kLevelStage), and none needs splitting without one of more than kBfsCap.
     static_assert(kLevelVerts * kBfsSortSmall <= kLevelStage, "small groups always fit");
+    static_assert(kHubDegree >= kBfsSortSmall, "segments need the jobs");
     const bool sorts = max_degree > kBfsSortSmall, splits = max_degree > kBfsCap;
+    const bool hubs = max_degree > kHubDegree;
     TmpBuf<int4> jobs(sorts ? 2 * (size_t)N : 0);
-    TmpBuf<int> njobs(2), lpos(splits ? N : 0), rpos(splits ? N : 0), children(kLevelBlocks);
+    TmpBuf<int> counters(kCounters), lpos(splits ? N : 0), rpos(splits ? N : 0);
+    TmpBuf<int> children(kLevelBlocks), block_segs(hubs ? kLevelBlocks : 0);
+    // every vertex ends at most one segment that is not full
+    TmpBuf<int4> segs(hubs ? (size_t)N + (size_t)(E / kSegment) : 0);
+    // Passes that halve the largest possible group down to kBfsCap, and one more; ranges above it
+    // number at most N / kBfsCap.
+    const int passes = splits ? std::min(bits_for((u64)(max_degree / kBfsCap)) + 1, kSplitPasses) : 0;
+    TmpBuf<int4> ranges0(splits ? N / kBfsCap + 1 : 0), ranges1(splits ? N / kBfsCap + 1 : 0);
     int4 s = make_int4(roots, roots, 1, 0);
     VCSRMC_HIP(hipMemcpyAsync(state.p, &s, sizeof s, hipMemcpyHostToDevice, st));
     int cur = 0;
+    const dim3 grid(kLevelBlocks), block(64 * kLevelWaves);
+    const auto level = [&](auto with_hubs, const int4* now, int4* next) {
+        constexpr bool HUBS = decltype(with_hubs)::value;
+        if constexpr (HUBS) {
+            hipLaunchKernelGGL(k_level_seg_count, grid, dim3(256), 0, st, walk.p, head.p, now,
+                               max_level, block_segs.p, counters.p);
+            VCSRMC_HIP(hipGetLastError());
+            hipLaunchKernelGGL(k_level_seg_write, grid, dim3(256), 0, st, walk.p, head.p, now,
+                               max_level, block_segs.p, segs.p, jobs.p, counters.p);
+            VCSRMC_HIP(hipGetLastError());
+        }
+        hipLaunchKernelGGL((k_level_claim<HUBS>), grid, block, 0, st, walk.p, head.p, adj.p, segs.p,
+                           seq.p, claim.p, now, max_level, counters.p);
+        VCSRMC_HIP(hipGetLastError());
+        hipLaunchKernelGGL((k_level_count<HUBS>), grid, block, 0, st, walk.p, head.p, adj.p, segs.p,
+                           claim.p, now, max_level, children.p, counters.p);
+        VCSRMC_HIP(hipGetLastError());
+        hipLaunchKernelGGL((k_level_place<HUBS>), grid, block, 0, st, walk.p, head.p, adj.p, segs.p,
+                           seq.p, claim.p, now, next, max_level, children.p, child.p, jobs.p,
+                           counters.p);
+        VCSRMC_HIP(hipGetLastError());
+    };
     for (int batch = 1; s.y < N && !s.w && s.z <= max_level; batch = std::min(2 * batch, 16)) {
         // levels inside one work-group while they are small, then `batch` of any size
         hipLaunchKernelGGL(k_bfs_levels, dim3(1), dim3(kBfsThreads), 0, st, walk.p, head.p, adj.p,
                            seq.p, claim.p, N, max_level, state.p + cur);
         VCSRMC_HIP(hipGetLastError());
         for (int i = 0; i < batch; ++i, cur ^= 1) {
-            const dim3 grid(kLevelBlocks), block(64 * kLevelWaves);
             const int4* now = state.p + cur;
-            hipLaunchKernelGGL(k_level_claim, grid, block, 0, st, walk.p, head.p, adj.p, seq.p,
-                               claim.p, now, max_level, njobs.p);
-            VCSRMC_HIP(hipGetLastError());
-            hipLaunchKernelGGL(k_level_count, grid, block, 0, st, walk.p, head.p, adj.p, claim.p,
-                               now, max_level, children.p);
-            VCSRMC_HIP(hipGetLastError());
-            hipLaunchKernelGGL(k_level_place, grid, block, 0, st, walk.p, head.p, adj.p, seq.p,
-                               claim.p, now, state.p + (cur ^ 1), max_level, children.p, child.p,
-                               jobs.p, njobs.p);
-            VCSRMC_HIP(hipGetLastError());
+            if (hubs) level(std::true_type{}, now, state.p + (cur ^ 1));
+            else level(std::false_type{}, now, state.p + (cur ^ 1));
+            const int4* src = jobs.p;
+            for (int pass = 0; pass < passes; ++pass) {
+                int4* dst = pass % 2 ? ranges1.p : ranges0.p;
+                hipLaunchKernelGGL(k_level_split_pass, dim3(256), dim3(kBfsThreads), 0, st, src, pass,
+                                   dst, jobs.p, counters.p, child.p, lpos.p, rpos.p);
+                VCSRMC_HIP(hipGetLastError());
+                src = dst;
+            }
             if (splits) {
-                hipLaunchKernelGGL(k_level_split, dim3(256), dim3(kBfsThreads), 0, st, jobs.p,
-                                   njobs.p, child.p, lpos.p, rpos.p);
+                hipLaunchKernelGGL(k_level_split, dim3(256), dim3(kBfsThreads), 0, st, src, passes,
+                                   jobs.p, counters.p, child.p, lpos.p, rpos.p);
                 VCSRMC_HIP(hipGetLastError());
             }
             if (sorts) {
                 hipLaunchKernelGGL(k_level_sort, dim3(256), dim3(kBfsThreads), 0, st, jobs.p,
-                                   njobs.p, now, child.p, walk.p, seq.p);
+                                   counters.p, now, child.p, walk.p, seq.p);
                 VCSRMC_HIP(hipGetLastError());
             }
         }
