@@ -491,10 +491,24 @@ __global__ void k_big_store(Positions pos, const int* __restrict__ big,
         sval[out] = entry_value<FP32>(val[bsrc[i]] * inv_scale, r);
         if constexpr (FP32) srow[out] = (unsigned char)r;
     }
-    // one addition per wave where it holds one panel's elements
+    // One addition a work-group where it holds one panel's elements, else one a wave that does (8 M
+    // nonzeros in one panel, an addition a wave: 1.4 ms).
+    __shared__ int s_q, s_heads, s_mixed;
+    if (threadIdx.x == 0) {
+        s_q = q;
+        s_heads = s_mixed = 0;
+    }
+    __syncthreads();
+    const int heads = __popcll(__ballot(head));
+    if (i < total && q != s_q) s_mixed = 1;
+    if ((threadIdx.x & 63) == 0) atomicAdd(&s_heads, heads);
+    __syncthreads();
+    if (!s_mixed) {
+        if (threadIdx.x == 0 && s_heads) atomicAdd(&ndist[big[q]], s_heads);
+        return;
+    }
     const int q0 = __builtin_amdgcn_readfirstlane(q);
     if (__ballot(q != q0) == 0) {
-        const int heads = __popcll(__ballot(head));
         if (q0 >= 0 && (threadIdx.x & 63) == 0) atomicAdd(&ndist[big[q0]], heads);
     } else if (head) {
         atomicAdd(&ndist[big[q]], 1);
@@ -580,8 +594,39 @@ __global__ void k_panel_compact(Positions pos, const int* __restrict__ nch,
     pmask[i] = pmask_all[j];
 }
 
+// One sorted nonzero, the lr-th distinct column of its panel (whose tiles start at c0): its entry,
+// and, where it is the column's first (head), the column in its tile.
+template <bool FP32>
+__device__ __forceinline__ void fill_entry(long long i, int c0, int lr, bool head, uint32_t col,
+                                           uint32_t val, const unsigned char* __restrict__ srow,
+                                           uint32_t* __restrict__ entries,
+                                           int* __restrict__ chunk_cols,
+                                           int* __restrict__ chunk_eptr) {
+    const int tile = c0 + lr / kChunkCols, k = lr % kChunkCols;
+    if constexpr (FP32) {
+        *reinterpret_cast<uint2*>(entries + 2 * i) =
+            make_uint2((uint32_t)srow[i] | ((uint32_t)k << 4), val);
+    } else {
+        entries[i] = val | ((uint32_t)k << 20);
+    }
+    if (head) {
+        // FP32 formats keep a tile's columns in K-step order: lane group g of the kernel
+        // reads columns 4 s + g (s = 0..7) as eight consecutive words.
+        const int slot = FP32 ? (k & 3) * 8 + (k >> 2) : k;
+        chunk_cols[(long long)tile * kChunkCols + slot] = (int)col;
+        if (k == 0) chunk_eptr[tile] = (int)i;
+    }
+}
+
+// The unused column k of a panel's last tile.
+template <bool FP32>
+__device__ __forceinline__ void fill_pad(long long tile, int k, int* __restrict__ chunk_cols) {
+    chunk_cols[tile * kChunkCols + (FP32 ? (k & 3) * 8 + (k >> 2) : k)] = kPadSlot;
+}
+
 // Tiles of one panel per work-group, from its sorted nonzeros: the running number of distinct
-// columns gives each nonzero its tile and column in it.
+// columns gives each nonzero its tile and column in it.  Panels above kSortMid nonzeros take
+// k_big_fill.
 template <bool FP32>
 __global__ __launch_bounds__(256) void k_panel_fill(
     const int* __restrict__ pstart, const int* __restrict__ cbase, int NP,
@@ -593,6 +638,7 @@ __global__ __launch_bounds__(256) void k_panel_fill(
     if (j >= NP) return;  // the whole work-group
     const int t = threadIdx.x, w = t >> 6, lane = t & 63;
     const int p0 = pstart[j], p1 = pstart[j + 1], c0 = cbase[j];
+    if (p1 - p0 > kSortMid) return;
     const uint64_t upto = ~0ull >> (63 - lane);
     int run = 0, phase = 0;  // distinct columns before this round's nonzeros
     for (int i0 = p0; i0 < p1; i0 += 256, phase ^= 1) {
@@ -614,29 +660,44 @@ __global__ __launch_bounds__(256) void k_panel_fill(
             all += h;
         }
         run += all;
-        if (i < p1) {
-            const int lr = before + __popcll(m & upto) - 1;
-            const int tile = c0 + lr / kChunkCols, k = lr % kChunkCols;
-            if constexpr (FP32) {
-                *reinterpret_cast<uint2*>(entries + 2 * (long long)i) =
-                    make_uint2((uint32_t)srow[i] | ((uint32_t)k << 4), sval[i]);
-            } else {
-                entries[i] = sval[i] | ((uint32_t)k << 20);
-            }
-            if (head) {
-                // FP32 formats keep a tile's columns in K-step order: lane group g of the kernel
-                // reads columns 4 s + g (s = 0..7) as eight consecutive words.
-                const int slot = FP32 ? (k & 3) * 8 + (k >> 2) : k;
-                chunk_cols[(long long)tile * kChunkCols + slot] = (int)c;
-                if (k == 0) chunk_eptr[tile] = i;
-            }
-        }
+        if (i < p1)
+            fill_entry<FP32>(i, c0, before + __popcll(m & upto) - 1, head, c, sval[i], srow,
+                             entries, chunk_cols, chunk_eptr);
     }
-    // the last tile's unused columns
-    if (run % kChunkCols != 0 && t >= run % kChunkCols && t < kChunkCols) {
-        const int slot = FP32 ? (t & 3) * 8 + (t >> 2) : t;
-        chunk_cols[(long long)(c0 + run / kChunkCols) * kChunkCols + slot] = kPadSlot;
-    }
+    if (run % kChunkCols != 0 && t >= run % kChunkCols && t < kChunkCols)
+        fill_pad<FP32>(c0 + run / kChunkCols, t, chunk_cols);
+}
+
+// The same for large panels, a thread an element: the running number of distinct columns is a scan
+// of `head` over their elements laid one after another.  One work-group a panel took 5 ns a nonzero
+// (16 rows of 2 M columns each, one panel: the build 152 ms, now 8.2).
+__global__ void k_big_heads(Positions pos, const int* __restrict__ big,
+                            const int* __restrict__ bofs, int nbig, long long total,
+                            const uint32_t* __restrict__ scol, int* __restrict__ head) {
+    const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= total) return;
+    const int q = big_of(bofs, nbig, e);
+    const long long i = (long long)pos.begin(big[q] * kPanelRows) + (e - bofs[q]);
+    head[e] = e == bofs[q] || scol[i - 1] != scol[i];
+}
+
+template <bool FP32>
+__global__ void k_big_fill(Positions pos, const int* __restrict__ big, const int* __restrict__ bofs,
+                           int nbig, long long total, const int* __restrict__ cbase_all,
+                           const int* __restrict__ head, const int* __restrict__ distinct,
+                           const uint32_t* __restrict__ scol, const uint32_t* __restrict__ sval,
+                           const unsigned char* __restrict__ srow, uint32_t* __restrict__ entries,
+                           int* __restrict__ chunk_cols, int* __restrict__ chunk_eptr) {
+    const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= total) return;
+    const int q = big_of(bofs, nbig, e), panel = big[q];
+    const long long i = (long long)pos.begin(panel * kPanelRows) + (e - bofs[q]);
+    const int lr = distinct[e] - distinct[bofs[q]], c0 = cbase_all[panel];
+    fill_entry<FP32>(i, c0, lr, head[e] != 0, scol[i], sval[i], srow, entries, chunk_cols,
+                     chunk_eptr);
+    if (e + 1 == bofs[q + 1] && (lr + 1) % kChunkCols != 0)  // the panel's last
+        for (int k = (lr + 1) % kChunkCols; k < kChunkCols; ++k)
+            fill_pad<FP32>(c0 + lr / kChunkCols, k, chunk_cols);
 }
 
 __global__ void k_dense_flags(const int* __restrict__ eptr, int NC, int dmin,
@@ -936,6 +997,10 @@ struct PanelSet {
     const int* row_map = nullptr;
     TmpBuf<int> at, pmask, ndist;
     int pairs = 0, NC = 0, NP = 0, max_tiles = 0;
+    // Panels above kSortMid nonzeros, and where each starts in their elements laid one after another.
+    TmpBuf<int> big, bofs;
+    int nbig = 0;
+    long long big_total = 0;
     Positions positions(const int* rp, int M) const { return Positions{rp, row_map, at.p, M}; }
 };
 
@@ -956,11 +1021,12 @@ static PanelSet sort_panels(int M, const int* rp, const int* row_map, const int*
     const Positions pos = P.positions(rp, M);
     P.pmask.alloc(P.panels);
     P.ndist.alloc(P.panels);
-    TmpBuf<int> mid(P.panels), big(P.panels), bsize(P.panels);
+    P.big.alloc(P.panels);
+    TmpBuf<int> mid(P.panels), bsize(P.panels);
     TmpBuf<int> counts(6);  // {middle, large panels}, the totals
     fill<int>(counts.p, 6, 0, st);
-    LAUNCH(k_panel_classes, P.panels, pos, P.panels, P.pmask.p, P.ndist.p, mid.p, big.p, bsize.p,
-           counts.p);
+    LAUNCH(k_panel_classes, P.panels, pos, P.panels, P.pmask.p, P.ndist.p, mid.p, P.big.p,
+           bsize.p, counts.p);
     // One work-group a panel; more panels than nonzeros are mostly empty, and the others are listed
     // first (200 M rows, 1 M nonzeros: 12.5 M work-groups took 9.4 ms, the list and its own 0.9).
     int small = P.panels;
@@ -986,22 +1052,25 @@ static PanelSet sort_panels(int M, const int* rp, const int* row_map, const int*
                            S.val.p, S.row.p, P.ndist.p);
         VCSRMC_HIP(hipGetLastError());
     }
-    if (nsort[1] > 0) {
-        const int nbig = nsort[1];
-        TmpBuf<int> bofs((size_t)nbig + 1);
-        exclusive_sum<int, int>(bsize.p, bofs.p, nbig, st);
-        const long long total = read_scalar(bofs.p + nbig, st);
+    P.nbig = nsort[1];
+    if (P.nbig > 0) {
+        const int nbig = P.nbig;
+        const int* big = P.big.p;
+        P.bofs.alloc((size_t)nbig + 1);
+        const int* bofs = P.bofs.p;
+        exclusive_sum<int, int>(bsize.p, P.bofs.p, nbig, st);
+        const long long total = P.big_total = read_scalar(bofs + nbig, st);
         TmpBuf<uint32_t> c0(total), c1(total), s0(total), s1(total);
         TmpBuf<unsigned char> r0(total), r1(total);
-        LAUNCH(k_big_load, total, pos, big.p, bofs.p, nbig, total, col, c0.p, s0.p, r0.p);
+        LAUNCH(k_big_load, total, pos, big, bofs, nbig, total, col, c0.p, s0.p, r0.p);
         for (int s = 0; s < 4; ++s) {
-            LAUNCH(k_big_merge, total, pos, big.p, bofs.p, nbig, total, s, c0.p, s0.p, r0.p, c1.p,
+            LAUNCH(k_big_merge, total, pos, big, bofs, nbig, total, s, c0.p, s0.p, r0.p, c1.p,
                    s1.p, r1.p);
             std::swap(c0, c1);
             std::swap(s0, s1);
             std::swap(r0, r1);
         }
-        LAUNCH((k_big_store<FP32>), total, pos, big.p, bofs.p, nbig, total, c0.p, s0.p, r0.p, val,
+        LAUNCH((k_big_store<FP32>), total, pos, big, bofs, nbig, total, c0.p, s0.p, r0.p, val,
                inv_scale, S.col.p, S.val.p, S.row.p, P.ndist.p);
     }
     hipLaunchKernelGGL(k_panel_totals, dim3(grid_for(P.panels, 256 * kTotalsPerThread)), dim3(256),
@@ -1027,9 +1096,9 @@ static void fill_layout(DeviceFormat& F, const PanelSet& S, const SortedNonzeros
     F.chunk_cols.alloc((size_t)NC * kChunkCols);
     F.entries.alloc(F.fp32 ? 2 * n : n);
     TmpBuf<int> pstart((size_t)NP + 1), ppanel(NP), nch(NP), cbase((size_t)NP + 1), pmask(NP);
+    TmpBuf<int> cbase_all((size_t)S.panels + 1);
     {
-        TmpBuf<int> all(S.panels), some(S.panels), cbase_all((size_t)S.panels + 1),
-            pidx((size_t)S.panels + 1);
+        TmpBuf<int> all(S.panels), some(S.panels), pidx((size_t)S.panels + 1);
         LAUNCH(k_panel_tiles, S.panels, S.ndist.p, S.panels, all.p, some.p);
         exclusive_sum<int, int>(all.p, cbase_all.p, S.panels, st);
         exclusive_sum<int, int>(some.p, pidx.p, S.panels, st);
@@ -1037,15 +1106,25 @@ static void fill_layout(DeviceFormat& F, const PanelSet& S, const SortedNonzeros
                S.pmask.p, S.panels, NP, NC, (int)n, ppanel.p, pstart.p, cbase.p, nch.p, pmask.p,
                F.chunk_eptr.p);
     }
-    if (F.fp32)
-        hipLaunchKernelGGL((k_panel_fill<true>), grid_of(NP), dim3(256), 0, st, pstart.p, cbase.p,
-                           NP, nz.col.p, nz.val.p, nz.row.p, F.entries.p, F.chunk_cols.p,
+    const auto fill_tiles = [&](auto fp32) {
+        constexpr bool FP32 = decltype(fp32)::value;
+        hipLaunchKernelGGL((k_panel_fill<FP32>), grid_of(NP), dim3(256), 0, st, pstart.p, cbase.p, NP,
+                           nz.col.p, nz.val.p, nz.row.p, F.entries.p, F.chunk_cols.p,
                            F.chunk_eptr.p);
-    else
-        hipLaunchKernelGGL((k_panel_fill<false>), grid_of(NP), dim3(256), 0, st, pstart.p, cbase.p,
-                           NP, nz.col.p, nz.val.p, nz.row.p, F.entries.p, F.chunk_cols.p,
-                           F.chunk_eptr.p);
-    VCSRMC_HIP(hipGetLastError());
+        VCSRMC_HIP(hipGetLastError());
+        if (S.nbig == 0) return;
+        const Positions pos = S.positions(rp, F.M);
+        TmpBuf<int> head(S.big_total), distinct(S.big_total);
+        LAUNCH(k_big_heads, S.big_total, pos, S.big.p, S.bofs.p, S.nbig, S.big_total, nz.col.p,
+               head.p);
+        inclusive_sum<int, int>(head.p, distinct.p, S.big_total, st);
+        LAUNCH((k_big_fill<FP32>), S.big_total, pos, S.big.p, S.bofs.p, S.nbig, S.big_total,
+               cbase_all.p, head.p, distinct.p, nz.col.p, nz.val.p, nz.row.p, F.entries.p,
+               F.chunk_cols.p, F.chunk_eptr.p);
+    };
+    if (F.fp32) fill_tiles(std::true_type{});
+    else fill_tiles(std::false_type{});
+    cbase_all.release();
 
     // dense copies of well-filled tiles
     {
