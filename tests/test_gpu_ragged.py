@@ -116,3 +116,39 @@ def test_operands_around_the_32_bit_reach(fp32, O, more):
     err = (C.double() - want).abs().sum(1)
     assert bool((err <= (40 * 2.0 ** -24 if fp32 else 2e-3) * bound + 1e-30).all()), \
         float((err / bound).max())
+
+
+@pytest.mark.parametrize("add", [True, False])
+@pytest.mark.parametrize("empty", [0.0, 0.5])
+@pytest.mark.parametrize("fp32,half_b", [(True, False), (False, True), (False, False)])
+def test_operand_beyond_the_last_level_cache(fp32, half_b, empty, add):
+    """B above 256 MB in tiles of few nonzeros, in natural order and with the empty rows moved last.
+    Bound as in test_row_numbers_around_24_bits."""
+    import torch
+    rng = np.random.default_rng(11)
+    M, O = 1500, 128
+    N = (270 << 20) // (O * (2 if half_b else 4))
+    lens = np.where(rng.random(M) < empty, 0, rng.integers(1, 38, M))
+    cols = [np.unique(rng.integers(0, N, k)) for k in lens]
+    rp = np.zeros(M + 1, np.int32)
+    rp[1:] = np.cumsum([len(x) for x in cols])
+    c = np.concatenate(cols).astype(np.int32)
+    v = rng.uniform(-1, 1, c.size).astype(np.float32)
+    say("far operand", fp32, half_b, empty, add)
+    B = torch.empty((N, O), device="cuda", dtype=torch.float16 if half_b else torch.float32)
+    B.uniform_(-0.5, 0.5)
+    C0 = torch.rand((M, O), device="cuda")
+    row = torch.repeat_interleave(torch.arange(M, device="cuda"), dev(np.diff(rp)).long())
+    P = dev(v).double()[:, None] * B[dev(c).long()].double()
+    sums = torch.zeros((M, O), device="cuda", dtype=torch.float64).index_add_(0, row, P)
+    used = dev(np.diff(rp) > 0)[:, None]
+    want = C0.double() + sums if add else torch.where(used, sums, C0.double())
+    bound = torch.zeros_like(want).index_add_(0, row, P.abs()).sum(1) + C0.double().sum(1) * add
+    with vm.DeviceFormat.from_device_csr(dev(rp), dev(c), dev(v), M, N, fp32, 32) as f:
+        assert (f.row_map() is not None) == (empty > 0) and c.size < 48 * f.info()["num_chunks"]
+        C = C0.clone()
+        f.spmm(B, C, overwrite=not add)
+        torch.cuda.synchronize()
+    err = (C.double() - want).abs().sum(1)
+    assert bool((err <= (40 * 2.0 ** -24 if fp32 else 2e-3) * bound + 1e-30).all()), \
+        float((err / bound).max())

@@ -153,13 +153,15 @@ __device__ __forceinline__ auto load_b_row(const TB* __restrict__ B, int slot, l
     }
 }
 
-// A pause of 16 cycles after each load of a B row (FAR), in the launches that read C non-temporally:
-// those that accumulate, are aligned, and whose B and C together exceed the last-level cache.  A wave
-// that issues its eight rows back to back ends up slower where they come from beyond that cache.
-// With the pause / without, us: R-MAT scale 22 FP16 2430 / 2491, scale 20 FP16 O = 256 946 / 953,
-// scale 19 FP32 O = 256 817 / 822, stencil 100^3 401 / 403, blocks FP32 250.7 / 250.5, FP16 160.6 /
-// 159.9 (64 cycles, scale 20: 472 -> 496).  Launches of those sizes that overwrite C, or are ragged,
-// go without.
+// A pause of 16 cycles after each load of a B row (FAR): a wave that issues its eight rows back to
+// back ends up slower where they come from beyond the last-level cache.  Taken by aligned launches
+// that accumulate with B and C together above that cache (the ones that read C non-temporally), or
+// overwrite with sparse tiles and B alone above it.  With the pause / without, us: accumulating,
+// R-MAT scale 22 FP16 2430 / 2491, scale 20 FP16 O = 256 946 / 953, scale 19 FP32 O = 256 817 / 822,
+// stencil 100^3 401 / 403, blocks FP32 250.7 / 250.5, FP16 160.6 / 159.9 (64 cycles, scale 20: 472 ->
+// 496); overwriting, scale 22 FP16 2403 / 2457, FP32 5153 / 5188, scale 20 862 / 863, scale 19 FP32
+// 779 / 782, uniform 600,000^2 with 8 per row O = 256 450 / 449; kept without, blocks FP16 131 / 127,
+// power-law 10^6 (B 244 MB) 388 / 384.
 __device__ __forceinline__ void space_loads() {
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("s_nop 15");
@@ -599,7 +601,7 @@ __global__ __launch_bounds__(64 * kWaves, (f16_min_waves<TB>())) void k_spmm_f16
     // counting sees one fixed sequence of loads on each.
     if (heavy) {
         CAhead<TK, kWaves> ca;
-        read_c_ahead<TK, kWaves, NTC>(ca, U, pr, k0, O, ACC, C);
+        read_c_ahead<TK, kWaves, NTC && ACC>(ca, U, pr, k0, O, ACC, C);
         tiles_f16<TK, TB, ALIGNED, WIDE, NTC>(U.y + wave, U.z, kWaves, lane, n, g, cb, ldb,
                                    chunk_eptr, chunk_cols, chunk_dense, entries, dense_a, Bt,
                                    As[wave], acc, [] {});
@@ -608,7 +610,7 @@ __global__ __launch_bounds__(64 * kWaves, (f16_min_waves<TB>())) void k_spmm_f16
         CAhead<TK, 1> ca;
         tiles_f16<TK, TB, ALIGNED, WIDE, NTC>(U.y, U.z, 1, lane, n, g, cb, ldb, chunk_eptr,
                                    chunk_cols, chunk_dense, entries, dense_a, Bt, As[wave], acc,
-                                   [&] { read_c_ahead<TK, 1, NTC>(ca, U, pr, k0, O, ACC, C); });
+                                   [&] { read_c_ahead<TK, 1, NTC && ACC>(ca, U, pr, k0, O, ACC, C); });
         merge_into_c<TK, 1, ALIGNED, ACC>(acc, scale, U, pr, k0, O, C, P, ca);
     }
 }
@@ -898,12 +900,12 @@ __global__ __launch_bounds__(64 * kWaves, 3) void k_spmm_f32(
     };
     if (heavy) {
         CAhead<TK, kWaves> ca;
-        read_c_ahead<TK, kWaves, NTC>(ca, U, pr, k0, O, ACC, C);
+        read_c_ahead<TK, kWaves, NTC && ACC>(ca, U, pr, k0, O, ACC, C);
         run(U.y + wave, kWaves, [] {});
         merge_into_c<TK, kWaves, ALIGNED, ACC>(acc, 1.0f, U, pr, k0, O, C, P, ca);
     } else {
         CAhead<TK, 1> ca;
-        run(U.y, 1, [&] { read_c_ahead<TK, 1, NTC>(ca, U, pr, k0, O, ACC, C); });
+        run(U.y, 1, [&] { read_c_ahead<TK, 1, NTC && ACC>(ca, U, pr, k0, O, ACC, C); });
         merge_into_c<TK, 1, ALIGNED, ACC>(acc, 1.0f, U, pr, k0, O, C, P, ca);
     }
 }
@@ -916,7 +918,8 @@ static bool fits_32(const DeviceFormat& F, bool b_f16, int O) {
 }
 
 // NTC: C read ahead with non-temporal loads (accumulating launches whose C and B exceed the
-// last-level cache, see load_c4); only the aligned variants take it.
+// last-level cache, see load_c4) and B rows loaded with pauses between them (those, and overwriting
+// launches with a far B, see space_loads); only the aligned variants take it.
 template <int TK, bool ACC, bool MAPPED, bool NTC, bool WIDE>
 static void launch_tk_mode(const DeviceFormat& F, const void* dB, bool b_f16, bool b_tiled, int O,
                            float* dC, hipStream_t st) {
@@ -992,14 +995,17 @@ static void launch_tk_mode(const DeviceFormat& F, const void* dB, bool b_f16, bo
 
 template <int TK, bool WIDE>
 static void launch_tk_wide(const DeviceFormat& F, const void* dB, bool b_f16, bool b_tiled, int O,
-                           float* dC, bool accumulate, bool nt_c, hipStream_t st) {
+                           float* dC, bool accumulate, bool far, hipStream_t st) {
     const bool mapped = F.row_map.n > 0;
-    if (accumulate && nt_c) {
+    if (accumulate && far) {
         if (mapped) launch_tk_mode<TK, true, true, true, WIDE>(F, dB, b_f16, b_tiled, O, dC, st);
         else launch_tk_mode<TK, true, false, true, WIDE>(F, dB, b_f16, b_tiled, O, dC, st);
     } else if (accumulate) {
         if (mapped) launch_tk_mode<TK, true, true, false, WIDE>(F, dB, b_f16, b_tiled, O, dC, st);
         else launch_tk_mode<TK, true, false, false, WIDE>(F, dB, b_f16, b_tiled, O, dC, st);
+    } else if (far) {
+        if (mapped) launch_tk_mode<TK, false, true, true, WIDE>(F, dB, b_f16, b_tiled, O, dC, st);
+        else launch_tk_mode<TK, false, false, true, WIDE>(F, dB, b_f16, b_tiled, O, dC, st);
     } else {
         if (mapped) launch_tk_mode<TK, false, true, false, WIDE>(F, dB, b_f16, b_tiled, O, dC, st);
         else launch_tk_mode<TK, false, false, false, WIDE>(F, dB, b_f16, b_tiled, O, dC, st);
@@ -1008,11 +1014,11 @@ static void launch_tk_wide(const DeviceFormat& F, const void* dB, bool b_f16, bo
 
 template <int TK>
 static void launch_tk(const DeviceFormat& F, const void* dB, bool b_f16, bool b_tiled, int O,
-                      float* dC, bool accumulate, bool nt_c, hipStream_t st) {
+                      float* dC, bool accumulate, bool far, hipStream_t st) {
     if (fits_32(F, b_f16, O))
-        launch_tk_wide<TK, false>(F, dB, b_f16, b_tiled, O, dC, accumulate, nt_c, st);
+        launch_tk_wide<TK, false>(F, dB, b_f16, b_tiled, O, dC, accumulate, far, st);
     else
-        launch_tk_wide<TK, true>(F, dB, b_f16, b_tiled, O, dC, accumulate, nt_c, st);
+        launch_tk_wide<TK, true>(F, dB, b_f16, b_tiled, O, dC, accumulate, far, st);
 }
 
 // Before an overwriting launch (C = A.B), the rows of every split panel are set to zero: their
@@ -1168,10 +1174,12 @@ SpmmPlan plan_spmm(const DeviceFormat& F, const void* dB, bool b_f16, int O, int
     // half of 256-byte rows, which reach only half of an L2's sets (R-MAT scale 22, O tiles of
     // 64: 2.44 -> 2.29 ms; O tiles of 32: 4.78 -> 3.96 ms).  Same values either way.
     p.b_tiled = p.convert_to != nullptr && O > p.tk && O % p.tk == 0;
-    // C read non-temporally where C and B together exceed the 256 MB last-level cache (load_c4)
-    const long long c_bytes = (long long)F.M * O * 4;
+    // beyond the 256 MB last-level cache: C and B together (load_c4, space_loads), or, overwriting, B
+    // alone, in tiles of few nonzeros (space_loads)
+    const long long c_bytes = (long long)F.M * O * 4, far_bytes = 256LL << 20;
     const long long b_bytes = (long long)F.N * O * (p.b_f16 ? 2 : 4);
-    p.nt_c = accumulate && c_bytes + b_bytes > (256LL << 20);
+    p.far = accumulate ? c_bytes + b_bytes > far_bytes
+                       : b_bytes > far_bytes && F.nnz < (long long)kSparseTileNnz * F.num_chunks;
     p.launch = true;
     return p;
 }
@@ -1193,10 +1201,10 @@ void run_spmm(const SpmmPlan& p, hipStream_t st) {
         VCSRMC_HIP(hipGetLastError());
     }
     switch (p.tk) {
-        case 16: launch_tk<16>(F, dB, p.b_f16, p.b_tiled, p.O, p.dC, p.accumulate, p.nt_c, st); break;
-        case 32: launch_tk<32>(F, dB, p.b_f16, p.b_tiled, p.O, p.dC, p.accumulate, p.nt_c, st); break;
-        case 64: launch_tk<64>(F, dB, p.b_f16, p.b_tiled, p.O, p.dC, p.accumulate, p.nt_c, st); break;
-        default: launch_tk<128>(F, dB, p.b_f16, p.b_tiled, p.O, p.dC, p.accumulate, p.nt_c, st); break;
+        case 16: launch_tk<16>(F, dB, p.b_f16, p.b_tiled, p.O, p.dC, p.accumulate, p.far, st); break;
+        case 32: launch_tk<32>(F, dB, p.b_f16, p.b_tiled, p.O, p.dC, p.accumulate, p.far, st); break;
+        case 64: launch_tk<64>(F, dB, p.b_f16, p.b_tiled, p.O, p.dC, p.accumulate, p.far, st); break;
+        default: launch_tk<128>(F, dB, p.b_f16, p.b_tiled, p.O, p.dC, p.accumulate, p.far, st); break;
     }
 }
 
